@@ -16,25 +16,20 @@ namespace gdtp {
     if (e_ != hipSuccess) throw std::runtime_error(std::string(#call) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
-// Exact triangular solves of an LDL^T factor, split into independent elimination-subtree
-// teams (one workgroup each) and a top part solved by a single workgroup.
+// Exact triangular solves of an LDL^T factor on the device: the staged form (LdltStages).
 struct DevLdlt {
-  int n = 0;
-  int *perm = nullptr;
-  int *lrRowptr = nullptr, *lrCol = nullptr, *lcRowptr = nullptr, *lcCol = nullptr;
-  double *lrVal = nullptr, *lcVal = nullptr, *dinv = nullptr;
-  // teams: team t owns forward levels [teamLevPtr[t], teamLevPtr[t+1]) of levRowPtr -> levRows
-  int nTeams = 0;
-  int *teamFwdLev = nullptr, *teamBwdLev = nullptr;  // nTeams+1 each, indices into the level tables
-  int *fwdLevPtr = nullptr, *fwdRows = nullptr, *bwdLevPtr = nullptr, *bwdRows = nullptr;
-  int topFwdLevBegin = 0, topFwdLevEnd = 0, topBwdLevBegin = 0, topBwdLevEnd = 0;
-  int maxTeamRows = 0;
-  // dense top (when the top has at most kDenseTopMax rows): the top rows (permuted indices), their
-  // coupling to team rows (CSR over the top rows), the inverse of the unit-lower top block and its
-  // transpose (row-major s x s), and a [kcap][s] scratch vector
-  int nTop = 0, kcap = 0;
-  int *topRows = nullptr, *topCplRowptr = nullptr, *topCplCol = nullptr;
-  double *topCplVal = nullptr, *topInv = nullptr, *topInvT = nullptr, *topBuf = nullptr;
+  int n = 0, wideBegin = 0;
+  std::vector<LdltStage> stages;
+  int* perm = nullptr;
+  double* dinv = nullptr;
+  int* compPtr = nullptr;
+  int *fwdPtr = nullptr, *fwdCol = nullptr, *bwdPtr = nullptr, *bwdCol = nullptr;
+  double *fwdVal = nullptr, *bwdVal = nullptr;
+  long *fwdMatPtr = nullptr, *bwdMatPtr = nullptr;
+  double *fwdMat = nullptr, *bwdMat = nullptr;
+  int* rowComp = nullptr;      // component of each row of the wide stages (row - wideBegin)
+  double* wideBuf = nullptr;   // [2][kcap][n - wideBegin]: right-hand sides of the wide products
+  int kcap = 0;
 };
 
 struct DevCsr {
@@ -75,8 +70,8 @@ struct DeviceSystem {
   ~DeviceSystem();
 };
 
-// Upload an LDL^T factor with its team / top level schedule; LdltSolve solves for K columns,
-// gathering src[perm] and scattering into dst (through `map` when not null).
+// Upload an LDL^T factor's staged triangular solves; LdltSolve solves for K columns (at most kcap),
+// gathering src[perm] and scattering into dst (through `map` when not null; dst may be src).  y: [K][n] scratch.
 void UploadLdlt(std::vector<void*>& allocations, const Ldlt& F, DevLdlt& d, int kcap);
 // Bytes uploaded / allocated by this thread's device uploads so far (monotone counter).
 size_t UploadByteCounter();

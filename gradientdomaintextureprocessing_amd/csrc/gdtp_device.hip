@@ -2,6 +2,7 @@
 //
 // Vectors are column-major: column c of a level-l vector starts at c*ld.  Deep stencils are
 // stored structure-of-arrays, [10][D], so every stencil slot is a coalesced stream.
+#include <algorithm>
 #include <stdexcept>
 
 #include "gdtp_device.h"
@@ -11,7 +12,6 @@
 namespace gdtp {
 
 static constexpr int kWave = 64;
-static constexpr int kDenseTopMax = 4096;  // largest LDL^T top solved through a dense inverse
 
 // ------------------------------------------------------------------ band Gauss-Seidel
 // The reference smoother (IterativeSolvers.inl:398-558 with residual, :174-395 without):
@@ -263,63 +263,155 @@ __global__ void KBoundaryResidual(int B, const int* __restrict__ bgi, const int*
 }
 
 // ------------------------------------------------------------------ exact LDL^T solves
-__global__ void KLdltGather(int n, const int* __restrict__ perm, const double* __restrict__ src, int lds, double* y, int K) {
-  long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)n * K) return;
-  int k = idx % n, c = idx / n;
-  y[(size_t)c * n + k] = src[(size_t)c * lds + perm[k]];
+// The staged triangular solves (LdltStages): forward stages r = src[perm] - L y(earlier stages),
+// y = inv(L_cc) r per component, then backward r = y / D - L^T x(later stages), x = inv(L_cc)^T r.
+//
+// What bounds them: a dependency chain.  The level-scheduled solve they replace walked the elimination
+// tree's 250-450 levels (subtree teams of one workgroup, a barrier per level, one thread per row), each
+// level a round trip to memory: 1.75 ms for the 175,580 boundary rows of a 4096^2 atlas and three
+// columns, 0.25 ms for 3840 rows.  Explicit inverses of components of up to 128 (first stage) or a few
+// hundred rows leave two passes per stage, each a gather and a product with loads that wait for
+// nothing; the inverses are 2-4 times the factor's bytes.
+
+// Lanes' sum over groups of G lanes.
+template <int G>
+__device__ __forceinline__ double GroupSum(double v) {
+#pragma unroll
+  for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, G);
+  return v;
 }
 
-__global__ void KLdltScatter(int n, const int* __restrict__ perm, const int* __restrict__ map, const double* __restrict__ y, double* dst,
-                             int ldd, int K) {
-  long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)n * K) return;
-  int k = idx % n, c = idx / n;
-  int t = perm[k];
-  if (map) t = map[t];
-  dst[(size_t)c * ldd + t] = y[(size_t)c * n + k];
+// One row's coupling sums with the stages solved before, by a group of G lanes, for up to KC columns.
+template <int G, int KC>
+__device__ __forceinline__ void CouplingSums(const int* __restrict__ col, const double* __restrict__ val, int p0, int p1, int lane,
+                                             const double* y, int n, int kc, double (&s)[KC]) {
+#pragma unroll
+  for (int c = 0; c < KC; c++) s[c] = 0.0;
+  for (int p = p0 + lane; p < p1; p += G) {
+    const double v = val[p];
+    const int j = col[p];
+#pragma unroll
+    for (int c = 0; c < KC; c++)
+      if (c < kc) s[c] += v * y[(size_t)c * n + j];
+  }
+#pragma unroll
+  for (int c = 0; c < KC; c++) s[c] = GroupSum<G>(s[c]);
 }
 
-__global__ void KLdltDiag(int n, const double* __restrict__ dinv, double* y, int K) {
-  long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)n * K) return;
-  y[idx] *= dinv[idx % n];
-}
+// The 16 waves of a narrow component's workgroup are divided over its row blocks (at most four) in
+// proportion to the blocks' columns (forward: later blocks have more; backward: mirrored).
+__device__ __constant__ const unsigned char kWaveSplit[4][5] = {{0, 16, 16, 16, 16}, {0, 5, 16, 16, 16}, {0, 3, 8, 16, 16}, {0, 2, 5, 10, 16}};
 
-// Teams: one workgroup per elimination subtree, its dependency levels separated by barriers.
-__global__ __launch_bounds__(256) void KLdltTeams(const int* __restrict__ teamLev, const int* __restrict__ levPtr,
-                                                  const int* __restrict__ rows, const int* __restrict__ rp, const int* __restrict__ cl,
-                                                  const double* __restrict__ vl, double* y, int n, int K) {
-  const int t = blockIdx.x;
-  for (int lv = teamLev[t]; lv < teamLev[t + 1]; lv++) {
-    const int r0 = levPtr[lv], cnt = levPtr[lv + 1] - r0;
-    for (int q = threadIdx.x; q < cnt * K; q += blockDim.x) {
-      int row = rows[r0 + q % cnt], c = q / cnt;
-      double* Y = y + (size_t)c * n;
-      double s = Y[row];
-      for (int k = rp[row]; k < rp[row + 1]; k++) s -= vl[k] * Y[cl[k]];
-      Y[row] = s;
+// A narrow stage: one workgroup of 16 waves per component of at most kLdltNarrowRows rows and chunk of
+// up to KC columns.  The component's right-hand side is staged in LDS; a wave then owns one row per
+// lane and a share of its block's columns, so the inverse's loads are whole lines that wait for nothing
+// and most of a component is one memory round trip; the waves' parts are added in a fixed order.
+template <bool kForward, int G, int KC>
+__global__ __launch_bounds__(1024) void KLdltNarrow(int comp0, const int* __restrict__ compPtr, const long* __restrict__ matPtr,
+                                                    const double* __restrict__ mat, const int* __restrict__ rp, const int* __restrict__ col,
+                                                    const double* __restrict__ val, const int* __restrict__ perm,
+                                                    const double* __restrict__ dinv, const double* src, int lds, double* y, int n, double* dst,
+                                                    int ldd, const int* __restrict__ map, int K) {
+  __shared__ double R[KC][kLdltNarrowRows];
+  __shared__ double P[16][KC][kLdltBlock];
+  const int comp = comp0 + blockIdx.x, w0 = compPtr[comp], m = compPtr[comp + 1] - w0;
+  const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
+  y += (size_t)c0 * n;
+  for (int i = threadIdx.x / G; i < m; i += 1024 / G) {
+    const int w = w0 + i, lane = threadIdx.x % G;
+    double s[KC];
+    CouplingSums<G, KC>(col, val, rp[w], rp[w + 1], lane, y, n, kc, s);
+#pragma unroll
+    for (int c = 0; c < KC; c++)
+      if (lane == c % G && c < kc) R[c][i] = (kForward ? src[(size_t)(c0 + c) * lds + perm[w]] : y[(size_t)c * n + w] * dinv[w]) - s[c];
+  }
+  __syncthreads();
+  const int blocks = (m + kLdltBlock - 1) / kLdltBlock, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  // this wave's block: the split's k-th (backward: mirrored, so that the widest block gets the most waves)
+  int k = 0;
+  while (wave >= kWaveSplit[blocks - 1][k + 1]) k++;
+  const int part = wave - kWaveSplit[blocks - 1][k], parts = kWaveSplit[blocks - 1][k + 1] - kWaveSplit[blocks - 1][k];
+  const int rb = kForward ? k : blocks - 1 - k, r0 = rb * kLdltBlock, nr = min(kLdltBlock, m - r0);
+  const int j0 = kForward ? 0 : r0, j1 = kForward ? r0 + nr : m;
+  // the blocks before this one: kLdltBlock rows each (only the last is shorter)
+  const long off = matPtr[comp] + (kForward ? (long)kLdltBlock * kLdltBlock * (rb * (rb + 1) / 2)
+                                            : (long)kLdltBlock * rb * m - (long)kLdltBlock * kLdltBlock * (rb * (rb - 1) / 2));
+  const double* M = mat + off + min(lane, nr - 1);
+  double acc[KC] = {};
+#pragma unroll 8
+  for (int j = j0 + part; j < j1; j += parts) {
+    const double a = M[(size_t)(j - j0) * nr];
+#pragma unroll
+    for (int c = 0; c < KC; c++) acc[c] += a * R[c][j];
+  }
+#pragma unroll
+  for (int c = 0; c < KC; c++) P[wave][c][lane] = acc[c];
+  __syncthreads();
+  for (int t = threadIdx.x; t < m * kc; t += 1024) {
+    const int c = t / m, i = t % m, b = i / kLdltBlock, kk = kForward ? b : blocks - 1 - b;
+    double s = 0.0;
+    for (int q = kWaveSplit[blocks - 1][kk]; q < kWaveSplit[blocks - 1][kk + 1]; q++) s += P[q][c][i % kLdltBlock];
+    y[(size_t)c * n + w0 + i] = s;
+    if (!kForward) {
+      const int g = perm[w0 + i];
+      dst[(size_t)(c0 + c) * ldd + (map ? map[g] : g)] = s;
     }
-    __syncthreads();
   }
 }
 
-// Top of the elimination tree: one workgroup, a wavefront per (row, column) dot product.
-__global__ __launch_bounds__(1024) void KLdltTop(int lev0, int lev1, const int* __restrict__ levPtr, const int* __restrict__ rows,
-                                                 const int* __restrict__ rp, const int* __restrict__ cl, const double* __restrict__ vl, double* y,
-                                                 int n, int K) {
-  const int lane = threadIdx.x % kWave, wv = threadIdx.x / kWave, nw = blockDim.x / kWave;
-  for (int lv = lev0; lv < lev1; lv++) {
-    const int r0 = levPtr[lv], cnt = levPtr[lv + 1] - r0;
-    for (int q = wv; q < cnt * K; q += nw) {
-      int row = rows[r0 + q % cnt], c = q / cnt;
-      double* Y = y + (size_t)c * n;
-      double s = 0;
-      for (int k = rp[row] + lane; k < rp[row + 1]; k += kWave) s += vl[k] * Y[cl[k]];
-      for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
-      if (lane == 0) Y[row] -= s;
+// A wide stage's right-hand sides (its rows [row0, row1), one wave per row and chunk of columns).
+template <bool kForward, int KC>
+__global__ __launch_bounds__(256) void KLdltCouple(int row0, int row1, int wideBegin, const int* __restrict__ rp, const int* __restrict__ col,
+                                                   const double* __restrict__ val, const int* __restrict__ perm,
+                                                   const double* __restrict__ dinv, const double* src, int lds, const double* y, int n,
+                                                   double* buf, int nWide, int K) {
+  const int w = row0 + blockIdx.x * (256 / kWave) + (int)threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  if (w >= row1) return;
+  const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
+  y += (size_t)c0 * n;
+  double s[KC];
+  CouplingSums<kWave, KC>(col, val, rp[w], rp[w + 1], lane, y, n, kc, s);
+#pragma unroll
+  for (int c = 0; c < KC; c++)
+    if (lane == c && c < kc)
+      buf[(size_t)(c0 + c) * nWide + w - wideBegin] = (kForward ? src[(size_t)(c0 + c) * lds + perm[w]] : y[(size_t)c * n + w] * dinv[w]) - s[c];
+}
+
+// A wide stage's product with its components' inverses, one wave per row and chunk of columns: the
+// forward result to y, or for the top scaled by 1 / D to `top` (the backward product's input); the
+// backward result to y and dst.
+template <bool kForward, int KC>
+__global__ __launch_bounds__(256) void KLdltWide(int row0, int row1, int wideBegin, const int* __restrict__ rowComp,
+                                                 const int* __restrict__ compPtr, const long* __restrict__ matPtr,
+                                                 const double* __restrict__ mat, const double* __restrict__ buf, int nWide,
+                                                 const int* __restrict__ perm, const double* __restrict__ dinv, double* y, int n, double* top,
+                                                 double* dst, int ldd, const int* __restrict__ map, int K) {
+  const int w = row0 + blockIdx.x * (256 / kWave) + (int)threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  if (w >= row1) return;
+  const int comp = rowComp[w - wideBegin], w0 = compPtr[comp], m = compPtr[comp + 1] - w0, i = w - w0;
+  const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
+  const double* row = mat + matPtr[comp] + (size_t)i * m;
+  const double* in = buf + (size_t)c0 * nWide + w0 - wideBegin;
+  double acc[KC] = {};
+  const int j1 = kForward ? i + 1 : m;
+#pragma unroll 4
+  for (int j = (kForward ? 0 : i / kWave * kWave) + lane; j < j1; j += kWave) {  // backward: entries before i are zero
+    const double a = row[j];
+#pragma unroll
+    for (int c = 0; c < KC; c++)
+      if (c < kc) acc[c] += a * in[(size_t)c * nWide + j];
+  }
+#pragma unroll
+  for (int c = 0; c < KC; c++) acc[c] = GroupSum<kWave>(acc[c]);
+#pragma unroll
+  for (int c = 0; c < KC; c++) {
+    if (lane != c || c >= kc) continue;
+    if (kForward && top) top[(size_t)(c0 + c) * nWide + w - wideBegin] = acc[c] * dinv[w];
+    else y[(size_t)(c0 + c) * n + w] = acc[c];
+    if (!kForward) {
+      const int g = perm[w];
+      dst[(size_t)(c0 + c) * ldd + (map ? map[g] : g)] = acc[c];
     }
-    __syncthreads();
   }
 }
 
@@ -495,42 +587,6 @@ __global__ void KZeroStrided(int N, double* x, int ld, int K) {
   x[(t / N) * ld + t % N] = 0.0;
 }
 
-// ------------------------------------------------------------------ dense top of an LDL^T solve
-// buf[c][a] = y[c][top[a]] - sum over team columns of L[top[a]][i] y[c][i]   (one wave per top row)
-__global__ __launch_bounds__(256) void KTopCouple(int st, const int* __restrict__ top, const int* __restrict__ rp,
-                                                  const int* __restrict__ cl, const double* __restrict__ vl, const double* __restrict__ y,
-                                                  int n, double* buf, int K) {
-  const int a = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  if (a >= st) return;
-  for (int c = 0; c < K; c++) {
-    const double* Y = y + (long)c * n;
-    double s = 0.0;
-    for (int p = rp[a] + lane; p < rp[a + 1]; p += kWave) s += vl[p] * Y[cl[p]];
-    for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
-    if (lane == 0) buf[(long)c * st + a] = Y[top[a]] - s;
-  }
-}
-// buf[c][a] = y[c][top[a]]
-__global__ void KTopGather(int st, const int* __restrict__ top, const double* __restrict__ y, int n, double* buf, int K) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)st * K) return;
-  buf[t] = y[(t / st) * n + top[t % st]];
-}
-// y[c][top[a]] = sum_b M[a][b] buf[c][b]   (one wave per row; M row-major st x st)
-__global__ __launch_bounds__(256) void KTopDense(int st, const int* __restrict__ top, const double* __restrict__ M,
-                                                 const double* __restrict__ buf, double* y, int n, int K) {
-  const int a = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  if (a >= st) return;
-  const double* row = M + (long)a * st;
-  for (int c = 0; c < K; c++) {
-    const double* in = buf + (long)c * st;
-    double s = 0.0;
-    for (int b = lane; b < st; b += kWave) s += row[b] * in[b];
-    for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
-    if (lane == 0) y[(long)c * n + top[a]] = s;
-  }
-}
-
 static thread_local size_t g_uploadBytes = 0;
 size_t UploadByteCounter() { return g_uploadBytes; }
 
@@ -626,122 +682,21 @@ static std::vector<double> SymStencil(const std::vector<double>& aos, const std:
   return s;
 }
 
-// Partition the elimination tree into subtree teams (at most `smax` rows) plus the top part, and
-// group rows by dependency level inside each team and inside the top.
 void UploadLdlt(std::vector<void*>& ds, const Ldlt& F, DevLdlt& d, int kcap) {
-  const int n = F.n;
-  d.n = n;
-  d.perm = UploadTo(ds, F.perm);
-  d.lrRowptr = UploadTo(ds, F.Lrows.rowptr), d.lrCol = UploadTo(ds, F.Lrows.col), d.lrVal = UploadTo(ds, F.Lrows.val);
-  d.lcRowptr = UploadTo(ds, F.Lcols.rowptr), d.lcCol = UploadTo(ds, F.Lcols.col), d.lcVal = UploadTo(ds, F.Lcols.val);
-  std::vector<double> dinv(n);
-  for (int i = 0; i < n; i++) dinv[i] = 1.0 / F.D[i];
-  d.dinv = UploadTo(ds, dinv);
-  std::vector<int> parent(n, -1), size(n, 1), team(n, -1);
-  for (int i = 0; i < n; i++)
-    if (F.Lcols.rowptr[i + 1] > F.Lcols.rowptr[i]) parent[i] = F.Lcols.col[F.Lcols.rowptr[i]];
-  for (int i = 0; i < n; i++)
-    if (parent[i] >= 0) size[parent[i]] += size[i];
-  const int smax = std::max(64, n / 256);
-  int nTeams = 0;
-  for (int v = n - 1; v >= 0; v--) {
-    if (size[v] > smax) continue;
-    if (parent[v] < 0 || size[parent[v]] > smax) team[v] = nTeams++;
-    else team[v] = team[parent[v]];
-  }
-  // forward levels (dependencies within the same team, or within the top)
-  std::vector<int> lev(n, 0);
-  for (int k = 0; k < n; k++) {
-    int l = 0;
-    for (int p = F.Lrows.rowptr[k]; p < F.Lrows.rowptr[k + 1]; p++) {
-      int i = F.Lrows.col[p];
-      if (team[i] == team[k]) l = std::max(l, lev[i] + 1);
-    }
-    lev[k] = l;
-  }
-  auto build = [&](std::vector<int>& levPtr, std::vector<int>& rows, std::vector<int>& teamLev, int& top0, int& top1) {
-    // group key (team, level); teams first in team order, then the top part
-    int G = nTeams + 1;
-    std::vector<int> maxLev(G, -1);
-    for (int k = 0; k < n; k++) {
-      int g = team[k] < 0 ? nTeams : team[k];
-      maxLev[g] = std::max(maxLev[g], lev[k]);
-    }
-    std::vector<int> groupBase(G + 1, 0);
-    for (int g = 0; g < G; g++) groupBase[g + 1] = groupBase[g] + maxLev[g] + 1;
-    int nGroups = groupBase[G];
-    std::vector<int> cnt(nGroups + 1, 0);
-    for (int k = 0; k < n; k++) {
-      int g = team[k] < 0 ? nTeams : team[k];
-      cnt[groupBase[g] + lev[k] + 1]++;
-    }
-    for (int i = 0; i < nGroups; i++) cnt[i + 1] += cnt[i];
-    levPtr = cnt;
-    rows.assign(n, 0);
-    std::vector<int> fillp(cnt.begin(), cnt.end() - 1);
-    for (int k = 0; k < n; k++) {
-      int g = team[k] < 0 ? nTeams : team[k];
-      rows[fillp[groupBase[g] + lev[k]]++] = k;
-    }
-    teamLev.assign(groupBase.begin(), groupBase.begin() + nTeams + 1);
-    top0 = groupBase[nTeams], top1 = groupBase[G];
-    int mr = 0;
-    for (int i = 0; i < groupBase[nTeams]; i++) mr = std::max(mr, levPtr[i + 1] - levPtr[i]);
-    d.maxTeamRows = std::max(d.maxTeamRows, mr);
-  };
-  std::vector<int> fLevPtr, fRows, fTeamLev, bLevPtr, bRows, bTeamLev;
-  build(fLevPtr, fRows, fTeamLev, d.topFwdLevBegin, d.topFwdLevEnd);
-  // backward levels: dependencies on ancestors in the same team (the top is solved first)
-  std::fill(lev.begin(), lev.end(), 0);
-  for (int i = n - 1; i >= 0; i--) {
-    int l = 0;
-    for (int p = F.Lcols.rowptr[i]; p < F.Lcols.rowptr[i + 1]; p++) {
-      int k = F.Lcols.col[p];
-      if (team[k] == team[i]) l = std::max(l, lev[k] + 1);
-    }
-    lev[i] = l;
-  }
-  build(bLevPtr, bRows, bTeamLev, d.topBwdLevBegin, d.topBwdLevEnd);
-  d.nTeams = nTeams;
-  d.fwdLevPtr = UploadTo(ds, fLevPtr), d.fwdRows = UploadTo(ds, fRows), d.teamFwdLev = UploadTo(ds, fTeamLev);
-  d.bwdLevPtr = UploadTo(ds, bLevPtr), d.bwdRows = UploadTo(ds, bRows), d.teamBwdLev = UploadTo(ds, bTeamLev);
-  // dense top: the top rows form a unit-lower block L_TT (separators after fill, nearly dense);
-  // its inverse turns the sequential top solve into two dense matrix-vector products
-  std::vector<int> top, local(n, -1);
-  for (int k = 0; k < n; k++)
-    if (team[k] < 0) local[k] = (int)top.size(), top.push_back(k);
-  const int st = (int)top.size();
-  if (st == 0 || st > kDenseTopMax || kcap < 1) return;
-  std::vector<int> crp(1, 0), ccl;
-  std::vector<double> cvl, Ltt((size_t)st * st, 0.0);
-  for (int a = 0; a < st; a++) {
-    const int k = top[a];
-    Ltt[(size_t)a * st + a] = 1.0;
-    for (int p = F.Lrows.rowptr[k]; p < F.Lrows.rowptr[k + 1]; p++) {
-      const int i = F.Lrows.col[p];
-      if (local[i] >= 0) Ltt[(size_t)a * st + local[i]] = F.Lrows.val[p];
-      else ccl.push_back(i), cvl.push_back(F.Lrows.val[p]);
-    }
-    crp.push_back((int)ccl.size());
-  }
-  std::vector<double> inv((size_t)st * st, 0.0), invT((size_t)st * st, 0.0);
-#pragma omp parallel for schedule(dynamic, 16)
-  for (int j = 0; j < st; j++) {  // column j of the inverse: forward substitution from e_j
-    std::vector<double> z(st, 0.0);
-    z[j] = 1.0;
-    for (int a = j + 1; a < st; a++) {
-      double v = 0.0;
-      const double* row = &Ltt[(size_t)a * st];
-      for (int b = j; b < a; b++) v -= row[b] * z[b];
-      z[a] = v;
-    }
-    for (int a = j; a < st; a++) inv[(size_t)a * st + j] = z[a], invT[(size_t)j * st + a] = z[a];
-  }
-  d.nTop = st, d.kcap = kcap;
-  d.topRows = UploadTo(ds, top);
-  d.topCplRowptr = UploadTo(ds, crp), d.topCplCol = UploadTo(ds, ccl), d.topCplVal = UploadTo(ds, cvl);
-  d.topInv = UploadTo(ds, inv), d.topInvT = UploadTo(ds, invT);
-  d.topBuf = UploadTo(ds, std::vector<double>((size_t)st * kcap, 0.0));
+  LdltStages S;
+  BuildLdltStages(F, S);
+  d.n = S.n, d.wideBegin = S.wideBegin, d.kcap = kcap;
+  d.stages = S.stages;
+  d.perm = UploadTo(ds, S.perm), d.dinv = UploadTo(ds, S.dinv), d.compPtr = UploadTo(ds, S.compPtr);
+  d.fwdPtr = UploadTo(ds, S.fwdPtr), d.fwdCol = UploadTo(ds, S.fwdCol), d.fwdVal = UploadTo(ds, S.fwdVal);
+  d.bwdPtr = UploadTo(ds, S.bwdPtr), d.bwdCol = UploadTo(ds, S.bwdCol), d.bwdVal = UploadTo(ds, S.bwdVal);
+  d.fwdMatPtr = UploadTo(ds, S.fwdMatPtr), d.bwdMatPtr = UploadTo(ds, S.bwdMatPtr);
+  d.fwdMat = UploadTo(ds, S.fwdMat), d.bwdMat = UploadTo(ds, S.bwdMat);
+  std::vector<int> rowComp(S.n - S.wideBegin);
+  for (size_t c = 0; c + 1 < S.compPtr.size(); c++)
+    for (int w = std::max(S.compPtr[c], S.wideBegin); w < S.compPtr[c + 1]; w++) rowComp[w - S.wideBegin] = (int)c;
+  d.rowComp = UploadTo(ds, rowComp);
+  if (kcap > 0 && !rowComp.empty()) d.wideBuf = UploadTo(ds, std::vector<double>(2 * (size_t)kcap * rowComp.size(), 0.0));
 }
 
 void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOperator& op, int kcap, DeviceSystem& ds) {
@@ -803,27 +758,54 @@ void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOpe
   ds.bytes = g_uploadBytes;
 }
 
+// Columns in chunks of KC = min(K, 4); a stage's launches cover all chunks.
+template <int KC>
+static void LdltSolveChunks(DevLdlt& F, const double* src, int lds, double* dst, int ldd, const int* map, double* y, int K, hipStream_t s) {
+  const int n = F.n, nWide = n - F.wideBegin, last = (int)F.stages.size() - 1;
+  const unsigned chunks = (unsigned)((K + KC - 1) / KC);
+  double *buf = F.wideBuf, *top = F.wideBuf + (size_t)F.kcap * nWide;
+  auto wideGrid = [&](const LdltStage& T) { return dim3(Blocks(T.rowEnd - T.rowBegin, 256 / kWave), chunks); };
+  for (int k = 0; k <= last; k++) {
+    const LdltStage& T = F.stages[k];
+    if (T.rowBegin == T.rowEnd) continue;
+    if (!T.wide) {
+      // the first stage has no couplings; the next stages' rows have tens (C2 level 0: 43 on average)
+      const auto kernel = k == 0 ? KLdltNarrow<true, 8, KC> : KLdltNarrow<true, 16, KC>;
+      kernel<<<dim3(T.compEnd - T.compBegin, chunks), 1024, 0, s>>>(T.compBegin, F.compPtr, F.fwdMatPtr, F.fwdMat, F.fwdPtr, F.fwdCol, F.fwdVal,
+                                                                    F.perm, F.dinv, src, lds, y, n, nullptr, 0, nullptr, K);
+      continue;
+    }
+    KLdltCouple<true, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.fwdPtr, F.fwdCol, F.fwdVal, F.perm, F.dinv, src, lds,
+                                                      y, n, buf, nWide, K);
+    KLdltWide<true, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.rowComp, F.compPtr, F.fwdMatPtr, F.fwdMat, buf, nWide,
+                                                    F.perm, F.dinv, y, n, k == last ? top : nullptr, nullptr, 0, nullptr, K);
+  }
+  for (int k = last; k >= 0; k--) {
+    const LdltStage& T = F.stages[k];
+    if (T.rowBegin == T.rowEnd) continue;
+    if (!T.wide) {
+      KLdltNarrow<false, 8, KC><<<dim3(T.compEnd - T.compBegin, chunks), 1024, 0, s>>>(T.compBegin, F.compPtr, F.bwdMatPtr, F.bwdMat, F.bwdPtr,
+                                                                                       F.bwdCol, F.bwdVal, F.perm, F.dinv, nullptr, 0, y, n, dst,
+                                                                                       ldd, map, K);
+      continue;
+    }
+    if (k < last)
+      KLdltCouple<false, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.bwdPtr, F.bwdCol, F.bwdVal, F.perm, F.dinv, nullptr,
+                                                         0, y, n, buf, nWide, K);
+    KLdltWide<false, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.rowComp, F.compPtr, F.bwdMatPtr, F.bwdMat,
+                                                     k == last ? top : buf, nWide, F.perm, F.dinv, y, n, nullptr, dst, ldd, map, K);
+  }
+}
+
 void LdltSolve(DevLdlt& F, const double* src, int lds, double* dst, int ldd, const int* map, double* y, int K, hipStream_t s) {
-  const int n = F.n;
-  if (n == 0) return;
-  const long nk = (long)n * K;
-  KLdltGather<<<Blocks(nk, 256), 256, 0, s>>>(n, F.perm, src, lds, y, K);
-  if (F.nTeams) KLdltTeams<<<F.nTeams, 256, 0, s>>>(F.teamFwdLev, F.fwdLevPtr, F.fwdRows, F.lrRowptr, F.lrCol, F.lrVal, y, n, K);
-  const bool dense = F.nTop > 0 && K <= F.kcap;
-  const unsigned topBlocks = Blocks(F.nTop, 256 / kWave);
-  if (dense) {
-    KTopCouple<<<topBlocks, 256, 0, s>>>(F.nTop, F.topRows, F.topCplRowptr, F.topCplCol, F.topCplVal, y, n, F.topBuf, K);
-    KTopDense<<<topBlocks, 256, 0, s>>>(F.nTop, F.topRows, F.topInv, F.topBuf, y, n, K);
-  } else if (F.topFwdLevEnd > F.topFwdLevBegin)
-    KLdltTop<<<1, 1024, 0, s>>>(F.topFwdLevBegin, F.topFwdLevEnd, F.fwdLevPtr, F.fwdRows, F.lrRowptr, F.lrCol, F.lrVal, y, n, K);
-  KLdltDiag<<<Blocks(nk, 256), 256, 0, s>>>(n, F.dinv, y, K);
-  if (dense) {
-    KTopGather<<<Blocks((long)F.nTop * K, 256), 256, 0, s>>>(F.nTop, F.topRows, y, n, F.topBuf, K);
-    KTopDense<<<topBlocks, 256, 0, s>>>(F.nTop, F.topRows, F.topInvT, F.topBuf, y, n, K);
-  } else if (F.topBwdLevEnd > F.topBwdLevBegin)
-    KLdltTop<<<1, 1024, 0, s>>>(F.topBwdLevBegin, F.topBwdLevEnd, F.bwdLevPtr, F.bwdRows, F.lcRowptr, F.lcCol, F.lcVal, y, n, K);
-  if (F.nTeams) KLdltTeams<<<F.nTeams, 256, 0, s>>>(F.teamBwdLev, F.bwdLevPtr, F.bwdRows, F.lcRowptr, F.lcCol, F.lcVal, y, n, K);
-  KLdltScatter<<<Blocks(nk, 256), 256, 0, s>>>(n, F.perm, map, y, dst, ldd, K);
+  if (F.n == 0) return;
+  if (K < 1 || K > F.kcap) throw std::runtime_error("column count outside [1, capacity]");
+  switch (std::min(K, 4)) {
+    case 1: LdltSolveChunks<1>(F, src, lds, dst, ldd, map, y, K, s); break;
+    case 2: LdltSolveChunks<2>(F, src, lds, dst, ldd, map, y, K, s); break;
+    case 3: LdltSolveChunks<3>(F, src, lds, dst, ldd, map, y, K, s); break;
+    default: LdltSolveChunks<4>(F, src, lds, dst, ldd, map, y, K, s); break;
+  }
 }
 
 static void CheckK(const DeviceSystem& ds, int K) {

@@ -1,5 +1,6 @@
 #include "gdtp_ldlt.h"
 
+#include <algorithm>
 #include <cmath>
 #include <functional>
 
@@ -160,32 +161,156 @@ int FactorLdlt(const Csr& A, Ldlt& F, std::string& err) {
   for (int k = 0; k < n; k++) Lc.rowptr[k + 1] = (int)Lp[k + 1];
   Lc.col = Li, Lc.val = Lx;
   F.Lrows = Lc.Transpose();
-  // dependency levels
-  std::vector<int> lev(n, 0);
-  int maxL = 0;
-  for (int k = 0; k < n; k++) {
-    int l = 0;
-    for (int p = F.Lrows.rowptr[k]; p < F.Lrows.rowptr[k + 1]; p++) l = std::max(l, lev[F.Lrows.col[p]] + 1);
-    lev[k] = l, maxL = std::max(maxL, l);
-  }
-  auto bucket = [&](std::vector<int>& ptr, std::vector<int>& rows, int nl) {
-    ptr.assign(nl + 2, 0);
-    for (int k = 0; k < n; k++) ptr[lev[k] + 1]++;
-    for (int l = 0; l <= nl; l++) ptr[l + 1] += ptr[l];
-    rows.assign(n, 0);
-    std::vector<int> f(ptr.begin(), ptr.end() - 1);
-    for (int k = 0; k < n; k++) rows[f[lev[k]]++] = k;
-    ptr.resize(nl + 2);
-  };
-  bucket(F.fwdLevelPtr, F.fwdRows, maxL);
-  maxL = 0;
-  for (int i = n - 1; i >= 0; i--) {
-    int l = 0;
-    for (int p = Lc.rowptr[i]; p < Lc.rowptr[i + 1]; p++) l = std::max(l, lev[Lc.col[p]] + 1);
-    lev[i] = l, maxL = std::max(maxL, l);
-  }
-  bucket(F.bwdLevelPtr, F.bwdRows, maxL);
   return 1;
+}
+
+void BuildLdltStages(const Ldlt& F, LdltStages& S, int topRows) {
+  const int n = F.n;
+  S = LdltStages();
+  S.n = n;
+  if (n == 0) return;
+  // elimination tree (a column's first entry below the diagonal) and subtree sizes
+  std::vector<int> parent(n, -1), size(n, 1);
+  for (int i = 0; i < n; i++) {
+    int p = n;
+    for (int k = F.Lcols.rowptr[i]; k < F.Lcols.rowptr[i + 1]; k++) p = std::min(p, F.Lcols.col[k]);
+    if (p < n) parent[i] = p;
+  }
+  for (int i = 0; i < n; i++)
+    if (parent[i] >= 0) size[parent[i]] += size[i];
+  // stage limits: rows whose subtree exceeds the last limit form the top
+  std::vector<int> limit;
+  if (n > topRows)
+    for (long s = kLdltLeafRows, last = n;; s *= kLdltStageGrowth) {
+      long above = 0;
+      for (int i = 0; i < n; i++) above += size[i] > s;
+      // no row left for the top: what the last stage left is the top unless that is far too many
+      if (above == 0 && !limit.empty() && last <= 2 * (long)topRows) break;
+      limit.push_back((int)std::min<long>(s, n));
+      if (above <= topRows) break;
+      last = above;
+    }
+  const int nStages = (int)limit.size() + 1;
+  std::vector<int> stage(n), comp(n), compStage;
+  for (int i = 0; i < n; i++) stage[i] = (int)(std::lower_bound(limit.begin(), limit.end(), size[i]) - limit.begin());
+  // components: a row joins its parent's when both are of one stage; the top is one component
+  for (int i = n - 1, top = -1; i >= 0; i--) {
+    if (stage[i] == nStages - 1 && top >= 0) comp[i] = top;
+    else if (stage[i] < nStages - 1 && parent[i] >= 0 && stage[parent[i]] == stage[i]) comp[i] = comp[parent[i]];
+    else {
+      comp[i] = (int)compStage.size();
+      compStage.push_back(stage[i]);
+      if (stage[i] == nStages - 1) top = comp[i];
+    }
+  }
+  // new numbering: components by stage, rows of a component in elimination order
+  const int nComp = (int)compStage.size();
+  std::vector<int> order(nComp), rank(nComp), count(nComp, 0);
+  for (int c = 0; c < nComp; c++) order[c] = c;
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return compStage[a] < compStage[b]; });
+  for (int c = 0; c < nComp; c++) rank[order[c]] = c;
+  for (int i = 0; i < n; i++) count[rank[comp[i]]]++;
+  S.compPtr.assign(nComp + 1, 0);
+  for (int c = 0; c < nComp; c++) S.compPtr[c + 1] = S.compPtr[c] + count[c];
+  std::vector<int> next(S.compPtr.begin(), S.compPtr.end() - 1), rowOf(n), at(n);
+  for (int i = 0; i < n; i++) {
+    at[i] = next[rank[comp[i]]]++;
+    rowOf[at[i]] = i;
+  }
+  S.stages.assign(nStages, LdltStage());
+  for (int c = 0, s = 0; s < nStages; s++) {
+    LdltStage& T = S.stages[s];
+    T.compBegin = c;
+    while (c < nComp && compStage[order[c]] == s) T.wide = T.wide || count[c] > kLdltNarrowRows, c++;
+    T.compEnd = c;
+    T.rowBegin = S.compPtr[T.compBegin], T.rowEnd = S.compPtr[T.compEnd];
+    // the top, and every stage after a wide one
+    T.wide = T.wide || s == nStages - 1 || (s > 0 && S.stages[s - 1].wide);
+  }
+  S.wideBegin = n;
+  for (int s = nStages - 1; s >= 0 && S.stages[s].wide; s--) S.wideBegin = S.stages[s].rowBegin;
+  S.perm.resize(n), S.dinv.resize(n);
+  for (int w = 0; w < n; w++) S.perm[w] = F.perm[rowOf[w]], S.dinv[w] = 1.0 / F.D[rowOf[w]];
+  auto couplings = [&](const Csr& L, std::vector<int>& ptr, std::vector<int>& col, std::vector<double>& val) {
+    ptr.assign(n + 1, 0);
+    for (int w = 0; w < n; w++) {
+      const int i = rowOf[w];
+      for (int k = L.rowptr[i]; k < L.rowptr[i + 1]; k++)
+        if (comp[L.col[k]] != comp[i]) col.push_back(at[L.col[k]]), val.push_back(L.val[k]);
+      ptr[w + 1] = (int)col.size();
+    }
+  };
+  couplings(F.Lrows, S.fwdPtr, S.fwdCol, S.fwdVal);
+  couplings(F.Lcols, S.bwdPtr, S.bwdCol, S.bwdVal);
+  // inverses of the components' unit-lower blocks
+  S.fwdMatPtr.assign(nComp + 1, 0), S.bwdMatPtr.assign(nComp + 1, 0);
+  std::vector<char> wide(nComp, 0);
+  for (const LdltStage& T : S.stages)
+    for (int c = T.compBegin; c < T.compEnd; c++) wide[c] = T.wide;
+  for (int c = 0; c < nComp; c++) {
+    const int m = count[c];
+    long f = 0, b = 0;
+    if (wide[c]) f = b = (long)m * m;
+    else
+      for (int r0 = 0; r0 < m; r0 += kLdltBlock) {
+        const int nr = std::min(kLdltBlock, m - r0);
+        f += (long)nr * (r0 + nr), b += (long)nr * (m - r0);
+      }
+    S.fwdMatPtr[c + 1] = S.fwdMatPtr[c] + f, S.bwdMatPtr[c + 1] = S.bwdMatPtr[c] + b;
+  }
+  S.fwdMat.assign(S.fwdMatPtr[nComp], 0.0), S.bwdMat.assign(S.bwdMatPtr[nComp], 0.0);
+  // inv: row-major m x m, the inverse; its column j by forward substitution from e_j
+  auto column = [&](int m, const std::vector<double>& L, std::vector<double>& inv, int j, std::vector<double>& z) {
+    z[j] = 1.0;
+    inv[(size_t)j * m + j] = 1.0;
+    for (int a = j + 1; a < m; a++) {
+      double v = 0.0;
+      const double* row = &L[(size_t)a * m];
+      for (int b = j; b < a; b++) v -= row[b] * z[b];
+      z[a] = v;
+      inv[(size_t)a * m + j] = v;
+    }
+  };
+  auto load = [&](int c, std::vector<double>& L) {
+    const int m = count[c], w0 = S.compPtr[c];
+    L.assign((size_t)m * m, 0.0);
+    for (int a = 0; a < m; a++) {
+      const int i = rowOf[w0 + a];
+      for (int k = F.Lrows.rowptr[i]; k < F.Lrows.rowptr[i + 1]; k++)
+        if (comp[F.Lrows.col[k]] == comp[i]) L[(size_t)a * m + at[F.Lrows.col[k]] - w0] = F.Lrows.val[k];
+    }
+  };
+  const int nNarrow = (int)(std::find(wide.begin(), wide.end(), 1) - wide.begin());
+#pragma omp parallel for schedule(dynamic, 8)
+  for (int c = 0; c < nNarrow; c++) {
+    const int m = count[c];
+    std::vector<double> L, inv((size_t)m * m, 0.0), z(m);
+    load(c, L);
+    for (int j = 0; j < m; j++) column(m, L, inv, j, z);
+    double *f = S.fwdMat.data() + S.fwdMatPtr[c], *b = S.bwdMat.data() + S.bwdMatPtr[c];
+    for (int r0 = 0; r0 < m; r0 += kLdltBlock) {
+      const int nr = std::min(kLdltBlock, m - r0);
+      for (int j = 0; j < r0 + nr; j++)
+        for (int r = 0; r < nr; r++) *f++ = inv[(size_t)(r0 + r) * m + j];
+      for (int j = r0; j < m; j++)
+        for (int r = 0; r < nr; r++) *b++ = inv[(size_t)j * m + r0 + r];
+    }
+  }
+  for (int c = nNarrow; c < nComp; c++) {  // few and large: in parallel over the columns
+    const int m = count[c];
+    std::vector<double> L, inv((size_t)m * m, 0.0);
+    load(c, L);
+#pragma omp parallel
+    {
+      std::vector<double> z(m);
+#pragma omp for schedule(dynamic, 16)
+      for (int j = 0; j < m; j++) column(m, L, inv, j, z);
+    }
+    double *f = S.fwdMat.data() + S.fwdMatPtr[c], *b = S.bwdMat.data() + S.bwdMatPtr[c];
+#pragma omp parallel for schedule(static)
+    for (int r = 0; r < m; r++)
+      for (int j = 0; j < m; j++) f[(size_t)r * m + j] = inv[(size_t)r * m + j], b[(size_t)r * m + j] = inv[(size_t)j * m + r];
+  }
 }
 
 void SolveLdlt(const Ldlt& F, const double* b, double* x, int ncols, int ld) {

@@ -20,12 +20,48 @@ struct Ldlt {
   Csr Lrows;                  // strictly lower triangular L by rows (row k: entries l_ki, i < k), permuted space
   Csr Lcols;                  // the same entries by columns (row of L^T)
   std::vector<double> D;      // diagonal
-  // level schedules: rows grouped by dependency level, forward (L) and backward (L^T)
-  std::vector<int> fwdLevelPtr, fwdRows, bwdLevelPtr, bwdRows;
+};
+
+// The triangular solves of an LDL^T factor as a few passes whose rows are all independent, for the
+// GPU (partitioned inverses: F. L. Alvarado and R. Schreiber, "Optimal parallel solution of sparse
+// triangular systems", SIAM J. Sci. Comput. 14, 1993).  The elimination tree is cut by subtree size
+// into stages; a stage's connected pieces ("components") do not couple with each other, so a stage is
+// one gather of couplings with the stages already solved and one product with each component's
+// explicit inverse of its unit-lower block.  The last stage (the top of the tree) is one component.
+// Rows are renumbered by (stage, component, row): a component is a contiguous range.
+constexpr int kLdltLeafRows = 128;     // largest subtree of the first stage
+constexpr int kLdltStageGrowth = 8;    // each further stage takes subtrees this many times larger
+constexpr int kLdltTopRows = 2048;     // stages are added until the top has at most this many rows
+constexpr int kLdltNarrowRows = 256;   // components up to this size are solved by one workgroup
+constexpr int kLdltBlock = 64;         // rows per block of a narrow component's inverse
+
+struct LdltStage {
+  int rowBegin = 0, rowEnd = 0;        // rows (new numbering)
+  int compBegin = 0, compEnd = 0;      // components
+  bool wide = false;                   // some component has more than kLdltNarrowRows rows (or the top)
+};
+
+struct LdltStages {
+  int n = 0;
+  std::vector<LdltStage> stages;       // in forward order; the last is the top
+  std::vector<int> perm;               // new row -> row of the original matrix
+  std::vector<double> dinv;            // 1 / D
+  std::vector<int> compPtr;            // first row of each component (one more than components)
+  // couplings with other stages: of a row of L with the earlier stages, of a row of L^T with the later
+  std::vector<int> fwdPtr, fwdCol, bwdPtr, bwdCol;
+  std::vector<double> fwdVal, bwdVal;
+  // Inverses.  Narrow component: for each block of kLdltBlock rows the columns its rows can reach
+  // (forward: columns before the block's end; backward: from its begin), column-major, the block's
+  // rows contiguous.  Wide component: the whole matrix row-major (forward, then transposed).
+  std::vector<long> fwdMatPtr, bwdMatPtr;  // per component
+  std::vector<double> fwdMat, bwdMat;
+  int wideBegin = 0;                   // first row of the first wide stage (the later stages are all wide)
 };
 
 void NestedDissectionOrder(const Csr& A, std::vector<int>& perm);
 int FactorLdlt(const Csr& A, Ldlt& F, std::string& err);
+// The staged form of F's triangular solves; topRows: the largest top (kLdltTopRows, smaller in tests).
+void BuildLdltStages(const Ldlt& F, LdltStages& S, int topRows = kLdltTopRows);
 // Solve A x = b for ncols column-major vectors (host reference path).
 void SolveLdlt(const Ldlt& F, const double* b, double* x, int ncols, int ld);
 
