@@ -2004,7 +2004,7 @@ void UploadMixed(const Hierarchy& h, const OperatorHierarchy& oh, DeviceSystem& 
   ms.weights = Zeros<double>(ms, 2 * (size_t)kcap);
   {
     const size_t n0 = (size_t)ms.L[0].N * kcap;
-    ms.r64 = Zeros<double>(ms, n0), ms.p64 = Zeros<double>(ms, n0), ms.q64 = Zeros<double>(ms, n0), ms.z64 = Zeros<double>(ms, n0);
+    ms.r64 = Zeros<double>(ms, n0), ms.p64 = Zeros<double>(ms, n0), ms.q64 = Zeros<double>(ms, n0);
     ms.dots = Zeros<double>(ms, 3 * (size_t)kcap * kDotBlocks);
     ms.alpha = Zeros<double>(ms, kcap), ms.beta = Zeros<double>(ms, kcap), ms.pqPrev = Zeros<double>(ms, kcap);
     ms.first = Zeros<int>(ms, 1);
@@ -2311,71 +2311,180 @@ __global__ __launch_bounds__(256) void K64ApplyW(int deepBlocks, int D, const in
                           N, q, K, w);
 }
 
-// column dot products a_c . b_c: one partial sum per block (out[c][blockIdx.x]), no atomics, so
-// that the flexible-CG scalars are reproducible run to run (blockIdx.y = column)
-__global__ __launch_bounds__(256) void K64Dot(int N, const double* __restrict__ a, const double* __restrict__ b, double* out) {
-  const int ch = blockIdx.y;
-  double v = 0.0;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x) v += a[(long)ch * N + i] * b[(long)ch * N + i];
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  __shared__ double part[4];
-  if (threadIdx.x % 64 == 0) part[threadIdx.x / 64] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) out[(long)ch * kDotBlocks + blockIdx.x] = part[0] + part[1] + part[2] + part[3];
+// A flexible-CG step's vector passes stream columns of N doubles and are bound by memory, so they read
+// and write as little as they can: (z, q) and the direction take z straight from the FP32 correction
+// (never stored in FP64), the two dot products with p share one pass, and a thread takes up to four
+// columns for one read of its dense index (3.0 M texels x 64 columns: 128 bytes a value against 156,
+// 5.1-6 TB/s; the passes but the operator 92 -> 74 ms of a heat and a distance solve).
+// Dot products are reproducible run to run: one partial sum per block (out[c][blockIdx.x], no
+// atomics), added in block order.  The order of every addition is part of the result: the dot products
+// of nearly singular systems cancel, and another order moves unconverged iterates by 1e-8.
+
+// Sums over the wave of eight values per lane, 10 exchanges instead of 48: each step hands half of the
+// values to the partner lane.  Every lane returns the sum of value (lane / 8).
+__device__ __forceinline__ double WaveSum8(double (&v)[8]) {
+  const int lane = threadIdx.x % 64;
+#pragma unroll
+  for (int h = 4, o = 32; h >= 1; h /= 2, o /= 2) {
+    const bool hi = lane & o;
+#pragma unroll
+    for (int k = 0; k < h; k++) {
+      const double give = hi ? v[k] : v[k + h], keep = hi ? v[k + h] : v[k];
+      v[k] = keep + __shfl_xor(give, o, 64);
+    }
+  }
+#pragma unroll
+  for (int o = 4; o >= 1; o /= 2) v[0] += __shfl_xor(v[0], o, 64);
+  return v[0];
 }
 
-__device__ __forceinline__ double DotSum(const double* s, int n) {
+// Block sums of (z, q) with z the level-0 FP32 correction: parts[c][block]; blockIdx.y = chunk of columns.
+template <int KC>
+__global__ __launch_bounds__(256) void KFcgDotZq(int N, const int* __restrict__ g2d, const float* __restrict__ e0, long Nd,
+                                                 const double* __restrict__ q, double* parts, int K) {
+  const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
+  double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x) {
+    const long di = g2d[i];
+#pragma unroll
+    for (int c = 0; c < KC; c++)
+      if (c < kc) acc[c] += (double)e0[(long)(c0 + c) * Nd + di] * q[(long)(c0 + c) * N + i];
+  }
+  __shared__ double part[4][KC];
+  const double s = WaveSum8(acc);
+  const int lane = threadIdx.x % 64;
+  if (lane % 8 == 0 && lane / 8 < KC) part[threadIdx.x / 64][lane / 8] = s;
+  __syncthreads();
+  if ((int)threadIdx.x < kc)
+    parts[(long)(c0 + threadIdx.x) * kDotBlocks + blockIdx.x] = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
+}
+
+// Block sums of (r, p) into rp[c][block] and of (p, q) into pq[c][block]; blockIdx.y = chunk of columns.
+template <int KC>
+__global__ __launch_bounds__(256) void KFcgDots(int N, const double* __restrict__ r, const double* __restrict__ p, const double* __restrict__ q,
+                                                double* rp, double* pq, int K) {
+  const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
+  double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (long)gridDim.x * blockDim.x) {
+#pragma unroll
+    for (int c = 0; c < KC; c++)
+      if (c < kc) {
+        const long o = (long)(c0 + c) * N + i;
+        const double pv = p[o];
+        acc[c] += r[o] * pv, acc[4 + c] += pv * q[o];
+      }
+  }
+  __shared__ double part[4][8];
+  const double s = WaveSum8(acc);
+  if (threadIdx.x % 8 == 0) part[threadIdx.x / 64][threadIdx.x % 64 / 8] = s;
+  __syncthreads();
+  const int c = threadIdx.x % 4, w = threadIdx.x / 4;
+  if (w < 2 && c < kc) {
+    const double t = part[0][4 * w + c] + part[1][4 * w + c] + part[2][4 * w + c] + part[3][4 * w + c];
+    (w ? pq : rp)[(long)(c0 + c) * kDotBlocks + blockIdx.x] = t;
+  }
+}
+
+// The sum of n <= kDotBlocks block sums in block order, for each of the first two waves its own: the
+// values go to LDS in one round trip and one lane adds them.  (Added straight from memory, with one
+// thread per column, the 1024 values took 38 us for one sum and 95-168 us for two: a third of a 512^2
+// geodesic solve; from LDS 7-15 us.)  Every thread of the block calls it; the result is lane 0's of the sum's wave.
+static constexpr int kScalarThreads = 128;
+__device__ __forceinline__ double DotSum(const double* v, int n, double* lds) {
+#pragma unroll
+  for (int k = 0; k < kDotBlocks / 64; k++) {
+    const int i = (int)threadIdx.x % 64 + 64 * k;
+    lds[i] = i < n ? v[i] : 0.0;  // adding the zeros past n changes nothing (the sum is never -0)
+  }
+  __syncthreads();
   double t = 0.0;
-  for (int q = 0; q < n; q++) t += s[q];
+  if (threadIdx.x % 64 == 0) {
+#pragma unroll 32
+    for (int q = 0; q < (n + 31) / 32 * 32; q++) t += lds[q];
+  }
   return t;
 }
 
-// beta_c = (z, q_prev) / (p_prev, q_prev); zero on the first step of a solve (flag set by the host)
-__global__ void KFcgBeta(int K, int nb, const double* __restrict__ zq, const double* __restrict__ pqPrev, const int* __restrict__ first,
-                         double* beta) {
-  const int c = threadIdx.x;
-  if (c >= K) return;
-  beta[c] = (*first || !(pqPrev[c] > 0)) ? 0.0 : DotSum(zq + (long)c * kDotBlocks, nb) / pqPrev[c];
+// beta_c = (z, q_prev) / (p_prev, q_prev); zero on the first step of a solve (flag set by the host).
+// One wave per column.
+__global__ __launch_bounds__(64) void KFcgBeta(int nb, const double* __restrict__ zq, const double* __restrict__ pqPrev,
+                                               const int* __restrict__ first, double* beta) {
+  __shared__ double lds[kDotBlocks];
+  const int c = blockIdx.x;
+  const double s = DotSum(zq + (long)c * kDotBlocks, nb, lds);
+  if (threadIdx.x == 0) beta[c] = (*first || !(pqPrev[c] > 0)) ? 0.0 : s / pqPrev[c];
 }
 
-__global__ void KFcgDirection(long n, int N, const double* __restrict__ z, const double* __restrict__ beta, double* p) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const double bt = beta[t / N];
-  p[t] = bt == 0.0 ? z[t] : z[t] - bt * p[t];
-}
-
-// alpha_c = (r, p) / (p, q); keeps (p, q) for the next beta and clears the first-step flag
-__global__ void KFcgAlpha(int K, int nb, const double* __restrict__ rp, const double* __restrict__ pq, double* alpha, double* pqPrev,
-                          int* first) {
-  const int c = threadIdx.x;
-  if (c < K) {
-    const double d = DotSum(pq + (long)c * kDotBlocks, nb);
-    alpha[c] = d > 0 ? DotSum(rp + (long)c * kDotBlocks, nb) / d : 0.0;
-    pqPrev[c] = d;
+// p = z - beta p, a chunk of columns per thread (z from the FP32 correction, its dense index read once).
+template <int KC>
+__global__ __launch_bounds__(256) void KFcgDirection(int N, const int* __restrict__ g2d, const float* __restrict__ e0, long Nd,
+                                                     const double* __restrict__ beta, double* p, int K) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= N) return;
+  const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
+  const long di = g2d[i];
+  double z[KC], old[KC];
+#pragma unroll
+  for (int c = 0; c < KC; c++) {
+    if (c >= kc) continue;
+    z[c] = (double)e0[(long)(c0 + c) * Nd + di];
+    old[c] = beta[c0 + c] == 0.0 ? 0.0 : p[(long)(c0 + c) * N + i];
   }
-  if (c == 0) *first = 0;
+#pragma unroll
+  for (int c = 0; c < KC; c++) {
+    if (c >= kc) continue;
+    const double bt = beta[c0 + c];
+    p[(long)(c0 + c) * N + i] = bt == 0.0 ? z[c] : z[c] - bt * old[c];
+  }
 }
 
-// x += alpha p, r -= alpha q; the new residual into the FP32 correction rhs (e zeroed), its norms
+// alpha_c = (r, p) / (p, q); keeps (p, q) for the next beta, clears the first-step flag and the
+// column's norm slots (the update adds to them).  One block per column, a wave per dot product.
+__global__ __launch_bounds__(kScalarThreads) void KFcgAlpha(int nb, const double* __restrict__ rp, const double* __restrict__ pq, double* alpha,
+                                                            double* pqPrev, int* first, double* norms) {
+  __shared__ double lds[2][kDotBlocks], sum[2];
+  const int c = blockIdx.x, w = threadIdx.x / 64;
+  const double s = DotSum((w ? pq : rp) + (long)c * kDotBlocks, nb, lds[w]);
+  if (threadIdx.x % 64 == 0) sum[w] = s;
+  __syncthreads();
+  if (threadIdx.x < kSlots) norms[(long)c * kSlots + threadIdx.x] = 0.0;
+  if (threadIdx.x == 0) {
+    alpha[c] = sum[1] > 0 ? sum[0] / sum[1] : 0.0;
+    pqPrev[c] = sum[1];
+    if (c == 0) *first = 0;
+  }
+}
+
+// x += alpha p, r -= alpha q; the new residual into the FP32 correction rhs (e zeroed), its norms; a
+// chunk of columns per thread.  Every thread of a block reaches the block sums.
+template <int KC>
 __global__ __launch_bounds__(256) void KFcgUpdate(int N, const int* __restrict__ g2d, const double* __restrict__ alpha,
                                                   const double* __restrict__ p, const double* __restrict__ q, double* x, double* r,
-                                                  float* rhs0, float* e0, long Nd, double* norms) {
-  const int ch = blockIdx.y;
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  double a = 0.0;
+                                                  float* rhs0, float* e0, long Nd, double* norms, int K) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, c0 = blockIdx.y * KC, kc = min(KC, K - c0);
+  double sq[4] = {0, 0, 0, 0};
   if (i < N) {
-    const long o = (long)ch * N + i;
-    const double al = alpha[ch];
-    x[o] += al * p[o];
-    const double rv = r[o] - al * q[o];
-    r[o] = rv;
-    const long d = (long)ch * Nd + g2d[i];
-    rhs0[d] = (float)rv;
-    e0[d] = 0.0f;
-    a = rv * rv;
+    const long di = g2d[i];
+    double pv[KC], qv[KC], xv[KC], rv[KC];
+#pragma unroll
+    for (int c = 0; c < KC; c++) {
+      if (c >= kc) continue;
+      const long o = (long)(c0 + c) * N + i;
+      pv[c] = p[o], qv[c] = q[o], xv[c] = x[o], rv[c] = r[o];
+    }
+#pragma unroll
+    for (int c = 0; c < KC; c++) {
+      if (c >= kc) continue;
+      const long o = (long)(c0 + c) * N + i, dd = (long)(c0 + c) * Nd + di;
+      const double al = alpha[c0 + c], t = rv[c] - al * qv[c];
+      x[o] = xv[c] + al * pv[c];
+      r[o] = t;
+      rhs0[dd] = (float)t;
+      e0[dd] = 0.0f;
+      sq[c] = t * t;
+    }
   }
-  BlockAddSquares(a, norms + (long)ch * kSlots);
+  BlockAddSquares4(sq, kc, norms + (long)c0 * kSlots);
 }
 
 // The fused sweeps swap a level's two correction buffers.  Level 0's correction is consumed (x += e,
@@ -2416,18 +2525,19 @@ static void OuterResidual(DeviceSystem& ds, MixedSystem& ms, double* x, const do
 // One flexible-CG step after the V-cycle left z = V(r) in the level-0 FP32 correction:
 // beta = (z, q_prev)/(p_prev, q_prev), p = z - beta p, q = A p, alpha = (r, p)/(p, q),
 // x += alpha p, r -= alpha q (all scalars stay on the device).
-static void FcgStep(DeviceSystem& ds, MixedSystem& ms, double* x, int K, hipStream_t s) {
+static constexpr int kUpdateWideTexels = 1 << 21;
+template <int KC>
+static void FcgStepChunks(DeviceSystem& ds, MixedSystem& ms, double* x, int K, hipStream_t s) {
   DevLevel& L0 = ds.L[0];
   DevMixLevel& d = ms.L[0];
   const int N = d.N;
-  const long nk = (long)N * K;
   const size_t slab = (size_t)ms.kcap * kDotBlocks;
   double *zq = ms.dots, *rp = ms.dots + slab, *pq = ms.dots + 2 * slab;
-  const unsigned gb = std::min(NBlk(N, 256), (unsigned)kDotBlocks), cb = (unsigned)((K + 63) / 64 * 64);
-  KMixGather<<<NBlk(nk, 256), 256, 0, s>>>(N, d.g2d, d.e, d.Nd, ms.z64, K);
-  K64Dot<<<dim3(gb, K), 256, 0, s>>>(N, ms.z64, ms.q64, zq);
-  KFcgBeta<<<1, cb, 0, s>>>(K, (int)gb, zq, ms.pqPrev, ms.first, ms.beta);
-  KFcgDirection<<<NBlk(nk, 256), 256, 0, s>>>(nk, N, ms.z64, ms.beta, ms.p64);
+  const unsigned gb = std::min(NBlk(N, 256), (unsigned)kDotBlocks), chunks = (unsigned)((K + KC - 1) / KC);
+  const dim3 sums(gb, chunks), texels(NBlk(N, 256), chunks);
+  KFcgDotZq<KC><<<sums, 256, 0, s>>>(N, d.g2d, d.e, d.Nd, ms.q64, zq, K);
+  KFcgBeta<<<K, 64, 0, s>>>((int)gb, zq, ms.pqPrev, ms.first, ms.beta);
+  KFcgDirection<KC><<<texels, 256, 0, s>>>(N, d.g2d, d.e, d.Nd, ms.beta, ms.p64, K);
   const DevLevel &M = ds.mass0, &S = ds.stiff0;
   const int db = L0.nRaster > 0 ? (int)NBlk(L0.D, 256) : 0;
   const int bb = L0.B > 0 ? (int)NBlk((long)L0.B * kRowLanes64, 256) : 0;
@@ -2435,12 +2545,24 @@ static void FcgStep(DeviceSystem& ds, MixedSystem& ms, double* x, int K, hipStre
     K64ApplyW<<<db + bb, 256, 0, s>>>(db, L0.D, ms.deepLine, L0.raster, M.coefSym, S.coefSym, L0.B, L0.bgi, M.bd.rowptr, M.bd.col, M.bd.val,
                                       M.bb.rowptr, M.bb.col, M.bb.val, S.bd.rowptr, S.bd.col, S.bd.val, S.bb.rowptr, S.bb.col, S.bb.val,
                                       ms.p64, N, ms.q64, K, ms.weights);
-  K64Dot<<<dim3(gb, K), 256, 0, s>>>(N, ms.r64, ms.p64, rp);
-  K64Dot<<<dim3(gb, K), 256, 0, s>>>(N, ms.p64, ms.q64, pq);
-  KFcgAlpha<<<1, cb, 0, s>>>(K, (int)gb, rp, pq, ms.alpha, ms.pqPrev, ms.first);
-  KMixZeroD<<<NBlk((long)K * kSlots, 256), 256, 0, s>>>(K * kSlots, ms.norms);
-  HomeLevel0(ms);  // e was gathered above; the update zeroes the buffer the next step starts on
-  KFcgUpdate<<<dim3(NBlk(N, 256), K), 256, 0, s>>>(N, d.g2d, ms.alpha, ms.p64, ms.q64, x, ms.r64, d.rhs, d.e, d.Nd, ms.norms);
+  KFcgDots<KC><<<sums, 256, 0, s>>>(N, ms.r64, ms.p64, ms.q64, rp, pq, K);
+  KFcgAlpha<<<K, kScalarThreads, 0, s>>>((int)gb, rp, pq, ms.alpha, ms.pqPrev, ms.first, ms.norms);
+  HomeLevel0(ms);  // e was read above; the update zeroes the buffer the next step starts on
+  // eight streams a column: on large levels one column per thread keeps each stream's pages together
+  // (3.0 M texels, 64 columns: 2670 us a launch against 2950 with four; 0.75 M texels, 8 columns: 64 and 60)
+  if (N > kUpdateWideTexels)
+    KFcgUpdate<1><<<dim3(NBlk(N, 256), K), 256, 0, s>>>(N, d.g2d, ms.alpha, ms.p64, ms.q64, x, ms.r64, d.rhs, d.e, d.Nd, ms.norms, K);
+  else
+    KFcgUpdate<KC><<<texels, 256, 0, s>>>(N, d.g2d, ms.alpha, ms.p64, ms.q64, x, ms.r64, d.rhs, d.e, d.Nd, ms.norms, K);
+}
+
+static void FcgStep(DeviceSystem& ds, MixedSystem& ms, double* x, int K, hipStream_t s) {
+  switch (std::min(K, 4)) {
+    case 1: FcgStepChunks<1>(ds, ms, x, K, s); break;
+    case 2: FcgStepChunks<2>(ds, ms, x, K, s); break;
+    case 3: FcgStepChunks<3>(ds, ms, x, K, s); break;
+    default: FcgStepChunks<4>(ds, ms, x, K, s); break;
+  }
 }
 
 static void OuterUpdate(DeviceSystem& ds, MixedSystem& ms, double* x, int K, hipStream_t s) {
