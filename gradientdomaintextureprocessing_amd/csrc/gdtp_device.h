@@ -38,6 +38,12 @@ struct DevCsr {
   double* val = nullptr;
 };
 
+// One chart row of a band block: the texels its deep rows touch, base .. base + len - 1, and its pairs
+// of neighbouring deep texels.
+struct BandRow {
+  int base, len, pair0, pairs;
+};
+
 struct DevLevel {
   int N = 0, D = 0, B = 0;
   double* coef = nullptr;      // reciprocal (levels < L-1) deep stencil, SoA [10][D]
@@ -48,11 +54,11 @@ struct DevLevel {
   DevCsr bd, bb, brestr;       // A_BD, A_BB, boundary restriction to level+1
   // band tasks
   int nTasks = 0;
-  int *taskPtr = nullptr, *blockBegin = nullptr, *blockDeepEnd = nullptr, *blockPadEnd = nullptr;
-  int *blockStart = nullptr, *taskSteps = nullptr;  // pipeline schedule: first task step of each block, steps per task
-  int bandGroups = 1;                                // wave groups of the band launches (1 or kBandGroups)
-  int* lineElem = nullptr;                           // row elements of every band line (offsets)
-  int4* elems = nullptr;                             // (g, above, below, deep index or -d-1 at a segment start)
+  int* taskPtr = nullptr;
+  int* blockRow = nullptr;                           // first row of each block in bandRows
+  BandRow* bandRows = nullptr;
+  int4* pairs = nullptr;                             // (texel g, deep index, LDS places, 1: starts a segment | 2: g + 1 too)
+  long nPairs = 0;
   int nRaster = 0, nRestr = 0, nProl = 0;
   int *raster = nullptr, *restr = nullptr, *prol = nullptr;  // 5, 5, 6 ints per line
   DevLdlt factor;              // boundary factor (levels < L-1) or full coarse factor (level L-1)

@@ -3,6 +3,7 @@
 // Vectors are column-major: column c of a level-l vector starts at c*ld.  Deep stencils are
 // stored structure-of-arrays, [10][D], so every stencil slot is a coalesced stream.
 #include <algorithm>
+#include <climits>
 #include <stdexcept>
 
 #include "gdtp_device.h"
@@ -12,222 +13,196 @@
 namespace gdtp {
 
 static constexpr int kWave = 64;
+static constexpr int kBandColumns = 3;  // most columns of a band workgroup
 
 // ------------------------------------------------------------------ band Gauss-Seidel
 // The reference smoother (IterativeSolvers.inl:398-558 with residual, :174-395 without):
 // per band task, blocks left to right; inside a block, three lagged passes over the block's deep
-// rows (at step j rows j, j-1, j-2), each row a left-to-right Gauss-Seidel sweep of its deep
-// segments, and (pre-smoother) the true residual of padded row j-3.
-// The in-row dependence x_i = beta_i - c3_i x_{i-1} is a first-order linear recurrence, evaluated
-// with a wavefront-wide scan (two texels per lane, 128-texel rows).
+// rows (at step j rows j, j-1, j-2), each row a left-to-right Gauss-Seidel sweep of its deep segments.
+// The reference also computes a row's residual inside the sweep, from final values only; it equals
+// b - A x after the sweep, which is one streaming pass over the level (ResidualLevel).
+//
+// One workgroup per band task and chunk of KC columns.  The sweep is a chain: rows x passes of a block,
+// blocks one after another.  Within a block three waves run the passes as a pipeline, one row per wave
+// per step (step t: wave 0 row t first pass, wave 1 row t - 2 second, wave 2 row t - 4 third): each
+// operation sees exactly the values it sees in the reference's order, rows of one step are disjoint,
+// and a block of 16 rows takes 20 steps.  What bounds a launch is therefore the latency of a step, so
+// a step touches no memory but LDS on its chain: the rows' values live in a ring of eight LDS rows
+// (rows t - 5 .. t + 1 are read at step t, row t + 2 is filled meanwhile), a fourth wave streams the
+// rows in two steps ahead, a pass loads its next row's stencil and right-hand side as soon as the
+// current ones are used, and only the third pass stores.  The barrier of a step waits for LDS alone.
+// The in-row dependence x_i = beta_i - c3_i x_{i-1} is a first-order linear recurrence: two texels per
+// lane, then a wavefront scan by DPP moves.
+// (Measured, us per sweep of both colours, 4096^2 icosphere, three columns: level 0 739, level 1 274,
+// level 2 99; with x read and written through the L2, loads behind branches, the scan by LDS permutes
+// and the residual rows as a fourth pass 2690, 1015, 408 (3.5-6 us a step).  Tried: a load per line that
+// brings the next rows' stencils into the L2 ahead of the first pass (level 0 865 against 777 then), and
+// nine pass waves of one column each instead of three of three (level 0 1346, level 1 467: the stencil
+// loads of nine waves).  A lane's two neighbouring words as one 16-byte load: level 0 777 to 765.)
+constexpr int kBandRing = 8, kBandRowMax = 136;  // ring rows; texels of a row (132 at most), padded
 
-// Where one lane's texels of a row are: up to three elements (a pass takes elements 2 lane and
-// 2 lane + 1, for the scan; a residual row lane, lane + 64 and lane + 128), each with its global
-// index g, the rows above and below (p, n), its deep index d and whether it starts a segment.  The
-// host expands every band line into a table of such elements (BandTasks::elems), so that a wave
-// finds its elements with one load that waits on nothing, issued a step ahead (LoadRow); searching
-// the line's segments instead took three or four dependent memory round trips per step.
-struct RowLoc {
-  int g[3], p[3], n[3], d[3];
-  bool first[3];
-};
-
-// One left-to-right Gauss-Seidel sweep of a row (UpdateRow, IterativeSolvers.inl:448-470): the
-// in-row dependence x_i = beta_i - c3_i x_{i-1} as a wavefront scan over the lanes' element pairs,
-// columns in chunks of kKc (registers: the chunk's values and scan state).
-template <int kKc>
-__device__ __forceinline__ void GsRow(const RowLoc& L, const double* __restrict__ coef, int D, double* x, const double* __restrict__ b,
-                                      int K, int ld) {
-  const int lane = threadIdx.x % kWave;
-  double a[2] = {0, 0}, c[2][9];
-  for (int q = 0; q < 2; q++) {
-    if (L.g[q] >= 0) {
-      for (int k = 0; k < 9; k++) c[q][k] = coef[(size_t)k * D + L.d[q]];
-      a[q] = L.first[q] ? 0.0 : -c[q][3];
-    }
-  }
-  for (int c0 = 0; c0 < K; c0 += kKc) {
-    const int kc = min(kKc, K - c0);
-    double beta[2][kKc];
-    for (int q = 0; q < 2; q++)
-      for (int cc = 0; cc < kKc; cc++) {
-        beta[q][cc] = 0.0;
-        if (L.g[q] < 0 || cc >= kc) continue;
-        const double* X = x + (size_t)(c0 + cc) * ld;
-        const double* B = b + (size_t)(c0 + cc) * ld;
-        const int g = L.g[q], p = L.p[q], n = L.n[q];
-        double s = X[p - 1] * c[q][0] + X[p] * c[q][1] + X[p + 1] * c[q][2] + X[g + 1] * c[q][5] + X[n - 1] * c[q][6] + X[n] * c[q][7] +
-                   X[n + 1] * c[q][8];
-        double v = B[g] * c[q][4] - s;
-        if (L.first[q]) v -= X[g - 1] * c[q][3];
-        beta[q][cc] = v;
-      }
-    // lane-local composition of the two elements, then an inclusive wavefront scan
-    double A = a[1] * a[0];
-    double Bs[kKc];
-    for (int cc = 0; cc < kKc; cc++) Bs[cc] = a[1] * beta[0][cc] + beta[1][cc];
-    for (int o = 1; o < kWave; o <<= 1) {
-      double Au = __shfl_up(A, o, kWave);
-      double Bu[kKc];
-      for (int cc = 0; cc < kKc; cc++) Bu[cc] = __shfl_up(Bs[cc], o, kWave);
-      if (lane >= o) {
-        for (int cc = 0; cc < kKc; cc++) Bs[cc] = A * Bu[cc] + Bs[cc];
-        A = A * Au;
-      }
-    }
-    for (int cc = 0; cc < kKc; cc++) {
-      double prev = __shfl_up(Bs[cc], 1, kWave);
-      if (lane == 0) prev = 0.0;
-      double x0 = a[0] * prev + beta[0][cc];
-      double x1 = a[1] * x0 + beta[1][cc];
-      if (cc < kc) {
-        double* X = x + (size_t)(c0 + cc) * ld;
-        if (L.g[0] >= 0) X[L.g[0]] = x0;
-        if (L.g[1] >= 0) X[L.g[1]] = x1;
-      }
-    }
-  }
-}
-
-// The true residual of a padded row (UpdateResidual, IterativeSolvers.inl:473-495).
-__device__ __forceinline__ void ResRow(const RowLoc& L, const double* __restrict__ coef, int D, const double* x,
-                                       const double* __restrict__ b, double* r, int K, int ld) {
-  for (int q = 0; q < 3; q++) {
-    if (L.g[q] < 0) continue;
-    const int g = L.g[q], p = L.p[q], n = L.n[q];
-    double c[10];
-    for (int k = 0; k < 10; k++) c[k] = coef[(size_t)k * D + L.d[q]];
-    for (int cc = 0; cc < K; cc++) {
-      const double* X = x + (size_t)cc * ld;
-      double s = X[p - 1] * c[0] + X[p] * c[1] + X[p + 1] * c[2] + X[g - 1] * c[3] + X[g] + X[g + 1] * c[5] + X[n - 1] * c[6] +
-                 X[n] * c[7] + X[n + 1] * c[8];
-      r[(size_t)cc * ld + g] = b[(size_t)cc * ld + g] - s * c[9];
-    }
-  }
-}
-
-// One workgroup per band task.  Within a block the three lagged passes and the residual rows run as
-// a pipeline, one row per wave per step: at local step t wave 0 relaxes row t (first pass), wave 1
-// row t-2 (second pass), wave 2 row t-4 (third pass) and wave 3 computes the residual of padded row
-// t-6.  Each operation sees exactly the values it sees in the reference's order (step j: rows j,
-// j-1, j-2, then padded row j-3, IterativeSolvers.inl:497-509): a pass reads its row's neighbours
-// above after their own pass and below before it, which the two-step lag preserves, and a padded
-// row's residual reads deep rows up to one past its own index, final after their third pass (done
-// by step pr+5).  Rows of one step are disjoint.
-// With G = 1 the blocks of a task (left to right, overlapping by two columns,
-// IterativeSolvers.inl:511-515) run one after another.  With G = 3 they also overlap in time: three
-// groups of four waves take blocks in turn, block b running its local steps at task steps
-// blockStart[b] + t; the host schedule (BandSchedule) starts a block only once no chart row it
-// touches (reads or writes, rows and residuals, one row either side) is still touched by the block
-// before it, so every value is read and written in the reference's order.  G = 3 pays where a
-// launch has fewer tasks than CUs and several blocks per task; with more tasks, the 12-wave
-// workgroups (about 160 registers a lane) fit one per CU and the launch takes several rounds.
-struct BandBlock {  // one block's rows as the band kernel walks them
-  int r0 = 0, p0 = 0, nDeep = 0, nPad = 0, steps = 0;
-};
-__device__ __forceinline__ BandBlock LoadBlock(const int* __restrict__ blockBegin, const int* __restrict__ blockDeepEnd,
-                                               const int* __restrict__ blockPadEnd, int blk, int withResidual) {
-  BandBlock B;
-  B.r0 = blockBegin[blk], B.p0 = blockDeepEnd[blk];
-  B.nDeep = B.p0 - B.r0, B.nPad = blockPadEnd[blk] - B.p0;
-  B.steps = withResidual ? max(B.nDeep + 4, B.nPad + 6) : B.nDeep + 4;
-  return B;
-}
-// The line wave gw (0..3 in its group) works on at local step ls of block B, or -1; kind 1 pass, 2 residual.
-__device__ __forceinline__ int LineOfStep(const BandBlock& B, int gw, int ls, int withResidual, int& kind) {
-  kind = 0;
-  if (gw < 3) {
-    const int row = ls - 2 * gw;
-    if (row < 0 || row >= B.nDeep) return -1;
-    kind = 1;
-    return B.r0 + row;
-  }
-  const int pr = ls - 6;
-  if (!withResidual || pr < 0 || pr >= B.nPad) return -1;
-  kind = 2;
-  return B.p0 + pr;
-}
-// A lane's elements of a line from the row element table (no search, no load that waits on another):
-// a pass takes elements 2 lane and 2 lane + 1, a residual row lane, lane + 64 and lane + 128.
-__device__ __forceinline__ RowLoc LoadRow(const int4* __restrict__ elems, int o0, int o1, int kind) {
-  const int lane = threadIdx.x % kWave;
-  RowLoc L;
-#pragma unroll
-  for (int q = 0; q < 3; q++) {
-    const int e = kind == 1 ? 2 * lane + q : lane + kWave * q;
-    const bool in = kind != 0 && (kind == 2 || q < 2) && o0 + e < o1;
-    const int4 v = elems[in ? o0 + e : 0];  // unconditional (element 0 where not in), then selected: no branch
-    L.g[q] = in ? v.x : -1, L.p[q] = v.y, L.n[q] = v.z, L.d[q] = v.w >= 0 ? v.w : -v.w - 1, L.first[q] = v.w < 0;
-  }
-  return L;
-}
-// Where a group's blocks stand at a task step: the block it works on (or past the task's end) and
-// the task step that block starts at.  G = 1: the blocks one after another; G > 1: every G-th block
-// of the task, at the host schedule's blockStart.
-template <int G>
-struct BandCursor {
-  int blk, b1, start;
-  BandBlock B;
-  __device__ __forceinline__ void Init(int first, int last, const int* __restrict__ blockBegin, const int* __restrict__ blockDeepEnd,
-                                       const int* __restrict__ blockPadEnd, const int* __restrict__ blockStart, int withResidual) {
-    blk = first, b1 = last, start = 0;
-    if (blk < b1) {
-      B = LoadBlock(blockBegin, blockDeepEnd, blockPadEnd, blk, withResidual);
-      if (G > 1) start = blockStart[blk];
-    }
-  }
-  // move to task step st (non-decreasing); returns the line of wave gw there, or -1
-  __device__ __forceinline__ int At(int st, int gw, const int* __restrict__ blockBegin, const int* __restrict__ blockDeepEnd,
-                                    const int* __restrict__ blockPadEnd, const int* __restrict__ blockStart, int withResidual, int& kind) {
-    while (blk < b1 && st >= start + B.steps) {
-      const int end = start + B.steps;
-      blk += G;
-      if (blk < b1) B = LoadBlock(blockBegin, blockDeepEnd, blockPadEnd, blk, withResidual), start = G == 1 ? end : blockStart[blk];
-    }
-    kind = 0;
-    if (blk >= b1 || st < start) return -1;
-    return LineOfStep(B, gw, st - start, withResidual, kind);
-  }
-};
-template <int G, int KC>
-__global__ __launch_bounds__(G * 4 * kWave) void KBandGs(int color, int nTasks, const int* __restrict__ taskPtr,
-                                                         const int* __restrict__ blockBegin, const int* __restrict__ blockDeepEnd,
-                                                         const int* __restrict__ blockPadEnd, const int* __restrict__ lineElem,
-                                                         const int4* __restrict__ elems, const int* __restrict__ blockStart,
-                                                         const int* __restrict__ taskSteps, const double* __restrict__ coef, int D,
-                                                         double* x, const double* __restrict__ b, double* r, int K, int ld,
-                                                         int withResidual) {
-  const int t = 2 * blockIdx.x + color;
-  if (t >= nTasks) return;
-  const int wave = threadIdx.x / kWave, group = wave / 4, gw = wave % 4;
-  const int b0 = taskPtr[t], b1 = taskPtr[t + 1];
-  int total = 0;  // task steps
-  if constexpr (G == 1) {
-    for (int k = b0; k < b1; k++) total += LoadBlock(blockBegin, blockDeepEnd, blockPadEnd, k, withResidual).steps;
+// Wave-wide DPP move of a double; lanes without a source (and rows masked out) get `old`, or with kZero
+// zero (for unmasked moves: no initial value to set up).
+template <int kCtrl, int kRowMask = 0xf, bool kZero = false>
+__device__ __forceinline__ double DppMove(double v, double old) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v), o = __builtin_bit_cast(unsigned long long, old);
+  unsigned lo, hi;
+  if constexpr (kZero) {
+    lo = __builtin_amdgcn_mov_dpp((int)u, kCtrl, kRowMask, 0xf, true);
+    hi = __builtin_amdgcn_mov_dpp((int)(u >> 32), kCtrl, kRowMask, 0xf, true);
   } else {
-    total = taskSteps[t];
+    lo = __builtin_amdgcn_update_dpp((int)o, (int)u, kCtrl, kRowMask, 0xf, false);
+    hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(u >> 32), kCtrl, kRowMask, 0xf, false);
   }
-  // Two steps of lookahead per wave: the line of step st + 2 (its element range, scalar loads) and
-  // the elements of step st + 1 (vector loads) are fetched while step st computes, so a step waits
-  // only for its own stencil and x.
-  BandCursor<G> ahead;
-  ahead.Init(b0 + group, b1, blockBegin, blockDeepEnd, blockPadEnd, blockStart, withResidual);
-  int kind0, kind1;
-  const int l0 = ahead.At(0, gw, blockBegin, blockDeepEnd, blockPadEnd, blockStart, withResidual, kind0);
-  const int l1 = ahead.At(1, gw, blockBegin, blockDeepEnd, blockPadEnd, blockStart, withResidual, kind1);
-  RowLoc cur = LoadRow(elems, kind0 ? lineElem[l0] : 0, kind0 ? lineElem[l0 + 1] : 0, kind0);
-  int curKind = kind0, nextKind = kind1;
-  int n0 = kind1 ? lineElem[l1] : 0, n1 = kind1 ? lineElem[l1 + 1] : 0;
-  for (int st = 0; st < total; st++) {
-    int kind2;
-    const int l2 = ahead.At(st + 2, gw, blockBegin, blockDeepEnd, blockPadEnd, blockStart, withResidual, kind2);
-    const int m0 = kind2 ? lineElem[l2] : 0, m1 = kind2 ? lineElem[l2 + 1] : 0;
-    const RowLoc nxt = LoadRow(elems, n0, n1, nextKind);
-    if (curKind == 1) GsRow<KC>(cur, coef, D, x, b, K, ld);
-    else if (curKind == 2) ResRow(cur, coef, D, x, b, r, K, ld);
-    __syncthreads();
-    cur = nxt, curKind = nextKind;
-    nextKind = kind2, n0 = m0, n1 = m1;
+  return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+// One step of the inclusive scan of the maps x -> A x + B over the lanes (identity where no source).
+template <int kCtrl, int kRowMask, int KC>
+__device__ __forceinline__ void ScanStep(double& A, double (&B)[KC]) {
+  const double Au = DppMove<kCtrl, kRowMask>(A, 1.0);
+#pragma unroll
+  for (int c = 0; c < KC; c++) B[c] += A * DppMove<kCtrl, kRowMask, kRowMask == 0xf>(B[c], 0.0);
+  A *= Au;
+}
+
+// Two neighbouring doubles of a lane in one load (a pair starts at any texel: 8-byte alignment).
+struct __attribute__((packed, aligned(8))) Double2 {
+  double a, b;
+};
+__device__ __forceinline__ void LoadPair(const double* p, double& a, double& b) {
+  const Double2 v = *reinterpret_cast<const Double2*>(p);
+  a = v.a, b = v.b;
+}
+
+// All waves' LDS accesses before this point are done; global loads and stores stay in flight.
+__device__ __forceinline__ void LdsBarrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <int KC>
+__global__ __launch_bounds__(256) void KBandGs(int color, int nTasks, const int* __restrict__ taskPtr, const int* __restrict__ blockRow,
+                                               const BandRow* __restrict__ rows, const int4* __restrict__ pairs,
+                                               const double* __restrict__ coef, int D, double* x, const double* __restrict__ b, int K, int ld) {
+  __shared__ double S[KC][kBandRing][kBandRowMax];
+  const int task = 2 * blockIdx.x + color;
+  if (task >= nTasks) return;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  // column of each slot of the chunk; the last chunk's slots past K repeat column K - 1 (same values)
+  size_t col[KC];
+#pragma unroll
+  for (int c = 0; c < KC; c++) col[c] = (size_t)min((int)blockIdx.y * KC + c, K - 1) * ld;
+  for (int blk = taskPtr[task]; blk < taskPtr[task + 1]; blk++) {
+    // rows R[0 .. nr + 1]: the chart rows of the block's deep rows 1 .. nr and one row either side
+    const BandRow* R = rows + blockRow[blk];
+    const int nr = blockRow[blk + 1] - blockRow[blk] - 2, steps = nr + 4;
+    __syncthreads();  // the block before this one has stored its rows
+    if (wave == 3) {
+      constexpr int kLoads = (KC * kBandRowMax + kWave - 1) / kWave;
+      const double* from[kLoads];  // a lane's columns and places in a row, the same for every row
+      double* to[kLoads];
+      int at[kLoads];
+#pragma unroll
+      for (int k = 0; k < kLoads; k++) {
+        const int e = min(lane + kWave * k, KC * kBandRowMax - 1), c = e / kBandRowMax;
+        at[k] = e % kBandRowMax, to[k] = &S[c][0][at[k]];
+        from[k] = x + (c == 0 ? col[0] : c == 1 ? col[KC > 1 ? 1 : 0] : col[KC - 1]);
+      }
+      // (a row's places past its texels repeat the last one; their values are not used)
+      auto load = [&](int r, double (&v)[kLoads]) {
+        const BandRow W = R[min(r, nr + 1)];
+#pragma unroll
+        for (int k = 0; k < kLoads; k++) v[k] = from[k][W.base + min(at[k], max(W.len - 1, 0))];
+      };
+      auto put = [&](int r, const double (&v)[kLoads]) {
+#pragma unroll
+        for (int k = 0; k < kLoads; k++) to[k][(r % kBandRing) * kBandRowMax] = v[k];
+      };
+      double v0[kLoads], v1[kLoads], v2[kLoads];
+      load(0, v0), load(1, v1), load(2, v2);
+      put(0, v0), put(1, v1), put(2, v2);
+      load(3, v0), load(4, v1);
+      LdsBarrier();
+      for (int t = 0; t < steps; t += 2) {
+        put(t + 3, v0);
+        load(t + 5, v0);
+        LdsBarrier();
+        if (t + 1 == steps) break;
+        put(t + 4, v1);
+        load(t + 6, v1);
+        LdsBarrier();
+      }
+      continue;
+    }
+    // pair of this lane in row r: texels g, g + 1 with stencils d, d + 1 (first: g starts a segment;
+    // two: both are deep) and the LDS places of g, of the texel above g - 1 and of the one below g - 1
+    auto pairOf = [&](const BandRow& W) { return pairs[lane < W.pairs ? W.pair0 + lane : 0]; };
+    double c0[9], c1[9], b0[KC], b1[KC];
+    auto operands = [&](const int4& P) {
+#pragma unroll
+      for (int k = 0; k < 9; k++) LoadPair(coef + (size_t)k * D + P.y, c0[k], c1[k]);
+#pragma unroll
+      for (int c = 0; c < KC; c++) LoadPair(b + col[c] + P.x, b0[c], b1[c]);
+    };
+    int n0 = R[1].pairs;
+    int4 P0 = pairOf(R[1]);
+    operands(P0);
+    BandRow W1 = R[min(2, nr + 1)];
+    int4 P1 = pairOf(W1);
+    LdsBarrier();
+    for (int t = 0; t < steps; t++) {
+      const int r = t + 1 - 2 * wave;
+      if (r >= 1 && r <= nr) {
+        const BandRow W2 = R[min(r + 2, nr + 1)];
+        const int4 P2 = pairOf(W2);
+        const bool first = P0.w & 1, two = P0.w & 2, active = lane < n0;
+        const int og = P0.z & 255, oa = (P0.z >> 8) & 255, ob = (P0.z >> 16) & 255;
+        const double a0 = first ? 0.0 : -c0[3], a1 = two ? -c1[3] : 0.0;
+        double beta0[KC], beta1[KC];
+#pragma unroll
+        for (int c = 0; c < KC; c++) {
+          double* own = &S[c][r % kBandRing][og];
+          const double* up = &S[c][(r - 1) % kBandRing][oa];
+          const double* dn = &S[c][(r + 1) % kBandRing][ob];
+          const double u0 = up[0], u1 = up[1], u2 = up[2], u3 = up[3], w0 = dn[0], w1 = dn[1], w2 = dn[2], w3 = dn[3];
+          const double left = own[-1], right = own[1], far = own[2];
+          const double s0 = u0 * c0[0] + u1 * c0[1] + u2 * c0[2] + right * c0[5] + w0 * c0[6] + w1 * c0[7] + w2 * c0[8];
+          const double s1 = u1 * c1[0] + u2 * c1[1] + u3 * c1[2] + far * c1[5] + w1 * c1[6] + w2 * c1[7] + w3 * c1[8];
+          double v = b0[c] * c0[4] - s0;
+          if (first) v -= left * c0[3];
+          beta0[c] = v;
+          beta1[c] = two ? b1[c] * c1[4] - s1 : 0.0;
+        }
+        operands(P1);  // the next row's, in flight until the next step
+        // the lane's two texels as one map, then an inclusive scan over the wave
+        double A = a1 * a0, B[KC];
+#pragma unroll
+        for (int c = 0; c < KC; c++) B[c] = a1 * beta0[c] + beta1[c];
+        ScanStep<0x111, 0xf, KC>(A, B);  // row_shr:1, 2, 4, 8 within 16 lanes
+        ScanStep<0x112, 0xf, KC>(A, B);
+        ScanStep<0x114, 0xf, KC>(A, B);
+        ScanStep<0x118, 0xf, KC>(A, B);
+        ScanStep<0x142, 0xa, KC>(A, B);  // row_bcast:15 into rows 1 and 3
+        ScanStep<0x143, 0xc, KC>(A, B);  // row_bcast:31 into rows 2 and 3
+#pragma unroll
+        for (int c = 0; c < KC; c++) {
+          const double prev = DppMove<0x138, 0xf, true>(B[c], 0.0);  // wave_shr:1
+          const double x0 = a0 * prev + beta0[c], x1 = a1 * x0 + beta1[c];
+          if (active) {
+            double* own = &S[c][r % kBandRing][og];
+            own[0] = x0;
+            if (two) own[1] = x1;
+            if (wave == 2) {
+              x[col[c] + P0.x] = x0;
+              if (two) x[col[c] + P0.x + 1] = x1;
+            }
+          }
+        }
+        P0 = P1, P1 = P2, n0 = W1.pairs, W1 = W2;
+      }
+      LdsBarrier();
+    }
   }
 }
 
@@ -601,17 +576,43 @@ static T* UploadTo(std::vector<void*>& allocs, const std::vector<T>& v) {
   return p;
 }
 
-// Wave groups of a level's band launches: kBandGroups (blocks of a task overlapped in time) where a
-// launch has no more tasks than the device has CUs (its 12-wave workgroups then run in one round)
-// and the tasks have two or more blocks on average (else there is little to overlap); else 1.
-// (C2 4096^2: levels 0 and 1 have 640 and 320 tasks per launch, level 2 160 tasks of 2.2 blocks.)
-static int BandGroups(const BandTasks& T) {
-  const int nt = (int)T.taskPtr.size() - 1;
-  if (nt <= 0) return 1;
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 1;
-  const double blocksPerTask = double(T.blockBegin.size()) / nt;
-  return (nt + 1) / 2 <= cus && blocksPerTask >= 2.0 ? kBandGroups : 1;
+// The band kernel's tables: for every block the chart rows its deep rows touch (a row without deep
+// texels between two deep ones is a row without pairs), and each row's deep texels in pairs of
+// neighbours (a segment of odd length ends in a pair of one).  Segments of a row are at least one texel
+// apart, so 128 columns hold at most 64 pairs.
+static void BandTables(const BandTasks& T, std::vector<int>& blockRow, std::vector<BandRow>& rows, std::vector<int4>& pairs) {
+  blockRow.assign(1, 0), rows.clear(), pairs.clear();
+  const int nb = (int)T.blockBegin.size();
+  for (int k = 0; k < nb; k++) {
+    const int l0 = T.blockBegin[k], l1 = T.blockDeepEnd[k], y0 = l0 < l1 ? T.lineRow[l0] : 0;
+    const int nr = l0 < l1 ? T.lineRow[l1 - 1] - y0 + 1 : 0;
+    std::vector<int> lo(nr + 2, INT_MAX), hi(nr + 2, -1), line(nr + 2, -1);
+    auto touch = [&](int r, int g) { lo[r] = std::min(lo[r], g - 1), hi[r] = std::max(hi[r], g + 1); };
+    for (int l = l0; l < l1; l++) {
+      const int r = T.lineRow[l] - y0 + 1;
+      if (r < 1 || r > nr || line[r] >= 0) throw std::runtime_error("band block rows out of order");
+      line[r] = l;
+      for (int e = T.lineElem[l]; e < T.lineElem[l + 1]; e++) {
+        const int* E = &T.elems[4 * (size_t)e];
+        touch(r, E[0]), touch(r - 1, E[1]), touch(r + 1, E[2]);
+      }
+    }
+    for (int r = 0; r < nr + 2; r++) {
+      BandRow W{hi[r] < 0 ? 0 : lo[r], hi[r] < 0 ? 0 : hi[r] - lo[r] + 1, (int)pairs.size(), 0};
+      if (line[r] >= 0)
+        for (int e = T.lineElem[line[r]], end = T.lineElem[line[r] + 1]; e < end;) {
+          const int* E = &T.elems[4 * (size_t)e];
+          const bool first = E[3] < 0, two = e + 1 < end && E[7] >= 0;
+          pairs.push_back(make_int4(E[0], first ? -E[3] - 1 : E[3], (E[0] - lo[r]) | (E[1] - 1 - lo[r - 1]) << 8 | (E[2] - 1 - lo[r + 1]) << 16,
+                                    (first ? 1 : 0) | (two ? 2 : 0)));
+          W.pairs++, e += two ? 2 : 1;
+        }
+      // two more texels than a row holds are read (and not used) past a pair of one
+      if (W.len + 2 > kBandRowMax || W.pairs > kWave) throw std::runtime_error("band row wider than its block");
+      rows.push_back(W);
+    }
+    blockRow.push_back((int)rows.size());
+  }
 }
 
 template <class T>
@@ -718,14 +719,14 @@ void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOpe
     if (l + 1 < nl) d.brestr = UploadCsr(ds, H.boundaryRestriction);
     d.nTasks = (int)H.tasks.taskPtr.size() - 1;
     d.taskPtr = Upload(ds, H.tasks.taskPtr);
-    d.blockBegin = Upload(ds, H.tasks.blockBegin);
-    d.blockDeepEnd = Upload(ds, H.tasks.blockDeepEnd);
-    d.blockPadEnd = Upload(ds, H.tasks.blockPadEnd);
-    d.blockStart = Upload(ds, H.tasks.blockStart);
-    d.taskSteps = Upload(ds, H.tasks.taskSteps);
-    d.bandGroups = BandGroups(H.tasks);
-    d.lineElem = Upload(ds, H.tasks.lineElem);
-    d.elems = reinterpret_cast<int4*>(Upload(ds, H.tasks.elems));
+    {
+      std::vector<int> blockRow;
+      std::vector<BandRow> rows;
+      std::vector<int4> pairs;
+      BandTables(H.tasks, blockRow, rows, pairs);
+      d.blockRow = Upload(ds, blockRow), d.bandRows = Upload(ds, rows);
+      d.pairs = Upload(ds, pairs), d.nPairs = (long)pairs.size();
+    }
     std::vector<int> rl;
     for (auto& x : H.rasterLines) rl.insert(rl.end(), {x.start, x.end, x.prev, x.next, x.coeff});
     d.nRaster = (int)H.rasterLines.size();
@@ -825,34 +826,34 @@ void CoarseSolve(DeviceSystem& ds, const double* rhs, double* sol, int K, int ld
   LdltSolve(d.factor, rhs, ld, sol, ld, nullptr, d.y, K, s);
 }
 
+// The band sweep of a level's deep rows, columns in chunks of up to kBandColumns, every chunk a workgroup
+// of its own (columns are independent).  A step's latency grows with its columns (0.5 us with one, 1.0
+// with three) and each chunk reads the stencil again, so a launch takes one column per workgroup as long
+// as it then has at most two workgroups per CU (us per sweep, one / three columns per workgroup, K = 3:
+// 30 tasks a launch 59 / 102, 160 tasks 99 / 158, 320 tasks 346 / 274).
+static constexpr long kBandSplit = 512;
+static void BandSweep(DevLevel& d, double* x, const double* b, int K, int ld, hipStream_t s) {
+  if (d.nTasks == 0 || d.nPairs == 0) return;
+  const int chunks = (K + kBandColumns - 1) / kBandColumns;
+  const int kc = (d.nTasks + 1) / 2 * (long)K <= kBandSplit ? 1 : (K + chunks - 1) / chunks;
+  for (int color = 0; color < 2; color++) {
+    const int tasks = color == 0 ? (d.nTasks + 1) / 2 : d.nTasks / 2;
+    if (tasks == 0) continue;
+    const dim3 grid(tasks, (K + kc - 1) / kc);
+    const auto kernel = kc == 1 ? KBandGs<1> : kc == 2 ? KBandGs<2> : KBandGs<3>;
+    kernel<<<grid, 256, 0, s>>>(color, d.nTasks, d.taskPtr, d.blockRow, d.bandRows, d.pairs, d.coef, d.D, x, b, K, ld);
+  }
+}
+
+// Deep rows of y = A x, or with `b` of b - A x.
+static void DeepRows(DevLevel& d, const double* x, const double* b, double* y, int K, int ld, hipStream_t s) {
+  if (d.nRaster > 0) KApplyDeep<<<d.nRaster, 128, 0, s>>>(d.nRaster, d.raster, d.coefRaw, d.D, x, b, y, K, ld);
+}
+
 void BandSweepLevel(DeviceSystem& ds, int l, double* x, const double* b, double* r, int K, int ld, hipStream_t s) {
   CheckK(ds, K);
-  DevLevel& d = ds.L[l];
-  if (d.nTasks == 0) return;
-  const int withResidual = r != nullptr ? 1 : 0;
-#define GDTP_BAND(G, KC)                                                                                                       \
-  KBandGs<G, KC><<<blocks, G * 4 * kWave, 0, s>>>(color, d.nTasks, d.taskPtr, d.blockBegin, d.blockDeepEnd, d.blockPadEnd,  \
-                                                  d.lineElem, d.elems, d.blockStart, d.taskSteps, d.coef, d.D, x, b, r, K, ld,     \
-                                                  withResidual)
-  // column chunks of K up to three, else of two (a chunk of four needs 168-179 registers a lane:
-  // occupancy 2 or spills)
-#define GDTP_BAND_KC(G)             \
-  switch (K >= 4 ? 2 : K) {         \
-    case 1: GDTP_BAND(G, 1); break; \
-    case 2: GDTP_BAND(G, 2); break; \
-    default: GDTP_BAND(G, 3); break; \
-  }
-  for (int color = 0; color < 2; color++) {
-    const int blocks = color == 0 ? (d.nTasks + 1) / 2 : d.nTasks / 2;
-    if (blocks == 0) continue;
-    if (d.bandGroups == kBandGroups) {
-      GDTP_BAND_KC(kBandGroups)
-    } else {
-      GDTP_BAND_KC(1)
-    }
-  }
-#undef GDTP_BAND_KC
-#undef GDTP_BAND
+  BandSweep(ds.L[l], x, b, K, ld, s);
+  if (r) DeepRows(ds.L[l], x, b, r, K, ld, s);
 }
 
 void RelaxLevel(DeviceSystem& ds, int l, double* x, const double* b, double* r, int K, int ld, bool withResidual, hipStream_t s) {
@@ -863,12 +864,8 @@ void RelaxLevel(DeviceSystem& ds, int l, double* x, const double* b, double* r, 
     KBoundaryRhs<<<Blocks(bk, 256), 256, 0, s>>>(d.B, d.bgi, d.bd.rowptr, d.bd.col, d.bd.val, x, b, d.vb, K, ld);
     LdltSolve(d.factor, d.vb, d.B, x, ld, d.bgi, d.y, K, s);
   }
-  BandSweepLevel(ds, l, x, b, withResidual ? r : nullptr, K, ld, s);
-  if (withResidual && d.B > 0) {
-    const long bk = (long)d.B * K;
-    KBoundaryResidual<<<Blocks(bk, 256), 256, 0, s>>>(d.B, d.bgi, d.bd.rowptr, d.bd.col, d.bd.val, d.bb.rowptr, d.bb.col, d.bb.val, x, b, r,
-                                                       K, ld, ld);
-  }
+  BandSweep(d, x, b, K, ld, s);
+  if (withResidual) ResidualLevel(ds, l, x, b, r, K, ld, s);
 }
 
 void RestrictLevel(DeviceSystem& ds, int l, const double* rF, double* bC, int K, int ldF, int ldC, hipStream_t s) {

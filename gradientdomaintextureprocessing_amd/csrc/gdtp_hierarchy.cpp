@@ -576,7 +576,7 @@ int BuildHierarchy(const TexturedMesh& mesh, int W, int H, int numLevels, const 
   return 1;
 }
 
-// Pipeline schedule of the band tasks (the GPU band kernel): block b of a task runs its local steps
+// Overlapped schedule of the band tasks: block b of a task runs its local steps
 // t = 0 .. max(nDeep + 4, nPad + 6) - 1 at task steps blockStart[b] + t.  At local step t it touches (reads
 // or writes) chart rows Y - 1 .. Y + 1 of deep row i = t - 2w (passes w = 0, 1, 2) and of padded row
 // t - 6 (residual).  A block starts once every row it shares with the block before it is touched

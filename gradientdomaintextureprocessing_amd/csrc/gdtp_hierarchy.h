@@ -79,23 +79,24 @@ struct ProlongationLine { int start, length, center, prev, next, aligned; };
 // Flattened band tasks: task t owns blocks [taskPtr[t], taskPtr[t+1]); block b owns deep rows
 // [lineBegin[b], deepEnd[b]) then padded rows [deepEnd[b], padEnd[b]); row r owns segments
 // [linePtr[r], linePtr[r+1]).
-// Wave groups of the GPU band kernel: blocks of one band task in flight at once.
+// Blocks of one band task in flight at once in the overlapped schedule (BandSchedule).
 constexpr int kBandGroups = 3;
 
 struct BandTasks {
   std::vector<int> taskPtr{0}, blockBegin, blockDeepEnd, blockPadEnd, linePtr{0};
   std::vector<Segment> segments;
   std::vector<int> lineRow;    // chart grid row of every line (deep and padded)
-  std::vector<int> blockStart; // GPU pipeline: first task step of every block (BandSchedule)
-  std::vector<int> taskSteps;  // GPU pipeline: task steps of every task
-  // GPU row elements: line l's elements (its segments' texels in order) are lineElem[l] ..
+  std::vector<int> blockStart; // overlapped schedule: first task step of every block (BandSchedule)
+  std::vector<int> taskSteps;  // overlapped schedule: task steps of every task
+  // row elements: line l's elements (its segments' texels in order) are lineElem[l] ..
   // lineElem[l + 1] - 1, element e stored as 4 ints (global index, index above, index below, deep
   // index d; -d - 1 where the element starts a segment)
   std::vector<int> lineElem, elems;
 };
 
-// The GPU band kernel's pipeline schedule and row element table of T (fills blockStart, taskSteps,
-// lineElem and elems).
+// The row element table of T (the GPU band kernel's tables are built from it) and a schedule that
+// overlaps the blocks of a task in time without changing any access's order (exported; the GPU kernel,
+// whose steps are short, runs them one after another).  Fills lineElem, elems, blockStart, taskSteps.
 void BandSchedule(BandTasks& T);
 
 struct Level {
