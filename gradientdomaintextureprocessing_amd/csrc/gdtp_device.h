@@ -52,6 +52,8 @@ struct DevLevel {
                                // indices (slots 0-3: lower neighbours k = 0..3, slot 4: diagonal)
   int* bgi = nullptr;          // boundary -> global
   DevCsr bd, bb, brestr;       // A_BD, A_BB, boundary restriction to level+1
+  DevCsr rows;                 // A_BB's and (from rowMid on) A_BD's entries row by row, global columns
+  int* rowMid = nullptr;
   // band tasks
   int nTasks = 0;
   int* taskPtr = nullptr;

@@ -220,23 +220,6 @@ __global__ void KBoundaryRhs(int B, const int* __restrict__ bgi, const int* __re
   vb[(size_t)c * B + i] = b[(size_t)c * ld + bgi[i]] - s;
 }
 
-// r_B = b_B - A_BD x - A_BB x_B   (IterativeSolvers.inl:549-555)
-__global__ void KBoundaryResidual(int B, const int* __restrict__ bgi, const int* __restrict__ rpd, const int* __restrict__ cold,
-                                  const double* __restrict__ vald, const int* __restrict__ rpb, const int* __restrict__ colb,
-                                  const double* __restrict__ valb, const double* __restrict__ x, const double* __restrict__ b, double* r,
-                                  int K, int ld, int ldr) {
-  long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)B * K) return;
-  int i = idx % B, c = idx / B;
-  const double* X = x + (size_t)c * ld;
-  double s = 0;
-  for (int k = rpd[i]; k < rpd[i + 1]; k++) s += X[cold[k]] * vald[k];
-  double v = b[(size_t)c * ld + bgi[i]] - s;
-  double t = 0;
-  for (int k = rpb[i]; k < rpb[i + 1]; k++) t += X[bgi[colb[k]]] * valb[k];
-  r[(size_t)c * ldr + bgi[i]] = v - t;
-}
-
 // ------------------------------------------------------------------ exact LDL^T solves
 // The staged triangular solves (LdltStages): forward stages r = src[perm] - L y(earlier stages),
 // y = inv(L_cc) r per component, then backward r = y / D - L^T x(later stages), x = inv(L_cc)^T r.
@@ -391,34 +374,96 @@ __global__ __launch_bounds__(256) void KLdltWide(int row0, int row1, int wideBeg
 }
 
 // ------------------------------------------------------------------ transfers
-// coarse boundary rhs = R_B r   (IterativeSolvers.inl:1027-1030)
-__global__ void KCsrGatherScatter(int rows, const int* __restrict__ outMap, const int* __restrict__ rp, const int* __restrict__ cl,
-                                  const double* __restrict__ vl, const double* __restrict__ in, int ldi, double* out, int ldo, int K) {
-  long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)rows * K) return;
-  int i = idx % rows, c = idx / rows;
-  const double* X = in + (size_t)c * ldi;
-  double s = 0;
-  for (int k = rp[i]; k < rp[i + 1]; k++) s += X[cl[k]] * vl[k];
-  out[(size_t)c * ldo + outMap[i]] = s;
+// Sparse rows (boundary rows of an operator, of the restriction): kRowLanes lanes per row, so that a
+// row's entries are read together instead of one round trip after another.
+static constexpr int kRowLanes = 8;
+static constexpr int kRowBatch = 4 * kRowLanes;  // entries staged at a time
+static constexpr int kRowThreads = 128;          // threads of the kernels that take sparse rows and lines
+template <int KC, int kThreads>
+struct RowTerms {
+  double v[kThreads / kRowLanes][KC][kRowBatch + 1];
+};
+
+// Sum over entries [k0, mid) plus sum over [mid, k1) of val x[col] for column (lane of the row's group),
+// up to KC columns (lane < kc).  Seam rows cancel, so the order of the additions is kept: the lanes
+// stage an entry's terms in LDS, and lane c adds column c's in the row's order.
+template <int KC, int kThreads>
+__device__ __forceinline__ double RowSum(int k0, int mid, int k1, const int* __restrict__ cl, const double* __restrict__ vl,
+                                         const double* __restrict__ x, size_t ld, int kc, RowTerms<KC, kThreads>& terms) {
+  double(&T)[KC][kRowBatch + 1] = terms.v[threadIdx.x / kRowLanes];
+  const int lane = threadIdx.x % kRowLanes;
+  double first = 0.0, second = 0.0;
+  for (int at = k0; at < k1; at += kRowBatch) {
+    double v[kRowBatch / kRowLanes], xv[kRowBatch / kRowLanes][KC];
+#pragma unroll
+    for (int q = 0; q < kRowBatch / kRowLanes; q++) {
+      const int k = min(at + lane + kRowLanes * q, k1 - 1);
+      const int g = cl[k];
+      v[q] = vl[k];
+#pragma unroll
+      for (int c = 0; c < KC; c++) xv[q][c] = x[(size_t)min(c, kc - 1) * ld + g];
+    }
+#pragma unroll
+    for (int q = 0; q < kRowBatch / kRowLanes; q++)
+#pragma unroll
+      for (int c = 0; c < KC; c++) T[c][lane + kRowLanes * q] = v[q] * xv[q][c];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the group's lanes are of one wave
+    if (lane < kc) {
+      const int n = min(kRowBatch, k1 - at), m = min(max(mid - at, 0), n);
+      const double* t = T[lane];
+#pragma unroll 8
+      for (int k = 0; k < m; k++) first += t[k];
+#pragma unroll 8
+      for (int k = m; k < n; k++) second += t[k];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  return first + second;
 }
 
-// coarse deep rhs: 3x3 full weighting around the fine texel 2c (IterativeSolvers.inl:1034-1050)
-__global__ void KRestrictDeep(int nLines, const int* __restrict__ lines, const double* __restrict__ in, int ldi, double* out, int ldo, int K) {
-  const int l = blockIdx.x;
-  if (l >= nLines) return;
-  const int* L = lines + 5 * l;
+// Restriction into the next level in one launch (blockIdx.y = chunk of KC columns): blocks [0, rowBlocks)
+// take the coarse boundary rows (R_B r, IterativeSolvers.inl:1027-1030), the others one restriction line
+// each, coarse deep texels by 3x3 full weighting around the fine texel 2c (:1034-1050).  With `zero` the
+// coarse vector there is set to zero as well (the coarse correction of a V-cycle starts from zero).
+template <int KC>
+__global__ __launch_bounds__(kRowThreads) void KRestrict(int rowBlocks, int rows, const int* __restrict__ outMap, const int* __restrict__ rp,
+                                                         const int* __restrict__ cl, const double* __restrict__ vl, int nLines,
+                                                         const int* __restrict__ lines, const double* __restrict__ in, int ldi, double* out,
+                                                         double* zero, int ldo, int K) {
+  const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
+  in += (size_t)c0 * ldi, out += (size_t)c0 * ldo;
+  if (zero) zero += (size_t)c0 * ldo;
+  if ((int)blockIdx.x < rowBlocks) {
+    __shared__ RowTerms<KC, kRowThreads> terms;
+    const int row = (blockIdx.x * kRowThreads + (int)threadIdx.x) / kRowLanes, c = threadIdx.x % kRowLanes;
+    if (row >= rows) return;  // whole row groups leave together
+    const double s = RowSum(rp[row], rp[row + 1], rp[row + 1], cl, vl, in, ldi, kc, terms);
+    if (c < kc) {
+      const size_t o = (size_t)c * ldo + outMap[row];
+      out[o] = s;
+      if (zero) zero[o] = 0.0;
+    }
+    return;
+  }
+  const int* L = lines + 5 * (blockIdx.x - rowBlocks);
   const int start = L[0], end = L[1], prev = L[2], next = L[3], outStart = L[4];
   const int len = (end - start) / 2 + 1;
-  for (int i = threadIdx.x; i < len; i += blockDim.x) {
+  for (int i = threadIdx.x; i < len; i += kRowThreads) {
     const int j = 2 * i;
-    for (int c = 0; c < K; c++) {
-      const double* cu = in + (size_t)c * ldi + start;
-      const double* pv = in + (size_t)c * ldi + prev;
-      const double* nx = in + (size_t)c * ldi + next;
-      out[(size_t)c * ldo + outStart + i] = cu[j] + (pv[j] + cu[j - 1] + cu[j + 1] + nx[j]) * 0.5 +
-                                            (pv[j - 1] + pv[j + 1] + nx[j - 1] + nx[j + 1]) * 0.25;
+    double v[KC][9];
+#pragma unroll
+    for (int c = 0; c < KC; c++) {
+      const double* X = in + (size_t)min(c, kc - 1) * ldi;
+#pragma unroll
+      for (int k = 0; k < 9; k++) v[c][k] = X[(k < 3 ? prev : k < 6 ? start : next) + j + k % 3 - 1];
     }
+#pragma unroll
+    for (int c = 0; c < KC; c++)
+      if (c < kc) {
+        const double* R = v[c];
+        out[(size_t)c * ldo + outStart + i] = R[4] + (R[1] + R[3] + R[5] + R[7]) * 0.5 + (R[0] + R[2] + R[6] + R[8]) * 0.25;
+        if (zero) zero[(size_t)c * ldo + outStart + i] = 0.0;
+      }
   }
 }
 
@@ -439,40 +484,53 @@ __global__ void KProlongAdd(int nLines, const int* __restrict__ lines, const dou
 }
 
 // ------------------------------------------------------------------ operator application
-// Deep rows of y = A x with raw stencils (MultiplyBySystemMatrix_NoReciprocals, IterativeSolvers.inl:881-950);
-// with `b` given, writes the residual b - A x instead.
-__global__ void KApplyDeep(int nLines, const int* __restrict__ lines, const double* __restrict__ coef, int D, const double* __restrict__ x,
-                           const double* __restrict__ b, double* y, int K, int ld) {
-  const int l = blockIdx.x;
-  if (l >= nLines) return;
-  const int* L = lines + 5 * l;
-  const int start = L[0], len = L[1] - L[0] + 1, prev = L[2], next = L[3], d0 = L[4];
-  for (int i = threadIdx.x; i < len; i += blockDim.x) {
-    double c[9];
-    for (int k = 0; k < 9; k++) c[k] = coef[(size_t)k * D + d0 + i];
-    for (int cc = 0; cc < K; cc++) {
-      const double* X = x + (size_t)cc * ld;
-      double s = X[prev + i - 1] * c[0] + X[prev + i] * c[1] + X[prev + i + 1] * c[2] + X[start + i - 1] * c[3] + X[start + i] * c[4] +
-                 X[start + i + 1] * c[5] + X[next + i - 1] * c[6] + X[next + i] * c[7] + X[next + i + 1] * c[8];
-      y[(size_t)cc * ld + start + i] = b ? b[(size_t)cc * ld + start + i] - s : s;
+// y = A x with raw stencils (MultiplyBySystemMatrix_NoReciprocals, IterativeSolvers.inl:881-950), or with
+// `b` the residual b - A x, in one launch (blockIdx.y = chunk of KC columns, all of whose loads are in
+// flight together): blocks [0, rowBlocks) take the boundary rows, the others one raster line each.
+// (A small apply is its launches and round trips: one launch with kRowLanes lanes per row and global
+// columns took 6,936 texels x 3 columns from 14.1 to 4.0 us of kernels (13.3 to 10.1 a call) against a thread per row and column that
+// looked its A_BB columns up, beside the deep rows' own launch.)
+template <int KC>
+__global__ __launch_bounds__(kRowThreads) void KApply(int rowBlocks, int B, const int* __restrict__ bgi, const int* __restrict__ rp,
+                                                      const int* __restrict__ mid, const int* __restrict__ cl, const double* __restrict__ vl, const int* __restrict__ lines,
+                                                      const double* __restrict__ coef, int D, const double* __restrict__ x,
+                                                      const double* __restrict__ b, double* y, int K, int ld) {
+  const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
+  x += (size_t)c0 * ld, y += (size_t)c0 * ld;
+  if (b) b += (size_t)c0 * ld;
+  if ((int)blockIdx.x < rowBlocks) {
+    __shared__ RowTerms<KC, kRowThreads> terms;
+    const int row = (blockIdx.x * kRowThreads + (int)threadIdx.x) / kRowLanes, c = threadIdx.x % kRowLanes;
+    if (row >= B) return;  // whole row groups leave together
+    const double s = RowSum(rp[row], mid[row], rp[row + 1], cl, vl, x, ld, kc, terms);
+    if (c < kc) {
+      const size_t o = (size_t)c * ld + bgi[row];
+      y[o] = b ? b[o] - s : s;
     }
+    return;
   }
-}
-
-__global__ void KApplyBoundary(int B, const int* __restrict__ bgi, const int* __restrict__ rpd, const int* __restrict__ cold,
-                               const double* __restrict__ vald, const int* __restrict__ rpb, const int* __restrict__ colb,
-                               const double* __restrict__ valb, const double* __restrict__ x, const double* __restrict__ b, double* y, int K,
-                               int ld) {
-  long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)B * K) return;
-  int i = idx % B, c = idx / B;
-  const double* X = x + (size_t)c * ld;
-  double t = 0;
-  for (int k = rpb[i]; k < rpb[i + 1]; k++) t += X[bgi[colb[k]]] * valb[k];
-  double s = 0;
-  for (int k = rpd[i]; k < rpd[i + 1]; k++) s += X[cold[k]] * vald[k];
-  double v = t + s;
-  y[(size_t)c * ld + bgi[i]] = b ? b[(size_t)c * ld + bgi[i]] - v : v;
+  const int* L = lines + 5 * (blockIdx.x - rowBlocks);
+  const int start = L[0], len = L[1] - L[0] + 1, prev = L[2], next = L[3], d0 = L[4];
+  for (int i = threadIdx.x; i < len; i += kRowThreads) {
+    double a[9], v[KC][9], bv[KC];
+#pragma unroll
+    for (int k = 0; k < 9; k++) a[k] = coef[(size_t)k * D + d0 + i];
+#pragma unroll
+    for (int c = 0; c < KC; c++) {
+      const size_t o = (size_t)min(c, kc - 1) * ld;
+#pragma unroll
+      for (int k = 0; k < 9; k++) v[c][k] = x[o + (k < 3 ? prev : k < 6 ? start : next) + i + k % 3 - 1];
+      bv[c] = b ? b[o + start + i] : 0.0;
+    }
+#pragma unroll
+    for (int c = 0; c < KC; c++)
+      if (c < kc) {
+        double s = v[c][0] * a[0];
+#pragma unroll
+        for (int k = 1; k < 9; k++) s += v[c][k] * a[k];
+        y[(size_t)c * ld + start + i] = b ? bv[c] - s : s;
+      }
+  }
 }
 
 // Squared 2-norm of column blockIdx.y: a bounded grid strides over the column so that only a
@@ -638,6 +696,22 @@ static DevCsr UploadCsr(DeviceSystem& ds, const Csr& m) {
   return d;
 }
 
+// An operator's boundary rows with global columns: A_BB's entries, then A_BD's (from rowMid on).
+static void UploadBoundaryRows(DeviceSystem& ds, DevLevel& d, const Csr& bb, const Csr& bd, const std::vector<int>& bgi) {
+  Csr m;
+  std::vector<int> mid;
+  m.rows = bb.rows, m.cols = bd.cols;
+  m.col.reserve(bb.col.size() + bd.col.size()), m.val.reserve(m.col.capacity());
+  for (int r = 0; r < bb.rows; r++) {
+    for (int k = bb.rowptr[r]; k < bb.rowptr[r + 1]; k++) m.col.push_back(bgi[bb.col[k]]), m.val.push_back(bb.val[k]);
+    mid.push_back((int)m.col.size());
+    for (int k = bd.rowptr[r]; k < bd.rowptr[r + 1]; k++) m.col.push_back(bd.col[k]), m.val.push_back(bd.val[k]);
+    m.rowptr.push_back((int)m.col.size());
+  }
+  d.rows = UploadCsr(ds, m);
+  d.rowMid = Upload(ds, mid);
+}
+
 static std::vector<double> SoA10(const std::vector<double>& aos) {
   size_t D = aos.size() / 10;
   std::vector<double> s(aos.size());
@@ -716,6 +790,7 @@ void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOpe
     d.bgi = Upload(ds, H.boundaryGlobalIndex);
     d.bd = UploadCsr(ds, O.bd);
     d.bb = UploadCsr(ds, O.bb);
+    UploadBoundaryRows(ds, d, O.bb, O.bd, H.boundaryGlobalIndex);
     if (l + 1 < nl) d.brestr = UploadCsr(ds, H.boundaryRestriction);
     d.nTasks = (int)H.tasks.taskPtr.size() - 1;
     d.taskPtr = Upload(ds, H.tasks.taskPtr);
@@ -755,6 +830,8 @@ void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOpe
     d.coefSym = Upload(ds, SymStencil(which == 0 ? op.deepMass : op.deepStiffness, h.levels[0].rasterLines, l0.N));
     d.bd = UploadCsr(ds, which == 0 ? op.bdMass : op.bdStiffness);
     d.bb = UploadCsr(ds, which == 0 ? op.bbMass : op.bbStiffness);
+    if (which == 0) UploadBoundaryRows(ds, d, op.bbMass, op.bdMass, h.levels[0].boundaryGlobalIndex);
+    else UploadBoundaryRows(ds, d, op.bbStiffness, op.bdStiffness, h.levels[0].boundaryGlobalIndex);
   }
   ds.bytes = g_uploadBytes;
 }
@@ -845,15 +922,21 @@ static void BandSweep(DevLevel& d, double* x, const double* b, int K, int ld, hi
   }
 }
 
-// Deep rows of y = A x, or with `b` of b - A x.
-static void DeepRows(DevLevel& d, const double* x, const double* b, double* y, int K, int ld, hipStream_t s) {
-  if (d.nRaster > 0) KApplyDeep<<<d.nRaster, 128, 0, s>>>(d.nRaster, d.raster, d.coefRaw, d.D, x, b, y, K, ld);
+// y = A x of an operator's rows, or with `b` the residual b - A x; boundary: its boundary rows too.
+static void ApplyRows(DevLevel& d, const double* x, const double* b, double* y, int K, int ld, bool boundary, hipStream_t s) {
+  const int rowBlocks = boundary ? (int)Blocks((long)d.B * kRowLanes, kRowThreads) : 0;
+  if (rowBlocks + d.nRaster == 0) return;
+  // three columns at a time: 27 values of x in registers
+  const int chunks = (K + 2) / 3, kc = (K + chunks - 1) / chunks;
+  const auto kernel = kc == 1 ? KApply<1> : kc == 2 ? KApply<2> : KApply<3>;
+  kernel<<<dim3(rowBlocks + d.nRaster, (K + kc - 1) / kc), kRowThreads, 0, s>>>(rowBlocks, d.B, d.bgi, d.rows.rowptr, d.rowMid, d.rows.col, d.rows.val,
+                                                                                d.raster, d.coefRaw, d.D, x, b, y, K, ld);
 }
 
 void BandSweepLevel(DeviceSystem& ds, int l, double* x, const double* b, double* r, int K, int ld, hipStream_t s) {
   CheckK(ds, K);
   BandSweep(ds.L[l], x, b, K, ld, s);
-  if (r) DeepRows(ds.L[l], x, b, r, K, ld, s);
+  if (r) ApplyRows(ds.L[l], x, b, r, K, ld, false, s);
 }
 
 void RelaxLevel(DeviceSystem& ds, int l, double* x, const double* b, double* r, int K, int ld, bool withResidual, hipStream_t s) {
@@ -868,12 +951,20 @@ void RelaxLevel(DeviceSystem& ds, int l, double* x, const double* b, double* r, 
   if (withResidual) ResidualLevel(ds, l, x, b, r, K, ld, s);
 }
 
+// Restriction of level l's residual; zeroC (may be null): a level l + 1 vector set to zero with it.
+static void Restrict(DeviceSystem& ds, int l, const double* rF, double* bC, double* zeroC, int K, int ldF, int ldC, hipStream_t s) {
+  DevLevel &f = ds.L[l], &c = ds.L[l + 1];
+  const int rowBlocks = (int)Blocks((long)c.B * kRowLanes, kRowThreads);
+  if (rowBlocks + c.nRestr == 0) return;
+  const int chunks = (K + 2) / 3, kc = (K + chunks - 1) / chunks;
+  const auto kernel = kc == 1 ? KRestrict<1> : kc == 2 ? KRestrict<2> : KRestrict<3>;
+  kernel<<<dim3(rowBlocks + c.nRestr, (K + kc - 1) / kc), kRowThreads, 0, s>>>(rowBlocks, c.B, c.bgi, f.brestr.rowptr, f.brestr.col, f.brestr.val,
+                                                                              c.nRestr, c.restr, rF, ldF, bC, zeroC, ldC, K);
+}
+
 void RestrictLevel(DeviceSystem& ds, int l, const double* rF, double* bC, int K, int ldF, int ldC, hipStream_t s) {
   CheckK(ds, K);
-  DevLevel &f = ds.L[l], &c = ds.L[l + 1];
-  if (c.B > 0)
-    KCsrGatherScatter<<<Blocks((long)c.B * K, 256), 256, 0, s>>>(c.B, c.bgi, f.brestr.rowptr, f.brestr.col, f.brestr.val, rF, ldF, bC, ldC, K);
-  if (c.nRestr > 0) KRestrictDeep<<<c.nRestr, 128, 0, s>>>(c.nRestr, c.restr, rF, ldF, bC, ldC, K);
+  Restrict(ds, l, rF, bC, nullptr, K, ldF, ldC, s);
 }
 
 void ProlongAddLevel(DeviceSystem& ds, int l, const double* xC, double* xF, int K, int ldC, int ldF, hipStream_t s) {
@@ -888,10 +979,7 @@ void ApplyLevel(DeviceSystem& ds, int l, const double* x, double* y, int K, int 
 
 void ApplyOperator(DeviceSystem& ds, DevLevel& d, const double* x, double* y, int K, int ld, hipStream_t s) {
   CheckK(ds, K);
-  if (d.B > 0)
-    KApplyBoundary<<<Blocks((long)d.B * K, 256), 256, 0, s>>>(d.B, d.bgi, d.bd.rowptr, d.bd.col, d.bd.val, d.bb.rowptr, d.bb.col, d.bb.val, x,
-                                                              nullptr, y, K, ld);
-  if (d.nRaster > 0) KApplyDeep<<<d.nRaster, 128, 0, s>>>(d.nRaster, d.raster, d.coefRaw, d.D, x, nullptr, y, K, ld);
+  ApplyRows(d, x, nullptr, y, K, ld, true, s);
 }
 
 void SquaredNorms(const double* v, int N, int K, int ld, double* dNorms, hipStream_t s) {
@@ -901,27 +989,19 @@ void SquaredNorms(const double* v, int N, int K, int ld, double* dNorms, hipStre
 
 void ResidualLevel(DeviceSystem& ds, int l, const double* x, const double* b, double* r, int K, int ld, hipStream_t s) {
   CheckK(ds, K);
-  DevLevel& d = ds.L[l];
-  if (d.B > 0)
-    KApplyBoundary<<<Blocks((long)d.B * K, 256), 256, 0, s>>>(d.B, d.bgi, d.bd.rowptr, d.bd.col, d.bd.val, d.bb.rowptr, d.bb.col, d.bb.val, x, b,
-                                                              r, K, ld);
-  if (d.nRaster > 0) KApplyDeep<<<d.nRaster, 128, 0, s>>>(d.nRaster, d.raster, d.coefRaw, d.D, x, b, r, K, ld);
+  ApplyRows(ds.L[l], x, b, r, K, ld, true, s);
 }
 
 void VCycleReference(DeviceSystem& ds, double* x, const double* b, int K, int ld, hipStream_t s) {
   CheckK(ds, K);
   const int nl = ds.levels;
-  for (int l = 1; l < nl; l++) {
-    long n = (long)ds.L[l].N * K;
-    KZero<<<Blocks(n, 256), 256, 0, s>>>(n, ds.L[l].x);
-  }
   auto X = [&](int l) { return l == 0 ? x : ds.L[l].x; };
   auto Bv = [&](int l) { return l == 0 ? const_cast<double*>(b) : ds.L[l].b; };
   auto LD = [&](int l) { return l == 0 ? ld : ds.L[l].N; };
   for (int l = 0; l + 1 < nl; l++) {
     RelaxLevel(ds, l, X(l), Bv(l), ds.L[l].r, K, LD(l), true, s);
     // the level residual lives in r with the level's own stride
-    RestrictLevel(ds, l, ds.L[l].r, ds.L[l + 1].b, K, LD(l), ds.L[l + 1].N, s);
+    Restrict(ds, l, ds.L[l].r, ds.L[l + 1].b, ds.L[l + 1].x, K, LD(l), ds.L[l + 1].N, s);
   }
   CoarseSolve(ds, ds.L[nl - 1].b, ds.L[nl - 1].x, K, ds.L[nl - 1].N, s);
   for (int l = nl - 2; l >= 0; l--) {
@@ -1022,11 +1102,11 @@ void ModulatedStiffness(const DevModulation& m, const double* mask, double* out,
 // column in a fixed order, so repeated calls give bitwise identical norms.
 template <int KC>
 __global__ __launch_bounds__(256) void KResidualNormParts(int nLines, const int* __restrict__ lines, const double* __restrict__ coef, int D,
-                                                          int B, const int* __restrict__ bgi, const int* __restrict__ rpd,
-                                                          const int* __restrict__ cold, const double* __restrict__ vald,
-                                                          const int* __restrict__ rpb, const int* __restrict__ colb,
-                                                          const double* __restrict__ valb, const double* __restrict__ x,
-                                                          const double* __restrict__ b, int ld, int c0, double* parts) {
+                                                          int B, const int* __restrict__ bgi, const int* __restrict__ rp,
+                                                          const int* __restrict__ mid, const int* __restrict__ cl,
+                                                          const double* __restrict__ vl,
+                                                          const double* __restrict__ x, const double* __restrict__ b, int ld, int c0,
+                                                          double* parts) {
   double rr[KC], bn[KC];
 #pragma unroll
   for (int c = 0; c < KC; c++) rr[c] = 0.0, bn[c] = 0.0;
@@ -1048,17 +1128,14 @@ __global__ __launch_bounds__(256) void KResidualNormParts(int nLines, const int*
       }
     }
   }
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < B; i += gridDim.x * blockDim.x) {
-    const int g = bgi[i];
+  // boundary rows: kRowLanes lanes each; lane c of a row's group adds column c's terms
+  __shared__ RowTerms<KC, 256> terms;
+  const int lane = threadIdx.x % kRowLanes;
+  for (int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) / kRowLanes); i < B; i += (int)(gridDim.x * blockDim.x / kRowLanes)) {
+    const double s = RowSum(rp[i], mid[i], rp[i + 1], cl, vl, x + (size_t)c0 * ld, ld, KC, terms);
+    const double bv = b[(size_t)(c0 + min(lane, KC - 1)) * ld + bgi[i]], r = bv - s;
 #pragma unroll
-    for (int c = 0; c < KC; c++) {
-      const double* X = x + (size_t)(c0 + c) * ld;
-      double t = 0.0, s = 0.0;
-      for (int k = rpb[i]; k < rpb[i + 1]; k++) t += X[bgi[colb[k]]] * valb[k];
-      for (int k = rpd[i]; k < rpd[i + 1]; k++) s += X[cold[k]] * vald[k];
-      const double bv = b[(size_t)(c0 + c) * ld + g], r = bv - (t + s);
-      rr[c] += r * r, bn[c] += bv * bv;
-    }
+    for (int c = 0; c < KC; c++) rr[c] += lane == c ? r * r : 0.0, bn[c] += lane == c ? bv * bv : 0.0;
   }
   __shared__ double part[2 * KC][4];
 #pragma unroll
@@ -1092,8 +1169,8 @@ void ResidualNorms(DeviceSystem& ds, const double* x, const double* b, int K, in
   for (int c0 = 0; c0 < K; c0 += 4) {
     const int kc = std::min(4, K - c0);
 #define GDTP_NORM_PARTS(KC)                                                                                                         \
-  KResidualNormParts<KC><<<kNormParts, 256, 0, s>>>(d.nRaster, d.raster, d.coefRaw, d.D, d.B, d.bgi, d.bd.rowptr, d.bd.col, d.bd.val, \
-                                                    d.bb.rowptr, d.bb.col, d.bb.val, x, b, ld, c0, parts)
+  KResidualNormParts<KC><<<kNormParts, 256, 0, s>>>(d.nRaster, d.raster, d.coefRaw, d.D, d.B, d.bgi, d.rows.rowptr, d.rowMid, d.rows.col, \
+                                                    d.rows.val, x, b, ld, c0, parts)
     switch (kc) {
       case 4: GDTP_NORM_PARTS(4); break;
       case 3: GDTP_NORM_PARTS(3); break;
