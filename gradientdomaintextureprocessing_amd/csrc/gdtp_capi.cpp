@@ -525,7 +525,7 @@ int gdtp_direct_solve(gdtp_system* s, double* x, const double* b, int ncols, dou
         f->allocations.push_back(f->y);
         s->direct = std::move(f);
       }
-      LdltSolve(s->direct->d, b, N, x, N, nullptr, s->direct->y, ncols, st);
+      LdltSolve(s->direct->d, b, N, x, N, s->direct->y, ncols, st);
       SystemNorms(s, x, b, ncols, sq, st);
       if (method) *method = 0;
     } else {

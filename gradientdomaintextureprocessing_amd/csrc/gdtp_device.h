@@ -16,6 +16,12 @@ namespace gdtp {
     if (e_ != hipSuccess) throw std::runtime_error(std::string(#call) + ": " + hipGetErrorString(e_)); \
   } while (0)
 
+// A row of a wide stage: its component's first row and size, and where its rows of the two inverses begin.
+struct LdltWideRow {
+  int begin, rows;
+  long mat[2];  // forward, backward
+};
+
 // Exact triangular solves of an LDL^T factor on the device: the staged form (LdltStages).
 struct DevLdlt {
   int n = 0, wideBegin = 0;
@@ -27,8 +33,11 @@ struct DevLdlt {
   double *fwdVal = nullptr, *bwdVal = nullptr;
   long *fwdMatPtr = nullptr, *bwdMatPtr = nullptr;
   double *fwdMat = nullptr, *bwdMat = nullptr;
-  int* rowComp = nullptr;      // component of each row of the wide stages (row - wideBegin)
+  LdltWideRow* wideRows = nullptr;  // of each row of the wide stages (row - wideBegin)
   double* wideBuf = nullptr;   // [2][kcap][n - wideBegin]: right-hand sides of the wide products
+  // boundary factors: the texel of each row, and A_BD's rows in the factor's numbering
+  int *texel = nullptr, *rhsPtr = nullptr, *rhsCol = nullptr;
+  double* rhsVal = nullptr;
   int kcap = 0;
 };
 
@@ -65,7 +74,7 @@ struct DevLevel {
   int *raster = nullptr, *restr = nullptr, *prol = nullptr;  // 5, 5, 6 ints per line
   DevLdlt factor;              // boundary factor (levels < L-1) or full coarse factor (level L-1)
   // work vectors for up to `kcap` columns
-  double *x = nullptr, *b = nullptr, *r = nullptr, *vb = nullptr, *y = nullptr;
+  double *x = nullptr, *b = nullptr, *r = nullptr, *y = nullptr;
 };
 
 struct DeviceSystem {
@@ -78,12 +87,13 @@ struct DeviceSystem {
   ~DeviceSystem();
 };
 
-// Upload an LDL^T factor's staged triangular solves; LdltSolve solves for K columns (at most kcap),
-// gathering src[perm] and scattering into dst (through `map` when not null; dst may be src).  y: [K][n] scratch.
-void UploadLdlt(std::vector<void*>& allocations, const Ldlt& F, DevLdlt& d, int kcap);
+// Upload an LDL^T factor's staged triangular solves; LdltSolve solves for K columns (at most kcap); dst
+// may be src.  y: [K][n] scratch.
+void UploadLdlt(std::vector<void*>& allocations, const Ldlt& F, DevLdlt& d, int kcap, const Csr* bd = nullptr,
+                const std::vector<int>* bgi = nullptr);
 // Bytes uploaded / allocated by this thread's device uploads so far (monotone counter).
 size_t UploadByteCounter();
-void LdltSolve(DevLdlt& F, const double* src, int lds, double* dst, int ldd, const int* map, double* y, int K, hipStream_t s);
+void LdltSolve(DevLdlt& F, const double* src, int lds, double* dst, int ldd, double* y, int K, hipStream_t s);
 
 void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOperator& op, int kcap, DeviceSystem& ds);
 

@@ -206,20 +206,6 @@ __global__ __launch_bounds__(256) void KBandGs(int color, int nTasks, const int*
   }
 }
 
-// ------------------------------------------------------------------ boundary rows
-// vb = b_B - A_BD x   (IterativeSolvers.inl:410-419)
-__global__ void KBoundaryRhs(int B, const int* __restrict__ bgi, const int* __restrict__ rp, const int* __restrict__ col,
-                             const double* __restrict__ val, const double* __restrict__ x, const double* __restrict__ b, double* vb, int K,
-                             int ld) {
-  long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (long)B * K) return;
-  int i = idx % B, c = idx / B;
-  const double* X = x + (size_t)c * ld;
-  double s = 0;
-  for (int k = rp[i]; k < rp[i + 1]; k++) s += X[col[k]] * val[k];
-  vb[(size_t)c * B + i] = b[(size_t)c * ld + bgi[i]] - s;
-}
-
 // ------------------------------------------------------------------ exact LDL^T solves
 // The staged triangular solves (LdltStages): forward stages r = src[perm] - L y(earlier stages),
 // y = inv(L_cc) r per component, then backward r = y / D - L^T x(later stages), x = inv(L_cc)^T r.
@@ -227,7 +213,7 @@ __global__ void KBoundaryRhs(int B, const int* __restrict__ bgi, const int* __re
 // What bounds them: a dependency chain.  The level-scheduled solve they replace walked the elimination
 // tree's 250-450 levels (subtree teams of one workgroup, a barrier per level, one thread per row), each
 // level a round trip to memory: 1.75 ms for the 175,580 boundary rows of a 4096^2 atlas and three
-// columns, 0.25 ms for 3840 rows.  Explicit inverses of components of up to 128 (first stage) or a few
+// columns, 0.25 ms for 3840 rows; the stages take 0.12 and 0.03 ms.  Explicit inverses of components of up to 128 (first stage) or a few
 // hundred rows leave two passes per stage, each a gather and a product with loads that wait for
 // nothing; the inverses are 2-4 times the factor's bytes.
 
@@ -238,138 +224,179 @@ __device__ __forceinline__ double GroupSum(double v) {
   for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, G);
   return v;
 }
+// The wave's sum in lane 63, by DPP moves.
+__device__ __forceinline__ double WaveSumLast(double v) {
+  v += DppMove<0x111, 0xf, true>(v, 0.0);
+  v += DppMove<0x112, 0xf, true>(v, 0.0);
+  v += DppMove<0x114, 0xf, true>(v, 0.0);
+  v += DppMove<0x118, 0xf, true>(v, 0.0);
+  v += DppMove<0x142, 0xa>(v, 0.0);
+  v += DppMove<0x143, 0xc>(v, 0.0);
+  return v;
+}
 
-// One row's coupling sums with the stages solved before, by a group of G lanes, for up to KC columns.
+// The tables of one direction and the vectors of a solve.
+struct LdltPass {
+  const int* compPtr;
+  const long* matPtr;
+  const double* mat;
+  const int *ptr, *col;  // couplings with the stages solved before
+  const double* val;
+  const int* index;      // of each row in the right-hand side (forward) or the solution (backward)
+  const double* dinv;
+  // the relaxation's right-hand side b - A_BD x is formed by the forward stages: A_BD's rows
+  const int *rhsPtr, *rhsCol;
+  const double *rhsVal, *rhsX;
+};
+
+// A group of G lanes adds val y[col] over entries [p0, p1) to s, for up to KC columns.
 template <int G, int KC>
-__device__ __forceinline__ void CouplingSums(const int* __restrict__ col, const double* __restrict__ val, int p0, int p1, int lane,
-                                             const double* y, int n, int kc, double (&s)[KC]) {
-#pragma unroll
-  for (int c = 0; c < KC; c++) s[c] = 0.0;
+__device__ __forceinline__ void CouplingTerms(const int* __restrict__ col, const double* __restrict__ val, int p0, int p1, int lane,
+                                              const double* y, size_t n, int kc, double (&s)[KC]) {
   for (int p = p0 + lane; p < p1; p += G) {
     const double v = val[p];
     const int j = col[p];
 #pragma unroll
-    for (int c = 0; c < KC; c++)
-      if (c < kc) s[c] += v * y[(size_t)c * n + j];
+    for (int c = 0; c < KC; c++) s[c] += v * y[min(c, kc - 1) * n + j];
   }
+}
+
+// Row w's right-hand side of a stage in lane c (of the group) for column c: what is known of it
+// (forward: b, backward: y / D) less its couplings with the stages solved before.
+template <bool kForward, bool kRhs, int G, int KC>
+__device__ __forceinline__ double StageRhs(const LdltPass& P, int w, int lane, const double* src, int lds, const double* y, int n, int c0,
+                                           int kc) {
+  double s[KC] = {};
+  // column slots past kc repeat the last column, so that no load is behind a branch
+  const int c = min(min(lane, KC - 1), kc - 1);
+  const double known = kForward ? src[(size_t)(c0 + c) * lds + P.index[w]] : y[(size_t)c * n + w] * P.dinv[w];
+  CouplingTerms<G, KC>(P.col, P.val, P.ptr[w], P.ptr[w + 1], lane, y, n, kc, s);
+  if constexpr (kRhs) CouplingTerms<G, KC>(P.rhsCol, P.rhsVal, P.rhsPtr[w], P.rhsPtr[w + 1], lane, P.rhsX + (size_t)c0 * lds, lds, kc, s);
+  double mine = 0.0;
 #pragma unroll
-  for (int c = 0; c < KC; c++) s[c] = GroupSum<G>(s[c]);
+  for (int k = 0; k < KC; k++) {
+    const double t = GroupSum<G>(s[k]);
+    if (k == c) mine = t;
+  }
+  return known - mine;
 }
 
 // The 16 waves of a narrow component's workgroup are divided over its row blocks (at most four) in
 // proportion to the blocks' columns (forward: later blocks have more; backward: mirrored).
 __device__ __constant__ const unsigned char kWaveSplit[4][5] = {{0, 16, 16, 16, 16}, {0, 5, 16, 16, 16}, {0, 3, 8, 16, 16}, {0, 2, 5, 10, 16}};
+static constexpr int kEarlyColumns = 13; // loaded ahead: all of them for components of up to 128 rows
 
 // A narrow stage: one workgroup of 16 waves per component of at most kLdltNarrowRows rows and chunk of
-// up to KC columns.  The component's right-hand side is staged in LDS; a wave then owns one row per
-// lane and a share of its block's columns, so the inverse's loads are whole lines that wait for nothing
-// and most of a component is one memory round trip; the waves' parts are added in a fixed order.
-template <bool kForward, int G, int KC>
-__global__ __launch_bounds__(1024) void KLdltNarrow(int comp0, const int* __restrict__ compPtr, const long* __restrict__ matPtr,
-                                                    const double* __restrict__ mat, const int* __restrict__ rp, const int* __restrict__ col,
-                                                    const double* __restrict__ val, const int* __restrict__ perm,
-                                                    const double* __restrict__ dinv, const double* src, int lds, double* y, int n, double* dst,
-                                                    int ldd, const int* __restrict__ map, int K) {
+// up to KC columns.  A wave owns one row per lane and a share of its block's columns, so the inverse's
+// loads are whole lines that wait for nothing; they go out first and are in flight while the
+// component's right-hand side is gathered into LDS.  The waves' parts are added in a fixed order.
+template <bool kForward, bool kRhs, int G, int KC>
+__global__ __launch_bounds__(1024) void KLdltNarrow(int comp0, LdltPass P, const double* src, int lds, double* y, int n, double* dst, int ldd,
+                                                    int K) {
   __shared__ double R[KC][kLdltNarrowRows];
-  __shared__ double P[16][KC][kLdltBlock];
-  const int comp = comp0 + blockIdx.x, w0 = compPtr[comp], m = compPtr[comp + 1] - w0;
+  __shared__ double Q[16][KC][kLdltBlock];
+  const int comp = comp0 + blockIdx.x, w0 = P.compPtr[comp], m = P.compPtr[comp + 1] - w0;
   const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
   y += (size_t)c0 * n;
-  for (int i = threadIdx.x / G; i < m; i += 1024 / G) {
-    const int w = w0 + i, lane = threadIdx.x % G;
-    double s[KC];
-    CouplingSums<G, KC>(col, val, rp[w], rp[w + 1], lane, y, n, kc, s);
-#pragma unroll
-    for (int c = 0; c < KC; c++)
-      if (lane == c % G && c < kc) R[c][i] = (kForward ? src[(size_t)(c0 + c) * lds + perm[w]] : y[(size_t)c * n + w] * dinv[w]) - s[c];
-  }
-  __syncthreads();
   const int blocks = (m + kLdltBlock - 1) / kLdltBlock, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave), lane = threadIdx.x % kWave;
   // this wave's block: the split's k-th (backward: mirrored, so that the widest block gets the most waves)
   int k = 0;
   while (wave >= kWaveSplit[blocks - 1][k + 1]) k++;
   const int part = wave - kWaveSplit[blocks - 1][k], parts = kWaveSplit[blocks - 1][k + 1] - kWaveSplit[blocks - 1][k];
   const int rb = kForward ? k : blocks - 1 - k, r0 = rb * kLdltBlock, nr = min(kLdltBlock, m - r0);
-  const int j0 = kForward ? 0 : r0, j1 = kForward ? r0 + nr : m;
+  const int j0 = kForward ? 0 : r0, cols = kForward ? r0 + nr : m - r0;
   // the blocks before this one: kLdltBlock rows each (only the last is shorter)
-  const long off = matPtr[comp] + (kForward ? (long)kLdltBlock * kLdltBlock * (rb * (rb + 1) / 2)
-                                            : (long)kLdltBlock * rb * m - (long)kLdltBlock * kLdltBlock * (rb * (rb - 1) / 2));
-  const double* M = mat + off + min(lane, nr - 1);
-  double acc[KC] = {};
-#pragma unroll 8
-  for (int j = j0 + part; j < j1; j += parts) {
-    const double a = M[(size_t)(j - j0) * nr];
+  const long off = P.matPtr[comp] + (kForward ? (long)kLdltBlock * kLdltBlock * (rb * (rb + 1) / 2)
+                                              : (long)kLdltBlock * rb * m - (long)kLdltBlock * kLdltBlock * (rb * (rb - 1) / 2));
+  const double* M = P.mat + off + min(lane, nr - 1);
+  double early[kEarlyColumns];
 #pragma unroll
-    for (int c = 0; c < KC; c++) acc[c] += a * R[c][j];
+  for (int q = 0; q < kEarlyColumns; q++) early[q] = M[(size_t)min(part + q * parts, cols - 1) * nr];
+  const int outRow = min((int)threadIdx.x, m * KC - 1) % m;
+  const int out = kForward ? 0 : P.index[w0 + outRow];
+  for (int i = threadIdx.x / G; i < m; i += 1024 / G) {
+    const int gl = threadIdx.x % G;
+    const double v = StageRhs<kForward, kRhs, G, KC>(P, w0 + i, gl, src, lds, y, n, c0, kc);
+    if (gl < KC) R[gl][i] = v;
+  }
+  __syncthreads();
+  double acc[KC] = {};
+#pragma unroll
+  for (int q = 0; q < kEarlyColumns; q++) {
+    const int j = part + q * parts;
+    if (j >= cols) break;
+#pragma unroll
+    for (int c = 0; c < KC; c++) acc[c] += early[q] * R[c][j0 + j];
+  }
+#pragma unroll 8
+  for (int j = part + kEarlyColumns * parts; j < cols; j += parts) {
+    const double a = M[(size_t)j * nr];
+#pragma unroll
+    for (int c = 0; c < KC; c++) acc[c] += a * R[c][j0 + j];
   }
 #pragma unroll
-  for (int c = 0; c < KC; c++) P[wave][c][lane] = acc[c];
+  for (int c = 0; c < KC; c++) Q[wave][c][lane] = acc[c];
   __syncthreads();
-  for (int t = threadIdx.x; t < m * kc; t += 1024) {
-    const int c = t / m, i = t % m, b = i / kLdltBlock, kk = kForward ? b : blocks - 1 - b;
+  static_assert(kLdltNarrowRows * 4 <= 1024, "one result per thread");
+  if ((int)threadIdx.x < m * kc) {
+    const int c = threadIdx.x / m, i = outRow, b = i / kLdltBlock, kk = kForward ? b : blocks - 1 - b;
     double s = 0.0;
-    for (int q = kWaveSplit[blocks - 1][kk]; q < kWaveSplit[blocks - 1][kk + 1]; q++) s += P[q][c][i % kLdltBlock];
+    for (int q = kWaveSplit[blocks - 1][kk]; q < kWaveSplit[blocks - 1][kk + 1]; q++) s += Q[q][c][i % kLdltBlock];
     y[(size_t)c * n + w0 + i] = s;
-    if (!kForward) {
-      const int g = perm[w0 + i];
-      dst[(size_t)(c0 + c) * ldd + (map ? map[g] : g)] = s;
-    }
+    if (!kForward) dst[(size_t)(c0 + c) * ldd + out] = s;
   }
 }
 
 // A wide stage's right-hand sides (its rows [row0, row1), one wave per row and chunk of columns).
-template <bool kForward, int KC>
-__global__ __launch_bounds__(256) void KLdltCouple(int row0, int row1, int wideBegin, const int* __restrict__ rp, const int* __restrict__ col,
-                                                   const double* __restrict__ val, const int* __restrict__ perm,
-                                                   const double* __restrict__ dinv, const double* src, int lds, const double* y, int n,
-                                                   double* buf, int nWide, int K) {
+template <bool kForward, bool kRhs, int KC>
+__global__ __launch_bounds__(256) void KLdltCouple(int row0, int row1, int wideBegin, LdltPass P, const double* src, int lds, const double* y,
+                                                   int n, double* buf, int nWide, int K) {
   const int w = row0 + blockIdx.x * (256 / kWave) + (int)threadIdx.x / kWave, lane = threadIdx.x % kWave;
   if (w >= row1) return;
   const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
-  y += (size_t)c0 * n;
-  double s[KC];
-  CouplingSums<kWave, KC>(col, val, rp[w], rp[w + 1], lane, y, n, kc, s);
-#pragma unroll
-  for (int c = 0; c < KC; c++)
-    if (lane == c && c < kc)
-      buf[(size_t)(c0 + c) * nWide + w - wideBegin] = (kForward ? src[(size_t)(c0 + c) * lds + perm[w]] : y[(size_t)c * n + w] * dinv[w]) - s[c];
+  const double v = StageRhs<kForward, kRhs, kWave, KC>(P, w, lane, src, lds, y + (size_t)c0 * n, n, c0, kc);
+  if (lane < kc) buf[(size_t)(c0 + lane) * nWide + w - wideBegin] = v;
 }
 
-// A wide stage's product with its components' inverses, one wave per row and chunk of columns: the
-// forward result to y, or for the top scaled by 1 / D to `top` (the backward product's input); the
-// backward result to y and dst.
+// A wide stage's product with its components' inverses, one wave per row and chunk of columns, two
+// entries per lane and load: the forward result to y, or for the top scaled by 1 / D to `top` (the
+// backward product's input); the backward result to y and dst.  (1920 rows, three columns: forward
+// 26 and backward 20 us with one entry per load and the component looked up first, 13 and 8 us so.)
 template <bool kForward, int KC>
-__global__ __launch_bounds__(256) void KLdltWide(int row0, int row1, int wideBegin, const int* __restrict__ rowComp,
-                                                 const int* __restrict__ compPtr, const long* __restrict__ matPtr,
-                                                 const double* __restrict__ mat, const double* __restrict__ buf, int nWide,
-                                                 const int* __restrict__ perm, const double* __restrict__ dinv, double* y, int n, double* top,
-                                                 double* dst, int ldd, const int* __restrict__ map, int K) {
+__global__ __launch_bounds__(256) void KLdltWide(int row0, int row1, int wideBegin, const LdltWideRow* __restrict__ wideRows, LdltPass P,
+                                                 const double* __restrict__ buf, int nWide, double* y, int n, double* top, double* dst, int ldd,
+                                                 int K) {
   const int w = row0 + blockIdx.x * (256 / kWave) + (int)threadIdx.x / kWave, lane = threadIdx.x % kWave;
   if (w >= row1) return;
-  const int comp = rowComp[w - wideBegin], w0 = compPtr[comp], m = compPtr[comp + 1] - w0, i = w - w0;
+  const LdltWideRow T = wideRows[w - wideBegin];
+  const int i = w - T.begin, m = T.rows;
   const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
-  const double* row = mat + matPtr[comp] + (size_t)i * m;
-  const double* in = buf + (size_t)c0 * nWide + w0 - wideBegin;
+  const double* row = P.mat + T.mat[kForward ? 0 : 1];
+  const double* in = buf + (size_t)c0 * nWide + T.begin - wideBegin;
+  const double dinv = P.dinv[w];
+  const int out = kForward ? 0 : P.index[w];
   double acc[KC] = {};
   const int j1 = kForward ? i + 1 : m;
 #pragma unroll 4
-  for (int j = (kForward ? 0 : i / kWave * kWave) + lane; j < j1; j += kWave) {  // backward: entries before i are zero
-    const double a = row[j];
+  for (int j = (kForward ? 0 : i / 2 * 2) + 2 * lane; j < j1; j += 2 * kWave) {  // backward: entries before i are zero
+    double a0, a1;
+    LoadPair(row + j, a0, a1);
+    const bool both = j + 1 < m;  // (a row of odd length is padded with a zero; the vector is not)
 #pragma unroll
-    for (int c = 0; c < KC; c++)
-      if (c < kc) acc[c] += a * in[(size_t)c * nWide + j];
+    for (int c = 0; c < KC; c++) {
+      double v0, v1;
+      LoadPair(in + (size_t)min(c, kc - 1) * nWide + j, v0, v1);
+      acc[c] += a0 * v0;
+      if (both) acc[c] += a1 * v1;
+    }
   }
 #pragma unroll
-  for (int c = 0; c < KC; c++) acc[c] = GroupSum<kWave>(acc[c]);
-#pragma unroll
   for (int c = 0; c < KC; c++) {
-    if (lane != c || c >= kc) continue;
-    if (kForward && top) top[(size_t)(c0 + c) * nWide + w - wideBegin] = acc[c] * dinv[w];
-    else y[(size_t)(c0 + c) * n + w] = acc[c];
-    if (!kForward) {
-      const int g = perm[w];
-      dst[(size_t)(c0 + c) * ldd + (map ? map[g] : g)] = acc[c];
-    }
+    const double s = WaveSumLast(acc[c]);
+    if (lane != kWave - 1 || c >= kc) continue;
+    if (kForward && top) top[(size_t)(c0 + c) * nWide + w - wideBegin] = s * dinv;
+    else y[(size_t)(c0 + c) * n + w] = s;
+    if (!kForward) dst[(size_t)(c0 + c) * ldd + out] = s;
   }
 }
 
@@ -757,7 +784,9 @@ static std::vector<double> SymStencil(const std::vector<double>& aos, const std:
   return s;
 }
 
-void UploadLdlt(std::vector<void*>& ds, const Ldlt& F, DevLdlt& d, int kcap) {
+// bd, bgi (boundary factors; null for others): A_BD and the boundary texels, so that LdltRelaxSolve can
+// form its right-hand side itself and write into a level vector.
+void UploadLdlt(std::vector<void*>& ds, const Ldlt& F, DevLdlt& d, int kcap, const Csr* bd, const std::vector<int>* bgi) {
   LdltStages S;
   BuildLdltStages(F, S);
   d.n = S.n, d.wideBegin = S.wideBegin, d.kcap = kcap;
@@ -767,11 +796,29 @@ void UploadLdlt(std::vector<void*>& ds, const Ldlt& F, DevLdlt& d, int kcap) {
   d.bwdPtr = UploadTo(ds, S.bwdPtr), d.bwdCol = UploadTo(ds, S.bwdCol), d.bwdVal = UploadTo(ds, S.bwdVal);
   d.fwdMatPtr = UploadTo(ds, S.fwdMatPtr), d.bwdMatPtr = UploadTo(ds, S.bwdMatPtr);
   d.fwdMat = UploadTo(ds, S.fwdMat), d.bwdMat = UploadTo(ds, S.bwdMat);
-  std::vector<int> rowComp(S.n - S.wideBegin);
+  std::vector<LdltWideRow> wide(S.n - S.wideBegin);
   for (size_t c = 0; c + 1 < S.compPtr.size(); c++)
-    for (int w = std::max(S.compPtr[c], S.wideBegin); w < S.compPtr[c + 1]; w++) rowComp[w - S.wideBegin] = (int)c;
-  d.rowComp = UploadTo(ds, rowComp);
-  if (kcap > 0 && !rowComp.empty()) d.wideBuf = UploadTo(ds, std::vector<double>(2 * (size_t)kcap * rowComp.size(), 0.0));
+    for (int w = std::max(S.compPtr[c], S.wideBegin); w < S.compPtr[c + 1]; w++) {
+      const int m = S.compPtr[c + 1] - S.compPtr[c];
+      const long o = (long)(w - S.compPtr[c]) * LdltWideStride(m);
+      wide[w - S.wideBegin] = {S.compPtr[c], m, {S.fwdMatPtr[c] + o, S.bwdMatPtr[c] + o}};
+    }
+  d.wideRows = UploadTo(ds, wide);
+  if (kcap > 0 && !wide.empty())  // (one double more: a row of odd length is read in pairs)
+    d.wideBuf = UploadTo(ds, std::vector<double>(2 * (size_t)kcap * wide.size() + 1, 0.0));
+  if (!bd) return;
+  Csr rhs;
+  rhs.rows = S.n, rhs.cols = bd->cols;
+  std::vector<int> texel(S.n);
+  for (int w = 0; w < S.n; w++) {
+    const int r = S.perm[w];
+    rhs.col.insert(rhs.col.end(), bd->col.begin() + bd->rowptr[r], bd->col.begin() + bd->rowptr[r + 1]);
+    rhs.val.insert(rhs.val.end(), bd->val.begin() + bd->rowptr[r], bd->val.begin() + bd->rowptr[r + 1]);
+    rhs.rowptr.push_back((int)rhs.col.size());
+    texel[w] = (*bgi)[r];
+  }
+  d.texel = UploadTo(ds, texel);
+  d.rhsPtr = UploadTo(ds, rhs.rowptr), d.rhsCol = UploadTo(ds, rhs.col), d.rhsVal = UploadTo(ds, rhs.val);
 }
 
 void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOperator& op, int kcap, DeviceSystem& ds) {
@@ -814,12 +861,11 @@ void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOpe
     for (auto& x : H.prolongationLines) rl.insert(rl.end(), {x.start, x.length, x.center, x.prev, x.next, x.aligned});
     d.nProl = (int)H.prolongationLines.size();
     d.prol = Upload(ds, rl);
-    if (l + 1 < nl) UploadLdlt(ds.allocations, oh.boundaryFactor[l], d.factor, kcap);
+    if (l + 1 < nl) UploadLdlt(ds.allocations, oh.boundaryFactor[l], d.factor, kcap, &O.bd, &H.boundaryGlobalIndex);
     else UploadLdlt(ds.allocations, oh.coarseFactor, d.factor, kcap);
     d.x = Alloc(ds, (size_t)d.N * kcap);
     d.b = Alloc(ds, (size_t)d.N * kcap);
     d.r = Alloc(ds, (size_t)d.N * kcap);
-    d.vb = Alloc(ds, (size_t)std::max(d.B, 1) * kcap);
     d.y = Alloc(ds, (size_t)std::max(d.factor.n, 1) * kcap);
   }
   for (int which = 0; which < 2; which++) {
@@ -836,54 +882,64 @@ void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOpe
   ds.bytes = g_uploadBytes;
 }
 
-// Columns in chunks of KC = min(K, 4); a stage's launches cover all chunks.
-template <int KC>
-static void LdltSolveChunks(DevLdlt& F, const double* src, int lds, double* dst, int ldd, const int* map, double* y, int K, hipStream_t s) {
+// Columns in chunks of KC = min(K, 4); a stage's launches cover all chunks.  index: of each row in src and
+// dst; rhsX (kRhs): src is b, and A_BD rhsX is subtracted from it.
+template <bool kRhs, int KC>
+static void LdltSolveChunks(DevLdlt& F, const double* src, int lds, double* dst, int ldd, const int* index, const double* rhsX, double* y, int K,
+                            hipStream_t s) {
   const int n = F.n, nWide = n - F.wideBegin, last = (int)F.stages.size() - 1;
   const unsigned chunks = (unsigned)((K + KC - 1) / KC);
   double *buf = F.wideBuf, *top = F.wideBuf + (size_t)F.kcap * nWide;
   auto wideGrid = [&](const LdltStage& T) { return dim3(Blocks(T.rowEnd - T.rowBegin, 256 / kWave), chunks); };
+  const LdltPass fwd{F.compPtr, F.fwdMatPtr, F.fwdMat, F.fwdPtr, F.fwdCol, F.fwdVal, index, F.dinv, F.rhsPtr, F.rhsCol, F.rhsVal, rhsX};
+  const LdltPass bwd{F.compPtr, F.bwdMatPtr, F.bwdMat, F.bwdPtr, F.bwdCol, F.bwdVal, index, F.dinv, nullptr, nullptr, nullptr, nullptr};
   for (int k = 0; k <= last; k++) {
     const LdltStage& T = F.stages[k];
     if (T.rowBegin == T.rowEnd) continue;
     if (!T.wide) {
       // the first stage has no couplings; the next stages' rows have tens (C2 level 0: 43 on average)
-      const auto kernel = k == 0 ? KLdltNarrow<true, 8, KC> : KLdltNarrow<true, 16, KC>;
-      kernel<<<dim3(T.compEnd - T.compBegin, chunks), 1024, 0, s>>>(T.compBegin, F.compPtr, F.fwdMatPtr, F.fwdMat, F.fwdPtr, F.fwdCol, F.fwdVal,
-                                                                    F.perm, F.dinv, src, lds, y, n, nullptr, 0, nullptr, K);
+      const auto kernel = k == 0 ? KLdltNarrow<true, kRhs, 8, KC> : KLdltNarrow<true, kRhs, 16, KC>;
+      kernel<<<dim3(T.compEnd - T.compBegin, chunks), 1024, 0, s>>>(T.compBegin, fwd, src, lds, y, n, nullptr, 0, K);
       continue;
     }
-    KLdltCouple<true, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.fwdPtr, F.fwdCol, F.fwdVal, F.perm, F.dinv, src, lds,
-                                                      y, n, buf, nWide, K);
-    KLdltWide<true, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.rowComp, F.compPtr, F.fwdMatPtr, F.fwdMat, buf, nWide,
-                                                    F.perm, F.dinv, y, n, k == last ? top : nullptr, nullptr, 0, nullptr, K);
+    KLdltCouple<true, kRhs, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, fwd, src, lds, y, n, buf, nWide, K);
+    KLdltWide<true, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.wideRows, fwd, buf, nWide, y, n, k == last ? top : nullptr,
+                                                    nullptr, 0, K);
   }
   for (int k = last; k >= 0; k--) {
     const LdltStage& T = F.stages[k];
     if (T.rowBegin == T.rowEnd) continue;
     if (!T.wide) {
-      KLdltNarrow<false, 8, KC><<<dim3(T.compEnd - T.compBegin, chunks), 1024, 0, s>>>(T.compBegin, F.compPtr, F.bwdMatPtr, F.bwdMat, F.bwdPtr,
-                                                                                       F.bwdCol, F.bwdVal, F.perm, F.dinv, nullptr, 0, y, n, dst,
-                                                                                       ldd, map, K);
+      KLdltNarrow<false, false, 8, KC><<<dim3(T.compEnd - T.compBegin, chunks), 1024, 0, s>>>(T.compBegin, bwd, nullptr, 0, y, n, dst, ldd, K);
       continue;
     }
-    if (k < last)
-      KLdltCouple<false, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.bwdPtr, F.bwdCol, F.bwdVal, F.perm, F.dinv, nullptr,
-                                                         0, y, n, buf, nWide, K);
-    KLdltWide<false, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.rowComp, F.compPtr, F.bwdMatPtr, F.bwdMat,
-                                                     k == last ? top : buf, nWide, F.perm, F.dinv, y, n, nullptr, dst, ldd, map, K);
+    if (k < last) KLdltCouple<false, false, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, bwd, nullptr, 0, y, n, buf, nWide, K);
+    KLdltWide<false, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.wideRows, bwd, k == last ? top : buf, nWide, y, n, nullptr,
+                                                     dst, ldd, K);
   }
 }
 
-void LdltSolve(DevLdlt& F, const double* src, int lds, double* dst, int ldd, const int* map, double* y, int K, hipStream_t s) {
+template <bool kRhs>
+static void LdltSolveAny(DevLdlt& F, const double* src, int lds, double* dst, int ldd, const int* index, const double* rhsX, double* y, int K,
+                         hipStream_t s) {
   if (F.n == 0) return;
   if (K < 1 || K > F.kcap) throw std::runtime_error("column count outside [1, capacity]");
   switch (std::min(K, 4)) {
-    case 1: LdltSolveChunks<1>(F, src, lds, dst, ldd, map, y, K, s); break;
-    case 2: LdltSolveChunks<2>(F, src, lds, dst, ldd, map, y, K, s); break;
-    case 3: LdltSolveChunks<3>(F, src, lds, dst, ldd, map, y, K, s); break;
-    default: LdltSolveChunks<4>(F, src, lds, dst, ldd, map, y, K, s); break;
+    case 1: LdltSolveChunks<kRhs, 1>(F, src, lds, dst, ldd, index, rhsX, y, K, s); break;
+    case 2: LdltSolveChunks<kRhs, 2>(F, src, lds, dst, ldd, index, rhsX, y, K, s); break;
+    case 3: LdltSolveChunks<kRhs, 3>(F, src, lds, dst, ldd, index, rhsX, y, K, s); break;
+    default: LdltSolveChunks<kRhs, 4>(F, src, lds, dst, ldd, index, rhsX, y, K, s); break;
   }
+}
+
+void LdltSolve(DevLdlt& F, const double* src, int lds, double* dst, int ldd, double* y, int K, hipStream_t s) {
+  LdltSolveAny<false>(F, src, lds, dst, ldd, F.perm, nullptr, y, K, s);
+}
+
+// The boundary part of a relaxation: x_B = A_BB^-1 (b_B - A_BD x) on level vectors of stride ld
+// (IterativeSolvers.inl:410-419; the forward stages form the right-hand side, deep texels are read only).
+static void LdltRelaxSolve(DevLdlt& F, double* x, const double* b, int ld, double* y, int K, hipStream_t s) {
+  LdltSolveAny<true>(F, b, ld, x, ld, F.texel, x, y, K, s);
 }
 
 static void CheckK(const DeviceSystem& ds, int K) {
@@ -894,13 +950,13 @@ void BoundarySolveLevel(DeviceSystem& ds, int l, const double* rhs, double* sol,
   CheckK(ds, K);
   DevLevel& d = ds.L[l];
   if (l + 1 >= ds.levels) throw std::runtime_error("the coarsest level has no boundary solver");
-  LdltSolve(d.factor, rhs, ld, sol, ld, nullptr, d.y, K, s);
+  LdltSolve(d.factor, rhs, ld, sol, ld, d.y, K, s);
 }
 
 void CoarseSolve(DeviceSystem& ds, const double* rhs, double* sol, int K, int ld, hipStream_t s) {
   CheckK(ds, K);
   DevLevel& d = ds.L[ds.levels - 1];
-  LdltSolve(d.factor, rhs, ld, sol, ld, nullptr, d.y, K, s);
+  LdltSolve(d.factor, rhs, ld, sol, ld, d.y, K, s);
 }
 
 // The band sweep of a level's deep rows, columns in chunks of up to kBandColumns, every chunk a workgroup
@@ -942,11 +998,7 @@ void BandSweepLevel(DeviceSystem& ds, int l, double* x, const double* b, double*
 void RelaxLevel(DeviceSystem& ds, int l, double* x, const double* b, double* r, int K, int ld, bool withResidual, hipStream_t s) {
   CheckK(ds, K);
   DevLevel& d = ds.L[l];
-  if (d.B > 0) {
-    const long bk = (long)d.B * K;
-    KBoundaryRhs<<<Blocks(bk, 256), 256, 0, s>>>(d.B, d.bgi, d.bd.rowptr, d.bd.col, d.bd.val, x, b, d.vb, K, ld);
-    LdltSolve(d.factor, d.vb, d.B, x, ld, d.bgi, d.y, K, s);
-  }
+  LdltRelaxSolve(d.factor, x, b, ld, d.y, K, s);
   BandSweep(d, x, b, K, ld, s);
   if (withResidual) ResidualLevel(ds, l, x, b, r, K, ld, s);
 }

@@ -250,7 +250,7 @@ void BuildLdltStages(const Ldlt& F, LdltStages& S, int topRows) {
   for (int c = 0; c < nComp; c++) {
     const int m = count[c];
     long f = 0, b = 0;
-    if (wide[c]) f = b = (long)m * m;
+    if (wide[c]) f = b = (long)m * LdltWideStride(m);
     else
       for (int r0 = 0; r0 < m; r0 += kLdltBlock) {
         const int nr = std::min(kLdltBlock, m - r0);
@@ -309,7 +309,7 @@ void BuildLdltStages(const Ldlt& F, LdltStages& S, int topRows) {
     double *f = S.fwdMat.data() + S.fwdMatPtr[c], *b = S.bwdMat.data() + S.bwdMatPtr[c];
 #pragma omp parallel for schedule(static)
     for (int r = 0; r < m; r++)
-      for (int j = 0; j < m; j++) f[(size_t)r * m + j] = inv[(size_t)r * m + j], b[(size_t)r * m + j] = inv[(size_t)j * m + r];
+      for (int j = 0; j < m; j++) f[(size_t)r * LdltWideStride(m) + j] = inv[(size_t)r * m + j], b[(size_t)r * LdltWideStride(m) + j] = inv[(size_t)j * m + r];
   }
 }
 

@@ -41,6 +41,8 @@ struct LdltStage {
   bool wide = false;                   // some component has more than kLdltNarrowRows rows (or the top)
 };
 
+constexpr int LdltWideStride(int rows) { return (rows + 1) / 2 * 2; }  // even: rows are read in pairs
+
 struct LdltStages {
   int n = 0;
   std::vector<LdltStage> stages;       // in forward order; the last is the top
@@ -52,7 +54,8 @@ struct LdltStages {
   std::vector<double> fwdVal, bwdVal;
   // Inverses.  Narrow component: for each block of kLdltBlock rows the columns its rows can reach
   // (forward: columns before the block's end; backward: from its begin), column-major, the block's
-  // rows contiguous.  Wide component: the whole matrix row-major (forward, then transposed).
+  // rows contiguous.  Wide component: the whole matrix row-major (backward: transposed), rows of
+  // LdltWideStride doubles.
   std::vector<long> fwdMatPtr, bwdMatPtr;  // per component
   std::vector<double> fwdMat, bwdMat;
   int wideBegin = 0;                   // first row of the first wide stage (the later stages are all wide)

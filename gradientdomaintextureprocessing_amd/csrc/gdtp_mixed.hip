@@ -2215,7 +2215,7 @@ void MixedVCycle(DeviceSystem& ds, MixedSystem& ms, int K, hipStream_t s, bool z
       KMixDenseCoarse<<<c.N, 256, 0, s>>>(c.N, ms.coarseInv, c.g2d, c.rhs, c.e, c.Nd, K);
     } else {
       KMixGather<<<NBlk(nk, 256), 256, 0, s>>>(c.N, c.g2d, c.rhs, c.Nd, ms.coarseRhs, K);
-      LdltSolve(ms.coarse, ms.coarseRhs, c.N, ms.coarseX, c.N, nullptr, ms.coarseY, K, s);
+      LdltSolve(ms.coarse, ms.coarseRhs, c.N, ms.coarseX, c.N, ms.coarseY, K, s);
       KMixScatter<<<NBlk(nk, 256), 256, 0, s>>>(c.N, c.g2d, ms.coarseX, c.e, c.Nd, K);
     }
   }
