@@ -54,7 +54,8 @@ struct DevMixLevel {
   int8_t* type = nullptr;          // [Nd]: -1 inactive, 0/1 boundary, 2 deep
   int* g2d = nullptr;              // [N] compact global index -> dense index
   int nTiles = 0;
-  bool chartSweeps = false;         // small charts: one workgroup per chart runs all four colours of a sweep
+  bool chartSweeps = false;         // small charts: one workgroup per chart and column runs all four colours of a sweep
+  int chartPlane = 0;               // sub-grid positions of the largest chart
   int* tiles = nullptr;            // 3 ints per tile: chart, a0, b0 (sub-grid origin)
   unsigned long long* deepMask = nullptr;    // [tile][plane][tile row]: bit x set where texel (a0 + x, b0 + row) is deep
   unsigned long long* activeMask = nullptr;  // the same for active texels (deep or boundary)

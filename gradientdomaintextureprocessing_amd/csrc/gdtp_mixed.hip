@@ -27,7 +27,7 @@ namespace gdtp {
 static constexpr int kTA = 64, kTB = 4;  // tile of the sub-grid per workgroup: 64 x 4 (256 threads)
 static constexpr int kDenseCoarseMax = 6000;  // coarsest levels up to this size use a dense inverse
 static constexpr int kDotBlocks = 1024;       // partial sums per column of the flexible-CG dot products
-static constexpr long kChartSweepMax = 2048;  // largest chart colour plane (texels) swept by one workgroup
+static constexpr long kChartSweepMax = 2048;  // largest chart colour plane (texels) swept by one workgroup (two per thread)
 static inline unsigned NBlk(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 __device__ __forceinline__ long DenseIdx(const MixChart& c, long plane, int i, int j) {
@@ -126,37 +126,13 @@ __device__ __forceinline__ float GsStencil(long idx, long Nd, const float* __res
   }
 }
 
-// kHalf: the stencil as FP16 ratios with an FP32 row-sum correction (stc, sth), else the FP32
-// stencil st.
-template <bool kHalf>
-__device__ __forceinline__ void DeepGsTexel(const MixChart& c, long plane, long Nd, int q, int a, int b, const float* __restrict__ st,
-                                            const float2* __restrict__ stc, const uint4* __restrict__ sth, float* e,
-                                            const float* __restrict__ rhs, int K) {
-  const int i = 2 * a + (q & 1), j = 2 * b + (q >> 1);
-  if (i >= c.w || j >= c.h) return;
-  const long idx = (long)q * plane + c.base2 + (long)b * c.w2 + a;
-  float corr, cf[9];
-  const float c4 = GsStencil<kHalf>(idx, Nd, st, stc, sth, corr, cf);
-  if (c4 == 0.0f) return;
-  int nb[9];
-#pragma unroll
-  for (int k = 0; k < 9; k++) nb[k] = DenseByte(c, plane, i + k % 3 - 1, j + k / 3 - 1);
-  ForColumnChunks(K, [&](int c0, auto kc) {
-    constexpr int KC = decltype(kc)::value;
-    float v[KC][9], r[KC];
-#pragma unroll
-    for (int ch = 0; ch < KC; ch++) {
-#pragma unroll
-      for (int k = 0; k < 9; k++)
-        if (k != 4) v[ch][k] = Ld(e + (c0 + ch) * Nd, nb[k]);
-      r[ch] = Ld(rhs + (c0 + ch) * Nd, nb[4]);
-    }
-#pragma unroll
-    for (int ch = 0; ch < KC; ch++) e[(long)(c0 + ch) * Nd + idx] = GsValue<kHalf>(cf, v[ch], c4, corr, r[ch]);
-  });
-}
+// An FP32 stencil's off-diagonal ratios.
+struct Stencil9 {
+  float v[9];
+};
 
-// One colour plane of a tiled level: wave w of the workgroup takes row w of its 64 x 4 tile, whose
+// One colour plane of a tiled level (kHalf: the stencil as FP16 ratios with an FP32 row-sum correction
+// stc, sth, else the FP32 stencil st): wave w of the workgroup takes row w of its 64 x 4 tile, whose
 // deep texels it reads from a host-built bit mask (one uniform 64-bit load per wave) instead of
 // from the stencil, so that a deep texel's stencil, neighbour and rhs loads all go out together
 // (one memory round trip instead of two).  Tiles in XCD-contiguous order (XcdTile).
@@ -201,64 +177,106 @@ __global__ __launch_bounds__(256) void KMixDeepGs(int q, int nTiles, const int* 
   });
 }
 
-// DeepGsTexel for the small levels swept one chart per workgroup, which latency bounds: a texel
-// whose 3x3 neighbourhood lies inside the chart (a test on its position alone; every deep texel
-// passes it) issues its stencil, neighbour and rhs loads together and only then learns from c4
-// whether it is deep, one memory round trip instead of two.  (The other texels cannot be deep.)
+// Four-colour sweeps of the levels whose charts are small, one workgroup per chart and column, colours
+// in order (post: 3..0) separated by barriers: deep stencils never reach across charts, so this is
+// exactly the launches of KMixDeepGs in one, for levels whose charts are small enough that latency, not
+// memory, bounds a sweep.  `sweeps` consecutive sweeps (post-smoothing runs its sweeps back to back) run
+// in one launch.  The chart's four planes of e live in LDS and every texel's stencil and rhs in
+// registers (kIt texels per thread and colour), all loaded in one round trip before the first colour; a
+// colour then waits for LDS only.  (A 512^2 cube, three columns, us a launch: 11.7 with e and each
+// colour's operands read through the L2 colour by colour; 3.9 on levels of up to 1024 positions, and 11
+// on the level of 1764, where the one CU's arithmetic bounds a colour.)  A texel
+// whose 3x3 neighbourhood lies inside the chart (every deep texel) loads its stencil, and learns from
+// c4 whether it is deep.  All threads reach every barrier.
 template <bool kHalf>
-__device__ __forceinline__ void ChartGsTexel(const MixChart& c, long plane, long Nd, int q, int a, int b, const float* __restrict__ st,
-                                             const float2* __restrict__ stc, const uint4* __restrict__ sth, float* e,
-                                             const float* __restrict__ rhs, int K) {
-  const int i = 2 * a + (q & 1), j = 2 * b + (q >> 1);
-  if (i < 1 || j < 1 || i + 1 >= c.w || j + 1 >= c.h) return;
-  const int idx = (int)((long)q * plane + c.base2 + (long)b * c.w2 + a);
-  float c4, corr = 0.0f, cf[9];
-  if constexpr (kHalf) {
-    const float2 cd = stc[idx];
-    const uint4 w = sth[idx];
-    c4 = cd.x, corr = 0.125f * cd.y;
-    Unpack<true>(w, cf);
-  } else {
-    c4 = st[4 * Nd + idx];
-#pragma unroll
-    for (int k = 0; k < 9; k++) cf[k] = k == 4 ? 0.0f : st[k * Nd + idx];
-  }
-  int nb[9];
-#pragma unroll
-  for (int k = 0; k < 9; k++) nb[k] = DenseByte(c, plane, i + k % 3 - 1, j + k / 3 - 1);
-  ForColumnChunks(K, [&](int c0, auto kc) {
-    constexpr int KC = decltype(kc)::value;
-    float v[KC][9], r[KC];
-#pragma unroll
-    for (int ch = 0; ch < KC; ch++) {
-#pragma unroll
-      for (int k = 0; k < 9; k++)
-        if (k != 4) v[ch][k] = Ld(e + (c0 + ch) * Nd, nb[k]);
-      r[ch] = Ld(rhs + (c0 + ch) * Nd, nb[4]);
-    }
-    if (c4 == 0.0f) return;  // not deep: nothing to update
-#pragma unroll
-    for (int ch = 0; ch < KC; ch++) e[(long)(c0 + ch) * Nd + idx] = GsValue<kHalf>(cf, v[ch], c4, corr, r[ch]);
-  });
-}
-
-// The same four-colour sweep with one 1024-thread workgroup per chart, colours in order (post:
-// 3..0) separated by barriers: deep stencils never reach across charts, so this is exactly the
-// four launches of KMixDeepGs in one, for levels whose charts are small enough that launch
-// latency, not memory, bounds a sweep.  `sweeps` consecutive sweeps (post-smoothing runs its sweeps
-// back to back) in one launch.  All threads reach every barrier.
-template <bool kHalf>
+struct ChartOperands {
+  typename std::conditional<kHalf, uint4, Stencil9>::type sten;
+  float c4, corr, r;
+};
+template <bool kHalf, int kIt>
 __global__ __launch_bounds__(1024) void KMixChartGs(int post, int sweeps, const MixChart* __restrict__ charts, long plane, long Nd,
                                                     const float* __restrict__ st, const float2* __restrict__ stc,
-                                                    const uint4* __restrict__ sth, float* e, const float* __restrict__ rhs, int K) {
+                                                    const uint4* __restrict__ sth, float* e, const float* __restrict__ rhs) {
+  extern __shared__ float sm[];  // [4][n]
   const MixChart c = charts[blockIdx.x];
   const int aw = (c.w + 1) / 2, n = aw * c.h2;
-  for (int sw = 0; sw < sweeps; sw++)
-    for (int qq = 0; qq < 4; qq++) {
-      const int q = post ? 3 - qq : qq;
-      for (int t = threadIdx.x; t < n; t += blockDim.x) ChartGsTexel<kHalf>(c, plane, Nd, q, t % aw, t / aw, st, stc, sth, e, rhs, K);
-      __syncthreads();
+  e += (long)blockIdx.y * Nd, rhs += (long)blockIdx.y * Nd;
+  ChartOperands<kHalf> op[4][kIt];
+  float old[4][kIt];
+  int at[kIt];  // dense index in plane 0 of the thread's sub-grid positions
+#pragma unroll
+  for (int it = 0; it < kIt; it++) {
+    const int t = min((int)(threadIdx.x + blockDim.x * it), n - 1), a = t % aw, b = t / aw;
+    at[it] = c.base2 + b * c.w2 + a;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int idx = q * (int)plane + at[it];
+      ChartOperands<kHalf>& o = op[q][it];
+      if constexpr (kHalf) {
+        const float2 cd = stc[idx];
+        o.sten = sth[idx];
+        o.c4 = cd.x, o.corr = 0.125f * cd.y;
+      } else {
+        o.c4 = st[4 * Nd + idx], o.corr = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 9; k++) o.sten.v[k] = k == 4 ? 0.0f : st[k * Nd + idx];
+      }
+      o.r = rhs[idx];
+      old[q][it] = e[idx];
     }
+  }
+#pragma unroll
+  for (int it = 0; it < kIt; it++) {
+    const int t = threadIdx.x + blockDim.x * it, a = t % aw, b = t / aw;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int i = 2 * a + (q & 1), j = 2 * b + (q >> 1);
+      if (t < n) sm[q * n + t] = old[q][it];
+      if (t >= n || i < 1 || j < 1 || i + 1 >= c.w || j + 1 >= c.h) op[q][it].c4 = 0.0f;
+    }
+  }
+  __syncthreads();
+  auto colour = [&](auto qc) {
+    constexpr int q = decltype(qc)::value;
+#pragma unroll
+    for (int it = 0; it < kIt; it++) {
+      const ChartOperands<kHalf>& o = op[q][it];
+      if (o.c4 == 0.0f) continue;  // not deep: nothing to update
+      const int t = threadIdx.x + blockDim.x * it;
+      float cf[9], v[9];
+      if constexpr (kHalf) Unpack<true>(o.sten, cf);
+      else {
+#pragma unroll
+        for (int k = 0; k < 9; k++) cf[k] = o.sten.v[k];
+      }
+#pragma unroll
+      for (int k = 0; k < 9; k++) {
+        if (k == 4) {
+          v[k] = 0.0f;
+          continue;
+        }
+        // neighbour (i + di, j + dj): plane p, sub-grid offset (da, db) (floor division by 2)
+        const int ni = (q & 1) + k % 3 - 1, nj = (q >> 1) + k / 3 - 1;
+        v[k] = sm[((ni & 1) | (nj & 1) << 1) * n + t + (nj >> 1) * aw + (ni >> 1)];
+      }
+      sm[q * n + t] = GsValue<kHalf>(cf, v, o.c4, o.corr, o.r);
+    }
+    __syncthreads();
+  };
+  for (int sw = 0; sw < sweeps; sw++) {
+    if (post) {
+      colour(std::integral_constant<int, 3>()), colour(std::integral_constant<int, 2>());
+      colour(std::integral_constant<int, 1>()), colour(std::integral_constant<int, 0>());
+    } else {
+      colour(std::integral_constant<int, 0>()), colour(std::integral_constant<int, 1>());
+      colour(std::integral_constant<int, 2>()), colour(std::integral_constant<int, 3>());
+    }
+  }
+#pragma unroll
+  for (int it = 0; it < kIt; it++)
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (op[q][it].c4 != 0.0f) e[(long)q * plane + at[it]] = sm[q * n + threadIdx.x + blockDim.x * it];
 }
 
 // ------------------------------------------------------------------ colour pairs
@@ -464,9 +482,6 @@ __host__ __device__ constexpr FusedBox FusedRegion(bool post, int q) {
 // The operands one thread fetches for its texels of one colour's region (at most kIt of them):
 // stencil (FP16 ratios still packed, or FP32), rhs and, for the first colour, the texel's old
 // value where it is not deep.
-struct Stencil9 {
-  float v[9];
-};
 template <bool kHalf, bool kFirst, int KC, int kIt>
 struct FusedOperands {
   float c4[kIt], corr[kIt], r[kIt][KC], old[kFirst ? kIt : 1][KC];
@@ -1671,6 +1686,7 @@ void UploadMixed(const Hierarchy& h, const OperatorHierarchy& oh, DeviceSystem& 
       long largest = 0;
       for (const MixChart& m : d.hcharts) largest = std::max(largest, (long)((m.w + 1) / 2) * m.h2);
       d.chartSweeps = largest <= kChartSweepMax;
+      d.chartPlane = (int)largest;
     }
     d.plane = base, d.Nd = 4 * base;
     if (4 * d.Nd >= (1L << 31)) throw std::runtime_error("texel atlas too large for the mixed-precision solver (2 GiB per dense FP32 column)");
@@ -2148,6 +2164,23 @@ static void BoundarySweeps(MixedSystem& ms, DevMixLevel& d, int K, hipStream_t s
   }
 }
 
+// `sweeps` four-colour sweeps of a level swept one chart per workgroup.
+static void ChartLaunch(DevMixLevel& d, bool post, int sweeps, int K, hipStream_t s) {
+  // one texel of each colour per thread up to 1024 sub-grid positions, else two (kChartSweepMax)
+  const int threads = std::min(1024, (d.chartPlane + 63) / 64 * 64);
+  const size_t lds = 4 * (size_t)d.chartPlane * sizeof(float);
+  const dim3 grid(d.nCharts, K);
+#define GDTP_CHART(H, IT) KMixChartGs<H, IT><<<grid, threads, lds, s>>>(post ? 1 : 0, sweeps, d.charts, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.e, d.rhs)
+  if (d.chartPlane <= 1024) {
+    if (d.stencilH) GDTP_CHART(true, 1);
+    else GDTP_CHART(false, 1);
+  } else {
+    if (d.stencilH) GDTP_CHART(true, 2);
+    else GDTP_CHART(false, 2);
+  }
+#undef GDTP_CHART
+}
+
 // Pre-smoothing: (boundary Schwarz, deep colours 0..3) x nuPre; post-smoothing: (deep colours
 // 3..0) x nuPost, then one boundary Schwarz step (a Schwarz step after every post sweep converged
 // marginally faster per V-cycle but cost more per digit: C2 15.1 against 13.9 ms per solve).
@@ -2161,10 +2194,7 @@ static void Smooth(MixedSystem& ms, int l, int K, bool post, hipStream_t s, bool
     if (d.nTiles > 0 && d.chartSweeps) {
       // post-smoothing's deep sweeps follow one another with nothing between them: one launch
       const int sweeps = post ? nu : 1;
-      if (d.stencilH)
-        KMixChartGs<true><<<d.nCharts, 1024, 0, s>>>(post ? 1 : 0, sweeps, d.charts, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.e, d.rhs, K);
-      else
-        KMixChartGs<false><<<d.nCharts, 1024, 0, s>>>(post ? 1 : 0, sweeps, d.charts, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.e, d.rhs, K);
+      ChartLaunch(d, post, sweeps, K, s);
       if (post) it = nu - 1;
     } else if (d.nTiles > 0) {
       DeepSweep(ms, d, post, K, s, it == 0 ? prolong : nullptr);
