@@ -28,7 +28,7 @@ static constexpr int kTA = 64, kTB = 4;  // tile of the sub-grid per workgroup: 
 static constexpr int kDenseCoarseMax = 6000;  // coarsest levels up to this size use a dense inverse
 static constexpr int kDotBlocks = 1024;       // partial sums per column of the flexible-CG dot products
 static constexpr long kChartSweepMax = 2048;  // largest chart colour plane (texels) swept by one workgroup (two per thread)
-static inline unsigned NBlk(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
+__host__ __device__ static inline unsigned NBlk(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 __device__ __forceinline__ long DenseIdx(const MixChart& c, long plane, int i, int j) {
   int q = (i & 1) | ((j & 1) << 1);
@@ -56,20 +56,36 @@ __device__ __forceinline__ int XcdTile(int b, int n) {
   return x * per + min(x, rem) + k;
 }
 
-// Columns in chunks of up to four with the chunk width as a compile-time constant, so that a
-// kernel can issue every load of a chunk before its first store (one memory round trip per chunk
-// instead of one per column).
-// kMax: the widest chunk (4, or 3 where a kernel holds many values per column and the register
+// Columns in chunks of up to kMax, a chunk per workgroup: workgroups are numbered tile by tile and
+// within a tile chunk by chunk, in XCD-contiguous order, so that a tile's chunks run on one XCD one
+// after another and read its stencil, masks and row tables from that XCD's L2.  (With the chunks in a
+// loop inside the workgroup, each waited for the one before it: 3.0 M texels x 64 columns, V-cycle
+// residual of level 0 1027 us, 896 so; one colour pair of level 0, 16 launches, 554 us, one launch 448; a
+// solve pair 348 to 292 ms.)
+struct TileChunk {
+  int tile, c0;
+};
+template <int kMax>
+__device__ __forceinline__ TileChunk TileOf(int b, int nTiles, int K) {
+  const int chunks = (K + kMax - 1) / kMax;
+  if (chunks == 1) return {XcdTile(b, nTiles), 0};
+  const int v = XcdTile(b, nTiles * chunks);
+  return {v / chunks, v % chunks * kMax};
+}
+template <int kMax>
+static inline unsigned ChunkBlocks(long blocks, int K) { return (unsigned)(blocks * ((K + kMax - 1) / kMax)); }
+
+// f(chunk width as a compile-time constant), so that a kernel can issue every load of its chunk before
+// its first store (one memory round trip per chunk instead of one per column).
+// kMax: the widest chunk (4, or less where a kernel holds many values per column and the register
 // count of the widest chunk would halve its occupancy).
 template <int kMax = 4, class F>
-__device__ __forceinline__ void ForColumnChunks(int K, F&& f) {
-  for (int c0 = 0; c0 < K; c0 += kMax) {
-    switch (min(kMax, K - c0)) {
-      case 4: if constexpr (kMax >= 4) f(c0, std::integral_constant<int, 4>()); break;
-      case 3: f(c0, std::integral_constant<int, 3>()); break;
-      case 2: f(c0, std::integral_constant<int, 2>()); break;
-      default: f(c0, std::integral_constant<int, 1>()); break;
-    }
+__device__ __forceinline__ void ForChunk(int K, int c0, F&& f) {
+  switch (min(kMax, K - c0)) {
+    case 4: if constexpr (kMax >= 4) f(std::integral_constant<int, 4>()); break;
+    case 3: if constexpr (kMax >= 3) f(std::integral_constant<int, 3>()); break;
+    case 2: f(std::integral_constant<int, 2>()); break;
+    default: f(std::integral_constant<int, 1>()); break;
   }
 }
 
@@ -141,7 +157,8 @@ __global__ __launch_bounds__(256) void KMixDeepGs(int q, int nTiles, const int* 
                                                   const unsigned long long* __restrict__ deepMask, const MixChart* __restrict__ charts,
                                                   long plane, long Nd, const float* __restrict__ st, const float2* __restrict__ stc,
                                                   const uint4* __restrict__ sth, float* e, const float* __restrict__ rhs, int K) {
-  const int tile = XcdTile(blockIdx.x, nTiles), row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
+  const TileChunk v = TileOf<4>(blockIdx.x, nTiles, K);
+  const int tile = v.tile, c0 = v.c0, row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
   const unsigned long long m = deepMask[((long)tile * 4 + q) * kTB + row];
   if (!((m >> tx) & 1ull)) return;
   const int* T = tiles + 3 * tile;
@@ -162,7 +179,7 @@ __global__ __launch_bounds__(256) void KMixDeepGs(int q, int nTiles, const int* 
   int nb[9];
 #pragma unroll
   for (int k = 0; k < 9; k++) nb[k] = DenseByte(c, plane, i + k % 3 - 1, j + k / 3 - 1);
-  ForColumnChunks(K, [&](int c0, auto kc) {
+  ForChunk(K, c0, [&](auto kc) {
     constexpr int KC = decltype(kc)::value;
     float v[KC][9], r[KC];
 #pragma unroll
@@ -378,17 +395,20 @@ __device__ __forceinline__ void PairUpdate(PairTexel<kHalf, KC>& T, bool second,
 }
 
 template <bool kHalf, int KC, int NT, int P>
-__global__ __launch_bounds__(NT) void KMixPairGs(int qa, const int* __restrict__ rows, const unsigned long long* __restrict__ rowMask,
+__global__ __launch_bounds__(NT) void KMixPairGs(int qa, int chunks, const int* __restrict__ rows, const unsigned long long* __restrict__ rowMask,
                                                            int nRows, const MixChart* __restrict__ charts, long plane, long Nd,
                                                            const float* __restrict__ st, const float2* __restrict__ stc,
                                                            const uint4* __restrict__ sth, float* e, const float* __restrict__ rhs) {
   __shared__ float sm[KC][P * NT];
   const int qb = qa ^ 1;
+  // workgroups as in TileOf: a workgroup's rows for one chunk of columns
+  const int vb = XcdTile(blockIdx.x, nRows * chunks), rowBlock = vb / chunks;
+  e += (long)(vb % chunks) * KC * Nd, rhs += (long)(vb % chunks) * KC * Nd;
   if constexpr (P == 1) {
     // packed rows: wave w takes the 64 texels [R.z, R.z + 64) of row (chart R.x, R.y), clipped to
     // the row's span end R.w; a row's waves are consecutive, so its texels have consecutive LDS
     // slots.  One texel per thread and colour; both colours' stencils are loaded together.
-    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), slot = XcdTile(blockIdx.x, nRows) * (NT / 64) + w;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), slot = rowBlock * (NT / 64) + w;
     const int4 R = reinterpret_cast<const int4*>(rows)[slot];
     const MixChart c = charts[R.x];
     const int b = R.y, a1 = R.w, t = threadIdx.x, a = R.z + t % 64;
@@ -406,7 +426,7 @@ __global__ __launch_bounds__(NT) void KMixPairGs(int qa, const int* __restrict__
     __syncthreads();
     PairUpdate(B, true, qb, t, sm, e, Nd);
   } else {  // one row per workgroup: span [R.z, R.w) of row (chart R.x, R.y)
-    const int4 R = reinterpret_cast<const int4*>(rows)[XcdTile(blockIdx.x, nRows)];
+    const int4 R = reinterpret_cast<const int4*>(rows)[rowBlock];
     const MixChart c = charts[R.x];
     const int b = R.y, a0 = R.z, a1 = R.w;
     for (int p = 0; p < P; p++) {
@@ -624,14 +644,19 @@ struct FusedPhase {
 // on at most one colour's compute), or all at the start (kFusedAllAhead: one memory round trip per
 // tile).  NT threads per workgroup; kXcd: XCD-contiguous tile order (XcdTile).
 template <bool kHalf, bool kPost, bool kProlong, int TA, int TB, int NT, int KC, int kAhead, bool kXcd>
-__global__ __launch_bounds__(NT) void KMixDeepGsFused(const int* __restrict__ tiles, const MixChart* __restrict__ charts, long plane,
+__global__ __launch_bounds__(NT) void KMixDeepGsFused(int chunks, const int* __restrict__ tiles, const MixChart* __restrict__ charts, long plane,
                                                       long Nd, const float* __restrict__ st, const float2* __restrict__ stc,
                                                       const uint4* __restrict__ sth, const int8_t* __restrict__ type,
                                                       const float* __restrict__ eIn, float* __restrict__ eOut,
                                                       const float* __restrict__ rhs, FusedProlong pr) {
   constexpr int WX = TA + 4, WN = WX * (TB + 2), kLoads = (3 * WN + NT - 1) / NT;
   __shared__ float sm[KC * 4 * WN];
-  const int* T = tiles + 3 * (kXcd ? XcdTile(blockIdx.x, gridDim.x) : (int)blockIdx.x);
+  // workgroups as in TileOf: a tile for one chunk of columns
+  const int vb = kXcd ? XcdTile(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+  const long off = (long)(vb % chunks) * KC * Nd;
+  eIn += off, eOut += off, rhs += off;
+  if constexpr (kProlong) pr.ce += (long)(vb % chunks) * KC * pr.cNd;
+  const int* T = tiles + 3 * (vb / chunks);
   const MixChart c = charts[T[0]];
   MixChart cc{};
   if constexpr (kProlong) cc = pr.cch[T[0]];
@@ -728,7 +753,7 @@ __global__ __launch_bounds__(NT) void KMixDeepGsFused(const int* __restrict__ ti
 // registers, eight waves per SIMD instead of six, level 0 at C2 219 against 221 us; 4 on small
 // levels, which are latency-bound and pay for a second round trip).
 template <int kChunk>
-__device__ __forceinline__ void ResidualDeepTile(int vb, const int* __restrict__ tiles, const unsigned long long* __restrict__ deepMask,
+__device__ __forceinline__ void ResidualDeepTile(int vb, int c0, const int* __restrict__ tiles, const unsigned long long* __restrict__ deepMask,
                                                  const MixChart* __restrict__ charts, long plane, long Nd, const float* __restrict__ sym,
                                                  const float* __restrict__ e, const float* __restrict__ rhs, float* res, int K, int zeroQ) {
   const int row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
@@ -741,7 +766,7 @@ __device__ __forceinline__ void ResidualDeepTile(int vb, const int* __restrict__
     const int i = 2 * a + (q & 1), j = 2 * b + (q >> 1);
     const long idx = (long)q * plane + c.base2 + (long)b * c.w2 + a;
     if (q == zeroQ) {  // relaxed last by the FP32 smoother: its deep rows hold exactly, so the residual is zero
-      for (int ch = 0; ch < K; ch++) res[(long)ch * Nd + idx] = 0.0f;
+      for (int ch = c0; ch < min(K, c0 + kChunk); ch++) res[(long)ch * Nd + idx] = 0.0f;
       continue;
     }
     const float a4 = sym[4 * Nd + idx];
@@ -751,7 +776,7 @@ __device__ __forceinline__ void ResidualDeepTile(int vb, const int* __restrict__
     // own lower couplings and a4; upper coupling k from slot 8-k of that neighbour
     const float cf[9] = {sym[idx], sym[Nd + idx], sym[2 * Nd + idx], sym[3 * Nd + idx], a4,
                          Ld(sym + 3 * Nd, nb[5]), Ld(sym + 2 * Nd, nb[6]), Ld(sym + Nd, nb[7]), Ld(sym, nb[8])};
-    ForColumnChunks<kChunk>(K, [&](int c0, auto kc) {
+    ForChunk<kChunk>(K, c0, [&](auto kc) {
       constexpr int KC = decltype(kc)::value;
       float v[KC][9], r[KC];
 #pragma unroll
@@ -789,15 +814,15 @@ __device__ __forceinline__ T Pick(const T (&a)[4], int q) {
 // Boundary-row residual rhs - A e (FP32).  out: compact [K][B] when `compact`, else the dense
 // vector [K][Nd] at the row's texel.  A row entry is one 64-bit word (dense column, FP32 value
 // bits): one load per entry instead of two.
-__device__ __forceinline__ void BoundaryResidualRows(int vb, int B, const int* __restrict__ bdIdx, const int* __restrict__ rp,
+__device__ __forceinline__ void BoundaryResidualRows(int vb, int c0, int B, const int* __restrict__ bdIdx, const int* __restrict__ rp,
                                                      const int2* __restrict__ ent, const float* __restrict__ dg, const float* __restrict__ e,
                                                      const float* __restrict__ rhs, float* out, int compact, long Nd, int K) {
   const int r = (int)(((long)vb * blockDim.x + threadIdx.x) / kRowLanes), lane = threadIdx.x % kRowLanes;
   if (r >= B) return;  // whole row groups leave together
   const int k0 = rp[r], k1 = rp[r + 1];
   const long d = bdIdx[r];
-  for (int c0 = 0; c0 < K; c0 += 4) {
-    const int kc = min(4, K - c0);
+  const int kc = min(4, K - c0);
+  {
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int k = k0 + lane; k < k1; k += kRowLanes) {
       const int2 w = ent[k];
@@ -822,11 +847,12 @@ __global__ __launch_bounds__(256) void KMixBoundaryResidual(int B, const int* __
                                                             const int2* __restrict__ ent, const float* __restrict__ dg,
                                                             const float* __restrict__ e, const float* __restrict__ rhs, float* out,
                                                             int compact, long Nd, int K) {
-  BoundaryResidualRows(blockIdx.x, B, bdIdx, rp, ent, dg, e, rhs, out, compact, Nd, K);
+  const TileChunk v = TileOf<4>(blockIdx.x, NBlk((long)B * kRowLanes, 256), K);
+  BoundaryResidualRows(v.tile, v.c0, B, bdIdx, rp, ent, dg, e, rhs, out, compact, Nd, K);
 }
 
 static constexpr int kResidualWideTiles = 1024;  // levels with more 64 x 4 tiles load two columns at a time
-// The residual of a level after pre-smoothing in one launch: blocks [0, nTiles) take the deep tiles,
+// The residual of a level after pre-smoothing in one launch: the first blocks take the deep tiles,
 // the others the boundary rows (disjoint outputs, so the two parts overlap on the device).
 template <int kChunk>
 __global__ __launch_bounds__(256) void KMixResidual(int nTiles, const int* __restrict__ tiles, const unsigned long long* __restrict__ deepMask,
@@ -835,9 +861,14 @@ __global__ __launch_bounds__(256) void KMixResidual(int nTiles, const int* __res
                                                     const float* __restrict__ rhs, float* res, int K, int zeroQ, int B,
                                                     const int* __restrict__ bdIdx, const int* __restrict__ rp, const int2* __restrict__ ent,
                                                     const float* __restrict__ dg) {
-  if ((int)blockIdx.x < nTiles)
-    ResidualDeepTile<kChunk>(XcdTile(blockIdx.x, nTiles), tiles, deepMask, charts, plane, Nd, sym, e, rhs, res, K, zeroQ);
-  else BoundaryResidualRows(blockIdx.x - nTiles, B, bdIdx, rp, ent, dg, e, rhs, res, 0, Nd, K);
+  const int deepBlocks = nTiles * ((K + kChunk - 1) / kChunk);
+  if ((int)blockIdx.x < deepBlocks) {
+    const TileChunk v = TileOf<kChunk>(blockIdx.x, nTiles, K);
+    ResidualDeepTile<kChunk>(v.tile, v.c0, tiles, deepMask, charts, plane, Nd, sym, e, rhs, res, K, zeroQ);
+  } else {
+    const TileChunk v = TileOf<4>(blockIdx.x - deepBlocks, NBlk((long)B * kRowLanes, 256), K);
+    BoundaryResidualRows(v.tile, v.c0, B, bdIdx, rp, ent, dg, e, rhs, res, 0, Nd, K);
+  }
 }
 
 // Restricted additive Schwarz over the boundary rows: one workgroup of W waves per block, the
@@ -880,7 +911,9 @@ __global__ __launch_bounds__(64 * W) void KMixSchwarz(const int* __restrict__ co
   static_assert(kBlockExtMax % kJ == 0, "padded extended rows fit the staged residual");
   __shared__ float R[4 * kBlockExtMax];
   __shared__ float P[W][4][kBlockCore];
-  const int b = blockIdx.x, c0 = corePtr[b], nc = corePtr[b + 1] - c0, x0 = extPtr[b], nx = extPtr[b + 1] - x0;
+  const TileChunk v = TileOf<4>(blockIdx.x, gridDim.x / ((K + 3) / 4), K);
+  const int b = v.tile, ch0 = v.c0, kc = min(4, K - ch0);
+  const int c0 = corePtr[b], nc = corePtr[b + 1] - c0, x0 = extPtr[b], nx = extPtr[b + 1] - x0;
   const TM* M = mat + matPtr[b];
   const int i = threadIdx.x % 64, part = threadIdx.x / 64;
   // The first kPre of this lane's loads of the block inverse (row i, load slots part, part + W,
@@ -900,8 +933,7 @@ __global__ __launch_bounds__(64 * W) void KMixSchwarz(const int* __restrict__ co
       for (int t = 0; t < kJ; t++) mv[ss][t] = 0.0f;
   }
   const int nxPad = (nx + kJ - 1) / kJ * kJ;  // a quad's rows past nx read a zero residual
-  for (int ch0 = 0; ch0 < K; ch0 += 4) {
-    const int kc = min(4, K - ch0);
+  {
     for (int j = threadIdx.x; j < nxPad; j += 64 * W)
       for (int q = 0; q < kc; q++)  // resB null: e is zero on this level, the residual is the rhs
         R[q * kBlockExtMax + j] = j >= nx ? 0.0f : resB ? resB[(long)(ch0 + q) * B + ext[x0 + j]] : rhs[(long)(ch0 + q) * Nd + bdIdx[ext[x0 + j]]];
@@ -941,7 +973,6 @@ __global__ __launch_bounds__(64 * W) void KMixSchwarz(const int* __restrict__ co
         e[(long)(ch0 + q) * Nd + core[c0 + i]] += omega * v;
       }
     }
-    __syncthreads();
   }
 }
 
@@ -951,7 +982,7 @@ __global__ __launch_bounds__(64 * W) void KMixSchwarz(const int* __restrict__ co
 // deep texels from the tile's bit masks, so no load waits on the texel type).
 // (Measured and not kept: the tile's (4 x 64 + 1) x (4 x 4 + 1) fine window staged in LDS one
 // column at a time by row-contiguous loads: 101 instead of 95 us at C2 level 0.)
-__device__ __forceinline__ void RestrictDeepTile(int vb, const int* __restrict__ tiles, const unsigned long long* __restrict__ cDeepMask,
+__device__ __forceinline__ void RestrictDeepTile(int vb, int c0, const int* __restrict__ tiles, const unsigned long long* __restrict__ cDeepMask,
                                                  const MixChart* __restrict__ cch, const MixChart* __restrict__ fch, long cplane, long cNd,
                                                  long fplane, long fNd, const float* __restrict__ fres, float* crhs, float* ce, int K) {
   const int row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
@@ -967,7 +998,7 @@ __device__ __forceinline__ void RestrictDeepTile(int vb, const int* __restrict__
     int n[9];
 #pragma unroll
     for (int k = 0; k < 9; k++) n[k] = DenseByte(f, fplane, fi + k % 3 - 1, fj + k / 3 - 1);
-    ForColumnChunks(K, [&](int c0, auto kc) {
+    ForChunk(K, c0, [&](auto kc) {
       constexpr int KC = decltype(kc)::value;
       float v[KC][9];
 #pragma unroll
@@ -987,15 +1018,15 @@ __device__ __forceinline__ void RestrictDeepTile(int vb, const int* __restrict__
 // Coarse boundary rhs: the boundary restriction matrix (fine dense columns); kRowLanes lanes per
 // coarse row read its entries coalesced, once for up to four columns, summed by shuffles.  An entry
 // is one 64-bit word (fine dense column, FP32 weight bits).
-__device__ __forceinline__ void RestrictBoundaryRows(int vb, int B, const int* __restrict__ bdIdx, const int* __restrict__ rp,
+__device__ __forceinline__ void RestrictBoundaryRows(int vb, int c0, int B, const int* __restrict__ bdIdx, const int* __restrict__ rp,
                                                      const int2* __restrict__ ent, const float* __restrict__ fres, long fNd, float* crhs, float* ce, long cNd,
                                                      int K) {
   const int r = (int)(((long)vb * blockDim.x + threadIdx.x) / kRowLanes), lane = threadIdx.x % kRowLanes;
   if (r >= B) return;  // whole row groups leave together
   const int k0 = rp[r], k1 = rp[r + 1];
   const long d = bdIdx[r];
-  for (int c0 = 0; c0 < K; c0 += 4) {
-    const int kc = min(4, K - c0);
+  const int kc = min(4, K - c0);
+  {
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int k = k0 + lane; k < k1; k += kRowLanes) {
       const int2 w = ent[k];
@@ -1014,15 +1045,20 @@ __device__ __forceinline__ void RestrictBoundaryRows(int vb, int B, const int* _
   }
 }
 
-// Restriction into a level in one launch: blocks [0, nTiles) take the coarse deep tiles, the others
+// Restriction into a level in one launch: the first blocks take the coarse deep tiles, the others
 // the coarse boundary rows (disjoint outputs).
 __global__ __launch_bounds__(256) void KMixRestrict(int nTiles, const int* __restrict__ tiles, const unsigned long long* __restrict__ cDeepMask,
                                                     const MixChart* __restrict__ cch, const MixChart* __restrict__ fch, long cplane, long cNd,
                                                     long fplane, long fNd, const float* __restrict__ fres, float* crhs, float* ce, int K, int B,
                                                     const int* __restrict__ bdIdx, const int* __restrict__ rp, const int2* __restrict__ ent) {
-  if ((int)blockIdx.x < nTiles)
-    RestrictDeepTile(XcdTile(blockIdx.x, nTiles), tiles, cDeepMask, cch, fch, cplane, cNd, fplane, fNd, fres, crhs, ce, K);
-  else RestrictBoundaryRows(blockIdx.x - nTiles, B, bdIdx, rp, ent, fres, fNd, crhs, ce, cNd, K);
+  const int deepBlocks = nTiles * ((K + 3) / 4);
+  if ((int)blockIdx.x < deepBlocks) {
+    const TileChunk v = TileOf<4>(blockIdx.x, nTiles, K);
+    RestrictDeepTile(v.tile, v.c0, tiles, cDeepMask, cch, fch, cplane, cNd, fplane, fNd, fres, crhs, ce, K);
+  } else {
+    const TileChunk v = TileOf<4>(blockIdx.x - deepBlocks, NBlk((long)B * kRowLanes, 256), K);
+    RestrictBoundaryRows(v.tile, v.c0, B, bdIdx, rp, ent, fres, fNd, crhs, ce, cNd, K);
+  }
 }
 
 // e_fine += P e_coarse at every active fine texel (bilinear, chart-centred coarse grid).  A thread
@@ -1036,9 +1072,10 @@ __global__ __launch_bounds__(256) void KMixRestrict(int nTiles, const int* __res
 __global__ __launch_bounds__(256) void KMixProlongAdd(const int* __restrict__ tiles, const unsigned long long* __restrict__ fDeepMask,
                                                       const unsigned long long* __restrict__ fActiveMask, const MixChart* __restrict__ fch,
                                                       const MixChart* __restrict__ cch, long fplane, long fNd, long cplane, long cNd,
-                                                      const float* __restrict__ ce, float* fe, int K, int skipQ) {
+                                                      const float* __restrict__ ce, float* fe, int K, int nTiles, int skipQ) {
   // active (and deep) fine texels from the tile's bit masks: no load waits on the texel type
-  const int tile = XcdTile(blockIdx.x, gridDim.x), row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
+  const TileChunk v = TileOf<4>(blockIdx.x, nTiles, K);
+  const int tile = v.tile, c0 = v.c0, row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
   const long mo = (long)tile * 4 * kTB + row;
   const int* T = tiles + 3 * tile;
   const MixChart f = fch[T[0]], c = cch[T[0]];
@@ -1064,7 +1101,7 @@ __global__ __launch_bounds__(256) void KMixProlongAdd(const int* __restrict__ ti
   int nb[4];
 #pragma unroll
   for (int n = 0; n < 4; n++) nb[n] = DenseByte(c, cplane, ci0 + (n & 1), cj0 + (n >> 1));
-  ForColumnChunks(K, [&](int c0, auto kc) {
+  ForChunk(K, c0, [&](auto kc) {
     constexpr int KC = decltype(kc)::value;
     float v[KC][4], old[KC][4];
 #pragma unroll
@@ -1105,8 +1142,8 @@ __global__ __launch_bounds__(256) void KMixDenseCoarse(int N, const double* __re
   const int i = blockIdx.x;
   const double* row = Ainv + (long)i * N;
   __shared__ double part[4][4];
-  for (int c0 = 0; c0 < K; c0 += 4) {
-    const int kc = min(4, K - c0);
+  const int c0 = 4 * blockIdx.y, kc = min(4, K - c0);
+  {
     double s[4] = {0.0, 0.0, 0.0, 0.0};
     for (int j = threadIdx.x; j < N; j += blockDim.x) {
       const double a = row[j];
@@ -1125,7 +1162,6 @@ __global__ __launch_bounds__(256) void KMixDenseCoarse(int N, const double* __re
       const int q = threadIdx.x;
       e[(long)(c0 + q) * Nd + g2d[i]] = (float)(part[q][0] + part[q][1] + part[q][2] + part[q][3]);
     }
-    __syncthreads();
   }
 }
 
@@ -1246,12 +1282,12 @@ __device__ __forceinline__ void SymRow(const double* __restrict__ sym, int N, in
 // raster line (no dependent index loads) 475 against 467 us: the launch time follows neither the
 // atomics, the load batching, the load count, the occupancy nor the index chain.)
 static constexpr int kDeepGroups = 4;
-__device__ __forceinline__ void K64ResidualDeepRows(int vb, int D, const int* __restrict__ deepLine, const int* __restrict__ lines,
+__device__ __forceinline__ void K64ResidualDeepRows(int vb, int c0, int D, const int* __restrict__ deepLine, const int* __restrict__ lines,
                                                     const double* __restrict__ sym, const double* __restrict__ x,
                                                     const double* __restrict__ b, int N, const int* __restrict__ g2d, float* rhs0,
                                                     float* e0, long Nd, double* norms, int K, double* bnorms) {
-  for (int c0 = 0; c0 < K; c0 += 3) {  // chunks of three columns: 27 x values in registers
-    const int kc = min(3, K - c0);
+  {
+    const int kc = min(3, K - c0);  // chunks of three columns: 27 x values in registers
     double acc[4] = {0, 0, 0, 0}, bacc[4] = {0, 0, 0, 0};
     for (int g = 0; g < kDeepGroups; g++) {
       const int d = (vb * kDeepGroups + g) * blockDim.x + threadIdx.x;
@@ -1288,13 +1324,13 @@ __device__ __forceinline__ void K64ResidualDeepRows(int vb, int D, const int* __
 // The same residual for per-column operators A_c = w[c][0] M + w[c][1] S (parametric solves: one
 // refinement loop serves columns with different weights, its FP32 V-cycle built for one nearby pair
 // of weights): both level-0 stencils read once per texel for a chunk of columns.
-__device__ __forceinline__ void K64ResidualDeepWRows(int vb, int D, const int* __restrict__ deepLine, const int* __restrict__ lines,
+__device__ __forceinline__ void K64ResidualDeepWRows(int vb, int c0, int D, const int* __restrict__ deepLine, const int* __restrict__ lines,
                                                      const double* __restrict__ symM, const double* __restrict__ symS,
                                                      const double* __restrict__ x, const double* __restrict__ b, int N,
                                                      const int* __restrict__ g2d, float* rhs0, float* e0, long Nd, double* norms, int K,
                                                      const double* __restrict__ w, double* r64, double* bnorms) {
-  for (int c0 = 0; c0 < K; c0 += 2) {  // chunks of two columns (two stencils in registers)
-    const int kc = min(2, K - c0);
+  {
+    const int kc = min(2, K - c0);  // chunks of two columns (two stencils in registers)
     double acc[4] = {0, 0, 0, 0}, bacc[4] = {0, 0, 0, 0};
     for (int g = 0; g < kDeepGroups; g++) {
       const int d = (vb * kDeepGroups + g) * blockDim.x + threadIdx.x;
@@ -1442,10 +1478,12 @@ __global__ __launch_bounds__(256) void K64Residual(int deepBlocks, int D, const 
                                                    const int* __restrict__ g2d, float* rhs0, float* e0, long Nd, double* norms, int K,
                                                    double* bnorms, int* fresh) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *fresh = 0;  // x is written from here on (read by the next update)
-  if ((int)blockIdx.x < deepBlocks)
-    K64ResidualDeepRows(XcdTile(blockIdx.x, deepBlocks), D, deepLine, lines, sym, x, b, N, g2d, rhs0, e0, Nd, norms, K, bnorms);
-  else
-    K64ResidualBoundaryRows(blockIdx.x - deepBlocks, B, bgi, rpd, cold, vald, rpb, colb, valb, x, b, N, g2d, rhs0, e0, Nd, norms, K, bnorms);
+  const int deep = deepBlocks * ((K + 2) / 3);
+  if ((int)blockIdx.x < deep) {
+    const TileChunk v = TileOf<3>(blockIdx.x, deepBlocks, K);
+    K64ResidualDeepRows(v.tile, v.c0, D, deepLine, lines, sym, x, b, N, g2d, rhs0, e0, Nd, norms, K, bnorms);
+  } else
+    K64ResidualBoundaryRows(blockIdx.x - deep, B, bgi, rpd, cold, vald, rpb, colb, valb, x, b, N, g2d, rhs0, e0, Nd, norms, K, bnorms);
 }
 
 // The same for per-column weights (M and S rows of both parts).
@@ -1460,11 +1498,12 @@ __global__ __launch_bounds__(256) void K64ResidualW(int deepBlocks, int D, const
                                                     const double* __restrict__ x, const double* __restrict__ b, int N,
                                                     const int* __restrict__ g2d, float* rhs0, float* e0, long Nd, double* norms, int K,
                                                     const double* __restrict__ w, double* r64, double* bnorms) {
-  if ((int)blockIdx.x < deepBlocks)
-    K64ResidualDeepWRows(XcdTile(blockIdx.x, deepBlocks), D, deepLine, lines, symM, symS, x, b, N, g2d, rhs0, e0, Nd, norms, K, w, r64,
-                         bnorms);
-  else
-    K64ResidualBoundaryWRows(blockIdx.x - deepBlocks, B, bgi, mrpd, mcold, mvald, mrpb, mcolb, mvalb, srpd, scold, svald, srpb, scolb,
+  const int deep = deepBlocks * ((K + 1) / 2);
+  if ((int)blockIdx.x < deep) {
+    const TileChunk v = TileOf<2>(blockIdx.x, deepBlocks, K);
+    K64ResidualDeepWRows(v.tile, v.c0, D, deepLine, lines, symM, symS, x, b, N, g2d, rhs0, e0, Nd, norms, K, w, r64, bnorms);
+  } else
+    K64ResidualBoundaryWRows(blockIdx.x - deep, B, bgi, mrpd, mcold, mvald, mrpb, mcolb, mvalb, srpd, scold, svald, srpb, scolb,
                              svalb, x, b, N, g2d, rhs0, e0, Nd, norms, K, w, r64, bnorms);
 }
 
@@ -2035,19 +2074,20 @@ void UploadMixed(const Hierarchy& h, const OperatorHierarchy& oh, DeviceSystem& 
 // else FP32.
 static void DeepGsLaunch(DevMixLevel& d, int q, int K, hipStream_t s) {
   if (d.stencilH)
-    KMixDeepGs<true><<<d.nTiles, 256, 0, s>>>(q, d.nTiles, d.tiles, d.deepMask, d.charts, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.e, d.rhs, K);
+    KMixDeepGs<true><<<ChunkBlocks<4>(d.nTiles, K), 256, 0, s>>>(q, d.nTiles, d.tiles, d.deepMask, d.charts, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.e, d.rhs, K);
   else
-    KMixDeepGs<false><<<d.nTiles, 256, 0, s>>>(q, d.nTiles, d.tiles, d.deepMask, d.charts, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.e, d.rhs, K);
+    KMixDeepGs<false><<<ChunkBlocks<4>(d.nTiles, K), 256, 0, s>>>(q, d.nTiles, d.tiles, d.deepMask, d.charts, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.e, d.rhs, K);
 }
 
 // One colour pair (first colour qa) of the deep sweep over the level's rows, columns in chunks of up
 // to four.
 template <bool kHalf>
 static void PairLaunch(DevMixLevel& d, int qa, int K, hipStream_t s) {
-  for (int c0 = 0; c0 < K; c0 += 4) {
+  for (int c0 = 0; c0 < K; c0 += K - c0 >= 4 ? (K - c0) / 4 * 4 : 4) {  // all chunks of four, then the rest
+    const int chunks = std::max(1, (K - c0) / 4);
     const long off = (long)c0 * d.Nd;
 #define GDTP_PAIR(KC, NT, P)                                                                                                \
-  KMixPairGs<kHalf, KC, NT, P><<<d.nRows, NT, 0, s>>>(qa, d.rows, d.rowMask, d.nRows, d.charts, d.plane, d.Nd, d.stencil,      \
+  KMixPairGs<kHalf, KC, NT, P><<<d.nRows * chunks, NT, 0, s>>>(qa, chunks, d.rows, d.rowMask, d.nRows, d.charts, d.plane, d.Nd, d.stencil,      \
                                                       d.stencilC, d.stencilH, d.e + off, d.rhs + off)
 #define GDTP_PAIR_SPAN(KC)                                                                \
   if (d.pairSpan == 1 && d.pairThreads == 256) GDTP_PAIR(KC, 256, 1);                    \
@@ -2070,13 +2110,14 @@ static void PairLaunch(DevMixLevel& d, int qa, int K, hipStream_t s) {
 template <bool kHalf, bool kPost, bool kProlong, int I>
 static void FusedLaunch(DevMixLevel& d, int K, hipStream_t s, FusedProlong pr) {
   constexpr FusedShapeInfo F = kFusedShape[I];
-  for (int c0 = 0; c0 < K; c0 += 4) {
+  for (int c0 = 0; c0 < K; c0 += K - c0 >= 4 ? (K - c0) / 4 * 4 : 4) {  // all chunks of four, then the rest
+    const int chunks = std::max(1, (K - c0) / 4);
     const long off = (long)c0 * d.Nd;
     FusedProlong p = pr;
     if (p.ce) p.ce += (long)c0 * p.cNd;
 #define GDTP_FUSED(KC)                                                                                                               \
   KMixDeepGsFused<kHalf, kPost, kProlong, F.ta, F.tb, F.threads, KC, F.variant & 3, (F.variant & kFusedXcd) != 0>                  \
-      <<<d.nFTiles[I], F.threads, 0, s>>>(d.ftiles[I], d.charts, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.type, d.e + off, \
+      <<<d.nFTiles[I] * chunks, F.threads, 0, s>>>(chunks, d.ftiles[I], d.charts, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.type, d.e + off, \
                                           d.e2 + off, d.rhs + off, p)
     switch (std::min(4, K - c0)) {
       case 4: GDTP_FUSED(4); break;
@@ -2124,11 +2165,11 @@ static int DeepSweep(MixedSystem& ms, DevMixLevel& d, bool post, int K, hipStrea
     } else {
       post ? FusedShapeLaunch<false, true, false>(d, shape, K, s, pr) : FusedShapeLaunch<false, false, false>(d, shape, K, s, pr);
     }
-    return (K + 3) / 4;
+    return K < 4 || K % 4 == 0 ? 1 : 2;
   }
   if (d.shape == kShapePairs && d.pairSpan > 0 && d.nRows > 0) {  // pairs (0, 1), (2, 3); post (3, 2), (1, 0)
     for (const int qa : {post ? 3 : 0, post ? 1 : 2}) d.stencilH ? PairLaunch<true>(d, qa, K, s) : PairLaunch<false>(d, qa, K, s);
-    return 2 * ((K + 3) / 4);
+    return 2 * (K < 4 || K % 4 == 0 ? 1 : 2);
   }
   for (int qq = 0; qq < 4; qq++) DeepGsLaunch(d, post ? 3 - qq : qq, K, s);
   return 4;
@@ -2138,10 +2179,10 @@ static int DeepSweep(MixedSystem& ms, DevMixLevel& d, bool post, int K, hipStrea
 template <int W, int kPre>
 static void SchwarzLaunch(MixedSystem& ms, DevMixLevel& d, const float* res, int K, hipStream_t s) {
   if (d.blkMatH && ms.schwarzHalf)
-    KMixSchwarz<W, kPre / 4, uint2><<<d.nBlocks, 64 * W, 0, s>>>(d.blkCorePtr, d.blkCore, d.blkExtPtr, d.blkExt, d.blkMatPtrH, d.blkMatH,
+    KMixSchwarz<W, kPre / 4, uint2><<<ChunkBlocks<4>(d.nBlocks, K), 64 * W, 0, s>>>(d.blkCorePtr, d.blkCore, d.blkExtPtr, d.blkExt, d.blkMatPtrH, d.blkMatH,
                                                                 d.blkScale, res, d.bdIdx, d.rhs, d.B, d.e, d.Nd, K, ms.omega);
   else
-    KMixSchwarz<W, kPre, float><<<d.nBlocks, 64 * W, 0, s>>>(d.blkCorePtr, d.blkCore, d.blkExtPtr, d.blkExt, d.blkMatPtr, d.blkMat,
+    KMixSchwarz<W, kPre, float><<<ChunkBlocks<4>(d.nBlocks, K), 64 * W, 0, s>>>(d.blkCorePtr, d.blkCore, d.blkExtPtr, d.blkExt, d.blkMatPtr, d.blkMat,
                                                             nullptr, res, d.bdIdx, d.rhs, d.B, d.e, d.Nd, K, ms.omega);
 }
 
@@ -2152,7 +2193,7 @@ static void BoundarySweeps(MixedSystem& ms, DevMixLevel& d, int K, hipStream_t s
   for (int sw = 0; sw < ms.boundarySweeps; sw++) {
     const bool fromRhs = zeroE && sw == 0;
     if (!fromRhs)
-      KMixBoundaryResidual<<<NBlk((long)d.B * kRowLanes, 256), 256, 0, s>>>(d.B, d.bdIdx, d.bRowptr, d.bEnt, d.bDiag, d.e, d.rhs,
+      KMixBoundaryResidual<<<ChunkBlocks<4>(NBlk((long)d.B * kRowLanes, 256), K), 256, 0, s>>>(d.B, d.bdIdx, d.bRowptr, d.bEnt, d.bDiag, d.e, d.rhs,
                                                                             d.tmpB, 1, d.Nd, K);
     const float* res = fromRhs ? nullptr : d.tmpB;
     if (d.nBlocks <= kSchwarzPrefetchBlocks)
@@ -2229,20 +2270,22 @@ void MixedVCycle(DeviceSystem& ds, MixedSystem& ms, int K, hipStream_t s, bool z
   for (int l = 0; l + 1 < nl; l++) {
     DevMixLevel &d = ms.L[l], &c = ms.L[l + 1];
     Smooth(ms, l, K, false, s, l > 0 || zeroE0);
-    const long rb = d.B > 0 ? NBlk((long)d.B * kRowLanes, 256) : 0, cb = c.B > 0 ? NBlk((long)c.B * kRowLanes, 256) : 0;
-    if (d.nTiles + rb > 0)
-      (d.nTiles > kResidualWideTiles ? KMixResidual<2> : KMixResidual<4>)<<<d.nTiles + rb, 256, 0, s>>>(
+    const long rb = ChunkBlocks<4>(NBlk((long)d.B * kRowLanes, 256), K), cb = ChunkBlocks<4>(NBlk((long)c.B * kRowLanes, 256), K);
+    const bool wide = d.nTiles > kResidualWideTiles;
+    const long db = wide ? ChunkBlocks<2>(d.nTiles, K) : ChunkBlocks<4>(d.nTiles, K), cd = ChunkBlocks<4>(c.nTiles, K);
+    if (db + rb > 0)
+      (wide ? KMixResidual<2> : KMixResidual<4>)<<<db + rb, 256, 0, s>>>(
           d.nTiles, d.tiles, d.deepMask, d.charts, d.plane, d.Nd, d.stencilSym, d.e, d.rhs, d.res, K, ms.nuPre > 0 && !d.stencilH ? 3 : -1,
           d.B, d.bdIdx, d.bRowptr, d.bEnt, d.bDiag);
-    if (c.nTiles + cb > 0)
-      KMixRestrict<<<c.nTiles + cb, 256, 0, s>>>(c.nTiles, c.tiles, c.deepMask, c.charts, d.charts, c.plane, c.Nd, d.plane, d.Nd, d.res, c.rhs,
+    if (cd + cb > 0)
+      KMixRestrict<<<cd + cb, 256, 0, s>>>(c.nTiles, c.tiles, c.deepMask, c.charts, d.charts, c.plane, c.Nd, d.plane, d.Nd, d.res, c.rhs,
                                                  c.e, K, c.B, c.bdIdx, c.rRowptr, c.rEnt);
   }
   {
     DevMixLevel& c = ms.L[nl - 1];
     const long nk = (long)c.N * K;
     if (ms.coarseInv) {
-      KMixDenseCoarse<<<c.N, 256, 0, s>>>(c.N, ms.coarseInv, c.g2d, c.rhs, c.e, c.Nd, K);
+      KMixDenseCoarse<<<dim3(c.N, (K + 3) / 4), 256, 0, s>>>(c.N, ms.coarseInv, c.g2d, c.rhs, c.e, c.Nd, K);
     } else {
       KMixGather<<<NBlk(nk, 256), 256, 0, s>>>(c.N, c.g2d, c.rhs, c.Nd, ms.coarseRhs, K);
       LdltSolve(ms.coarse, ms.coarseRhs, c.N, ms.coarseX, c.N, ms.coarseY, K, s);
@@ -2254,8 +2297,8 @@ void MixedVCycle(DeviceSystem& ds, MixedSystem& ms, int K, hipStream_t s, bool z
     // the first post-smoothing sweep of a fused level adds the prolongation itself
     const bool fuse = ms.fuseProlong && ms.nuPost > 0 && Fused(d);
     if (d.nTiles > 0 && !fuse)
-      KMixProlongAdd<<<d.nTiles, 256, 0, s>>>(d.tiles, d.deepMask, d.activeMask, d.charts, c.charts, d.plane, d.Nd, c.plane, c.Nd, c.e, d.e,
-                                              K, ms.nuPost > 0 ? 3 : -1);
+      KMixProlongAdd<<<ChunkBlocks<4>(d.nTiles, K), 256, 0, s>>>(d.tiles, d.deepMask, d.activeMask, d.charts, c.charts, d.plane, d.Nd, c.plane, c.Nd, c.e, d.e,
+                                              K, d.nTiles, ms.nuPost > 0 ? 3 : -1);
     FusedProlong pr;
     pr.cch = c.charts, pr.cplane = c.plane, pr.cNd = c.Nd, pr.ce = c.e;
     Smooth(ms, l, K, true, s, false, fuse ? &pr : nullptr);
@@ -2265,7 +2308,7 @@ void MixedVCycle(DeviceSystem& ds, MixedSystem& ms, int K, hipStream_t s, bool z
 
 // ------------------------------------------------------------------ flexible conjugate gradients
 // q = A p for per-column operators A_c = w[c][0] M + w[c][1] S (level 0; deep rows by raster line)
-__device__ __forceinline__ void K64ApplyDeepWRows(int vb, int D, const int* __restrict__ deepLine, const int* __restrict__ lines,
+__device__ __forceinline__ void K64ApplyDeepWRows(int vb, int c0, int D, const int* __restrict__ deepLine, const int* __restrict__ lines,
                                                   const double* __restrict__ symM, const double* __restrict__ symS,
                                                   const double* __restrict__ p, int N, double* q, int K, const double* __restrict__ w) {
   const int d = vb * blockDim.x + threadIdx.x;
@@ -2275,8 +2318,7 @@ __device__ __forceinline__ void K64ApplyDeepWRows(int vb, int D, const int* __re
   double cm[9], cs[9];
   SymRow(symM, N, cur, next, cm);
   SymRow(symS, N, cur, next, cs);
-  for (int c0 = 0; c0 < K; c0 += 3)
-    WithChunkWidth<3>(min(3, K - c0), [&](auto kcc) {
+  WithChunkWidth<3>(min(3, K - c0), [&](auto kcc) {
       constexpr int KC = decltype(kcc)::value;
       double pv[KC][9];
       RowValues<KC>(p, N, c0, prev, cur, next, pv);
@@ -2335,9 +2377,12 @@ __global__ __launch_bounds__(256) void K64ApplyW(int deepBlocks, int D, const in
                                                  const double* __restrict__ svald, const int* __restrict__ srpb, const int* __restrict__ scolb,
                                                  const double* __restrict__ svalb, const double* __restrict__ p, int N, double* q, int K,
                                                  const double* __restrict__ w) {
-  if ((int)blockIdx.x < deepBlocks) K64ApplyDeepWRows(XcdTile(blockIdx.x, deepBlocks), D, deepLine, lines, symM, symS, p, N, q, K, w);
-  else
-    K64ApplyBoundaryWRows(blockIdx.x - deepBlocks, B, bgi, mrpd, mcold, mvald, mrpb, mcolb, mvalb, srpd, scold, svald, srpb, scolb, svalb, p,
+  const int deep = deepBlocks * ((K + 2) / 3);
+  if ((int)blockIdx.x < deep) {
+    const TileChunk v = TileOf<3>(blockIdx.x, deepBlocks, K);
+    K64ApplyDeepWRows(v.tile, v.c0, D, deepLine, lines, symM, symS, p, N, q, K, w);
+  } else
+    K64ApplyBoundaryWRows(blockIdx.x - deep, B, bgi, mrpd, mcold, mvald, mrpb, mcolb, mvalb, srpd, scold, svald, srpb, scolb, svalb, p,
                           N, q, K, w);
 }
 
@@ -2543,12 +2588,12 @@ static void OuterResidual(DeviceSystem& ds, MixedSystem& ms, double* x, const do
   if (db + bb == 0) return;
   if (weighted) {
     const DevLevel &M = ds.mass0, &S = ds.stiff0;
-    K64ResidualW<<<db + bb, nt, 0, s>>>(db, L0.D, ms.deepLine, L0.raster, M.coefSym, S.coefSym, L0.B, L0.bgi, M.bd.rowptr, M.bd.col,
+    K64ResidualW<<<ChunkBlocks<2>(db, K) + bb, nt, 0, s>>>(db, L0.D, ms.deepLine, L0.raster, M.coefSym, S.coefSym, L0.B, L0.bgi, M.bd.rowptr, M.bd.col,
                                          M.bd.val, M.bb.rowptr, M.bb.col, M.bb.val, S.bd.rowptr, S.bd.col, S.bd.val, S.bb.rowptr, S.bb.col,
                                          S.bb.val, x, b, L0.N, d.g2d, d.rhs, d.e, d.Nd, ms.norms, K, ms.weights, r64, bnorms);
     return;
   }
-  K64Residual<<<db + bb, nt, 0, s>>>(db, L0.D, ms.deepLine, L0.raster, L0.coefSym, L0.B, L0.bgi, L0.bd.rowptr, L0.bd.col, L0.bd.val,
+  K64Residual<<<ChunkBlocks<3>(db, K) + bb, nt, 0, s>>>(db, L0.D, ms.deepLine, L0.raster, L0.coefSym, L0.B, L0.bgi, L0.bd.rowptr, L0.bd.col, L0.bd.val,
                                       L0.bb.rowptr, L0.bb.col, L0.bb.val, x, b, L0.N, d.g2d, d.rhs, d.e, d.Nd, ms.norms, K, bnorms, ms.fresh);
 }
 
@@ -2572,7 +2617,7 @@ static void FcgStepChunks(DeviceSystem& ds, MixedSystem& ms, double* x, int K, h
   const int db = L0.nRaster > 0 ? (int)NBlk(L0.D, 256) : 0;
   const int bb = L0.B > 0 ? (int)NBlk((long)L0.B * kRowLanes64, 256) : 0;
   if (db + bb > 0)
-    K64ApplyW<<<db + bb, 256, 0, s>>>(db, L0.D, ms.deepLine, L0.raster, M.coefSym, S.coefSym, L0.B, L0.bgi, M.bd.rowptr, M.bd.col, M.bd.val,
+    K64ApplyW<<<ChunkBlocks<3>(db, K) + bb, 256, 0, s>>>(db, L0.D, ms.deepLine, L0.raster, M.coefSym, S.coefSym, L0.B, L0.bgi, M.bd.rowptr, M.bd.col, M.bd.val,
                                       M.bb.rowptr, M.bb.col, M.bb.val, S.bd.rowptr, S.bd.col, S.bd.val, S.bb.rowptr, S.bb.col, S.bb.val,
                                       ms.p64, N, ms.q64, K, ms.weights);
   KFcgDots<KC><<<sums, 256, 0, s>>>(N, ms.r64, ms.p64, ms.q64, rp, pq, K);
