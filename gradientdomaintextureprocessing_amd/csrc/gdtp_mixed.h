@@ -8,6 +8,20 @@ namespace gdtp {
 struct MixChart {  // per chart geometry of one level
   int w, h, w2, h2, base2, cofx, cofy;
 };
+struct MixGrid {  // what addressing a chart's dense planes takes
+  int w2, base2, cofx, cofy;
+};
+// A 64 x 4 tile of a level's sub-grid: its origin and its chart on this level and the levels either
+// side, in one record (a kernel's first load instead of two that wait for each other).
+struct MixTile {
+  int a0, b0, pad[2];
+  MixGrid own, finer, coarser;
+};
+// A Schwarz block: ranges of its core and extended rows, where its inverse begins (FP32, FP16 quads).
+struct MixBlock {
+  int core0, cores, ext0, exts;
+  long mat[2];
+};
 
 // Tile shapes of the fused four-colour deep sweep: a tile of ta x tb sub-grid texels per
 // workgroup of `threads` threads, and a variant.  The system uses one of them per level (or, with
@@ -56,7 +70,7 @@ struct DevMixLevel {
   int nTiles = 0;
   bool chartSweeps = false;         // small charts: one workgroup per chart and column runs all four colours of a sweep
   int chartPlane = 0;               // sub-grid positions of the largest chart
-  int* tiles = nullptr;            // 3 ints per tile: chart, a0, b0 (sub-grid origin)
+  MixTile* tileRecs = nullptr;
   unsigned long long* deepMask = nullptr;    // [tile][plane][tile row]: bit x set where texel (a0 + x, b0 + row) is deep
   unsigned long long* activeMask = nullptr;  // the same for active texels (deep or boundary)
   int* ftiles[kFusedShapes] = {};  // the same for each fused-sweep tile shape
@@ -74,14 +88,14 @@ struct DevMixLevel {
   int2* bEnt = nullptr;  // off-diagonal entries: (dense column, FP32 value bits)
   float* bDiag = nullptr;
   // overlapping Schwarz blocks of boundary rows: block b updates its core rows (dense indices
-  // blkCore[blkCorePtr[b]..]) from the residual at its extended rows (boundary indices
-  // blkExt[blkExtPtr[b]..]) through the core rows of the inverse of A restricted to the extended
-  // rows, stored column-major at blkMat + blkMatPtr[b] ([ext][core]) in FP32, or at blkMatH +
-  // blkMatPtrH[b] as FP16 quads ([ext / 4][core], extended rows 4s .. 4s + 3 in one 64-bit word,
-  // lowest first) scaled per core row (entries |.| <= 1, core row r's scale blkScale[r])
+  // blkCore[core0 ..]) from the residual at its extended rows (boundary indices blkExt[ext0 ..], dense
+  // indices blkExtDense) through the core rows of the inverse of A restricted to the extended rows,
+  // stored column-major at blkMat + mat[0] ([ext][core]) in FP32, or at blkMatH + mat[1] as FP16 quads
+  // ([ext / 4][core], extended rows 4s .. 4s + 3 in one 64-bit word, lowest first) scaled per core row
+  // (entries |.| <= 1, core row r's scale blkScale[r])
   int nBlocks = 0;
-  int *blkCorePtr = nullptr, *blkCore = nullptr, *blkExtPtr = nullptr, *blkExt = nullptr;
-  long *blkMatPtr = nullptr, *blkMatPtrH = nullptr;
+  MixBlock* blocks = nullptr;
+  int *blkCore = nullptr, *blkExt = nullptr, *blkExtDense = nullptr;
   float* blkMat = nullptr;
   uint2* blkMatH = nullptr;
   float* blkScale = nullptr;

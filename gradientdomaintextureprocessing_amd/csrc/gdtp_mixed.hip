@@ -43,7 +43,8 @@ __device__ __forceinline__ float Ld(const float* column, int bytes) {
   const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(column), 0, 0x7fffffff, 0x00020000);
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, bytes, 0, 0));
 }
-__device__ __forceinline__ int DenseByte(const MixChart& c, long plane, int i, int j) {
+template <class G>  // MixChart or MixGrid
+__device__ __forceinline__ int DenseByte(const G& c, long plane, int i, int j) {
   return 4 * (((i & 1) | ((j & 1) << 1)) * (int)plane + c.base2 + (j >> 1) * c.w2 + (i >> 1));
 }
 
@@ -153,17 +154,16 @@ struct Stencil9 {
 // from the stencil, so that a deep texel's stencil, neighbour and rhs loads all go out together
 // (one memory round trip instead of two).  Tiles in XCD-contiguous order (XcdTile).
 template <bool kHalf>
-__global__ __launch_bounds__(256) void KMixDeepGs(int q, int nTiles, const int* __restrict__ tiles,
-                                                  const unsigned long long* __restrict__ deepMask, const MixChart* __restrict__ charts,
-                                                  long plane, long Nd, const float* __restrict__ st, const float2* __restrict__ stc,
+__global__ __launch_bounds__(256) void KMixDeepGs(int q, int nTiles, const MixTile* __restrict__ tiles,
+                                                  const unsigned long long* __restrict__ deepMask, long plane, long Nd, const float* __restrict__ st, const float2* __restrict__ stc,
                                                   const uint4* __restrict__ sth, float* e, const float* __restrict__ rhs, int K) {
   const TileChunk v = TileOf<4>(blockIdx.x, nTiles, K);
   const int tile = v.tile, c0 = v.c0, row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
   const unsigned long long m = deepMask[((long)tile * 4 + q) * kTB + row];
   if (!((m >> tx) & 1ull)) return;
-  const int* T = tiles + 3 * tile;
-  const MixChart c = charts[T[0]];
-  const int a = T[1] + tx, b = T[2] + row, i = 2 * a + (q & 1), j = 2 * b + (q >> 1);
+  const MixTile& T = tiles[tile];
+  const MixGrid c = T.own;
+  const int a = T.a0 + tx, b = T.b0 + row, i = 2 * a + (q & 1), j = 2 * b + (q >> 1);
   const int idx = (int)((long)q * plane + c.base2 + (long)b * c.w2 + a);
   float c4, corr = 0.0f, cf[9];
   if constexpr (kHalf) {
@@ -752,16 +752,21 @@ __global__ __launch_bounds__(NT) void KMixDeepGsFused(int chunks, const int* __r
 // kChunk: columns whose loads are in flight together (2 on large levels: 50 instead of 79
 // registers, eight waves per SIMD instead of six, level 0 at C2 219 against 221 us; 4 on small
 // levels, which are latency-bound and pay for a second round trip).
-template <int kChunk>
-__device__ __forceinline__ void ResidualDeepTile(int vb, int c0, const int* __restrict__ tiles, const unsigned long long* __restrict__ deepMask,
-                                                 const MixChart* __restrict__ charts, long plane, long Nd, const float* __restrict__ sym,
-                                                 const float* __restrict__ e, const float* __restrict__ rhs, float* res, int K, int zeroQ) {
+// kSplit: the workgroup's tile in one plane only (vb = 4 tile + plane; small levels: four times the
+// workgroups, and one round trip instead of one per plane: 5.7 us a launch to 4.4 on a 512^2 cube).
+template <int kChunk, bool kSplit>
+__device__ __forceinline__ void ResidualDeepTile(int vb, int c0, const MixTile* __restrict__ tiles,
+                                                 const unsigned long long* __restrict__ deepMask, long plane, long Nd,
+                                                 const float* __restrict__ sym, const float* __restrict__ e, const float* __restrict__ rhs,
+                                                 float* res, int K, int zeroQ) {
+  const int plane0 = kSplit ? vb % 4 : 0, plane1 = kSplit ? plane0 + 1 : 4;
+  if constexpr (kSplit) vb /= 4;
   const int row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
   const unsigned long long* mk = deepMask + (long)vb * 4 * kTB + row;
-  const int* T = tiles + 3 * vb;
-  const MixChart c = charts[T[0]];
-  const int a = T[1] + tx, b = T[2] + row;
-  for (int q = 0; q < 4; q++) {
+  const MixTile& T = tiles[vb];
+  const MixGrid c = T.own;
+  const int a = T.a0 + tx, b = T.b0 + row;
+  for (int q = plane0; q < plane1; q++) {
     if (!((mk[q * kTB] >> tx) & 1ull)) continue;
     const int i = 2 * a + (q & 1), j = 2 * b + (q >> 1);
     const long idx = (long)q * plane + c.base2 + (long)b * c.w2 + a;
@@ -811,6 +816,32 @@ __device__ __forceinline__ T Pick(const T (&a)[4], int q) {
   return q == 0 ? a[0] : q == 1 ? a[1] : q == 2 ? a[2] : a[3];
 }
 
+// A row's sum of value x src[column] over entries [k0, k1) for up to four columns, in every lane of the
+// row's group: two entries per lane in flight.
+__device__ __forceinline__ void RowTerms(const int2* __restrict__ ent, int k0, int k1, int lane, const float* __restrict__ src, long stride,
+                                         int kc, float (&acc)[4]) {
+#pragma unroll
+  for (int q = 0; q < 4; q++) acc[q] = 0.0f;
+  for (int k = k0 + lane; k < k1; k += 2 * kRowLanes) {
+    const bool two = k + kRowLanes < k1;
+    const int2 w0 = ent[k], w1 = ent[two ? k + kRowLanes : k];
+    float v0[4], v1[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      if (q >= kc) continue;
+      v0[q] = src[q * stride + w0.x], v1[q] = src[q * stride + w1.x];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      if (q >= kc) continue;
+      acc[q] += __int_as_float(w0.y) * v0[q];
+      if (two) acc[q] += __int_as_float(w1.y) * v1[q];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) acc[q] = RowSum(acc[q]);
+}
+
 // Boundary-row residual rhs - A e (FP32).  out: compact [K][B] when `compact`, else the dense
 // vector [K][Nd] at the row's texel.  A row entry is one 64-bit word (dense column, FP32 value
 // bits): one load per entry instead of two.
@@ -819,27 +850,15 @@ __device__ __forceinline__ void BoundaryResidualRows(int vb, int c0, int B, cons
                                                      const float* __restrict__ rhs, float* out, int compact, long Nd, int K) {
   const int r = (int)(((long)vb * blockDim.x + threadIdx.x) / kRowLanes), lane = threadIdx.x % kRowLanes;
   if (r >= B) return;  // whole row groups leave together
-  const int k0 = rp[r], k1 = rp[r + 1];
-  const long d = bdIdx[r];
-  const int kc = min(4, K - c0);
-  {
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k = k0 + lane; k < k1; k += kRowLanes) {
-      const int2 w = ent[k];
-      const float v = __int_as_float(w.y);
-      const long c = w.x;
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-        if (q < kc) acc[q] += v * e[(long)(c0 + q) * Nd + c];
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q++) acc[q] = RowSum(acc[q]);
-    if (lane < kc) {
-      const long o = (long)(c0 + lane) * Nd + d;
-      const float rv = rhs[o] - (dg[r] * e[o] + Pick(acc, lane));
-      if (compact) out[(long)(c0 + lane) * B + r] = rv;
-      else out[o] = rv;
-    }
+  const int k0 = rp[r], k1 = rp[r + 1], kc = min(4, K - c0);
+  const long o = (long)(c0 + min(lane, kc - 1)) * Nd + bdIdx[r];
+  const float own = e[o], b = rhs[o], diag = dg[r];  // in flight with the row's entries
+  float acc[4];
+  RowTerms(ent, k0, k1, lane, e + (long)c0 * Nd, Nd, kc, acc);
+  if (lane < kc) {
+    const float rv = b - (diag * own + Pick(acc, lane));
+    if (compact) out[(long)(c0 + lane) * B + r] = rv;
+    else out[o] = rv;
   }
 }
 
@@ -854,17 +873,17 @@ __global__ __launch_bounds__(256) void KMixBoundaryResidual(int B, const int* __
 static constexpr int kResidualWideTiles = 1024;  // levels with more 64 x 4 tiles load two columns at a time
 // The residual of a level after pre-smoothing in one launch: the first blocks take the deep tiles,
 // the others the boundary rows (disjoint outputs, so the two parts overlap on the device).
-template <int kChunk>
-__global__ __launch_bounds__(256) void KMixResidual(int nTiles, const int* __restrict__ tiles, const unsigned long long* __restrict__ deepMask,
-                                                    const MixChart* __restrict__ charts, long plane,
+template <int kChunk, bool kSplit>
+__global__ __launch_bounds__(256) void KMixResidual(int nTiles, const MixTile* __restrict__ tiles,
+                                                    const unsigned long long* __restrict__ deepMask, long plane,
                                                     long Nd, const float* __restrict__ sym, const float* __restrict__ e,
                                                     const float* __restrict__ rhs, float* res, int K, int zeroQ, int B,
                                                     const int* __restrict__ bdIdx, const int* __restrict__ rp, const int2* __restrict__ ent,
                                                     const float* __restrict__ dg) {
-  const int deepBlocks = nTiles * ((K + kChunk - 1) / kChunk);
+  const int parts = kSplit ? 4 * nTiles : nTiles, deepBlocks = parts * ((K + kChunk - 1) / kChunk);
   if ((int)blockIdx.x < deepBlocks) {
-    const TileChunk v = TileOf<kChunk>(blockIdx.x, nTiles, K);
-    ResidualDeepTile<kChunk>(v.tile, v.c0, tiles, deepMask, charts, plane, Nd, sym, e, rhs, res, K, zeroQ);
+    const TileChunk v = TileOf<kChunk>(blockIdx.x, parts, K);
+    ResidualDeepTile<kChunk, kSplit>(v.tile, v.c0, tiles, deepMask, plane, Nd, sym, e, rhs, res, K, zeroQ);
   } else {
     const TileChunk v = TileOf<4>(blockIdx.x - deepBlocks, NBlk((long)B * kRowLanes, 256), K);
     BoundaryResidualRows(v.tile, v.c0, B, bdIdx, rp, ent, dg, e, rhs, res, 0, Nd, K);
@@ -898,23 +917,26 @@ __device__ __forceinline__ void Entries(const uint2* M, long k, float (&m)[4]) {
   const uint2 w = M[k];
   m[0] = Half(w.x & 0xffff), m[1] = Half(w.x >> 16), m[2] = Half(w.y & 0xffff), m[3] = Half(w.y >> 16);
 }
-template <int W, int kPre, class TM>
-__global__ __launch_bounds__(64 * W) void KMixSchwarz(const int* __restrict__ corePtr, const int* __restrict__ core,
-                                                                  const int* __restrict__ extPtr, const int* __restrict__ ext,
-                                                                  const long* __restrict__ matPtr, const TM* __restrict__ mat,
-                                                                  const float* __restrict__ rowScale,
-                                                                  const float* __restrict__ resB, const int* __restrict__ bdIdx,
-                                                                  const float* __restrict__ rhs, int B, float* e, long Nd, int K,
-                                                                  float omega) {
+// A launch is one chain of loads (block record, row list, residual; inverse entries and the core rows'
+// old values beside it) and two barriers; KC columns at a time, their residuals side by side in LDS (one
+// 16-byte read for four).  (512^2 cube, three columns: 6.8 us a launch with the row list looked up
+// through the boundary index and the core rows loaded last, 4.7 us so.)
+template <int W, int kPre, class TM, int KC>
+__global__ __launch_bounds__(64 * W) void KMixSchwarz(const MixBlock* __restrict__ blocks, const int* __restrict__ core,
+                                                      const int* __restrict__ ext, const TM* __restrict__ mat,
+                                                      const float* __restrict__ rowScale, const float* __restrict__ src, long srcStride, float* e,
+                                                      long Nd, int K, float omega) {
   constexpr bool kScaled = !std::is_same<TM, float>::value;
   constexpr int kJ = kScaled ? (int)sizeof(TM) / 2 : 1;  // extended rows per load
+  constexpr int kPad = KC == 3 ? 4 : KC;
   static_assert(kBlockExtMax % kJ == 0, "padded extended rows fit the staged residual");
-  __shared__ float R[4 * kBlockExtMax];
-  __shared__ float P[W][4][kBlockCore];
-  const TileChunk v = TileOf<4>(blockIdx.x, gridDim.x / ((K + 3) / 4), K);
-  const int b = v.tile, ch0 = v.c0, kc = min(4, K - ch0);
-  const int c0 = corePtr[b], nc = corePtr[b + 1] - c0, x0 = extPtr[b], nx = extPtr[b + 1] - x0;
-  const TM* M = mat + matPtr[b];
+  __shared__ __align__(16) float R[kBlockExtMax][kPad];
+  __shared__ float P[W][KC][kBlockCore];
+  const TileChunk tc = TileOf<KC>(blockIdx.x, gridDim.x / ((K + KC - 1) / KC), K);
+  const int ch0 = tc.c0, kc = min(KC, K - ch0);
+  const MixBlock D = blocks[tc.tile];
+  const int nc = D.cores, nx = D.exts;
+  const TM* M = mat + D.mat[kScaled ? 1 : 0];
   const int i = threadIdx.x % 64, part = threadIdx.x / 64;
   // The first kPre of this lane's loads of the block inverse (row i, load slots part, part + W,
   // ..., each kJ extended rows) are issued before the residual is staged, so they are in flight with it;
@@ -932,47 +954,52 @@ __global__ __launch_bounds__(64 * W) void KMixSchwarz(const int* __restrict__ co
 #pragma unroll
       for (int t = 0; t < kJ; t++) mv[ss][t] = 0.0f;
   }
+  // the row this thread updates at the end: core row i, column part (wave q sums column q over the parts)
+  const bool out = part < kc && i < nc;
+  const long at = out ? (long)(ch0 + part) * Nd + core[D.core0 + i] : 0;
+  const float old = out ? e[at] : 0.0f;
+  float scale = 1.0f;
+  if constexpr (kScaled) scale = out ? rowScale[D.core0 + i] : 1.0f;
   const int nxPad = (nx + kJ - 1) / kJ * kJ;  // a quad's rows past nx read a zero residual
-  {
-    for (int j = threadIdx.x; j < nxPad; j += 64 * W)
-      for (int q = 0; q < kc; q++)  // resB null: e is zero on this level, the residual is the rhs
-        R[q * kBlockExtMax + j] = j >= nx ? 0.0f : resB ? resB[(long)(ch0 + q) * B + ext[x0 + j]] : rhs[(long)(ch0 + q) * Nd + bdIdx[ext[x0 + j]]];
-    __syncthreads();
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (i < nc) {
+  for (int j = threadIdx.x; j < nxPad; j += 64 * W) {
+    const int row = ext[D.ext0 + min(j, nx - 1)];
+    float r[KC];
 #pragma unroll
-      for (int ss = 0; ss < kPre; ss++) {
-        const int j = kJ * (part + W * ss);
-        if (j >= nx) break;
+    for (int q = 0; q < KC; q++) r[q] = src[(long)(ch0 + min(q, kc - 1)) * srcStride + row];
 #pragma unroll
-        for (int t = 0; t < kJ; t++)
+    for (int q = 0; q < KC; q++) R[j][q] = j >= nx ? 0.0f : r[q];
+  }
+  __syncthreads();
+  float acc[KC] = {};
+  auto add = [&](const float (&m)[kJ], int j) {
 #pragma unroll
-          for (int q = 0; q < 4; q++)
-            if (q < kc) acc[q] += mv[ss][t] * R[q * kBlockExtMax + j + t];
-      }
-      for (int sl = part + W * kPre; kJ * sl < nx; sl += W) {
-        float m[kJ];
-        Entries(M, (long)sl * nc + i, m);
-        const int j = kJ * sl;
+    for (int t = 0; t < kJ; t++)
 #pragma unroll
-        for (int t = 0; t < kJ; t++)
+      for (int q = 0; q < KC; q++) acc[q] += m[t] * R[j + t][q];
+  };
+  if (i < nc) {
 #pragma unroll
-          for (int q = 0; q < 4; q++)
-            if (q < kc) acc[q] += m[t] * R[q * kBlockExtMax + j + t];
-      }
+    for (int ss = 0; ss < kPre; ss++) {
+      const int j = kJ * (part + W * ss);
+      if (j >= nx) break;
+      add(mv[ss], j);
     }
-#pragma unroll
-    for (int q = 0; q < 4; q++) P[part][q][i] = acc[q];
-    __syncthreads();
-    if (threadIdx.x < 4 * 64) {  // wave q sums column q over the parts
-      const int q = threadIdx.x / 64;
-      if (q < kc && i < nc) {
-        float v = 0.0f;
-        for (int p = 0; p < W; p++) v += P[p][q][i];
-        if constexpr (kScaled) v *= rowScale[c0 + i];
-        e[(long)(ch0 + q) * Nd + core[c0 + i]] += omega * v;
-      }
+#pragma unroll 4
+    for (int sl = part + W * kPre; kJ * sl < nx; sl += W) {
+      float m[kJ];
+      Entries(M, (long)sl * nc + i, m);
+      add(m, kJ * sl);
     }
+  }
+#pragma unroll
+  for (int q = 0; q < KC; q++) P[part][q][i] = acc[q];
+  __syncthreads();
+  if (out) {
+    float v = 0.0f;
+#pragma unroll
+    for (int p = 0; p < W; p++) v += P[p][part][i];
+    if constexpr (kScaled) v *= scale;
+    e[at] = old + omega * v;
   }
 }
 
@@ -982,15 +1009,19 @@ __global__ __launch_bounds__(64 * W) void KMixSchwarz(const int* __restrict__ co
 // deep texels from the tile's bit masks, so no load waits on the texel type).
 // (Measured and not kept: the tile's (4 x 64 + 1) x (4 x 4 + 1) fine window staged in LDS one
 // column at a time by row-contiguous loads: 101 instead of 95 us at C2 level 0.)
-__device__ __forceinline__ void RestrictDeepTile(int vb, int c0, const int* __restrict__ tiles, const unsigned long long* __restrict__ cDeepMask,
-                                                 const MixChart* __restrict__ cch, const MixChart* __restrict__ fch, long cplane, long cNd,
-                                                 long fplane, long fNd, const float* __restrict__ fres, float* crhs, float* ce, int K) {
+// kSplit: one plane per workgroup, as in ResidualDeepTile.
+template <bool kSplit>
+__device__ __forceinline__ void RestrictDeepTile(int vb, int c0, const MixTile* __restrict__ tiles,
+                                                 const unsigned long long* __restrict__ cDeepMask, long cplane, long cNd, long fplane, long fNd,
+                                                 const float* __restrict__ fres, float* crhs, float* ce, int K) {
+  const int plane0 = kSplit ? vb % 4 : 0, plane1 = kSplit ? plane0 + 1 : 4;
+  if constexpr (kSplit) vb /= 4;
   const int row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
   const unsigned long long* mk = cDeepMask + (long)vb * 4 * kTB + row;
-  const int* T = tiles + 3 * vb;
-  const MixChart c = cch[T[0]], f = fch[T[0]];
-  const int a = T[1] + tx, b = T[2] + row;
-  for (int q = 0; q < 4; q++) {
+  const MixTile& T = tiles[vb];
+  const MixGrid c = T.own, f = T.finer;
+  const int a = T.a0 + tx, b = T.b0 + row;
+  for (int q = plane0; q < plane1; q++) {
     if (!((mk[q * kTB] >> tx) & 1ull)) continue;  // coarse deep texels from the tile's bit masks
     const int ci = 2 * a + (q & 1), cj = 2 * b + (q >> 1);
     const long idx = (long)q * cplane + c.base2 + (long)b * c.w2 + a;
@@ -1023,38 +1054,26 @@ __device__ __forceinline__ void RestrictBoundaryRows(int vb, int c0, int B, cons
                                                      int K) {
   const int r = (int)(((long)vb * blockDim.x + threadIdx.x) / kRowLanes), lane = threadIdx.x % kRowLanes;
   if (r >= B) return;  // whole row groups leave together
-  const int k0 = rp[r], k1 = rp[r + 1];
+  const int k0 = rp[r], k1 = rp[r + 1], kc = min(4, K - c0);
   const long d = bdIdx[r];
-  const int kc = min(4, K - c0);
-  {
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k = k0 + lane; k < k1; k += kRowLanes) {
-      const int2 w = ent[k];
-      const float v = __int_as_float(w.y);
-      const long c = w.x;
-#pragma unroll
-      for (int q = 0; q < 4; q++)
-        if (q < kc) acc[q] += v * fres[(long)(c0 + q) * fNd + c];
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q++) acc[q] = RowSum(acc[q]);
-    if (lane < kc) {
-      crhs[(long)(c0 + lane) * cNd + d] = Pick(acc, lane);
-      ce[(long)(c0 + lane) * cNd + d] = 0.0f;
-    }
+  float acc[4];
+  RowTerms(ent, k0, k1, lane, fres + (long)c0 * fNd, fNd, kc, acc);
+  if (lane < kc) {
+    crhs[(long)(c0 + lane) * cNd + d] = Pick(acc, lane);
+    ce[(long)(c0 + lane) * cNd + d] = 0.0f;
   }
 }
 
 // Restriction into a level in one launch: the first blocks take the coarse deep tiles, the others
 // the coarse boundary rows (disjoint outputs).
-__global__ __launch_bounds__(256) void KMixRestrict(int nTiles, const int* __restrict__ tiles, const unsigned long long* __restrict__ cDeepMask,
-                                                    const MixChart* __restrict__ cch, const MixChart* __restrict__ fch, long cplane, long cNd,
-                                                    long fplane, long fNd, const float* __restrict__ fres, float* crhs, float* ce, int K, int B,
+template <bool kSplit>
+__global__ __launch_bounds__(256) void KMixRestrict(int nTiles, const MixTile* __restrict__ tiles,
+                                                    const unsigned long long* __restrict__ cDeepMask, long cplane, long cNd, long fplane, long fNd, const float* __restrict__ fres, float* crhs, float* ce, int K, int B,
                                                     const int* __restrict__ bdIdx, const int* __restrict__ rp, const int2* __restrict__ ent) {
-  const int deepBlocks = nTiles * ((K + 3) / 4);
+  const int parts = kSplit ? 4 * nTiles : nTiles, deepBlocks = parts * ((K + 3) / 4);
   if ((int)blockIdx.x < deepBlocks) {
-    const TileChunk v = TileOf<4>(blockIdx.x, nTiles, K);
-    RestrictDeepTile(v.tile, v.c0, tiles, cDeepMask, cch, fch, cplane, cNd, fplane, fNd, fres, crhs, ce, K);
+    const TileChunk v = TileOf<4>(blockIdx.x, parts, K);
+    RestrictDeepTile<kSplit>(v.tile, v.c0, tiles, cDeepMask, cplane, cNd, fplane, fNd, fres, crhs, ce, K);
   } else {
     const TileChunk v = TileOf<4>(blockIdx.x - deepBlocks, NBlk((long)B * kRowLanes, 256), K);
     RestrictBoundaryRows(v.tile, v.c0, B, bdIdx, rp, ent, fres, fNd, crhs, ce, cNd, K);
@@ -1069,17 +1088,16 @@ __global__ __launch_bounds__(256) void KMixRestrict(int nTiles, const int* __res
 // mean of two (bx, bx + 1): bx = 0 for both when ui0 is even, bx = qi when ui0 is odd.  Deep texels of
 // plane `skipQ` are left alone: the Gauss-Seidel sweep that follows overwrites them without reading
 // them (skipQ = -1 when no sweep follows).
-__global__ __launch_bounds__(256) void KMixProlongAdd(const int* __restrict__ tiles, const unsigned long long* __restrict__ fDeepMask,
-                                                      const unsigned long long* __restrict__ fActiveMask, const MixChart* __restrict__ fch,
-                                                      const MixChart* __restrict__ cch, long fplane, long fNd, long cplane, long cNd,
+__global__ __launch_bounds__(256) void KMixProlongAdd(const MixTile* __restrict__ tiles, const unsigned long long* __restrict__ fDeepMask,
+                                                      const unsigned long long* __restrict__ fActiveMask, long fplane, long fNd, long cplane, long cNd,
                                                       const float* __restrict__ ce, float* fe, int K, int nTiles, int skipQ) {
   // active (and deep) fine texels from the tile's bit masks: no load waits on the texel type
   const TileChunk v = TileOf<4>(blockIdx.x, nTiles, K);
   const int tile = v.tile, c0 = v.c0, row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
   const long mo = (long)tile * 4 * kTB + row;
-  const int* T = tiles + 3 * tile;
-  const MixChart f = fch[T[0]], c = cch[T[0]];
-  const int a = T[1] + tx, b = T[2] + row;
+  const MixTile& T = tiles[tile];
+  const MixGrid f = T.own, c = T.coarser;
+  const int a = T.a0 + tx, b = T.b0 + row;
   const int ui0 = 2 * a - f.cofx, uj0 = 2 * b - f.cofy;
   const int ci0 = FloorHalf(ui0) + c.cofx, cj0 = FloorHalf(uj0) + c.cofy;
   const bool ei = (ui0 & 1) == 0, ej = (uj0 & 1) == 0;
@@ -1706,6 +1724,7 @@ void UploadMixed(const Hierarchy& h, const OperatorHierarchy& oh, DeviceSystem& 
   ms.levels = nl, ms.kcap = kcap;
   ms.L.assign(nl, DevMixLevel());
   std::vector<std::vector<long>> g2dAll(nl);
+  std::vector<std::vector<int>> tilesAll(nl);  // 3 ints per tile: chart, a0, b0 (sub-grid origin)
   for (int l = 0; l < nl; l++) {
     const Level& H = h.levels[l];
     DevMixLevel& d = ms.L[l];
@@ -1779,7 +1798,7 @@ void UploadMixed(const Hierarchy& h, const OperatorHierarchy& oh, DeviceSystem& 
     {
       const std::vector<int> tiles = buildTiles(kTA, kTB);
       d.nTiles = (int)tiles.size() / 3;
-      d.tiles = Up(ms, tiles);
+      tilesAll[l] = tiles;
       // deep and active texels of each tile: [tile][plane][tile row] 64-bit masks, bit = column in the tile
       std::vector<unsigned long long> deep((size_t)d.nTiles * 4 * kTB, 0ull), active(deep.size(), 0ull);
       static_assert(kTA == 64, "one 64-bit mask per tile row");
@@ -1966,8 +1985,13 @@ void UploadMixed(const Hierarchy& h, const OperatorHierarchy& oh, DeviceSystem& 
       SchwarzBlocks blk;
       BuildSchwarzBlocks(bb, bidx, blk);
       d.nBlocks = (int)blk.corePtr.size() - 1;
-      d.blkCorePtr = Up(ms, blk.corePtr), d.blkCore = Up(ms, blk.core), d.blkExtPtr = Up(ms, blk.extPtr), d.blkExt = Up(ms, blk.ext);
-      d.blkMatPtr = Up(ms, blk.matPtr);
+      d.blkCore = Up(ms, blk.core), d.blkExt = Up(ms, blk.ext);
+      std::vector<int> extDense(blk.ext.size());
+      for (size_t k = 0; k < blk.ext.size(); k++) extDense[k] = bidx[blk.ext[k]];
+      d.blkExtDense = Up(ms, extDense);
+      std::vector<MixBlock> records(d.nBlocks);
+      for (int b = 0; b < d.nBlocks; b++)
+        records[b] = {blk.corePtr[b], blk.corePtr[b + 1] - blk.corePtr[b], blk.extPtr[b], blk.extPtr[b + 1] - blk.extPtr[b], {blk.matPtr[b], 0}};
       // FP16 quads of extended rows, each core row scaled by its largest |entry|, where the step
       // streams its matrices; levels with at most one block per CU prefetch every entry and are
       // latency-bound, and keep FP32 (FP16 pairs' conversions made them 0.5-0.8 us slower).
@@ -1997,8 +2021,10 @@ void UploadMixed(const Hierarchy& h, const OperatorHierarchy& oh, DeviceSystem& 
               H[(size_t)sl * nc + i] = make_uint2(h(4 * sl) | h(4 * sl + 1) << 16, h(4 * sl + 2) | h(4 * sl + 3) << 16);
           }
         }
-        d.blkMatPtrH = Up(ms, hp), d.blkMatH = Up(ms, mh), d.blkScale = Up(ms, sc);
+        for (int b = 0; b < d.nBlocks; b++) records[b].mat[1] = hp[b];
+        d.blkMatH = Up(ms, mh), d.blkScale = Up(ms, sc);
       }
+      d.blocks = Up(ms, records);
     } else {
       std::vector<int> bidx(d.B);
       for (int r = 0; r < d.B; r++) bidx[r] = g2d[H.boundaryGlobalIndex[r]];
@@ -2032,6 +2058,18 @@ void UploadMixed(const Hierarchy& h, const OperatorHierarchy& oh, DeviceSystem& 
     d.rhs = Zeros<float>(ms, (size_t)d.Nd * kcap);
     d.res = Zeros<float>(ms, (size_t)d.Nd * kcap);
     d.tmpB = Zeros<float>(ms, (size_t)std::max(d.B, 1) * kcap);
+  }
+  for (int l = 0; l < nl; l++) {  // tile records, with the charts of the levels either side
+    std::vector<MixTile> recs(ms.L[l].nTiles);
+    auto grid = [&](int level, int chart) {
+      const MixChart& m = ms.L[level].hcharts[chart];
+      return MixGrid{m.w2, m.base2, m.cofx, m.cofy};
+    };
+    for (int t = 0; t < ms.L[l].nTiles; t++) {
+      const int* T = &tilesAll[l][3 * (size_t)t];
+      recs[t] = {T[1], T[2], {0, 0}, grid(l, T[0]), grid(std::max(l - 1, 0), T[0]), grid(std::min(l + 1, nl - 1), T[0])};
+    }
+    ms.L[l].tileRecs = Up(ms, recs);
   }
   const size_t before = UploadByteCounter();
   UploadLdlt(ms.allocations, oh.coarseFactor, ms.coarse, kcap);
@@ -2074,9 +2112,9 @@ void UploadMixed(const Hierarchy& h, const OperatorHierarchy& oh, DeviceSystem& 
 // else FP32.
 static void DeepGsLaunch(DevMixLevel& d, int q, int K, hipStream_t s) {
   if (d.stencilH)
-    KMixDeepGs<true><<<ChunkBlocks<4>(d.nTiles, K), 256, 0, s>>>(q, d.nTiles, d.tiles, d.deepMask, d.charts, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.e, d.rhs, K);
+    KMixDeepGs<true><<<ChunkBlocks<4>(d.nTiles, K), 256, 0, s>>>(q, d.nTiles, d.tileRecs, d.deepMask, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.e, d.rhs, K);
   else
-    KMixDeepGs<false><<<ChunkBlocks<4>(d.nTiles, K), 256, 0, s>>>(q, d.nTiles, d.tiles, d.deepMask, d.charts, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.e, d.rhs, K);
+    KMixDeepGs<false><<<ChunkBlocks<4>(d.nTiles, K), 256, 0, s>>>(q, d.nTiles, d.tileRecs, d.deepMask, d.plane, d.Nd, d.stencil, d.stencilC, d.stencilH, d.e, d.rhs, K);
 }
 
 // One colour pair (first colour qa) of the deep sweep over the level's rows, columns in chunks of up
@@ -2176,14 +2214,25 @@ static int DeepSweep(MixedSystem& ms, DevMixLevel& d, bool post, int K, hipStrea
 }
 
 // res: the boundary rows' residual, or null when e is zero on the level (the residual is the rhs)
-template <int W, int kPre>
+template <int W, int kPre, int KC>
 static void SchwarzLaunch(MixedSystem& ms, DevMixLevel& d, const float* res, int K, hipStream_t s) {
+  const unsigned grid = ChunkBlocks<KC>(d.nBlocks, K);
+  const int* ext = res ? d.blkExt : d.blkExtDense;
+  const float* src = res ? res : d.rhs;
+  const long stride = res ? d.B : d.Nd;
   if (d.blkMatH && ms.schwarzHalf)
-    KMixSchwarz<W, kPre / 4, uint2><<<ChunkBlocks<4>(d.nBlocks, K), 64 * W, 0, s>>>(d.blkCorePtr, d.blkCore, d.blkExtPtr, d.blkExt, d.blkMatPtrH, d.blkMatH,
-                                                                d.blkScale, res, d.bdIdx, d.rhs, d.B, d.e, d.Nd, K, ms.omega);
+    KMixSchwarz<W, kPre / 4, uint2, KC><<<grid, 64 * W, 0, s>>>(d.blocks, d.blkCore, ext, d.blkMatH, d.blkScale, src, stride, d.e, d.Nd, K, ms.omega);
   else
-    KMixSchwarz<W, kPre, float><<<ChunkBlocks<4>(d.nBlocks, K), 64 * W, 0, s>>>(d.blkCorePtr, d.blkCore, d.blkExtPtr, d.blkExt, d.blkMatPtr, d.blkMat,
-                                                            nullptr, res, d.bdIdx, d.rhs, d.B, d.e, d.Nd, K, ms.omega);
+    KMixSchwarz<W, kPre, float, KC><<<grid, 64 * W, 0, s>>>(d.blocks, d.blkCore, ext, d.blkMat, nullptr, src, stride, d.e, d.Nd, K, ms.omega);
+}
+template <int W, int kPre>
+static void SchwarzStep(MixedSystem& ms, DevMixLevel& d, const float* res, int K, hipStream_t s) {
+  switch (std::min(K, 4)) {
+    case 1: SchwarzLaunch<W, kPre, 1>(ms, d, res, K, s); break;
+    case 2: SchwarzLaunch<W, kPre, 2>(ms, d, res, K, s); break;
+    case 3: SchwarzLaunch<W, kPre, 3>(ms, d, res, K, s); break;
+    default: SchwarzLaunch<W, kPre, 4>(ms, d, res, K, s); break;
+  }
 }
 
 // zeroE: e is zero on the whole level (start of pre-smoothing), so the first sweep takes the rhs
@@ -2197,11 +2246,11 @@ static void BoundarySweeps(MixedSystem& ms, DevMixLevel& d, int K, hipStream_t s
                                                                             d.tmpB, 1, d.Nd, K);
     const float* res = fromRhs ? nullptr : d.tmpB;
     if (d.nBlocks <= kSchwarzPrefetchBlocks)
-      SchwarzLaunch<kSchwarzWaves, kBlockExtMax / kSchwarzWaves>(ms, d, res, K, s);
+      SchwarzStep<kSchwarzWaves, kBlockExtMax / kSchwarzWaves>(ms, d, res, K, s);
     else if (d.nBlocks < kSchwarzManyBlocks)
-      SchwarzLaunch<kSchwarzWaves, 0>(ms, d, res, K, s);
+      SchwarzStep<kSchwarzWaves, 0>(ms, d, res, K, s);
     else
-      SchwarzLaunch<kSchwarzWavesLarge, 0>(ms, d, res, K, s);
+      SchwarzStep<kSchwarzWavesLarge, 0>(ms, d, res, K, s);
   }
 }
 
@@ -2271,15 +2320,15 @@ void MixedVCycle(DeviceSystem& ds, MixedSystem& ms, int K, hipStream_t s, bool z
     DevMixLevel &d = ms.L[l], &c = ms.L[l + 1];
     Smooth(ms, l, K, false, s, l > 0 || zeroE0);
     const long rb = ChunkBlocks<4>(NBlk((long)d.B * kRowLanes, 256), K), cb = ChunkBlocks<4>(NBlk((long)c.B * kRowLanes, 256), K);
-    const bool wide = d.nTiles > kResidualWideTiles;
-    const long db = wide ? ChunkBlocks<2>(d.nTiles, K) : ChunkBlocks<4>(d.nTiles, K), cd = ChunkBlocks<4>(c.nTiles, K);
+    const bool wide = d.nTiles > kResidualWideTiles, wideC = c.nTiles > kResidualWideTiles;
+    const long db = wide ? ChunkBlocks<2>(d.nTiles, K) : ChunkBlocks<4>(4 * d.nTiles, K), cd = ChunkBlocks<4>(wideC ? c.nTiles : 4 * c.nTiles, K);
     if (db + rb > 0)
-      (wide ? KMixResidual<2> : KMixResidual<4>)<<<db + rb, 256, 0, s>>>(
-          d.nTiles, d.tiles, d.deepMask, d.charts, d.plane, d.Nd, d.stencilSym, d.e, d.rhs, d.res, K, ms.nuPre > 0 && !d.stencilH ? 3 : -1,
-          d.B, d.bdIdx, d.bRowptr, d.bEnt, d.bDiag);
+      (wide ? KMixResidual<2, false> : KMixResidual<4, true>)<<<db + rb, 256, 0, s>>>(
+          d.nTiles, d.tileRecs, d.deepMask, d.plane, d.Nd, d.stencilSym, d.e, d.rhs, d.res, K, ms.nuPre > 0 && !d.stencilH ? 3 : -1, d.B, d.bdIdx,
+          d.bRowptr, d.bEnt, d.bDiag);
     if (cd + cb > 0)
-      KMixRestrict<<<cd + cb, 256, 0, s>>>(c.nTiles, c.tiles, c.deepMask, c.charts, d.charts, c.plane, c.Nd, d.plane, d.Nd, d.res, c.rhs,
-                                                 c.e, K, c.B, c.bdIdx, c.rRowptr, c.rEnt);
+      (wideC ? KMixRestrict<false> : KMixRestrict<true>)<<<cd + cb, 256, 0, s>>>(c.nTiles, c.tileRecs, c.deepMask, c.plane, c.Nd, d.plane, d.Nd,
+                                                                                d.res, c.rhs, c.e, K, c.B, c.bdIdx, c.rRowptr, c.rEnt);
   }
   {
     DevMixLevel& c = ms.L[nl - 1];
@@ -2297,7 +2346,7 @@ void MixedVCycle(DeviceSystem& ds, MixedSystem& ms, int K, hipStream_t s, bool z
     // the first post-smoothing sweep of a fused level adds the prolongation itself
     const bool fuse = ms.fuseProlong && ms.nuPost > 0 && Fused(d);
     if (d.nTiles > 0 && !fuse)
-      KMixProlongAdd<<<ChunkBlocks<4>(d.nTiles, K), 256, 0, s>>>(d.tiles, d.deepMask, d.activeMask, d.charts, c.charts, d.plane, d.Nd, c.plane, c.Nd, c.e, d.e,
+      KMixProlongAdd<<<ChunkBlocks<4>(d.nTiles, K), 256, 0, s>>>(d.tileRecs, d.deepMask, d.activeMask, d.plane, d.Nd, c.plane, c.Nd, c.e, d.e,
                                               K, d.nTiles, ms.nuPost > 0 ? 3 : -1);
     FusedProlong pr;
     pr.cch = c.charts, pr.cplane = c.plane, pr.cNd = c.Nd, pr.ce = c.e;
