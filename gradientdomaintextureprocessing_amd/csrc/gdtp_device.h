@@ -60,7 +60,7 @@ struct DevLevel {
   double* coefSym = nullptr;   // level 0: A's deep couplings in symmetric five-word form, SoA [5][N] over global
                                // indices (slots 0-3: lower neighbours k = 0..3, slot 4: diagonal)
   int* bgi = nullptr;          // boundary -> global
-  DevCsr bd, bb, brestr;       // A_BD, A_BB, boundary restriction to level+1
+  DevCsr brestr;               // boundary restriction to level+1
   DevCsr rows;                 // A_BB's and (from rowMid on) A_BD's entries row by row, global columns
   int* rowMid = nullptr;
   // band tasks
@@ -80,7 +80,7 @@ struct DevLevel {
 struct DeviceSystem {
   int levels = 0, kcap = 0;
   std::vector<DevLevel> L;
-  DevLevel mass0, stiff0;      // level-0 mass and stiffness (raw stencils and boundary rows only)
+  DevLevel mass0, stiff0;      // level-0 mass and stiffness (raw stencils and boundary rows only; the rows share their columns)
   std::vector<void*> allocations;
   size_t bytes = 0;
   hipStream_t stream = nullptr;

@@ -7,6 +7,7 @@
 #include <stdexcept>
 
 #include "gdtp_device.h"
+#include "gdtp_tiles.h"
 
 #include <mutex>
 
@@ -512,22 +513,26 @@ __global__ void KProlongAdd(int nLines, const int* __restrict__ lines, const dou
 
 // ------------------------------------------------------------------ operator application
 // y = A x with raw stencils (MultiplyBySystemMatrix_NoReciprocals, IterativeSolvers.inl:881-950), or with
-// `b` the residual b - A x, in one launch (blockIdx.y = chunk of KC columns, all of whose loads are in
-// flight together): blocks [0, rowBlocks) take the boundary rows, the others one raster line each.
+// `b` the residual b - A x, in one launch: first the boundary rows (rowBlocks blocks per chunk of KC
+// columns, all of whose loads are in flight together), then a raster line and chunk per workgroup.
 // (A small apply is its launches and round trips: one launch with kRowLanes lanes per row and global
 // columns took 6,936 texels x 3 columns from 14.1 to 4.0 us of kernels (13.3 to 10.1 a call) against a thread per row and column that
-// looked its A_BB columns up, beside the deep rows' own launch.)
+// looked its A_BB columns up, beside the deep rows' own launch.  A large one is bound by memory: a line's
+// chunks and its neighbours in one XCD's L2 (TileOf) took 3.3 M texels x 16 columns from 551 to 473 us.)
 template <int KC>
-__global__ __launch_bounds__(kRowThreads) void KApply(int rowBlocks, int B, const int* __restrict__ bgi, const int* __restrict__ rp,
+__global__ __launch_bounds__(kRowThreads) void KApply(int rowBlocks, int nLines, int B, const int* __restrict__ bgi, const int* __restrict__ rp,
                                                       const int* __restrict__ mid, const int* __restrict__ cl, const double* __restrict__ vl, const int* __restrict__ lines,
                                                       const double* __restrict__ coef, int D, const double* __restrict__ x,
                                                       const double* __restrict__ b, double* y, int K, int ld) {
-  const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
+  const int rowWork = rowBlocks * ((K + KC - 1) / KC);
+  const bool onBoundary = (int)blockIdx.x < rowWork;
+  const TileChunk v0 = onBoundary ? TileOf<KC>(blockIdx.x, rowBlocks, K) : TileOf<KC>(blockIdx.x - rowWork, nLines, K);
+  const int c0 = v0.c0, kc = min(KC, K - c0);
   x += (size_t)c0 * ld, y += (size_t)c0 * ld;
   if (b) b += (size_t)c0 * ld;
-  if ((int)blockIdx.x < rowBlocks) {
+  if (onBoundary) {
     __shared__ RowTerms<KC, kRowThreads> terms;
-    const int row = (blockIdx.x * kRowThreads + (int)threadIdx.x) / kRowLanes, c = threadIdx.x % kRowLanes;
+    const int row = (v0.tile * kRowThreads + (int)threadIdx.x) / kRowLanes, c = threadIdx.x % kRowLanes;
     if (row >= B) return;  // whole row groups leave together
     const double s = RowSum(rp[row], mid[row], rp[row + 1], cl, vl, x, ld, kc, terms);
     if (c < kc) {
@@ -536,7 +541,7 @@ __global__ __launch_bounds__(kRowThreads) void KApply(int rowBlocks, int B, cons
     }
     return;
   }
-  const int* L = lines + 5 * (blockIdx.x - rowBlocks);
+  const int* L = lines + 5 * v0.tile;
   const int start = L[0], len = L[1] - L[0] + 1, prev = L[2], next = L[3], d0 = L[4];
   for (int i = threadIdx.x; i < len; i += kRowThreads) {
     double a[9], v[KC][9], bv[KC];
@@ -835,8 +840,6 @@ void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOpe
     d.coefRaw = Upload(ds, SoA10(O.deepRaw));
     if (l == 0) d.coefSym = Upload(ds, SymStencil(O.deepRaw, H.rasterLines, H.numTexels));
     d.bgi = Upload(ds, H.boundaryGlobalIndex);
-    d.bd = UploadCsr(ds, O.bd);
-    d.bb = UploadCsr(ds, O.bb);
     UploadBoundaryRows(ds, d, O.bb, O.bd, H.boundaryGlobalIndex);
     if (l + 1 < nl) d.brestr = UploadCsr(ds, H.boundaryRestriction);
     d.nTasks = (int)H.tasks.taskPtr.size() - 1;
@@ -874,10 +877,22 @@ void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOpe
     d.N = l0.N, d.D = l0.D, d.B = l0.B, d.bgi = l0.bgi, d.nRaster = l0.nRaster, d.raster = l0.raster;
     d.coefRaw = Upload(ds, SoA10(which == 0 ? op.deepMass : op.deepStiffness));
     d.coefSym = Upload(ds, SymStencil(which == 0 ? op.deepMass : op.deepStiffness, h.levels[0].rasterLines, l0.N));
-    d.bd = UploadCsr(ds, which == 0 ? op.bdMass : op.bdStiffness);
-    d.bb = UploadCsr(ds, which == 0 ? op.bbMass : op.bbStiffness);
-    if (which == 0) UploadBoundaryRows(ds, d, op.bbMass, op.bdMass, h.levels[0].boundaryGlobalIndex);
-    else UploadBoundaryRows(ds, d, op.bbStiffness, op.bdStiffness, h.levels[0].boundaryGlobalIndex);
+  }
+  {  // one pattern for both (an entry only one of them has: zero in the other)
+    const std::vector<int>& bgi = h.levels[0].boundaryGlobalIndex;
+    auto widened = [](const Csr& m, const Csr& other) {
+      return m.rowptr == other.rowptr && m.col == other.col ? m : m.Combine(1.0, other, 0.0);
+    };
+    UploadBoundaryRows(ds, ds.mass0, widened(op.bbMass, op.bbStiffness), widened(op.bdMass, op.bdStiffness), bgi);
+    const Csr bbS = widened(op.bbStiffness, op.bbMass), bdS = widened(op.bdStiffness, op.bdMass);
+    std::vector<double> val;
+    val.reserve(bbS.val.size() + bdS.val.size());
+    for (int r = 0; r < bbS.rows; r++) {
+      val.insert(val.end(), bbS.val.begin() + bbS.rowptr[r], bbS.val.begin() + bbS.rowptr[r + 1]);
+      val.insert(val.end(), bdS.val.begin() + bdS.rowptr[r], bdS.val.begin() + bdS.rowptr[r + 1]);
+    }
+    ds.stiff0.rows = ds.mass0.rows, ds.stiff0.rowMid = ds.mass0.rowMid;
+    ds.stiff0.rows.val = Upload(ds, val);
   }
   ds.bytes = g_uploadBytes;
 }
@@ -985,7 +1000,7 @@ static void ApplyRows(DevLevel& d, const double* x, const double* b, double* y, 
   // three columns at a time: 27 values of x in registers
   const int chunks = (K + 2) / 3, kc = (K + chunks - 1) / chunks;
   const auto kernel = kc == 1 ? KApply<1> : kc == 2 ? KApply<2> : KApply<3>;
-  kernel<<<dim3(rowBlocks + d.nRaster, (K + kc - 1) / kc), kRowThreads, 0, s>>>(rowBlocks, d.B, d.bgi, d.rows.rowptr, d.rowMid, d.rows.col, d.rows.val,
+  kernel<<<(unsigned)((long)(rowBlocks + d.nRaster) * ((K + kc - 1) / kc)), kRowThreads, 0, s>>>(rowBlocks, d.nRaster, d.B, d.bgi, d.rows.rowptr, d.rowMid, d.rows.col, d.rows.val,
                                                                                 d.raster, d.coefRaw, d.D, x, b, y, K, ld);
 }
 

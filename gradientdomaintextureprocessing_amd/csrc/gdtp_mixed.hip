@@ -14,6 +14,7 @@
 // Transfers are the reference's: 3x3 full weighting / the boundary restriction matrix, and
 // bilinear prolongation (IterativeSolvers.inl:1009-1168), evaluated from chart geometry.
 #include "gdtp_mixed.h"
+#include "gdtp_tiles.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -47,34 +48,6 @@ template <class G>  // MixChart or MixGrid
 __device__ __forceinline__ int DenseByte(const G& c, long plane, int i, int j) {
   return 4 * (((i & 1) | ((j & 1) << 1)) * (int)plane + c.base2 + (j >> 1) * c.w2 + (i >> 1));
 }
-
-// Tile (or block of rows) of workgroup b when the eight XCDs (workgroup b runs on XCD b % 8) each
-// take a contiguous eighth of the n tiles, in order: XCD x owns tiles [x per + min(x, rem), ...),
-// per + (x < rem) of them (a bijection on [0, n)).  Neighbouring tiles then share an L2, so the halo
-// texels a tile reads from its neighbours are mostly L2 hits instead of HBM re-reads.
-__device__ __forceinline__ int XcdTile(int b, int n) {
-  const int x = b % 8, k = b / 8, per = n / 8, rem = n % 8;
-  return x * per + min(x, rem) + k;
-}
-
-// Columns in chunks of up to kMax, a chunk per workgroup: workgroups are numbered tile by tile and
-// within a tile chunk by chunk, in XCD-contiguous order, so that a tile's chunks run on one XCD one
-// after another and read its stencil, masks and row tables from that XCD's L2.  (With the chunks in a
-// loop inside the workgroup, each waited for the one before it: 3.0 M texels x 64 columns, V-cycle
-// residual of level 0 1027 us, 896 so; one colour pair of level 0, 16 launches, 554 us, one launch 448; a
-// solve pair 348 to 292 ms.)
-struct TileChunk {
-  int tile, c0;
-};
-template <int kMax>
-__device__ __forceinline__ TileChunk TileOf(int b, int nTiles, int K) {
-  const int chunks = (K + kMax - 1) / kMax;
-  if (chunks == 1) return {XcdTile(b, nTiles), 0};
-  const int v = XcdTile(b, nTiles * chunks);
-  return {v / chunks, v % chunks * kMax};
-}
-template <int kMax>
-static inline unsigned ChunkBlocks(long blocks, int K) { return (unsigned)(blocks * ((K + kMax - 1) / kMax)); }
 
 // f(chunk width as a compile-time constant), so that a kernel can issue every load of its chunk before
 // its first store (one memory round trip per chunk instead of one per column).
@@ -1341,157 +1314,148 @@ __device__ __forceinline__ void K64ResidualDeepRows(int vb, int c0, int D, const
 
 // The same residual for per-column operators A_c = w[c][0] M + w[c][1] S (parametric solves: one
 // refinement loop serves columns with different weights, its FP32 V-cycle built for one nearby pair
-// of weights): both level-0 stencils read once per texel for a chunk of columns.
+// of weights): both level-0 stencils read once per texel for a chunk of four columns.  (3.3 M texels x 4
+// columns: 366 us a launch with chunks of two, all of whose values are loaded together; 292 so.)
 __device__ __forceinline__ void K64ResidualDeepWRows(int vb, int c0, int D, const int* __restrict__ deepLine, const int* __restrict__ lines,
                                                      const double* __restrict__ symM, const double* __restrict__ symS,
                                                      const double* __restrict__ x, const double* __restrict__ b, int N,
                                                      const int* __restrict__ g2d, float* rhs0, float* e0, long Nd, double* norms, int K,
                                                      const double* __restrict__ w, double* r64, double* bnorms) {
-  {
-    const int kc = min(2, K - c0);  // chunks of two columns (two stencils in registers)
-    double acc[4] = {0, 0, 0, 0}, bacc[4] = {0, 0, 0, 0};
-    for (int g = 0; g < kDeepGroups; g++) {
-      const int d = (vb * kDeepGroups + g) * blockDim.x + threadIdx.x;
-      if (d >= D) break;
-      int cur, prev, next;
-      DeepRow(deepLine, lines, d, cur, prev, next);
-      double cm[9], cs[9];
-      SymRow(symM, N, cur, next, cm);
-      SymRow(symS, N, cur, next, cs);
-      const long di = g2d[cur];
-      WithChunkWidth<2>(kc, [&](auto kcc) {
-        constexpr int KC = decltype(kcc)::value;
-        double xv[KC][9], bv[KC];
-        RowValues<KC>(x, N, c0, prev, cur, next, xv);
+  const int kc = min(4, K - c0);  // two stencils in registers, a column in use and the next one's values on their way
+  double acc[4] = {0, 0, 0, 0}, bacc[4] = {0, 0, 0, 0};
+  for (int g = 0; g < kDeepGroups; g++) {
+    const int d = (vb * kDeepGroups + g) * blockDim.x + threadIdx.x;
+    if (d >= D) break;
+    int cur, prev, next;
+    DeepRow(deepLine, lines, d, cur, prev, next);
+    double cm[9], cs[9], xv[2][1][9], bv[2];
+    SymRow(symM, N, cur, next, cm);
+    SymRow(symS, N, cur, next, cs);
+    const long di = g2d[cur];
+    RowValues<1>(x, N, c0, prev, cur, next, xv[0]);
+    bv[0] = b[(long)c0 * N + cur];
 #pragma unroll
-        for (int cc = 0; cc < KC; cc++) bv[cc] = b[(long)(c0 + cc) * N + cur];
+    for (int cc = 0; cc < 4; cc++) {
+      if (cc >= kc) break;
+      const int ch = c0 + cc, ahead = min(ch + 1, K - 1);
+      if (cc < 3) {
+        RowValues<1>(x, N, ahead, prev, cur, next, xv[(cc + 1) % 2]);
+        bv[(cc + 1) % 2] = b[(long)ahead * N + cur];
+      }
+      const double (&v)[9] = xv[cc % 2][0];
+      double sm = 0.0, ss = 0.0;
 #pragma unroll
-        for (int cc = 0; cc < KC; cc++) {
-          const int ch = c0 + cc;
-          double sm = 0.0, ss = 0.0;
-#pragma unroll
-          for (int k = 0; k < 9; k++) sm += cm[k] * xv[cc][k], ss += cs[k] * xv[cc][k];
-          const double r = bv[cc] - (w[2 * ch] * sm + w[2 * ch + 1] * ss);
-          if (r64) r64[(long)ch * N + cur] = r;
-          rhs0[(long)ch * Nd + di] = (float)r;
-          e0[(long)ch * Nd + di] = 0.0f;
-          acc[cc] += r * r, bacc[cc] += bv[cc] * bv[cc];
-        }
-      });
+      for (int k = 0; k < 9; k++) sm += cm[k] * v[k], ss += cs[k] * v[k];
+      const double r = bv[cc % 2] - (w[2 * ch] * sm + w[2 * ch + 1] * ss);
+      if (r64) r64[(long)ch * N + cur] = r;
+      rhs0[(long)ch * Nd + di] = (float)r;
+      e0[(long)ch * Nd + di] = 0.0f;
+      acc[cc] += r * r, bacc[cc] += bv[cc % 2] * bv[cc % 2];
     }
-    BlockAddSquares4(acc, kc, norms + (long)c0 * kSlots);  // every thread of the block
-    if (bnorms) BlockAddSquares4(bacc, kc, bnorms + (long)c0 * kSlots);
+  }
+  BlockAddSquares4(acc, kc, norms + (long)c0 * kSlots);  // every thread of the block
+  if (bnorms) BlockAddSquares4(bacc, kc, bnorms + (long)c0 * kSlots);
+}
+
+// Level-0 boundary rows, columns global: A_BB's entries, then (from mid on) A_BD's; two values per entry
+// where a pass takes M and S together (PairRows).
+struct Rows64 {
+  const int *rp, *mid, *col;
+  const double *v0, *v1;
+};
+
+// A boundary row's sums for up to four columns, in every lane of the row's group.  A row has about 14
+// A_BB entries and one A_BD entry: two rounds of the lanes over the first and one over the second are
+// loaded together, then added in the row's order.  Two operators share the columns and the gathered x
+// (a gather costs a cache line per lane).  (87 k rows x 64 columns in a launch of 1.1 ms for
+// its deep rows: M's and S's rows loaded ahead but apart 378 us, so 245.)
+template <bool kPair>
+__device__ __forceinline__ void RowSums64(const Rows64& R, int r, int lane, const double* __restrict__ x, long N, int kc, double (&s0)[4],
+                                          double (&s1)[4]) {
+  const int k0 = R.rp[r], km = R.mid[r], k1 = R.rp[r + 1];
+  double v0[3], v1[3], xv[3][4];
+#pragma unroll
+  for (int t = 0; t < 3; t++) {
+    const int k = (t < 2 ? k0 + t * kRowLanes64 : km) + lane;
+    const bool in = k < (t < 2 ? km : k1);
+    const int g = in ? R.col[k] : 0;
+    v0[t] = in ? R.v0[k] : 0.0;
+    v1[t] = kPair && in ? R.v1[k] : 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) xv[t][q] = in && q < kc ? x[(long)q * N + g] : 0.0;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) s0[q] = s1[q] = 0.0;
+  auto add = [&](double a, double b, const double (&v)[4]) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      if (q >= kc) continue;
+      s0[q] += a * v[q];
+      if (kPair) s1[q] += b * v[q];
+    }
+  };
+  auto rest = [&](int k, int end) {
+    for (; k < end; k += kRowLanes64) {
+      const int g = R.col[k];
+      double v[4];
+#pragma unroll
+      for (int q = 0; q < 4; q++) v[q] = q < kc ? x[(long)q * N + g] : 0.0;
+      add(R.v0[k], kPair ? R.v1[k] : 0.0, v);
+    }
+  };
+#pragma unroll
+  for (int t = 0; t < 2; t++)
+    if (k0 + t * kRowLanes64 + lane < km) add(v0[t], v1[t], xv[t]);
+  rest(k0 + 2 * kRowLanes64 + lane, km);
+  if (km + lane < k1) add(v0[2], v1[2], xv[2]);
+  rest(km + kRowLanes64 + lane, k1);
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    s0[q] = RowSum<double, kRowLanes64>(s0[q]);
+    if (kPair) s1[q] = RowSum<double, kRowLanes64>(s1[q]);
   }
 }
 
-// Boundary rows of the per-column-weights residual: rows of M (A_BB, A_BD) then of S.
-__device__ __forceinline__ void K64ResidualBoundaryWRows(int vb, int B, const int* __restrict__ bgi, const int* __restrict__ mrpd,
-                                                         const int* __restrict__ mcold, const double* __restrict__ mvald,
-                                                         const int* __restrict__ mrpb, const int* __restrict__ mcolb,
-                                                         const double* __restrict__ mvalb, const int* __restrict__ srpd,
-                                                         const int* __restrict__ scold, const double* __restrict__ svald,
-                                                         const int* __restrict__ srpb, const int* __restrict__ scolb,
-                                                         const double* __restrict__ svalb, const double* __restrict__ x,
-                                                         const double* __restrict__ b, int N, const int* __restrict__ g2d, float* rhs0,
-                                                         float* e0, long Nd, double* norms, int K, const double* __restrict__ w,
-                                                         double* r64, double* bnorms) {
+// r = b - A x at the boundary rows (kPair: A_c = w[c][0] M + w[c][1] S), kRowLanes64 lanes per row, four
+// columns per workgroup; no early exit: every thread takes part in the block sums.
+template <bool kPair>
+__device__ __forceinline__ void K64ResidualBoundaryRows(int vb, int c0, int B, const int* __restrict__ bgi, const Rows64& R,
+                                                        const double* __restrict__ x, const double* __restrict__ b, int N,
+                                                        const int* __restrict__ g2d, float* rhs0, float* e0, long Nd, double* norms, int K,
+                                                        const double* __restrict__ w, double* r64, double* bnorms) {
   const int r = (int)(((long)vb * blockDim.x + threadIdx.x) / kRowLanes64), lane = threadIdx.x % kRowLanes64;
-  const bool active = r < B;
-  for (int c0 = 0; c0 < K; c0 += 4) {
-    const int kc = min(4, K - c0);
-    double am[4] = {0.0, 0.0, 0.0, 0.0}, as[4] = {0.0, 0.0, 0.0, 0.0};
-    if (active) {
-      auto rows = [&](const int* rp, const int* cl, const double* vl, bool viaBoundary, double (&acc)[4]) {
-        for (int k = rp[r] + lane; k < rp[r + 1]; k += kRowLanes64) {
-          const double v = vl[k];
-          const int g = viaBoundary ? bgi[cl[k]] : cl[k];
-#pragma unroll
-          for (int q = 0; q < 4; q++)
-            if (q < kc) acc[q] += v * x[(long)(c0 + q) * N + g];
-        }
-      };
-      rows(mrpb, mcolb, mvalb, true, am);
-      rows(mrpd, mcold, mvald, false, am);
-      rows(srpb, scolb, svalb, true, as);
-      rows(srpd, scold, svald, false, as);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q++) am[q] = RowSum<double, kRowLanes64>(am[q]), as[q] = RowSum<double, kRowLanes64>(as[q]);
-    double sq = 0.0, bq = 0.0;
-    if (active && lane < kc) {
-      const int ch = c0 + lane, g = bgi[r];
-      const double bv = b[(long)ch * N + g], rv = bv - (w[2 * ch] * Pick(am, lane) + w[2 * ch + 1] * Pick(as, lane));
-      if (r64) r64[(long)ch * N + g] = rv;
-      rhs0[(long)ch * Nd + g2d[g]] = (float)rv;
-      e0[(long)ch * Nd + g2d[g]] = 0.0f;
+  const int kc = min(4, K - c0), ch = c0 + min(lane, kc - 1);
+  double sq = 0.0, bq = 0.0;
+  if (r < B) {
+    const int g = bgi[r];
+    const long o = (long)ch * Nd + g2d[g];
+    const double bv = b[(long)ch * N + g];
+    double s0[4], s1[4];
+    RowSums64<kPair>(R, r, lane, x + (long)c0 * N, N, kc, s0, s1);
+    if (lane < kc) {
+      double rv;
+      if constexpr (kPair) rv = bv - (w[2 * ch] * Pick(s0, lane) + w[2 * ch + 1] * Pick(s1, lane));
+      else rv = bv - Pick(s0, lane);
+      if (kPair && r64) r64[(long)ch * N + g] = rv;
+      rhs0[o] = (float)rv;
+      e0[o] = 0.0f;
       sq = rv * rv, bq = bv * bv;
     }
-    {
-      const double sqs[4] = {lane == 0 ? sq : 0.0, lane == 1 ? sq : 0.0, lane == 2 ? sq : 0.0, lane == 3 ? sq : 0.0};
-      BlockAddSquares4(sqs, kc, norms + (long)c0 * kSlots);
-    }
-    if (bnorms) {
-      const double bqs[4] = {lane == 0 ? bq : 0.0, lane == 1 ? bq : 0.0, lane == 2 ? bq : 0.0, lane == 3 ? bq : 0.0};
-      BlockAddSquares4(bqs, kc, bnorms + (long)c0 * kSlots);
-    }
+  }
+  const double sqs[4] = {lane == 0 ? sq : 0.0, lane == 1 ? sq : 0.0, lane == 2 ? sq : 0.0, lane == 3 ? sq : 0.0};
+  BlockAddSquares4(sqs, kc, norms + (long)c0 * kSlots);
+  if (bnorms) {
+    const double bqs[4] = {lane == 0 ? bq : 0.0, lane == 1 ? bq : 0.0, lane == 2 ? bq : 0.0, lane == 3 ? bq : 0.0};
+    BlockAddSquares4(bqs, kc, bnorms + (long)c0 * kSlots);
   }
 }
 
-__device__ __forceinline__ void K64ResidualBoundaryRows(int vb, int B, const int* __restrict__ bgi, const int* __restrict__ rpd,
-                                                        const int* __restrict__ cold, const double* __restrict__ vald,
-                                                        const int* __restrict__ rpb, const int* __restrict__ colb,
-                                                        const double* __restrict__ valb, const double* __restrict__ x,
-                                                        const double* __restrict__ b, int N, const int* __restrict__ g2d, float* rhs0,
-                                                        float* e0, long Nd, double* norms, int K, double* bnorms) {
-  // kRowLanes64 lanes per boundary row (no early exit: every thread takes part in the block sums)
-  const int r = (int)(((long)vb * blockDim.x + threadIdx.x) / kRowLanes64), lane = threadIdx.x % kRowLanes64;
-  const bool active = r < B;
-  for (int c0 = 0; c0 < K; c0 += 4) {
-    const int kc = min(4, K - c0);
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    if (active) {
-      for (int k = rpb[r] + lane; k < rpb[r + 1]; k += kRowLanes64) {
-        const double v = valb[k];
-        const int g = bgi[colb[k]];
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          if (q < kc) acc[q] += v * x[(long)(c0 + q) * N + g];
-      }
-      for (int k = rpd[r] + lane; k < rpd[r + 1]; k += kRowLanes64) {
-        const double v = vald[k];
-        const int g = cold[k];
-#pragma unroll
-        for (int q = 0; q < 4; q++)
-          if (q < kc) acc[q] += v * x[(long)(c0 + q) * N + g];
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q++) acc[q] = RowSum<double, kRowLanes64>(acc[q]);
-    double sq = 0.0, bq = 0.0;
-    if (active && lane < kc) {
-      const int g = bgi[r];
-      const double bv = b[(long)(c0 + lane) * N + g], rv = bv - Pick(acc, lane);
-      rhs0[(long)(c0 + lane) * Nd + g2d[g]] = (float)rv;
-      e0[(long)(c0 + lane) * Nd + g2d[g]] = 0.0f;
-      sq = rv * rv, bq = bv * bv;
-    }
-    {
-      const double sqs[4] = {lane == 0 ? sq : 0.0, lane == 1 ? sq : 0.0, lane == 2 ? sq : 0.0, lane == 3 ? sq : 0.0};
-      BlockAddSquares4(sqs, kc, norms + (long)c0 * kSlots);
-    }
-    if (bnorms) {
-      const double bqs[4] = {lane == 0 ? bq : 0.0, lane == 1 ? bq : 0.0, lane == 2 ? bq : 0.0, lane == 3 ? bq : 0.0};
-      BlockAddSquares4(bqs, kc, bnorms + (long)c0 * kSlots);
-    }
-  }
-}
+__host__ __device__ static inline unsigned RowBlocks64(int B) { return NBlk((long)B * kRowLanes64, 256); }
 
 // The level-0 FP64 residual in one launch: blocks [0, deepBlocks) take the deep rows, the others
 // the boundary rows (disjoint rows; every block takes part in its own norm sums).
 __global__ __launch_bounds__(256) void K64Residual(int deepBlocks, int D, const int* __restrict__ deepLine, const int* __restrict__ lines,
-                                                   const double* __restrict__ sym, int B, const int* __restrict__ bgi,
-                                                   const int* __restrict__ rpd, const int* __restrict__ cold, const double* __restrict__ vald,
-                                                   const int* __restrict__ rpb, const int* __restrict__ colb, const double* __restrict__ valb,
+                                                   const double* __restrict__ sym, int B, const int* __restrict__ bgi, Rows64 rows,
                                                    const double* __restrict__ x, const double* __restrict__ b, int N,
                                                    const int* __restrict__ g2d, float* rhs0, float* e0, long Nd, double* norms, int K,
                                                    double* bnorms, int* fresh) {
@@ -1500,29 +1464,26 @@ __global__ __launch_bounds__(256) void K64Residual(int deepBlocks, int D, const 
   if ((int)blockIdx.x < deep) {
     const TileChunk v = TileOf<3>(blockIdx.x, deepBlocks, K);
     K64ResidualDeepRows(v.tile, v.c0, D, deepLine, lines, sym, x, b, N, g2d, rhs0, e0, Nd, norms, K, bnorms);
-  } else
-    K64ResidualBoundaryRows(blockIdx.x - deep, B, bgi, rpd, cold, vald, rpb, colb, valb, x, b, N, g2d, rhs0, e0, Nd, norms, K, bnorms);
+  } else {
+    const TileChunk v = TileOf<4>(blockIdx.x - deep, RowBlocks64(B), K);
+    K64ResidualBoundaryRows<false>(v.tile, v.c0, B, bgi, rows, x, b, N, g2d, rhs0, e0, Nd, norms, K, nullptr, nullptr, bnorms);
+  }
 }
 
 // The same for per-column weights (M and S rows of both parts).
 __global__ __launch_bounds__(256) void K64ResidualW(int deepBlocks, int D, const int* __restrict__ deepLine, const int* __restrict__ lines,
                                                     const double* __restrict__ symM, const double* __restrict__ symS, int B,
-                                                    const int* __restrict__ bgi, const int* __restrict__ mrpd, const int* __restrict__ mcold,
-                                                    const double* __restrict__ mvald, const int* __restrict__ mrpb,
-                                                    const int* __restrict__ mcolb, const double* __restrict__ mvalb,
-                                                    const int* __restrict__ srpd, const int* __restrict__ scold,
-                                                    const double* __restrict__ svald, const int* __restrict__ srpb,
-                                                    const int* __restrict__ scolb, const double* __restrict__ svalb,
-                                                    const double* __restrict__ x, const double* __restrict__ b, int N,
-                                                    const int* __restrict__ g2d, float* rhs0, float* e0, long Nd, double* norms, int K,
-                                                    const double* __restrict__ w, double* r64, double* bnorms) {
-  const int deep = deepBlocks * ((K + 1) / 2);
+                                                    const int* __restrict__ bgi, Rows64 rows, const double* __restrict__ x,
+                                                    const double* __restrict__ b, int N, const int* __restrict__ g2d, float* rhs0, float* e0,
+                                                    long Nd, double* norms, int K, const double* __restrict__ w, double* r64, double* bnorms) {
+  const int deep = deepBlocks * ((K + 3) / 4);
   if ((int)blockIdx.x < deep) {
-    const TileChunk v = TileOf<2>(blockIdx.x, deepBlocks, K);
+    const TileChunk v = TileOf<4>(blockIdx.x, deepBlocks, K);
     K64ResidualDeepWRows(v.tile, v.c0, D, deepLine, lines, symM, symS, x, b, N, g2d, rhs0, e0, Nd, norms, K, w, r64, bnorms);
-  } else
-    K64ResidualBoundaryWRows(blockIdx.x - deep, B, bgi, mrpd, mcold, mvald, mrpb, mcolb, mvalb, srpd, scold, svald, srpb, scolb,
-                             svalb, x, b, N, g2d, rhs0, e0, Nd, norms, K, w, r64, bnorms);
+  } else {
+    const TileChunk v = TileOf<4>(blockIdx.x - deep, RowBlocks64(B), K);
+    K64ResidualBoundaryRows<true>(v.tile, v.c0, B, bgi, rows, x, b, N, g2d, rhs0, e0, Nd, norms, K, w, r64, bnorms);
+  }
 }
 
 // The first residual of a solve from a zero guess: r = b exactly, so no operator is applied.  r goes
@@ -2356,83 +2317,59 @@ void MixedVCycle(DeviceSystem& ds, MixedSystem& ms, int K, hipStream_t s, bool z
 }
 
 // ------------------------------------------------------------------ flexible conjugate gradients
-// q = A p for per-column operators A_c = w[c][0] M + w[c][1] S (level 0; deep rows by raster line)
-__device__ __forceinline__ void K64ApplyDeepWRows(int vb, int c0, int D, const int* __restrict__ deepLine, const int* __restrict__ lines,
+// q = A_c p for columns [c0, c1) with per-column operators A_c = w[c][0] M + w[c][1] S: a thread keeps its
+// row's two stencils in registers and takes the columns one after another, the next one's values on
+// their way while one is added.  (3.0 M texels x 64 columns, deep rows: 1840 us with a workgroup per
+// three columns, whose threads load both stencils again for each; 1100 so (3.4 GB), against 1130 and 1200 with 32
+// and 16 columns a workgroup.  Whole launches, boundary rows included: 2220 us at
+// the first form, 1357 so; 0.75 M texels x 8 columns 91 and 58.)
+__device__ __forceinline__ void K64ApplyDeepWRows(int vb, int c0, int c1, int D, const int* __restrict__ deepLine, const int* __restrict__ lines,
                                                   const double* __restrict__ symM, const double* __restrict__ symS,
-                                                  const double* __restrict__ p, int N, double* q, int K, const double* __restrict__ w) {
+                                                  const double* __restrict__ p, int N, double* q, const double* __restrict__ w) {
   const int d = vb * blockDim.x + threadIdx.x;
   if (d >= D) return;
   int cur, prev, next;
   DeepRow(deepLine, lines, d, cur, prev, next);
-  double cm[9], cs[9];
+  double cm[9], cs[9], A[1][9], B[1][9];
   SymRow(symM, N, cur, next, cm);
   SymRow(symS, N, cur, next, cs);
-  WithChunkWidth<3>(min(3, K - c0), [&](auto kcc) {
-      constexpr int KC = decltype(kcc)::value;
-      double pv[KC][9];
-      RowValues<KC>(p, N, c0, prev, cur, next, pv);
+  auto put = [&](const double (&v)[9], int ch) {
+    double sm = 0.0, ss = 0.0;
 #pragma unroll
-      for (int cc = 0; cc < KC; cc++) {
-        const int ch = c0 + cc;
-        double sm = 0.0, ss = 0.0;
-#pragma unroll
-        for (int k = 0; k < 9; k++) sm += cm[k] * pv[cc][k], ss += cs[k] * pv[cc][k];
-        q[(long)ch * N + cur] = w[2 * ch] * sm + w[2 * ch + 1] * ss;
-      }
-    });
-}
-
-__device__ __forceinline__ void K64ApplyBoundaryWRows(int vb, int B, const int* __restrict__ bgi, const int* __restrict__ mrpd,
-                                                      const int* __restrict__ mcold, const double* __restrict__ mvald,
-                                                      const int* __restrict__ mrpb, const int* __restrict__ mcolb,
-                                                      const double* __restrict__ mvalb, const int* __restrict__ srpd,
-                                                      const int* __restrict__ scold, const double* __restrict__ svald,
-                                                      const int* __restrict__ srpb, const int* __restrict__ scolb,
-                                                      const double* __restrict__ svalb, const double* __restrict__ p, int N, double* q,
-                                                      int K, const double* __restrict__ w) {
-  const int r = (int)(((long)vb * blockDim.x + threadIdx.x) / kRowLanes64), lane = threadIdx.x % kRowLanes64;
-  if (r >= B) return;  // whole row groups leave together
-  for (int c0 = 0; c0 < K; c0 += 4) {
-    const int kc = min(4, K - c0);
-    double am[4] = {0.0, 0.0, 0.0, 0.0}, as[4] = {0.0, 0.0, 0.0, 0.0};
-    auto rows = [&](const int* rp, const int* cl, const double* vl, bool viaBoundary, double (&acc)[4]) {
-      for (int k = rp[r] + lane; k < rp[r + 1]; k += kRowLanes64) {
-        const double v = vl[k];
-        const int g = viaBoundary ? bgi[cl[k]] : cl[k];
-#pragma unroll
-        for (int qq = 0; qq < 4; qq++)
-          if (qq < kc) acc[qq] += v * p[(long)(c0 + qq) * N + g];
-      }
-    };
-    rows(mrpb, mcolb, mvalb, true, am);
-    rows(mrpd, mcold, mvald, false, am);
-    rows(srpb, scolb, svalb, true, as);
-    rows(srpd, scold, svald, false, as);
-#pragma unroll
-    for (int qq = 0; qq < 4; qq++) am[qq] = RowSum<double, kRowLanes64>(am[qq]), as[qq] = RowSum<double, kRowLanes64>(as[qq]);
-    if (lane < kc) {
-      const int ch = c0 + lane;
-      q[(long)ch * N + bgi[r]] = w[2 * ch] * Pick(am, lane) + w[2 * ch + 1] * Pick(as, lane);
-    }
+    for (int k = 0; k < 9; k++) sm += cm[k] * v[k], ss += cs[k] * v[k];
+    q[(long)ch * N + cur] = w[2 * ch] * sm + w[2 * ch + 1] * ss;
+  };
+  RowValues<1>(p, N, c0, prev, cur, next, A);
+  for (int c = c0; c < c1; c += 2) {
+    RowValues<1>(p, N, min(c + 1, c1 - 1), prev, cur, next, B);
+    put(A[0], c);
+    RowValues<1>(p, N, min(c + 2, c1 - 1), prev, cur, next, A);
+    if (c + 1 < c1) put(B[0], c + 1);
   }
 }
 
-// q = A p for per-column operators in one launch: deep rows, then boundary rows.
-__global__ __launch_bounds__(256) void K64ApplyW(int deepBlocks, int D, const int* __restrict__ deepLine, const int* __restrict__ lines,
-                                                 const double* __restrict__ symM, const double* __restrict__ symS, int B,
-                                                 const int* __restrict__ bgi, const int* __restrict__ mrpd, const int* __restrict__ mcold,
-                                                 const double* __restrict__ mvald, const int* __restrict__ mrpb, const int* __restrict__ mcolb,
-                                                 const double* __restrict__ mvalb, const int* __restrict__ srpd, const int* __restrict__ scold,
-                                                 const double* __restrict__ svald, const int* __restrict__ srpb, const int* __restrict__ scolb,
-                                                 const double* __restrict__ svalb, const double* __restrict__ p, int N, double* q, int K,
-                                                 const double* __restrict__ w) {
-  const int deep = deepBlocks * ((K + 2) / 3);
+// q = A p for per-column operators in one launch: deep rows (blocks deepBlocks x chunks of `wide` columns),
+// then boundary rows (chunks of four).
+__global__ __launch_bounds__(256) void K64ApplyW(int deepBlocks, int wide, int D, const int* __restrict__ deepLine,
+                                                 const int* __restrict__ lines, const double* __restrict__ symM,
+                                                 const double* __restrict__ symS, int B, const int* __restrict__ bgi, Rows64 rows,
+                                                 const double* __restrict__ p, int N, double* q, int K, const double* __restrict__ w) {
+  const int deep = deepBlocks * ((K + wide - 1) / wide);
   if ((int)blockIdx.x < deep) {
-    const TileChunk v = TileOf<3>(blockIdx.x, deepBlocks, K);
-    K64ApplyDeepWRows(v.tile, v.c0, D, deepLine, lines, symM, symS, p, N, q, K, w);
-  } else
-    K64ApplyBoundaryWRows(blockIdx.x - deep, B, bgi, mrpd, mcold, mvald, mrpb, mcolb, mvalb, srpd, scold, svald, srpb, scolb, svalb, p,
-                          N, q, K, w);
+    const TileChunk v = TileOf(wide, blockIdx.x, deepBlocks, K);
+    K64ApplyDeepWRows(v.tile, v.c0, min(v.c0 + wide, K), D, deepLine, lines, symM, symS, p, N, q, w);
+    return;
+  }
+  const TileChunk v = TileOf<4>(blockIdx.x - deep, RowBlocks64(B), K);
+  const int r = (int)(((long)v.tile * blockDim.x + threadIdx.x) / kRowLanes64), lane = threadIdx.x % kRowLanes64;
+  if (r >= B) return;  // whole row groups leave together
+  const int kc = min(4, K - v.c0), g = bgi[r];
+  double am[4], as[4];
+  RowSums64<true>(rows, r, lane, p + (long)v.c0 * N, N, kc, am, as);
+  if (lane < kc) {
+    const int ch = v.c0 + lane;
+    q[(long)ch * N + g] = w[2 * ch] * Pick(am, lane) + w[2 * ch + 1] * Pick(as, lane);
+  }
 }
 
 // A flexible-CG step's vector passes stream columns of N doubles and are bound by memory, so they read
@@ -2620,6 +2557,11 @@ static void HomeLevel0(MixedSystem& ms) {
   if (d.e2 && d.e != d.eHome) std::swap(d.e, d.e2);
 }
 
+static Rows64 PairRows(const DeviceSystem& ds) {
+  const DevCsr& M = ds.mass0.rows;
+  return {M.rowptr, ds.mass0.rowMid, M.col, M.val, ds.stiff0.rows.val};
+}
+
 // residual of the level-0 FP64 system into the FP32 correction rhs, squared norms into norms[0..K)
 // bnorms (first residual of a solve): |b|^2 per column into bnorms[ch][slot] as well.
 static void OuterResidual(DeviceSystem& ds, MixedSystem& ms, double* x, const double* b, int K, bool weighted, hipStream_t s,
@@ -2633,23 +2575,24 @@ static void OuterResidual(DeviceSystem& ds, MixedSystem& ms, double* x, const do
   }
   // deep rows: kDeepGroups x 256 per block; boundary rows: kRowLanes64 lanes each
   const int nt = 256, db = L0.nRaster > 0 ? (int)NBlk(L0.D, 256 * kDeepGroups) : 0;
-  const int bb = L0.B > 0 ? (int)NBlk((long)L0.B * kRowLanes64, nt) : 0;
+  const int bb = (int)RowBlocks64(L0.B);
   if (db + bb == 0) return;
   if (weighted) {
     const DevLevel &M = ds.mass0, &S = ds.stiff0;
-    K64ResidualW<<<ChunkBlocks<2>(db, K) + bb, nt, 0, s>>>(db, L0.D, ms.deepLine, L0.raster, M.coefSym, S.coefSym, L0.B, L0.bgi, M.bd.rowptr, M.bd.col,
-                                         M.bd.val, M.bb.rowptr, M.bb.col, M.bb.val, S.bd.rowptr, S.bd.col, S.bd.val, S.bb.rowptr, S.bb.col,
-                                         S.bb.val, x, b, L0.N, d.g2d, d.rhs, d.e, d.Nd, ms.norms, K, ms.weights, r64, bnorms);
+    K64ResidualW<<<ChunkBlocks<4>(db, K) + ChunkBlocks<4>(bb, K), nt, 0, s>>>(db, L0.D, ms.deepLine, L0.raster, M.coefSym, S.coefSym, L0.B, L0.bgi,
+                                                                             PairRows(ds), x, b, L0.N, d.g2d, d.rhs, d.e, d.Nd, ms.norms, K,
+                                                                             ms.weights, r64, bnorms);
     return;
   }
-  K64Residual<<<ChunkBlocks<3>(db, K) + bb, nt, 0, s>>>(db, L0.D, ms.deepLine, L0.raster, L0.coefSym, L0.B, L0.bgi, L0.bd.rowptr, L0.bd.col, L0.bd.val,
-                                      L0.bb.rowptr, L0.bb.col, L0.bb.val, x, b, L0.N, d.g2d, d.rhs, d.e, d.Nd, ms.norms, K, bnorms, ms.fresh);
+  K64Residual<<<ChunkBlocks<3>(db, K) + ChunkBlocks<4>(bb, K), nt, 0, s>>>(db, L0.D, ms.deepLine, L0.raster, L0.coefSym, L0.B, L0.bgi,
+                                                                          {L0.rows.rowptr, L0.rowMid, L0.rows.col, L0.rows.val, nullptr}, x, b,
+                                                                          L0.N, d.g2d, d.rhs, d.e, d.Nd, ms.norms, K, bnorms, ms.fresh);
 }
 
 // One flexible-CG step after the V-cycle left z = V(r) in the level-0 FP32 correction:
 // beta = (z, q_prev)/(p_prev, q_prev), p = z - beta p, q = A p, alpha = (r, p)/(p, q),
 // x += alpha p, r -= alpha q (all scalars stay on the device).
-static constexpr int kUpdateWideTexels = 1 << 21;
+static constexpr int kUpdateWideTexels = 1 << 21, kApplyBlocks = 2048;
 template <int KC>
 static void FcgStepChunks(DeviceSystem& ds, MixedSystem& ms, double* x, int K, hipStream_t s) {
   DevLevel& L0 = ds.L[0];
@@ -2664,11 +2607,12 @@ static void FcgStepChunks(DeviceSystem& ds, MixedSystem& ms, double* x, int K, h
   KFcgDirection<KC><<<texels, 256, 0, s>>>(N, d.g2d, d.e, d.Nd, ms.beta, ms.p64, K);
   const DevLevel &M = ds.mass0, &S = ds.stiff0;
   const int db = L0.nRaster > 0 ? (int)NBlk(L0.D, 256) : 0;
-  const int bb = L0.B > 0 ? (int)NBlk((long)L0.B * kRowLanes64, 256) : 0;
+  const int bb = (int)RowBlocks64(L0.B);
+  // as many columns per workgroup as leave kApplyBlocks workgroups (eight per CU)
+  const int wide = (int)std::clamp((long)db * K / kApplyBlocks, 1L, (long)K);
   if (db + bb > 0)
-    K64ApplyW<<<ChunkBlocks<3>(db, K) + bb, 256, 0, s>>>(db, L0.D, ms.deepLine, L0.raster, M.coefSym, S.coefSym, L0.B, L0.bgi, M.bd.rowptr, M.bd.col, M.bd.val,
-                                      M.bb.rowptr, M.bb.col, M.bb.val, S.bd.rowptr, S.bd.col, S.bd.val, S.bb.rowptr, S.bb.col, S.bb.val,
-                                      ms.p64, N, ms.q64, K, ms.weights);
+    K64ApplyW<<<db * ((K + wide - 1) / wide) + ChunkBlocks<4>(bb, K), 256, 0, s>>>(db, wide, L0.D, ms.deepLine, L0.raster, M.coefSym, S.coefSym, L0.B,
+                                                                                  L0.bgi, PairRows(ds), ms.p64, N, ms.q64, K, ms.weights);
   KFcgDots<KC><<<sums, 256, 0, s>>>(N, ms.r64, ms.p64, ms.q64, rp, pq, K);
   KFcgAlpha<<<K, kScalarThreads, 0, s>>>((int)gb, rp, pq, ms.alpha, ms.pqPrev, ms.first, ms.norms);
   HomeLevel0(ms);  // e was read above; the update zeroes the buffer the next step starts on
