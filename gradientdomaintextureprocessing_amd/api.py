@@ -330,6 +330,14 @@ class MultigridSystem:
         _lib.check(_lib.load().gdtp_residual_norms(self._h, px, pb, K, rel.ctypes.data, norms.ctypes.data, _stream()))
         return rel, norms[0::2].copy(), norms[1::2].copy()
 
+    def weighted_residual_norms(self, x, b, weights):
+        """(||b - (weights[c][0] M + weights[c][1] S) x||, ||b||) per column, FP64, level 0."""
+        (px, pb), K = self._pair(x, b, self._texels[0])
+        w = np.ascontiguousarray(np.asarray(weights, np.float64).reshape(K, 2))
+        norms = np.zeros(2 * K)
+        _lib.check(_lib.load().gdtp_weighted_residual_norms(self._h, px, pb, K, w.ctypes.data, norms.ctypes.data, _stream()))
+        return norms[0::2].copy(), norms[1::2].copy()
+
     def direct_solve(self, x, b):
         """Exact FP64 solve of A x = b on level 0 (the apps' --useDirectSolver path): LDL^T of the
         full matrix up to 2^20 texels, else FP64 V-cycles to the FP64 residual floor.  Returns
@@ -698,12 +706,9 @@ class LineIntegralConvolution:
         return x, self._weighted_residuals(x, b, lengths)
 
     def _weighted_residuals(self, x, b, lengths):
-        import torch
-        m, s = torch.empty_like(x), torch.empty_like(x)
-        self.lic.apply(OPERATOR_MASS, x, m)
-        self.lic.apply(OPERATOR_STIFFNESS, x, s)
-        lam = torch.tensor(np.asarray(lengths, np.float64), device=x.device)[:, None]
-        return ((b - m - lam * s).norm(dim=1) / b.norm(dim=1)).cpu().numpy()
+        r, bn = self.lic.weighted_residual_norms(x, b, [[1.0, float(l)] for l in lengths])
+        with np.errstate(divide="ignore", invalid="ignore"):  # a zero column: 0 / 0
+            return r / bn
 
     def convolve(self, noise, passes=4, tol=None, mode="fp64", max_iters=200, between_rounds=None):
         """(x, y): the anisotropically diffused noise and its sharpened version ([K, N] FP64).

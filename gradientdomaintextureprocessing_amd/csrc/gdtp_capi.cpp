@@ -488,11 +488,12 @@ static void FinishNorms(const double* sq, int K, double* relRes, double* norms) 
 
 // Squared residual / rhs norms of K level-0 columns into the host vector sq (2 K entries), through
 // the system's norm scratch (allocated on first use).
-static void SystemNorms(gdtp_system* s, const double* x, const double* b, int K, std::vector<double>& sq, hipStream_t st) {
+static void SystemNorms(gdtp_system* s, const double* x, const double* b, int K, std::vector<double>& sq, hipStream_t st,
+                        const double* weights = nullptr) {
   DeviceSystem& ds = *s->ds;
   if (!s->dNormParts) GDTP_HIP(hipMalloc(&s->dNormParts, (NormPartsSize(s->kcap) + 2 * (size_t)s->kcap) * sizeof(double)));
   double* out = s->dNormParts + NormPartsSize(s->kcap);
-  ResidualNorms(ds, x, b, K, ds.L[0].N, s->dNormParts, out, st);
+  ResidualNorms(ds, x, b, K, ds.L[0].N, s->dNormParts, out, st, weights);
   sq.assign(2 * (size_t)K, 0.0);
   GDTP_HIP(hipMemcpyAsync(sq.data(), out, sq.size() * sizeof(double), hipMemcpyDeviceToHost, st));
   GDTP_HIP(hipStreamSynchronize(st));
@@ -503,6 +504,15 @@ int gdtp_residual_norms(gdtp_system* s, const double* x, const double* b, int nc
     std::vector<double> sq;
     SystemNorms(s, x, b, ncols, sq, st);
     FinishNorms(sq.data(), ncols, rel_res, norms);
+  })
+}
+
+int gdtp_weighted_residual_norms(gdtp_system* s, const double* x, const double* b, int ncols, const double* weights, double* norms,
+                                 void* stream) {
+  GDTP_DEVICE_OP(x && b && weights && norms, {
+    std::vector<double> sq;
+    SystemNorms(s, x, b, ncols, sq, st, weights);
+    FinishNorms(sq.data(), ncols, nullptr, norms);
   })
 }
 

@@ -119,7 +119,9 @@ void ResidualLevel(DeviceSystem& ds, int level, const double* x, const double* b
 // doubles, every entry of which the call overwrites.
 constexpr int kNormParts = 512;
 constexpr size_t NormPartsSize(int K) { return (size_t)2 * K * kNormParts; }
-void ResidualNorms(DeviceSystem& ds, const double* x, const double* b, int K, int ld, double* parts, double* out, hipStream_t s);
+// weights: null, or two per column (host): column c's operator is weights[2c] M + weights[2c + 1] S.
+void ResidualNorms(DeviceSystem& ds, const double* x, const double* b, int K, int ld, double* parts, double* out, hipStream_t s,
+                   const double* weights = nullptr);
 // The same with the scratch in a static device array (no allocation): at most kNoAllocMaxCols
 // columns; the 2 K squared norms are copied to hostSquares and the stream is synchronised.
 constexpr int kNoAllocMaxCols = 64;

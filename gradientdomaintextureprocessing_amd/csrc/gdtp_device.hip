@@ -1167,13 +1167,21 @@ void ModulatedStiffness(const DevModulation& m, const double* mask, double* out,
 // kNormParts blocks strides over the raster lines (deep rows, raw stencil) and the boundary rows,
 // each block writes one partial per (column, quantity), and a second pass adds the partials of a
 // column in a fixed order, so repeated calls give bitwise identical norms.
+// kPair: column c's operator is w.m[c] M + w.s[c] S (coef, vl: M's; coefS, vlS: S's).  Memory bounds it:
+// both stencils (144 bytes a texel) once per four columns.  (3.3 M texels x 16 columns: 730 us; the two products
+// written, combined and summed in passes of their own 3.2 ms.)
 template <int KC>
+struct PairWeights {
+  double m[KC], s[KC];
+};
+template <int KC, bool kPair>
 __global__ __launch_bounds__(256) void KResidualNormParts(int nLines, const int* __restrict__ lines, const double* __restrict__ coef, int D,
                                                           int B, const int* __restrict__ bgi, const int* __restrict__ rp,
                                                           const int* __restrict__ mid, const int* __restrict__ cl,
                                                           const double* __restrict__ vl,
                                                           const double* __restrict__ x, const double* __restrict__ b, int ld, int c0,
-                                                          double* parts) {
+                                                          double* parts, const double* __restrict__ coefS, const double* __restrict__ vlS,
+                                                          PairWeights<KC> w) {
   double rr[KC], bn[KC];
 #pragma unroll
   for (int c = 0; c < KC; c++) rr[c] = 0.0, bn[c] = 0.0;
@@ -1181,12 +1189,26 @@ __global__ __launch_bounds__(256) void KResidualNormParts(int nLines, const int*
     const int* L = lines + 5 * l;
     const int start = L[0], len = L[1] - L[0] + 1, prev = L[2], next = L[3], d0 = L[4];
     for (int i = threadIdx.x; i < len; i += blockDim.x) {
-      double cf[9];
+      double cf[9], cs[9];
 #pragma unroll
       for (int k = 0; k < 9; k++) cf[k] = coef[(size_t)k * D + d0 + i];
+      if constexpr (kPair)
+#pragma unroll
+        for (int k = 0; k < 9; k++) cs[k] = coefS[(size_t)k * D + d0 + i];
 #pragma unroll
       for (int c = 0; c < KC; c++) {
         const double* X = x + (size_t)(c0 + c) * ld;
+        if constexpr (kPair) {
+          double sm = 0.0, ss = 0.0;
+#pragma unroll
+          for (int k = 0; k < 9; k++) {
+            const double v = X[(k < 3 ? prev : k < 6 ? start : next) + i + k % 3 - 1];
+            sm += v * cf[k], ss += v * cs[k];
+          }
+          const double t = b[(size_t)(c0 + c) * ld + start + i], r = t - w.m[c] * sm - w.s[c] * ss;
+          rr[c] += r * r, bn[c] += t * t;
+          continue;
+        }
         const double s = X[prev + i - 1] * cf[0] + X[prev + i] * cf[1] + X[prev + i + 1] * cf[2] + X[start + i - 1] * cf[3] +
                          X[start + i] * cf[4] + X[start + i + 1] * cf[5] + X[next + i - 1] * cf[6] + X[next + i] * cf[7] +
                          X[next + i + 1] * cf[8];
@@ -1200,7 +1222,15 @@ __global__ __launch_bounds__(256) void KResidualNormParts(int nLines, const int*
   const int lane = threadIdx.x % kRowLanes;
   for (int i = (int)((blockIdx.x * blockDim.x + threadIdx.x) / kRowLanes); i < B; i += (int)(gridDim.x * blockDim.x / kRowLanes)) {
     const double s = RowSum(rp[i], mid[i], rp[i + 1], cl, vl, x + (size_t)c0 * ld, ld, KC, terms);
-    const double bv = b[(size_t)(c0 + min(lane, KC - 1)) * ld + bgi[i]], r = bv - s;
+    const double bv = b[(size_t)(c0 + min(lane, KC - 1)) * ld + bgi[i]];
+    double r = bv - s;
+    if constexpr (kPair) {
+      const double t = RowSum(rp[i], mid[i], rp[i + 1], cl, vlS, x + (size_t)c0 * ld, ld, KC, terms);
+      double wm = w.m[0], ws = w.s[0];
+#pragma unroll
+      for (int c = 1; c < KC; c++) wm = lane == c ? w.m[c] : wm, ws = lane == c ? w.s[c] : ws;
+      r = bv - wm * s - ws * t;
+    }
 #pragma unroll
     for (int c = 0; c < KC; c++) rr[c] += lane == c ? r * r : 0.0, bn[c] += lane == c ? bv * bv : 0.0;
   }
@@ -1231,20 +1261,30 @@ __global__ __launch_bounds__(256) void KNormPartsSum(const double* __restrict__ 
   if (threadIdx.x == 0) out[q] = (w[0] + w[1]) + (w[2] + w[3]);
 }
 
-void ResidualNorms(DeviceSystem& ds, const double* x, const double* b, int K, int ld, double* parts, double* out, hipStream_t s) {
-  DevLevel& d = ds.L[0];
+// weights (host, 2 per column: M's and S's) or null for the system's operator
+template <int KC>
+static void NormParts(DeviceSystem& ds, const double* x, const double* b, int c0, int ld, double* parts, const double* weights, hipStream_t s) {
+  const DevLevel &d = ds.L[0], &M = ds.mass0, &S = ds.stiff0;
+  PairWeights<KC> w = {};
+  if (weights) {
+    for (int c = 0; c < KC; c++) w.m[c] = weights[2 * (c0 + c)], w.s[c] = weights[2 * (c0 + c) + 1];
+    KResidualNormParts<KC, true><<<kNormParts, 256, 0, s>>>(d.nRaster, d.raster, M.coefRaw, d.D, d.B, d.bgi, M.rows.rowptr, M.rowMid, M.rows.col,
+                                                            M.rows.val, x, b, ld, c0, parts, S.coefRaw, S.rows.val, w);
+  } else {
+    KResidualNormParts<KC, false><<<kNormParts, 256, 0, s>>>(d.nRaster, d.raster, d.coefRaw, d.D, d.B, d.bgi, d.rows.rowptr, d.rowMid, d.rows.col,
+                                                             d.rows.val, x, b, ld, c0, parts, nullptr, nullptr, w);
+  }
+}
+
+void ResidualNorms(DeviceSystem& ds, const double* x, const double* b, int K, int ld, double* parts, double* out, hipStream_t s,
+                   const double* weights) {
   for (int c0 = 0; c0 < K; c0 += 4) {
-    const int kc = std::min(4, K - c0);
-#define GDTP_NORM_PARTS(KC)                                                                                                         \
-  KResidualNormParts<KC><<<kNormParts, 256, 0, s>>>(d.nRaster, d.raster, d.coefRaw, d.D, d.B, d.bgi, d.rows.rowptr, d.rowMid, d.rows.col, \
-                                                    d.rows.val, x, b, ld, c0, parts)
-    switch (kc) {
-      case 4: GDTP_NORM_PARTS(4); break;
-      case 3: GDTP_NORM_PARTS(3); break;
-      case 2: GDTP_NORM_PARTS(2); break;
-      default: GDTP_NORM_PARTS(1); break;
+    switch (std::min(4, K - c0)) {
+      case 4: NormParts<4>(ds, x, b, c0, ld, parts, weights, s); break;
+      case 3: NormParts<3>(ds, x, b, c0, ld, parts, weights, s); break;
+      case 2: NormParts<2>(ds, x, b, c0, ld, parts, weights, s); break;
+      default: NormParts<1>(ds, x, b, c0, ld, parts, weights, s); break;
     }
-#undef GDTP_NORM_PARTS
   }
   KNormPartsSum<<<2 * K, 256, 0, s>>>(parts, kNormParts, out);
 }

@@ -123,6 +123,11 @@ int gdtp_residual(gdtp_system* s, const double* x, const double* b, double* r, i
  * ComputeSystemResdiual followed by the apps' residual-norm printout (IterativeSolvers.inl:953-1007,
  * TextureFiltering.cpp:540-558). */
 int gdtp_residual_norms(gdtp_system* s, const double* x, const double* b, int ncols, double* rel_res, double* norms, void* stream);
+/* norms[2c] = ||b_c - (weights[2c] M + weights[2c + 1] S) x_c|| and norms[2c + 1] = ||b_c|| (host arrays of
+ * 2 ncols; x, b device): the norms of gdtp_residual_norms for the per-column operators of
+ * gdtp_solve_weighted. */
+int gdtp_weighted_residual_norms(gdtp_system* s, const double* x, const double* b, int ncols, const double* weights, double* norms,
+                                 void* stream);
 /* Exact FP64 solve of A x = b on level 0: the apps' --useDirectSolver path (FullMatrixConstruction
  * and solve(directSolver, ...), UpdateCoefficients.inl:137-219, TextureFiltering.cpp:509-558,
  * Geodesics.cpp:259-301).  Up to 2^20 texels: LDL^T of the full level-0 matrix (nested dissection,
