@@ -713,64 +713,119 @@ __global__ __launch_bounds__(NT) void KMixDeepGsFused(int chunks, const int* __r
 #undef GDTP_FUSED_FETCH
 #undef GDTP_FUSED_APPLY
 
-// res = rhs - A e at deep texels (raw A: the symmetric five-word stencil, a4 the diagonal).  A
-// workgroup covers its tile in all four colour planes, so the planes' shared neighbourhoods of e are
-// fetched once rather than once per plane; its deep texels come from the tile's bit masks (one
-// uniform load per wave and plane), so a texel's stencil, neighbour and rhs loads go out together.
-// (Measured and not kept: a thread owning the 2x2 block of texels of one sub-grid position, its 4x4
-// window of e and all four stencils loaded before any is used: one memory round trip per thread,
-// but 138 registers and 232 instead of 221 us at C2; the tile's window of e in all four planes
-// staged in LDS by row-contiguous loads, seven instead of 36 loads per column per thread: 220 us,
-// as the HBM bytes, not the load count, bound the launch.)
-// kChunk: columns whose loads are in flight together (2 on large levels: 50 instead of 79
-// registers, eight waves per SIMD instead of six, level 0 at C2 219 against 221 us; 4 on small
-// levels, which are latency-bound and pay for a second round trip).
-// kSplit: the workgroup's tile in one plane only (vb = 4 tile + plane; small levels: four times the
-// workgroups, and one round trip instead of one per plane: 5.7 us a launch to 4.4 on a 512^2 cube).
-template <int kChunk, bool kSplit>
-__device__ __forceinline__ void ResidualDeepTile(int vb, int c0, const MixTile* __restrict__ tiles,
-                                                 const unsigned long long* __restrict__ deepMask, long plane, long Nd,
-                                                 const float* __restrict__ sym, const float* __restrict__ e, const float* __restrict__ rhs,
-                                                 float* res, int K, int zeroQ) {
-  const int plane0 = kSplit ? vb % 4 : 0, plane1 = kSplit ? plane0 + 1 : 4;
-  if constexpr (kSplit) vb /= 4;
-  const int row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
-  const unsigned long long* mk = deepMask + (long)vb * 4 * kTB + row;
-  const MixTile& T = tiles[vb];
+// res = rhs - A e at deep texels (raw A: the symmetric five-word stencil, slot 4 the diagonal; upper
+// coupling k from slot 8-k of that neighbour).  Deep texels come from the tile's bit masks (one uniform load
+// per wave and plane), so a texel's stencil, neighbour and rhs loads go out together.  The texels of
+// plane zeroQ were relaxed last by the FP32 smoother: their rows hold exactly, so the residual is zero.
+//
+// Small levels: vb = 4 tile + plane, one texel and up to four columns per thread, every load in flight
+// (latency bounds it; four planes one after another in a workgroup 5.7 us on a 512^2 cube, 4.4 so).
+__device__ __forceinline__ void ResidualDeepPlane(int vb, int c0, const MixTile* __restrict__ tiles,
+                                                  const unsigned long long* __restrict__ deepMask, long plane, long Nd,
+                                                  const float* __restrict__ sym, const float* __restrict__ e, const float* __restrict__ rhs,
+                                                  float* res, int K, int zeroQ) {
+  const int q = vb % 4, row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
+  if (!((deepMask[(long)vb * kTB + row] >> tx) & 1ull)) return;
+  const MixTile& T = tiles[vb / 4];
   const MixGrid c = T.own;
-  const int a = T.a0 + tx, b = T.b0 + row;
-  for (int q = plane0; q < plane1; q++) {
-    if (!((mk[q * kTB] >> tx) & 1ull)) continue;
-    const int i = 2 * a + (q & 1), j = 2 * b + (q >> 1);
-    const long idx = (long)q * plane + c.base2 + (long)b * c.w2 + a;
-    if (q == zeroQ) {  // relaxed last by the FP32 smoother: its deep rows hold exactly, so the residual is zero
-      for (int ch = c0; ch < min(K, c0 + kChunk); ch++) res[(long)ch * Nd + idx] = 0.0f;
-      continue;
+  const int a = T.a0 + tx, b = T.b0 + row, i = 2 * a + (q & 1), j = 2 * b + (q >> 1);
+  const long idx = (long)q * plane + c.base2 + (long)b * c.w2 + a;
+  if (q == zeroQ) {
+    for (int ch = c0; ch < min(K, c0 + 4); ch++) res[(long)ch * Nd + idx] = 0.0f;
+    return;
+  }
+  int nb[9];
+#pragma unroll
+  for (int k = 0; k < 9; k++) nb[k] = DenseByte(c, plane, i + k % 3 - 1, j + k / 3 - 1);
+  const float cf[9] = {sym[idx], sym[Nd + idx], sym[2 * Nd + idx], sym[3 * Nd + idx], sym[4 * Nd + idx],
+                       Ld(sym + 3 * Nd, nb[5]), Ld(sym + 2 * Nd, nb[6]), Ld(sym + Nd, nb[7]), Ld(sym, nb[8])};
+  ForChunk<4>(K, c0, [&](auto kc) {
+    constexpr int KC = decltype(kc)::value;
+    float v[KC][9], r[KC];
+#pragma unroll
+    for (int ch = 0; ch < KC; ch++) {
+#pragma unroll
+      for (int k = 0; k < 9; k++) v[ch][k] = Ld(e + (c0 + ch) * Nd, nb[k]);
+      r[ch] = Ld(rhs + (c0 + ch) * Nd, nb[4]);
     }
-    const float a4 = sym[4 * Nd + idx];
-    int nb[9];
 #pragma unroll
-    for (int k = 0; k < 9; k++) nb[k] = DenseByte(c, plane, i + k % 3 - 1, j + k / 3 - 1);
-    // own lower couplings and a4; upper coupling k from slot 8-k of that neighbour
-    const float cf[9] = {sym[idx], sym[Nd + idx], sym[2 * Nd + idx], sym[3 * Nd + idx], a4,
-                         Ld(sym + 3 * Nd, nb[5]), Ld(sym + 2 * Nd, nb[6]), Ld(sym + Nd, nb[7]), Ld(sym, nb[8])};
-    ForChunk<kChunk>(K, c0, [&](auto kc) {
-      constexpr int KC = decltype(kc)::value;
-      float v[KC][9], r[KC];
+    for (int ch = 0; ch < KC; ch++) {
+      float s = 0.0f;
 #pragma unroll
-      for (int ch = 0; ch < KC; ch++) {
+      for (int k = 0; k < 9; k++) s += cf[k] * v[ch][k];
+      res[(long)(c0 + ch) * Nd + idx] = r[ch] - s;
+    }
+  });
+}
+
+// Large levels: a thread owns the 2 x 2 texels of one sub-grid position, one per plane; their four
+// stencils stay in registers over the workgroup's columns [c0, c1), a column's 4 x 4 window of e is
+// loaded once for all four, and the next column's is on its way while one is added.  What bounds a launch
+// is the L2's rate to the CUs (8 to 9 TB/s): a workgroup that went plane by plane read the window once a plane and
+// the stencils once per two columns, four to seven times what the level holds.
+// (12.1 M texels x 3 columns: 263 to 203 us a launch, the boundary rows' part included; 3.0 M x 3: 69 to 58; 3.0 M x 64: 1320 to
+// 1165.)
+__device__ __forceinline__ void ResidualDeepBlock(int tile, int c0, int c1, const MixTile* __restrict__ tiles,
+                                                  const unsigned long long* __restrict__ deepMask, long plane, long Nd,
+                                                  const float* __restrict__ sym, const float* __restrict__ e, const float* __restrict__ rhs,
+                                                  float* res, int zeroQ) {
+  const int row = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTA), tx = threadIdx.x % kTA;
+  const unsigned long long* mk = deepMask + (long)tile * 4 * kTB + row;
+  bool deep[4];
 #pragma unroll
-        for (int k = 0; k < 9; k++) v[ch][k] = Ld(e + (c0 + ch) * Nd, nb[k]);
-        r[ch] = Ld(rhs + (c0 + ch) * Nd, nb[4]);
-      }
+  for (int q = 0; q < 4; q++) deep[q] = (mk[q * kTB] >> tx) & 1ull;
+  if (!(deep[0] || deep[1] || deep[2] || deep[3])) return;
+  const MixTile& T = tiles[tile];
+  const MixGrid c = T.own;
+  const int at = 4 * (c.base2 + (T.b0 + row) * c.w2 + T.a0 + tx), step = 4 * (int)plane;  // bytes
+  const int any = at + (deep[0] ? 0 : deep[1] ? step : deep[2] ? 2 * step : 3 * step);
+  // window position (u, v) = texel (2a + u - 1, 2b + v - 1); those that no deep texel of the four reaches read `any`
+  int off[16];
 #pragma unroll
-      for (int ch = 0; ch < KC; ch++) {
-        float s = 0.0f;
+  for (int w = 0; w < 16; w++) {
+    const int u = w % 4 - 1, v = w / 4 - 1;
+    bool need = false;
 #pragma unroll
-        for (int k = 0; k < 9; k++) s += cf[k] * v[ch][k];
-        res[(long)(c0 + ch) * Nd + idx] = r[ch] - s;
-      }
-    });
+    for (int q = 0; q < 4; q++) {
+      const int du = u - (q & 1), dv = v - (q >> 1);
+      if (du >= -1 && du <= 1 && dv >= -1 && dv <= 1) need = need || deep[q];
+    }
+    const int o = at + ((u & 1) | ((v & 1) << 1)) * step + 4 * ((v == -1 ? -1 : v == 2 ? 1 : 0) * c.w2 + (u == -1 ? -1 : u == 2 ? 1 : 0));
+    off[w] = need ? o : any;
+  }
+  float cf[4][9];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const int w = 5 + (q & 1) + 4 * (q >> 1);
+#pragma unroll
+    for (int k = 0; k < 9; k++)
+      cf[q][k] = k < 5 ? Ld(sym + k * Nd, off[w]) : Ld(sym + (8 - k) * Nd, off[w + (k / 3 - 1) * 4 + k % 3 - 1]);
+  }
+  auto load = [&](float (&v)[16], float (&r)[4], int ch) {
+    const float *E = e + (long)ch * Nd, *R = rhs + (long)ch * Nd;
+#pragma unroll
+    for (int w = 0; w < 16; w++) v[w] = Ld(E, off[w]);
+#pragma unroll
+    for (int q = 0; q < 4; q++) r[q] = Ld(R, off[5 + (q & 1) + 4 * (q >> 1)]);
+  };
+  auto put = [&](const float (&v)[16], const float (&r)[4], int ch) {
+    float* O = res + (long)ch * Nd;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const int w = 5 + (q & 1) + 4 * (q >> 1);
+      float s = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 9; k++) s += cf[q][k] * v[w + (k / 3 - 1) * 4 + k % 3 - 1];
+      if (deep[q]) O[(at + q * step) / 4] = q == zeroQ ? 0.0f : r[q] - s;
+    }
+  };
+  float A[16], Ar[4], B[16], Br[4];
+  load(A, Ar, c0);
+  for (int ch = c0; ch < c1; ch += 2) {
+    load(B, Br, min(ch + 1, c1 - 1));
+    put(A, Ar, ch);
+    load(A, Ar, min(ch + 2, c1 - 1));
+    if (ch + 1 < c1) put(B, Br, ch + 1);
   }
 }
 
@@ -843,20 +898,22 @@ __global__ __launch_bounds__(256) void KMixBoundaryResidual(int B, const int* __
   BoundaryResidualRows(v.tile, v.c0, B, bdIdx, rp, ent, dg, e, rhs, out, compact, Nd, K);
 }
 
-static constexpr int kResidualWideTiles = 1024;  // levels with more 64 x 4 tiles load two columns at a time
-// The residual of a level after pre-smoothing in one launch: the first blocks take the deep tiles,
-// the others the boundary rows (disjoint outputs, so the two parts overlap on the device).
-template <int kChunk, bool kSplit>
+static constexpr int kResidualWideTiles = 1024;  // levels with more 64 x 4 tiles: a thread per 2 x 2 texels
+static constexpr int kColumnBlocks = 2048;       // workgroups (eight per CU) that columns are spread over before a workgroup takes several
+// The residual of a level after pre-smoothing in one launch: the first blocks take the deep tiles (`wide`
+// columns each on large levels), the others the boundary rows (disjoint outputs, so the two parts overlap
+// on the device).
+template <bool kSplit>
 __global__ __launch_bounds__(256) void KMixResidual(int nTiles, const MixTile* __restrict__ tiles,
-                                                    const unsigned long long* __restrict__ deepMask, long plane,
-                                                    long Nd, const float* __restrict__ sym, const float* __restrict__ e,
-                                                    const float* __restrict__ rhs, float* res, int K, int zeroQ, int B,
-                                                    const int* __restrict__ bdIdx, const int* __restrict__ rp, const int2* __restrict__ ent,
-                                                    const float* __restrict__ dg) {
-  const int parts = kSplit ? 4 * nTiles : nTiles, deepBlocks = parts * ((K + kChunk - 1) / kChunk);
+                                                    const unsigned long long* __restrict__ deepMask, long plane, long Nd,
+                                                    const float* __restrict__ sym, const float* __restrict__ e, const float* __restrict__ rhs,
+                                                    float* res, int K, int wide, int zeroQ, int B, const int* __restrict__ bdIdx,
+                                                    const int* __restrict__ rp, const int2* __restrict__ ent, const float* __restrict__ dg) {
+  const int parts = kSplit ? 4 * nTiles : nTiles, deepBlocks = parts * ((K + wide - 1) / wide);
   if ((int)blockIdx.x < deepBlocks) {
-    const TileChunk v = TileOf<kChunk>(blockIdx.x, parts, K);
-    ResidualDeepTile<kChunk, kSplit>(v.tile, v.c0, tiles, deepMask, plane, Nd, sym, e, rhs, res, K, zeroQ);
+    const TileChunk v = TileOf(wide, blockIdx.x, parts, K);
+    if constexpr (kSplit) ResidualDeepPlane(v.tile, v.c0, tiles, deepMask, plane, Nd, sym, e, rhs, res, K, zeroQ);
+    else ResidualDeepBlock(v.tile, v.c0, min(v.c0 + wide, K), tiles, deepMask, plane, Nd, sym, e, rhs, res, zeroQ);
   } else {
     const TileChunk v = TileOf<4>(blockIdx.x - deepBlocks, NBlk((long)B * kRowLanes, 256), K);
     BoundaryResidualRows(v.tile, v.c0, B, bdIdx, rp, ent, dg, e, rhs, res, 0, Nd, K);
@@ -2282,10 +2339,11 @@ void MixedVCycle(DeviceSystem& ds, MixedSystem& ms, int K, hipStream_t s, bool z
     Smooth(ms, l, K, false, s, l > 0 || zeroE0);
     const long rb = ChunkBlocks<4>(NBlk((long)d.B * kRowLanes, 256), K), cb = ChunkBlocks<4>(NBlk((long)c.B * kRowLanes, 256), K);
     const bool wide = d.nTiles > kResidualWideTiles, wideC = c.nTiles > kResidualWideTiles;
-    const long db = wide ? ChunkBlocks<2>(d.nTiles, K) : ChunkBlocks<4>(4 * d.nTiles, K), cd = ChunkBlocks<4>(wideC ? c.nTiles : 4 * c.nTiles, K);
+    const int cols = wide ? (int)std::clamp((long)d.nTiles * K / kColumnBlocks, 1L, (long)K) : 4;
+    const long db = (wide ? d.nTiles : 4L * d.nTiles) * ((K + cols - 1) / cols), cd = ChunkBlocks<4>(wideC ? c.nTiles : 4 * c.nTiles, K);
     if (db + rb > 0)
-      (wide ? KMixResidual<2, false> : KMixResidual<4, true>)<<<db + rb, 256, 0, s>>>(
-          d.nTiles, d.tileRecs, d.deepMask, d.plane, d.Nd, d.stencilSym, d.e, d.rhs, d.res, K, ms.nuPre > 0 && !d.stencilH ? 3 : -1, d.B, d.bdIdx,
+      (wide ? KMixResidual<false> : KMixResidual<true>)<<<db + rb, 256, 0, s>>>(
+          d.nTiles, d.tileRecs, d.deepMask, d.plane, d.Nd, d.stencilSym, d.e, d.rhs, d.res, K, cols, ms.nuPre > 0 && !d.stencilH ? 3 : -1, d.B, d.bdIdx,
           d.bRowptr, d.bEnt, d.bDiag);
     if (cd + cb > 0)
       (wideC ? KMixRestrict<false> : KMixRestrict<true>)<<<cd + cb, 256, 0, s>>>(c.nTiles, c.tileRecs, c.deepMask, c.plane, c.Nd, d.plane, d.Nd,
@@ -2592,7 +2650,7 @@ static void OuterResidual(DeviceSystem& ds, MixedSystem& ms, double* x, const do
 // One flexible-CG step after the V-cycle left z = V(r) in the level-0 FP32 correction:
 // beta = (z, q_prev)/(p_prev, q_prev), p = z - beta p, q = A p, alpha = (r, p)/(p, q),
 // x += alpha p, r -= alpha q (all scalars stay on the device).
-static constexpr int kUpdateWideTexels = 1 << 21, kApplyBlocks = 2048;
+static constexpr int kUpdateWideTexels = 1 << 21;
 template <int KC>
 static void FcgStepChunks(DeviceSystem& ds, MixedSystem& ms, double* x, int K, hipStream_t s) {
   DevLevel& L0 = ds.L[0];
@@ -2608,8 +2666,8 @@ static void FcgStepChunks(DeviceSystem& ds, MixedSystem& ms, double* x, int K, h
   const DevLevel &M = ds.mass0, &S = ds.stiff0;
   const int db = L0.nRaster > 0 ? (int)NBlk(L0.D, 256) : 0;
   const int bb = (int)RowBlocks64(L0.B);
-  // as many columns per workgroup as leave kApplyBlocks workgroups (eight per CU)
-  const int wide = (int)std::clamp((long)db * K / kApplyBlocks, 1L, (long)K);
+  // as many columns per workgroup as leave kColumnBlocks workgroups (eight per CU)
+  const int wide = (int)std::clamp((long)db * K / kColumnBlocks, 1L, (long)K);
   if (db + bb > 0)
     K64ApplyW<<<db * ((K + wide - 1) / wide) + ChunkBlocks<4>(bb, K), 256, 0, s>>>(db, wide, L0.D, ms.deepLine, L0.raster, M.coefSym, S.coefSym, L0.B,
                                                                                   L0.bgi, PairRows(ds), ms.p64, N, ms.q64, K, ms.weights);
