@@ -596,15 +596,23 @@ DeviceSystem::~DeviceSystem() {
 // ------------------------------------------------------------------ normalised-gradient integration
 // One thread per cell sample: the bilinear gradient at the sample from its 4 corners, normalised in
 // the metric, dotted with the 4 integrated basis gradients and added to the corners' rhs.
-__global__ void KVfCell(long n, const int* __restrict__ corners, const float* __restrict__ data, double invW, double invH,
-                        const double* __restrict__ u, int ldu, double* rhs, int ldr, int K) {
-  const long s = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
+// Atomic adds bound it: a triangle's samples run along its rows of cells, so the next lane's left corners
+// are mostly this lane's right ones, and the lane takes their terms along (DPP) before adding.
+// (4.4 M samples x 64 columns: 14.8 ms with four adds per sample, 11.6 so; sorted by texel 23.6.)
+__global__ __launch_bounds__(256) void KVfCell(long n, const int* __restrict__ corners, const float* __restrict__ data, double invW, double invH,
+                                               const double* __restrict__ u, int ldu, double* rhs, int ldr, int K) {
+  const long at = (long)blockIdx.x * blockDim.x + threadIdx.x, s = min(at, n - 1);
+  const bool active = at < n;  // every lane takes part in the moves
   int cn[4];
   for (int k = 0; k < 4; k++) cn[k] = corners[4 * s + k];
   const double x = data[s], y = data[n + s], t00 = data[2 * n + s], t01 = data[3 * n + s], t11 = data[4 * n + s];
   double vx[4], vy[4];
   for (int k = 0; k < 4; k++) vx[k] = data[(5 + 2 * k) * n + s], vy[k] = data[(6 + 2 * k) * n + s];
+  // corners 1 and 2 (right) against the next lane's 0 and 3 (left); -1 where there is none
+  const int next0 = __builtin_amdgcn_update_dpp(-1, active ? cn[0] : -1, 0x130, 0xf, 0xf, false);  // wave_shl:1
+  const int next3 = __builtin_amdgcn_update_dpp(-1, active ? cn[3] : -1, 0x130, 0xf, 0xf, false);
+  const int take1 = active && next0 == cn[1], take2 = active && next3 == cn[2];
+  const int give0 = __builtin_amdgcn_update_dpp(0, take1, 0x138, 0xf, 0xf, false), give3 = __builtin_amdgcn_update_dpp(0, take2, 0x138, 0xf, 0xf, false);
   for (int ch = 0; ch < K; ch++) {
     const double* U = u + (long)ch * ldu;
     const double c0 = U[cn[0]], c1 = U[cn[1]], c2 = U[cn[2]], c3 = U[cn[3]];
@@ -613,10 +621,18 @@ __global__ void KVfCell(long n, const int* __restrict__ corners, const float* __
     const double ny = -((1 - x) * (c3 - c0) + x * (c2 - c1)) * invH;
     const double ax = t00 * nx + t01 * ny, ay = t01 * nx + t11 * ny;
     const double len2 = nx * ax + ny * ay;
-    if (!(len2 > 0)) continue;
-    const double il = 1.0 / sqrt(len2);
+    const bool any = active && len2 > 0;
+    const double il = any ? 1.0 / sqrt(len2) : 0.0;
+    double v[4];
+    for (int k = 0; k < 4; k++) v[k] = any ? (ax * vx[k] + ay * vy[k]) * il : 0.0;
+    const double n0 = DppMove<0x130, 0xf, true>(v[0], 0.0), n3 = DppMove<0x130, 0xf, true>(v[3], 0.0);
+    if (take1) v[1] += n0;
+    if (take2) v[2] += n3;
     double* R = rhs + (long)ch * ldr;
-    for (int k = 0; k < 4; k++) atomicAdd(&R[cn[k]], (ax * vx[k] + ay * vy[k]) * il);
+    if (v[1] != 0.0) atomicAdd(&R[cn[1]], v[1]);
+    if (v[2] != 0.0) atomicAdd(&R[cn[2]], v[2]);
+    if (!give0 && v[0] != 0.0) atomicAdd(&R[cn[0]], v[0]);
+    if (!give3 && v[3] != 0.0) atomicAdd(&R[cn[3]], v[3]);
   }
 }
 
