@@ -33,6 +33,7 @@ struct DevLdlt {
   double *fwdVal = nullptr, *bwdVal = nullptr;
   long *fwdMatPtr = nullptr, *bwdMatPtr = nullptr;
   double *fwdMat = nullptr, *bwdMat = nullptr;
+  float *fwdLow = nullptr, *bwdLow = nullptr;
   LdltWideRow* wideRows = nullptr;  // of each row of the wide stages (row - wideBegin)
   double* wideBuf = nullptr;   // [2][kcap][n - wideBegin]: right-hand sides of the wide products
   // boundary factors: the texel of each row, and A_BD's rows in the factor's numbering

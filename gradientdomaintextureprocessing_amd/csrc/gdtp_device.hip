@@ -225,15 +225,46 @@ __device__ __forceinline__ double GroupSum(double v) {
   for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, G);
   return v;
 }
+// A sum in two doubles, v and what its additions rounded away, e (compensated summation: T. Ogita,
+// S. M. Rump and S. Oishi, "Accurate sum and dot product", SIAM J. Sci. Comput. 26, 2005).
+struct Sum2 {
+  double v, e;
+  // (the error terms are differences of rounded values: nothing here may be contracted)
+  __device__ __forceinline__ void Add(double b) {
+#pragma clang fp contract(off)
+    const double t = v + b, z = t - v;
+    e += (v - (t - z)) + (b - z);
+    v = t;
+  }
+  __device__ __forceinline__ void Add(const Sum2& s) {
+    Add(s.v);
+    e += s.e;
+  }
+  // + (high + low) x, the product's own rounding kept too.  (Add with the unrounded product in one fused
+  // step, three operations fewer, is not exact where the product exceeds the sum: residual 3 times larger.)
+  __device__ __forceinline__ void AddProduct(double high, float low, double x) {
+#pragma clang fp contract(off)
+    const double p = high * x;
+    e += __builtin_fma(high, x, -p);
+    e = __builtin_fma((double)low, x, e);
+    Add(p);
+  }
+  __device__ __forceinline__ double Value() const { return v + e; }
+};
+// A DPP move of a sum (zero where no source).
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ Sum2 DppMove(const Sum2& s) {
+  return {DppMove<kCtrl, kRowMask, kRowMask == 0xf>(s.v, 0.0), DppMove<kCtrl, kRowMask, kRowMask == 0xf>(s.e, 0.0)};
+}
 // The wave's sum in lane 63, by DPP moves.
-__device__ __forceinline__ double WaveSumLast(double v) {
-  v += DppMove<0x111, 0xf, true>(v, 0.0);
-  v += DppMove<0x112, 0xf, true>(v, 0.0);
-  v += DppMove<0x114, 0xf, true>(v, 0.0);
-  v += DppMove<0x118, 0xf, true>(v, 0.0);
-  v += DppMove<0x142, 0xa>(v, 0.0);
-  v += DppMove<0x143, 0xc>(v, 0.0);
-  return v;
+__device__ __forceinline__ double WaveSumLast(Sum2 s) {
+  s.Add(DppMove<0x111, 0xf>(s));
+  s.Add(DppMove<0x112, 0xf>(s));
+  s.Add(DppMove<0x114, 0xf>(s));
+  s.Add(DppMove<0x118, 0xf>(s));
+  s.Add(DppMove<0x142, 0xa>(s));
+  s.Add(DppMove<0x143, 0xc>(s));
+  return s.Value();
 }
 
 // The tables of one direction and the vectors of a solve.
@@ -241,6 +272,7 @@ struct LdltPass {
   const int* compPtr;
   const long* matPtr;
   const double* mat;
+  const float* low;
   const int *ptr, *col;  // couplings with the stages solved before
   const double* val;
   const int* index;      // of each row in the right-hand side (forward) or the solution (backward)
@@ -295,7 +327,7 @@ template <bool kForward, bool kRhs, int G, int KC>
 __global__ __launch_bounds__(1024) void KLdltNarrow(int comp0, LdltPass P, const double* src, int lds, double* y, int n, double* dst, int ldd,
                                                     int K) {
   __shared__ double R[KC][kLdltNarrowRows];
-  __shared__ double Q[16][KC][kLdltBlock];
+  __shared__ Sum2 Q[16][KC][kLdltBlock];
   const int comp = comp0 + blockIdx.x, w0 = P.compPtr[comp], m = P.compPtr[comp + 1] - w0;
   const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
   y += (size_t)c0 * n;
@@ -310,9 +342,14 @@ __global__ __launch_bounds__(1024) void KLdltNarrow(int comp0, LdltPass P, const
   const long off = P.matPtr[comp] + (kForward ? (long)kLdltBlock * kLdltBlock * (rb * (rb + 1) / 2)
                                               : (long)kLdltBlock * rb * m - (long)kLdltBlock * kLdltBlock * (rb * (rb - 1) / 2));
   const double* M = P.mat + off + min(lane, nr - 1);
+  const float* Ml = P.low + off + min(lane, nr - 1);
   double early[kEarlyColumns];
+  float earlyLow[kEarlyColumns];
 #pragma unroll
-  for (int q = 0; q < kEarlyColumns; q++) early[q] = M[(size_t)min(part + q * parts, cols - 1) * nr];
+  for (int q = 0; q < kEarlyColumns; q++) {
+    const size_t o = (size_t)min(part + q * parts, cols - 1) * nr;
+    early[q] = M[o], earlyLow[q] = Ml[o];
+  }
   const int outRow = min((int)threadIdx.x, m * KC - 1) % m;
   const int out = kForward ? 0 : P.index[w0 + outRow];
   for (int i = threadIdx.x / G; i < m; i += 1024 / G) {
@@ -321,19 +358,20 @@ __global__ __launch_bounds__(1024) void KLdltNarrow(int comp0, LdltPass P, const
     if (gl < KC) R[gl][i] = v;
   }
   __syncthreads();
-  double acc[KC] = {};
+  Sum2 acc[KC] = {};
 #pragma unroll
   for (int q = 0; q < kEarlyColumns; q++) {
     const int j = part + q * parts;
     if (j >= cols) break;
 #pragma unroll
-    for (int c = 0; c < KC; c++) acc[c] += early[q] * R[c][j0 + j];
+    for (int c = 0; c < KC; c++) acc[c].AddProduct(early[q], earlyLow[q], R[c][j0 + j]);
   }
-#pragma unroll 8
+#pragma unroll 4
   for (int j = part + kEarlyColumns * parts; j < cols; j += parts) {
     const double a = M[(size_t)j * nr];
+    const float al = Ml[(size_t)j * nr];
 #pragma unroll
-    for (int c = 0; c < KC; c++) acc[c] += a * R[c][j0 + j];
+    for (int c = 0; c < KC; c++) acc[c].AddProduct(a, al, R[c][j0 + j]);
   }
 #pragma unroll
   for (int c = 0; c < KC; c++) Q[wave][c][lane] = acc[c];
@@ -341,8 +379,9 @@ __global__ __launch_bounds__(1024) void KLdltNarrow(int comp0, LdltPass P, const
   static_assert(kLdltNarrowRows * 4 <= 1024, "one result per thread");
   if ((int)threadIdx.x < m * kc) {
     const int c = threadIdx.x / m, i = outRow, b = i / kLdltBlock, kk = kForward ? b : blocks - 1 - b;
-    double s = 0.0;
-    for (int q = kWaveSplit[blocks - 1][kk]; q < kWaveSplit[blocks - 1][kk + 1]; q++) s += Q[q][c][i % kLdltBlock];
+    Sum2 sum = {};
+    for (int q = kWaveSplit[blocks - 1][kk]; q < kWaveSplit[blocks - 1][kk + 1]; q++) sum.Add(Q[q][c][i % kLdltBlock]);
+    const double s = sum.Value();
     y[(size_t)c * n + w0 + i] = s;
     if (!kForward) dst[(size_t)(c0 + c) * ldd + out] = s;
   }
@@ -373,22 +412,24 @@ __global__ __launch_bounds__(256) void KLdltWide(int row0, int row1, int wideBeg
   const int i = w - T.begin, m = T.rows;
   const int c0 = blockIdx.y * KC, kc = min(KC, K - c0);
   const double* row = P.mat + T.mat[kForward ? 0 : 1];
+  const float* low = P.low + T.mat[kForward ? 0 : 1];
   const double* in = buf + (size_t)c0 * nWide + T.begin - wideBegin;
   const double dinv = P.dinv[w];
   const int out = kForward ? 0 : P.index[w];
-  double acc[KC] = {};
+  Sum2 acc[KC] = {};
   const int j1 = kForward ? i + 1 : m;
 #pragma unroll 4
   for (int j = (kForward ? 0 : i / 2 * 2) + 2 * lane; j < j1; j += 2 * kWave) {  // backward: entries before i are zero
     double a0, a1;
     LoadPair(row + j, a0, a1);
+    const float l0 = low[j], l1 = low[j + 1];
     const bool both = j + 1 < m;  // (a row of odd length is padded with a zero; the vector is not)
 #pragma unroll
     for (int c = 0; c < KC; c++) {
       double v0, v1;
       LoadPair(in + (size_t)min(c, kc - 1) * nWide + j, v0, v1);
-      acc[c] += a0 * v0;
-      if (both) acc[c] += a1 * v1;
+      acc[c].AddProduct(a0, l0, v0);
+      if (both) acc[c].AddProduct(a1, l1, v1);
     }
   }
 #pragma unroll
@@ -823,6 +864,7 @@ void UploadLdlt(std::vector<void*>& ds, const Ldlt& F, DevLdlt& d, int kcap, con
   d.bwdPtr = UploadTo(ds, S.bwdPtr), d.bwdCol = UploadTo(ds, S.bwdCol), d.bwdVal = UploadTo(ds, S.bwdVal);
   d.fwdMatPtr = UploadTo(ds, S.fwdMatPtr), d.bwdMatPtr = UploadTo(ds, S.bwdMatPtr);
   d.fwdMat = UploadTo(ds, S.fwdMat), d.bwdMat = UploadTo(ds, S.bwdMat);
+  d.fwdLow = UploadTo(ds, S.fwdLow), d.bwdLow = UploadTo(ds, S.bwdLow);
   std::vector<LdltWideRow> wide(S.n - S.wideBegin);
   for (size_t c = 0; c + 1 < S.compPtr.size(); c++)
     for (int w = std::max(S.compPtr[c], S.wideBegin); w < S.compPtr[c + 1]; w++) {
@@ -928,8 +970,8 @@ static void LdltSolveChunks(DevLdlt& F, const double* src, int lds, double* dst,
   const unsigned chunks = (unsigned)((K + KC - 1) / KC);
   double *buf = F.wideBuf, *top = F.wideBuf + (size_t)F.kcap * nWide;
   auto wideGrid = [&](const LdltStage& T) { return dim3(Blocks(T.rowEnd - T.rowBegin, 256 / kWave), chunks); };
-  const LdltPass fwd{F.compPtr, F.fwdMatPtr, F.fwdMat, F.fwdPtr, F.fwdCol, F.fwdVal, index, F.dinv, F.rhsPtr, F.rhsCol, F.rhsVal, rhsX};
-  const LdltPass bwd{F.compPtr, F.bwdMatPtr, F.bwdMat, F.bwdPtr, F.bwdCol, F.bwdVal, index, F.dinv, nullptr, nullptr, nullptr, nullptr};
+  const LdltPass fwd{F.compPtr, F.fwdMatPtr, F.fwdMat, F.fwdLow, F.fwdPtr, F.fwdCol, F.fwdVal, index, F.dinv, F.rhsPtr, F.rhsCol, F.rhsVal, rhsX};
+  const LdltPass bwd{F.compPtr, F.bwdMatPtr, F.bwdMat, F.bwdLow, F.bwdPtr, F.bwdCol, F.bwdVal, index, F.dinv, nullptr, nullptr, nullptr, nullptr};
   for (int k = 0; k <= last; k++) {
     const LdltStage& T = F.stages[k];
     if (T.rowBegin == T.rowEnd) continue;

@@ -1,8 +1,10 @@
 #include "gdtp_ldlt.h"
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <functional>
+#include <limits>
 
 namespace gdtp {
 
@@ -233,11 +235,19 @@ void BuildLdltStages(const Ldlt& F, LdltStages& S, int topRows) {
   for (int w = 0; w < n; w++) S.perm[w] = F.perm[rowOf[w]], S.dinv[w] = 1.0 / F.D[rowOf[w]];
   auto couplings = [&](const Csr& L, std::vector<int>& ptr, std::vector<int>& col, std::vector<double>& val) {
     ptr.assign(n + 1, 0);
+#pragma omp parallel for schedule(static)
     for (int w = 0; w < n; w++) {
       const int i = rowOf[w];
+      for (int k = L.rowptr[i]; k < L.rowptr[i + 1]; k++) ptr[w + 1] += comp[L.col[k]] != comp[i];
+    }
+    for (int w = 0; w < n; w++) ptr[w + 1] += ptr[w];
+    col.resize(ptr[n]), val.resize(ptr[n]);
+#pragma omp parallel for schedule(static)
+    for (int w = 0; w < n; w++) {
+      const int i = rowOf[w];
+      int p = ptr[w];
       for (int k = L.rowptr[i]; k < L.rowptr[i + 1]; k++)
-        if (comp[L.col[k]] != comp[i]) col.push_back(at[L.col[k]]), val.push_back(L.val[k]);
-      ptr[w + 1] = (int)col.size();
+        if (comp[L.col[k]] != comp[i]) col[p] = at[L.col[k]], val[p] = L.val[k], p++;
     }
   };
   couplings(F.Lrows, S.fwdPtr, S.fwdCol, S.fwdVal);
@@ -259,57 +269,93 @@ void BuildLdltStages(const Ldlt& F, LdltStages& S, int topRows) {
     S.fwdMatPtr[c + 1] = S.fwdMatPtr[c] + f, S.bwdMatPtr[c + 1] = S.bwdMatPtr[c] + b;
   }
   S.fwdMat.assign(S.fwdMatPtr[nComp], 0.0), S.bwdMat.assign(S.bwdMatPtr[nComp], 0.0);
-  // inv: row-major m x m, the inverse; its column j by forward substitution from e_j
-  auto column = [&](int m, const std::vector<double>& L, std::vector<double>& inv, int j, std::vector<double>& z) {
-    z[j] = 1.0;
-    inv[(size_t)j * m + j] = 1.0;
-    for (int a = j + 1; a < m; a++) {
-      double v = 0.0;
-      const double* row = &L[(size_t)a * m];
-      for (int b = j; b < a; b++) v -= row[b] * z[b];
-      z[a] = v;
-      inv[(size_t)a * m + j] = v;
-    }
+  S.fwdLow.assign(S.fwdMat.size(), 0.0f), S.bwdLow.assign(S.bwdMat.size(), 0.0f);
+  static_assert(std::numeric_limits<long double>::digits >= 64, "the inverses' low parts come from 64-bit significands");
+  auto split = [](long double v, double& high, float& low) { high = (double)v, low = (float)(v - high); };
+  // a component's block of L by rows without its unit diagonal, and each row's parent in it (or -1)
+  struct Block {
+    std::vector<int> ptr, col, up;
+    std::vector<double> val;
   };
-  auto load = [&](int c, std::vector<double>& L) {
-    const int m = count[c], w0 = S.compPtr[c];
-    L.assign((size_t)m * m, 0.0);
-    for (int a = 0; a < m; a++) {
+  auto load = [&](int c, Block& L) {
+    const int w0 = S.compPtr[c];
+    L.ptr.assign(1, 0), L.col.clear(), L.up.clear(), L.val.clear();
+    for (int a = 0; a < count[c]; a++) {
       const int i = rowOf[w0 + a];
       for (int k = F.Lrows.rowptr[i]; k < F.Lrows.rowptr[i + 1]; k++)
-        if (comp[F.Lrows.col[k]] == comp[i]) L[(size_t)a * m + at[F.Lrows.col[k]] - w0] = F.Lrows.val[k];
+        if (comp[F.Lrows.col[k]] == comp[i]) L.col.push_back(at[F.Lrows.col[k]] - w0), L.val.push_back(F.Lrows.val[k]);
+      L.ptr.push_back((int)L.col.size());
+      L.up.push_back(parent[i] >= 0 && comp[parent[i]] == comp[i] ? at[parent[i]] - w0 : -1);
+    }
+  };
+  // Columns j0 .. j1 - 1 (at most kColumns, each the next one's child) of the block's inverse by forward
+  // substitution from the unit vectors: z[a][j - j0] for row a.  A column's rows are its ancestors.
+  constexpr int kColumns = 4;
+  using Row = std::array<long double, kColumns>;
+  auto group = [](const Block& L, int m, int j0) {
+    int j1 = j0 + 1;
+    while (j1 < m && j1 < j0 + kColumns && L.up[j1 - 1] == j1) j1++;
+    return j1;
+  };
+  auto columns = [](const Block& L, int j0, int j1, std::vector<Row>& z) {
+    std::fill(z.begin(), z.end(), Row{});
+    for (int a = j0; a >= 0; a = L.up[a]) {
+      Row v{};
+      if (a < j1) v[a - j0] = 1.0L;
+      for (int p = L.ptr[a]; p < L.ptr[a + 1]; p++) {
+        const Row& x = z[L.col[p]];
+        for (int q = 0; q < kColumns; q++) v[q] -= L.val[p] * x[q];
+      }
+      z[a] = v;
     }
   };
   const int nNarrow = (int)(std::find(wide.begin(), wide.end(), 1) - wide.begin());
 #pragma omp parallel for schedule(dynamic, 8)
   for (int c = 0; c < nNarrow; c++) {
     const int m = count[c];
-    std::vector<double> L, inv((size_t)m * m, 0.0), z(m);
+    Block L;
+    std::vector<double> high((size_t)m * m, 0.0);
+    std::vector<float> low((size_t)m * m, 0.0f);
+    std::vector<Row> z(m);
     load(c, L);
-    for (int j = 0; j < m; j++) column(m, L, inv, j, z);
-    double *f = S.fwdMat.data() + S.fwdMatPtr[c], *b = S.bwdMat.data() + S.bwdMatPtr[c];
+    for (int j0 = 0, j1; j0 < m; j0 = j1) {  // high, low: the inverse by columns
+      j1 = group(L, m, j0);
+      columns(L, j0, j1, z);
+      for (int a = j0; a >= 0; a = L.up[a])
+        for (int j = j0; j < j1; j++) split(z[a][j - j0], high[(size_t)j * m + a], low[(size_t)j * m + a]);
+    }
+    long f = S.fwdMatPtr[c], b = S.bwdMatPtr[c];
     for (int r0 = 0; r0 < m; r0 += kLdltBlock) {
       const int nr = std::min(kLdltBlock, m - r0);
       for (int j = 0; j < r0 + nr; j++)
-        for (int r = 0; r < nr; r++) *f++ = inv[(size_t)(r0 + r) * m + j];
+        for (int r = 0; r < nr; r++, f++) S.fwdMat[f] = high[(size_t)j * m + r0 + r], S.fwdLow[f] = low[(size_t)j * m + r0 + r];
       for (int j = r0; j < m; j++)
-        for (int r = 0; r < nr; r++) *b++ = inv[(size_t)j * m + r0 + r];
+        for (int r = 0; r < nr; r++, b++) S.bwdMat[b] = high[(size_t)(r0 + r) * m + j], S.bwdLow[b] = low[(size_t)(r0 + r) * m + j];
     }
   }
   for (int c = nNarrow; c < nComp; c++) {  // few and large: in parallel over the columns
     const int m = count[c];
-    std::vector<double> L, inv((size_t)m * m, 0.0);
+    const size_t stride = LdltWideStride(m);
+    Block L;
     load(c, L);
+    double *f = S.fwdMat.data() + S.fwdMatPtr[c], *b = S.bwdMat.data() + S.bwdMatPtr[c];
+    float *fl = S.fwdLow.data() + S.fwdMatPtr[c], *bl = S.bwdLow.data() + S.bwdMatPtr[c];
+    std::vector<int> start;  // first column of each group
+    for (int j = 0; j < m; j = group(L, m, j)) start.push_back(j);
+    start.push_back(m);
 #pragma omp parallel
     {
-      std::vector<double> z(m);
-#pragma omp for schedule(dynamic, 16)
-      for (int j = 0; j < m; j++) column(m, L, inv, j, z);
+      std::vector<Row> z(m);
+#pragma omp for schedule(dynamic, 4)
+      for (int g = 0; g < (int)start.size() - 1; g++) {  // a column is a row of the transposed inverse
+        columns(L, start[g], start[g + 1], z);
+        for (int a = start[g]; a >= 0; a = L.up[a])
+          for (int j = start[g]; j < start[g + 1]; j++) split(z[a][j - start[g]], b[j * stride + a], bl[j * stride + a]);
+      }
+#pragma omp for schedule(static)
+      for (int r = 0; r < m; r++)
+        for (int j = 0; j <= r; j++) f[r * stride + j] = b[j * stride + r], fl[r * stride + j] = bl[j * stride + r];
     }
-    double *f = S.fwdMat.data() + S.fwdMatPtr[c], *b = S.bwdMat.data() + S.bwdMatPtr[c];
-#pragma omp parallel for schedule(static)
-    for (int r = 0; r < m; r++)
-      for (int j = 0; j < m; j++) f[(size_t)r * LdltWideStride(m) + j] = inv[(size_t)r * m + j], b[(size_t)r * LdltWideStride(m) + j] = inv[(size_t)j * m + r];
   }
 }
 

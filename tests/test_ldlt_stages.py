@@ -1,0 +1,93 @@
+"""The staged LDL^T solves on the host: the stages a factor is cut into, and their error against that of
+substitution, each against a solution refined in extended precision.
+
+The staged products carry their rounding errors (two-part inverses, compensated sums), so the staged solve
+rounds less often than substitution does: its error may be at most as large.  As a geometric mean over
+four right-hand sides the ratio of two such errors scatters by some ten percent: below 1.25."""
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import gradientdomaintextureprocessing_amd as g
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "gradientdomaintextureprocessing_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("ldlt") / "ldlt_stages")
+    r = subprocess.run([shutil.which("g++"), "-std=c++17", "-O2", "-fopenmp", "-I" + CSRC, os.path.join(ROOT, "tests", "cpp", "ldlt_stages.cpp"),
+                        os.path.join(CSRC, "gdtp_ldlt.cpp"), "-o", exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    return exe
+
+
+def run(program, path, A, top):
+    A = sp.csr_matrix(A)
+    A.sort_indices()
+    with open(path, "wb") as f:
+        f.write(np.array([A.shape[0], A.nnz], np.int64).tobytes() + A.indptr.astype(np.int32).tobytes() + A.indices.astype(np.int32).tobytes()
+                + A.data.astype(np.float64).tobytes())
+    r = subprocess.run([program, str(path), str(top)], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr
+    lines = [line.split() for line in r.stdout.splitlines()]
+    stages = [tuple(int(v) for v in line[1:]) for line in lines if line[0] == "stage"]
+    residual, error = (float(v) for v in lines[-1][1:])
+    print(f"[ldlt stages] n={A.shape[0]} top={top}: (rows, components, largest, wide) {stages}, residual x{residual:.2f}, error x{error:.2f}")
+    assert sum(s[0] for s in stages) == A.shape[0]
+    assert residual < 1.25 and error < 1.25
+    return stages
+
+
+def grid(w, h, seed):
+    """A weighted nine-point matrix of a w x h grid."""
+    rng = np.random.default_rng(seed)
+    at = np.arange(w * h).reshape(h, w)
+    pairs = [(at[:, :-1], at[:, 1:]), (at[:-1], at[1:]), (at[:-1, :-1], at[1:, 1:]), (at[:-1, 1:], at[1:, :-1])]
+    a, b = (np.concatenate([p[k].ravel() for p in pairs]) for k in (0, 1))
+    v = 10.0 ** rng.uniform(-3, 0, len(a))
+    off = sp.coo_matrix((-v, (a, b)), (w * h, w * h)).tocsr()
+    off = off + off.T
+    return sp.csr_matrix(off - sp.diags(np.asarray(off.sum(axis=1)).ravel() - 10.0 ** rng.uniform(-4, -2, w * h)))
+
+
+def test_top_alone(program, tmp_path):
+    assert run(program, tmp_path / "m", grid(17, 19, 1), 2048) == [(323, 1, 323, 1)]
+    assert run(program, tmp_path / "m", sp.identity(1), 2048) == [(1, 1, 1, 1)]
+
+
+def test_narrow_stages_of_several_blocks(program, tmp_path):
+    stages = run(program, tmp_path / "m", grid(91, 87, 2), 300)
+    assert len(stages) >= 3 and any(not s[3] and 128 < s[2] <= 256 for s in stages)
+
+
+def test_wide_stages_one_after_another(program, tmp_path):
+    stages = run(program, tmp_path / "m", grid(153, 149, 3), 100)
+    assert [s[3] for s in stages].count(1) >= 3 and max(s[2] for s in stages[:-1]) > 256
+
+
+def test_top_of_up_to_twice_the_limit(program, tmp_path):
+    A = sp.block_diag([grid(40, 40, k) for k in range(8)])  # trees of 1600 rows: nothing is left above the next limit
+    stages = run(program, tmp_path / "m", A, 400)
+    assert 400 < stages[-1][0] <= 800
+
+
+def test_forest_without_a_top(program, tmp_path):
+    A = sp.block_diag([grid(9 + k % 5, 11, k) for k in range(120)])  # every tree fits the first stage
+    stages = run(program, tmp_path / "m", A, 50)
+    assert stages[-1][0] == 0 and stages[0][1] == 120
+
+
+@pytest.mark.parametrize("width, height", [(166, 199), (236, 268)])
+def test_sliver_texels(program, tmp_path, width, height):
+    """Boundary matrix of an atlas whose exterior texels have supports down to 1e-12 of the others."""
+    H = g.InitializeHierarchy(g.TexturedMesh.icosphere(4, width, height, 0.05, 1), width, height, 3)
+    n = H.level_info(0)["boundary"]
+    M, K = (sp.csr_matrix((H.array(0, f"{m}.bb.val", np.float64), H.array(0, f"{m}.bb.col"), H.array(0, f"{m}.bb.rowptr")), (n, n))
+            for m in ("mass", "stiffness"))
+    run(program, tmp_path / "m", M + 1e-3 * K, 2048)
