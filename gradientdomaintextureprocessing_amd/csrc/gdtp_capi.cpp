@@ -516,12 +516,29 @@ int gdtp_weighted_residual_norms(gdtp_system* s, const double* x, const double* 
   })
 }
 
+// Device copy of columns for the length of a call.
+struct CopyOfColumns {
+  double* p = nullptr;
+  const double* Take(const double* from, size_t len, hipStream_t st) {
+    GDTP_HIP(hipMalloc(&p, len * sizeof(double)));
+    GDTP_HIP(hipMemcpyAsync(p, from, len * sizeof(double), hipMemcpyDeviceToDevice, st));
+    return p;
+  }
+  ~CopyOfColumns() {
+    if (p) (void)hipFree(p);  // waits for the device
+  }
+};
+
 // Largest level 0 that gdtp_direct_solve factorises (the host factorisation grows as N^1.5).
 static constexpr int kDirectMaxTexels = 1 << 20;
 
 int gdtp_direct_solve(gdtp_system* s, double* x, const double* b, int ncols, double* rel_res, int* method, void* stream) {
   GDTP_DEVICE_OP(x && b, {
     const int N = ds.L[0].N;
+    // b is read again after x is written (norms, V-cycles): a copy where they overlap
+    const size_t len = (size_t)ncols * N;
+    CopyOfColumns own;
+    if (x < b + len && b < x + len) b = own.Take(b, len, st);
     std::vector<double> sq;
     if (N <= kDirectMaxTexels) {
       if (!s->direct) {

@@ -133,8 +133,9 @@ int gdtp_weighted_residual_norms(gdtp_system* s, const double* x, const double* 
  * Geodesics.cpp:259-301).  Up to 2^20 texels: LDL^T of the full level-0 matrix (nested dissection,
  * factorised on the host by the first call after create / update and kept; triangular solves on
  * the GPU).  Larger levels: the FP64 direct-equivalent, reference-schedule V-cycles from x = 0
- * until the relative residual reaches 1e-14 or stops falling (the FP64 floor).  x is overwritten;
- * rel_res (host, ncols) and method (host: 0 factorisation, 1 V-cycles) may be NULL. */
+ * until the relative residual reaches 1e-14 or stops falling (the FP64 floor).  x is overwritten; it
+ * may be b or overlap it (b is then copied).  rel_res (host, ncols) and method (host: 0 factorisation,
+ * 1 V-cycles) may be NULL. */
 int gdtp_direct_solve(gdtp_system* s, double* x, const double* b, int ncols, double* rel_res, int* method, void* stream);
 /* gdtp_residual_norms for callers that cannot allocate device memory (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc): no counterpart in the reference.  Its
