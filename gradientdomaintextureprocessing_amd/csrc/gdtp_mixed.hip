@@ -31,11 +31,6 @@ static constexpr int kDotBlocks = 1024;       // partial sums per column of the 
 static constexpr long kChartSweepMax = 2048;  // largest chart colour plane (texels) swept by one workgroup (two per thread)
 __host__ __device__ static inline unsigned NBlk(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-__device__ __forceinline__ long DenseIdx(const MixChart& c, long plane, int i, int j) {
-  int q = (i & 1) | ((j & 1) << 1);
-  return (long)q * plane + c.base2 + (long)(j >> 1) * c.w2 + (i >> 1);
-}
-
 // Dense vectors are addressed with 32-bit byte offsets (each column is under 2 GiB, checked at
 // upload) from a uniform per-column base held in a buffer resource: one offset register per
 // neighbour serves all columns of a chunk, which keeps the register count low while every load
@@ -1039,7 +1034,7 @@ __global__ __launch_bounds__(64 * W) void KMixSchwarz(const MixBlock* __restrict
 // deep texels from the tile's bit masks, so no load waits on the texel type).
 // (Measured and not kept: the tile's (4 x 64 + 1) x (4 x 4 + 1) fine window staged in LDS one
 // column at a time by row-contiguous loads: 101 instead of 95 us at C2 level 0.)
-// kSplit: one plane per workgroup, as in ResidualDeepTile.
+// kSplit: one plane per workgroup, as in ResidualDeepPlane.
 template <bool kSplit>
 __device__ __forceinline__ void RestrictDeepTile(int vb, int c0, const MixTile* __restrict__ tiles,
                                                  const unsigned long long* __restrict__ cDeepMask, long cplane, long cNd, long fplane, long fNd,
@@ -1213,11 +1208,6 @@ __global__ __launch_bounds__(256) void KMixDenseCoarse(int N, const double* __re
   }
 }
 
-__global__ void KMixZero(long n, float* p) {
-  long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) p[t] = 0.0f;
-}
-
 __global__ void KMixZeroD(int n, double* p) {
   int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t < n) p[t] = 0.0;
@@ -1258,21 +1248,6 @@ __device__ __forceinline__ void BlockAddSquares4(const double (&v)[4], int kc, d
     double s = 0;
     for (int k = 0; k < (int)(blockDim.x / 64); k++) s += part[threadIdx.x][k];
     atomicAdd(target + (long)threadIdx.x * kSlots + (blockIdx.x % kSlots), s);
-  }
-  __syncthreads();
-}
-
-// Block-wide sum of v added to target[blockIdx.x % kSlots]; every thread of the block must call it.
-__device__ __forceinline__ void BlockAddSquares(double v, double* target) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  __shared__ double part[16];
-  const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
-  if (lane == 0) part[w] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double s = 0;
-    for (int k = 0; k < (int)(blockDim.x / 64); k++) s += part[k];
-    atomicAdd(target + (blockIdx.x % kSlots), s);
   }
   __syncthreads();
 }
