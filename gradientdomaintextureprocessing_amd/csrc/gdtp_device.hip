@@ -718,9 +718,9 @@ __global__ void KZeroStrided(int N, double* x, int ld, int K) {
 static thread_local size_t g_uploadBytes = 0;
 size_t UploadByteCounter() { return g_uploadBytes; }
 
-template <class T>
-static T* UploadTo(std::vector<void*>& allocs, const std::vector<T>& v) {
-  if (v.empty()) return nullptr;
+template <class V, class T = std::decay_t<decltype(*std::declval<const V&>().data())>>
+static T* UploadTo(std::vector<void*>& allocs, const V& v) {
+  if (v.size() == 0) return nullptr;
   T* p = nullptr;
   GDTP_HIP(hipMalloc(&p, v.size() * sizeof(T)));
   allocs.push_back(p);

@@ -182,7 +182,7 @@ void BuildLdltStages(const Ldlt& F, LdltStages& S, int topRows) {
     if (parent[i] >= 0) size[parent[i]] += size[i];
   // stage limits: rows whose subtree exceeds the last limit form the top
   std::vector<int> limit;
-  if (n > topRows)
+  if (n > std::min(topRows, kLdltDenseRows))
     for (long s = kLdltLeafRows, last = n;; s *= kLdltStageGrowth) {
       long above = 0;
       for (int i = 0; i < n; i++) above += size[i] > s;
@@ -268,8 +268,8 @@ void BuildLdltStages(const Ldlt& F, LdltStages& S, int topRows) {
       }
     S.fwdMatPtr[c + 1] = S.fwdMatPtr[c] + f, S.bwdMatPtr[c + 1] = S.bwdMatPtr[c] + b;
   }
-  S.fwdMat.assign(S.fwdMatPtr[nComp], 0.0), S.bwdMat.assign(S.bwdMatPtr[nComp], 0.0);
-  S.fwdLow.assign(S.fwdMat.size(), 0.0f), S.bwdLow.assign(S.bwdMat.size(), 0.0f);
+  S.fwdMat.Allocate(S.fwdMatPtr[nComp]), S.bwdMat.Allocate(S.bwdMatPtr[nComp]);
+  S.fwdLow.Allocate(S.fwdMat.size()), S.bwdLow.Allocate(S.bwdMat.size());
   static_assert(std::numeric_limits<long double>::digits >= 64, "the inverses' low parts come from 64-bit significands");
   auto split = [](long double v, double& high, float& low) { high = (double)v, low = (float)(v - high); };
   // a component's block of L by rows without its unit diagonal, and each row's parent in it (or -1)
@@ -289,7 +289,8 @@ void BuildLdltStages(const Ldlt& F, LdltStages& S, int topRows) {
     }
   };
   // Columns j0 .. j1 - 1 (at most kColumns, each the next one's child) of the block's inverse by forward
-  // substitution from the unit vectors: z[a][j - j0] for row a.  A column's rows are its ancestors.
+  // substitution from the unit vectors: z[a][j - j0] for row a.  A column's rows are its ancestors; z is zero
+  // before and elsewhere.
   constexpr int kColumns = 4;
   using Row = std::array<long double, kColumns>;
   auto group = [](const Block& L, int m, int j0) {
@@ -298,11 +299,11 @@ void BuildLdltStages(const Ldlt& F, LdltStages& S, int topRows) {
     return j1;
   };
   auto columns = [](const Block& L, int j0, int j1, std::vector<Row>& z) {
-    std::fill(z.begin(), z.end(), Row{});
     for (int a = j0; a >= 0; a = L.up[a]) {
       Row v{};
       if (a < j1) v[a - j0] = 1.0L;
-      for (int p = L.ptr[a]; p < L.ptr[a + 1]; p++) {
+      const int end = L.ptr[a + 1];  // entries in columns before j0 meet zeros
+      for (int p = (int)(std::lower_bound(L.col.begin() + L.ptr[a], L.col.begin() + end, j0) - L.col.begin()); p < end; p++) {
         const Row& x = z[L.col[p]];
         for (int q = 0; q < kColumns; q++) v[q] -= L.val[p] * x[q];
       }
@@ -316,21 +317,24 @@ void BuildLdltStages(const Ldlt& F, LdltStages& S, int topRows) {
     Block L;
     std::vector<double> high((size_t)m * m, 0.0);
     std::vector<float> low((size_t)m * m, 0.0f);
-    std::vector<Row> z(m);
+    std::vector<Row> z(m, Row{});
     load(c, L);
     for (int j0 = 0, j1; j0 < m; j0 = j1) {  // high, low: the inverse by columns
       j1 = group(L, m, j0);
       columns(L, j0, j1, z);
-      for (int a = j0; a >= 0; a = L.up[a])
+      for (int a = j0; a >= 0; a = L.up[a]) {
         for (int j = j0; j < j1; j++) split(z[a][j - j0], high[(size_t)j * m + a], low[(size_t)j * m + a]);
+        z[a] = Row{};
+      }
     }
-    long f = S.fwdMatPtr[c], b = S.bwdMatPtr[c];
+    double *f = S.fwdMat.data() + S.fwdMatPtr[c], *b = S.bwdMat.data() + S.bwdMatPtr[c];
+    float *fl = S.fwdLow.data() + S.fwdMatPtr[c], *bl = S.bwdLow.data() + S.bwdMatPtr[c];
     for (int r0 = 0; r0 < m; r0 += kLdltBlock) {
       const int nr = std::min(kLdltBlock, m - r0);
       for (int j = 0; j < r0 + nr; j++)
-        for (int r = 0; r < nr; r++, f++) S.fwdMat[f] = high[(size_t)j * m + r0 + r], S.fwdLow[f] = low[(size_t)j * m + r0 + r];
+        for (int r = 0; r < nr; r++) *f++ = high[(size_t)j * m + r0 + r], *fl++ = low[(size_t)j * m + r0 + r];
       for (int j = r0; j < m; j++)
-        for (int r = 0; r < nr; r++, b++) S.bwdMat[b] = high[(size_t)(r0 + r) * m + j], S.bwdLow[b] = low[(size_t)(r0 + r) * m + j];
+        for (int r = 0; r < nr; r++) *b++ = high[(size_t)(r0 + r) * m + j], *bl++ = low[(size_t)(r0 + r) * m + j];
     }
   }
   for (int c = nNarrow; c < nComp; c++) {  // few and large: in parallel over the columns
@@ -345,16 +349,21 @@ void BuildLdltStages(const Ldlt& F, LdltStages& S, int topRows) {
     start.push_back(m);
 #pragma omp parallel
     {
-      std::vector<Row> z(m);
+      std::vector<Row> z(m, Row{});
 #pragma omp for schedule(dynamic, 4)
       for (int g = 0; g < (int)start.size() - 1; g++) {  // a column is a row of the transposed inverse
         columns(L, start[g], start[g + 1], z);
-        for (int a = start[g]; a >= 0; a = L.up[a])
+        std::fill(b + start[g] * stride, b + start[g + 1] * stride, 0.0), std::fill(bl + start[g] * stride, bl + start[g + 1] * stride, 0.0f);
+        for (int a = start[g]; a >= 0; a = L.up[a]) {
           for (int j = start[g]; j < start[g + 1]; j++) split(z[a][j - start[g]], b[j * stride + a], bl[j * stride + a]);
+          z[a] = Row{};
+        }
       }
 #pragma omp for schedule(static)
-      for (int r = 0; r < m; r++)
+      for (int r = 0; r < m; r++) {
         for (int j = 0; j <= r; j++) f[r * stride + j] = b[j * stride + r], fl[r * stride + j] = bl[j * stride + r];
+        std::fill(f + r * stride + r + 1, f + (r + 1) * stride, 0.0), std::fill(fl + r * stride + r + 1, fl + (r + 1) * stride, 0.0f);
+      }
     }
   }
 }

@@ -7,6 +7,7 @@
 // breadth-first-level bisection (A. George, "Nested dissection of a regular finite element mesh",
 // SIAM J. Numer. Anal. 10, 1973).
 #pragma once
+#include <memory>
 #include <string>
 
 #include "gdtp_sparse.h"
@@ -32,6 +33,9 @@ struct Ldlt {
 constexpr int kLdltLeafRows = 128;     // largest subtree of the first stage
 constexpr int kLdltStageGrowth = 8;    // each further stage takes subtrees this many times larger
 constexpr int kLdltTopRows = 2048;     // stages are added until the top has at most this many rows
+// Matrices up to this size are the top alone.  (At 2048 a system of 1536 and 768 boundary rows, a 128^2 cube,
+// took 13 ms to create or to update instead of 7, for dense inverses of 70 MB; its V-cycle 296 us against 292.)
+constexpr int kLdltDenseRows = 512;
 constexpr int kLdltNarrowRows = 256;   // components up to this size are solved by one workgroup
 constexpr int kLdltBlock = 64;         // rows per block of a narrow component's inverse
 
@@ -42,6 +46,17 @@ struct LdltStage {
 };
 
 constexpr int LdltWideStride(int rows) { return (rows + 1) / 2 * 2; }  // even: rows are read in pairs
+
+// Values that the threads filling them touch first (a vector's one thread would clear them before).
+template <class T>
+struct LdltArray {
+  std::unique_ptr<T[]> values;
+  size_t count = 0;
+  void Allocate(size_t n) { values.reset(new T[n]), count = n; }
+  T* data() { return values.get(); }
+  const T* data() const { return values.get(); }
+  size_t size() const { return count; }
+};
 
 struct LdltStages {
   int n = 0;
@@ -55,13 +70,13 @@ struct LdltStages {
   // Inverses, a rounded part and what the rounding left (Low; single precision is enough for it): a product
   // with the rounded inverse alone, summed in double, is not backward stable, and where L's block is badly
   // conditioned (texels with a support of 1e-12 of the others) its error was up to 21 times that of
-  // substitution.  With both parts and a compensated sum it is no larger.  Narrow component: for each block of kLdltBlock rows the columns its rows can reach
-  // (forward: columns before the block's end; backward: from its begin), column-major, the block's
-  // rows contiguous.  Wide component: the whole matrix row-major (backward: transposed), rows of
-  // LdltWideStride doubles.
+  // substitution.  With both parts and a compensated sum it is no larger.
+  // Narrow component: for each block of kLdltBlock rows the columns its rows can reach (forward: columns
+  // before the block's end; backward: from its begin), column-major, the block's rows contiguous.  Wide
+  // component: the whole matrix row-major (backward: transposed), rows of LdltWideStride values.
   std::vector<long> fwdMatPtr, bwdMatPtr;  // per component
-  std::vector<double> fwdMat, bwdMat;
-  std::vector<float> fwdLow, bwdLow;
+  LdltArray<double> fwdMat, bwdMat;
+  LdltArray<float> fwdLow, bwdLow;
   int wideBegin = 0;                   // first row of the first wide stage (the later stages are all wide)
 };
 

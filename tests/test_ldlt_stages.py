@@ -61,6 +61,11 @@ def test_top_alone(program, tmp_path):
     assert run(program, tmp_path / "m", sp.identity(1), 2048) == [(1, 1, 1, 1)]
 
 
+def test_small_matrix_is_not_one_dense_top(program, tmp_path):
+    stages = run(program, tmp_path / "m", grid(40, 38, 4), 2048)  # a dense inverse of 1520 rows: 56 MB to build and upload
+    assert len(stages) == 2 and not stages[0][3] and stages[1][0] < 400
+
+
 def test_narrow_stages_of_several_blocks(program, tmp_path):
     stages = run(program, tmp_path / "m", grid(91, 87, 2), 300)
     assert len(stages) >= 3 and any(not s[3] and 128 < s[2] <= 256 for s in stages)
