@@ -214,9 +214,11 @@ __global__ __launch_bounds__(256) void KBandGs(int color, int nTasks, const int*
 // What bounds them: a dependency chain.  The level-scheduled solve they replace walked the elimination
 // tree's 250-450 levels (subtree teams of one workgroup, a barrier per level, one thread per row), each
 // level a round trip to memory: 1.75 ms for the 175,580 boundary rows of a 4096^2 atlas and three
-// columns, 0.25 ms for 3840 rows; the stages take 0.12 and 0.03 ms.  Explicit inverses of components of up to 128 (first stage) or a few
-// hundred rows leave two passes per stage, each a gather and a product with loads that wait for
-// nothing; the inverses are 2-4 times the factor's bytes.
+// columns, 0.25 ms for 3840 rows; the stages take 0.25 and 0.03 ms.  Explicit inverses of components of up
+// to 128 (first stage) or a few hundred rows leave two passes per stage, each a gather and a product with
+// loads that wait for nothing.  Inverses and couplings are 5 to 13 times the bytes of a boundary factor's L by
+// rows and by columns (2048^2 icosphere 183 MB against 34, 1200^2 cube 89 against 7), twice those of a
+// direct solve's (840 k texels: 5.0 GB against 2.4).
 
 // Lanes' sum over groups of G lanes.
 template <int G>
@@ -323,6 +325,9 @@ static constexpr int kEarlyColumns = 13; // loaded ahead: all of them for compon
 // up to KC columns.  A wave owns one row per lane and a share of its block's columns, so the inverse's
 // loads are whole lines that wait for nothing; they go out first and are in flight while the
 // component's right-hand side is gathered into LDS.  The waves' parts are added in a fixed order.
+// What bounds a launch: HBM where components are many (1981 of them, three columns: 55 us forward with rounded
+// inverses, 86 with both parts), else the chain of one workgroup, the FP64 additions of its sums among
+// it (52 components: 10.7 us with three columns a workgroup, 8.4 with one).
 template <bool kForward, bool kRhs, int G, int KC>
 __global__ __launch_bounds__(1024) void KLdltNarrow(int comp0, LdltPass P, const double* src, int lds, double* y, int n, double* dst, int ldd,
                                                     int K) {
@@ -401,7 +406,8 @@ __global__ __launch_bounds__(256) void KLdltCouple(int row0, int row1, int wideB
 // A wide stage's product with its components' inverses, one wave per row and chunk of columns, two
 // entries per lane and load: the forward result to y, or for the top scaled by 1 / D to `top` (the
 // backward product's input); the backward result to y and dst.  (1920 rows, three columns: forward
-// 26 and backward 20 us with one entry per load and the component looked up first, 13 and 8 us so.)
+// 26 and backward 20 us with one entry per load and the component looked up first, 13 and 8 us so; with
+// compensated sums 35 and 33 us with three columns a wave, 20 and 19 with one.)
 template <bool kForward, int KC>
 __global__ __launch_bounds__(256) void KLdltWide(int row0, int row1, int wideBegin, const LdltWideRow* __restrict__ wideRows, LdltPass P,
                                                  const double* __restrict__ buf, int nWide, double* y, int n, double* top, double* dst, int ldd,
@@ -563,9 +569,10 @@ __global__ void KProlongAdd(int nLines, const int* __restrict__ lines, const dou
 // `b` the residual b - A x, in one launch: first the boundary rows (rowBlocks blocks per chunk of KC
 // columns, all of whose loads are in flight together), then a raster line and chunk per workgroup.
 // (A small apply is its launches and round trips: one launch with kRowLanes lanes per row and global
-// columns took 6,936 texels x 3 columns from 14.1 to 4.0 us of kernels (13.3 to 10.1 a call) against a thread per row and column that
-// looked its A_BB columns up, beside the deep rows' own launch.  A large one is bound by memory: a line's
-// chunks and its neighbours in one XCD's L2 (TileOf) took 3.3 M texels x 16 columns from 551 to 473 us.)
+// columns took 6,936 texels x 3 columns from 14.1 to 4.4 us of kernels (13.2 to 9.9 a call) against a thread
+// per row and column that looked its A_BB columns up, beside the deep rows' own launch.  A large one is bound
+// by memory: a line's chunks and its neighbours in one XCD's L2 (TileOf) took 3.3 M texels x 16 columns from
+// 551 to 484 us.)
 template <int KC>
 __global__ __launch_bounds__(kRowThreads) void KApply(int rowBlocks, int nLines, int B, const int* __restrict__ bgi, const int* __restrict__ rp,
                                                       const int* __restrict__ mid, const int* __restrict__ cl, const double* __restrict__ vl, const int* __restrict__ lines,
@@ -961,40 +968,51 @@ void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOpe
   ds.bytes = g_uploadBytes;
 }
 
-// Columns in chunks of KC = min(K, 4); a stage's launches cover all chunks.  index: of each row in src and
-// dst; rhsX (kRhs): src is b, and A_BD rhsX is subtracted from it.
+// Columns in chunks of KC = min(K, 4), or one column per workgroup where a stage has so few workgroups that
+// the chip is not full; a stage's launches cover all chunks.  index: of each row in src and dst; rhsX (kRhs):
+// src is b, and A_BD rhsX is subtracted from it.
+// (V-cycle on a 512^2 cube 570 us with chunks everywhere, 501 so; on the 4096^2 icosphere 5274, 5049; the same bits.)
+static constexpr long kLdltNarrowSplit = 256, kLdltWideSplit = 2048;  // workgroups: one and eight per CU
 template <bool kRhs, int KC>
 static void LdltSolveChunks(DevLdlt& F, const double* src, int lds, double* dst, int ldd, const int* index, const double* rhsX, double* y, int K,
                             hipStream_t s) {
   const int n = F.n, nWide = n - F.wideBegin, last = (int)F.stages.size() - 1;
-  const unsigned chunks = (unsigned)((K + KC - 1) / KC);
   double *buf = F.wideBuf, *top = F.wideBuf + (size_t)F.kcap * nWide;
-  auto wideGrid = [&](const LdltStage& T) { return dim3(Blocks(T.rowEnd - T.rowBegin, 256 / kWave), chunks); };
   const LdltPass fwd{F.compPtr, F.fwdMatPtr, F.fwdMat, F.fwdLow, F.fwdPtr, F.fwdCol, F.fwdVal, index, F.dinv, F.rhsPtr, F.rhsCol, F.rhsVal, rhsX};
   const LdltPass bwd{F.compPtr, F.bwdMatPtr, F.bwdMat, F.bwdLow, F.bwdPtr, F.bwdCol, F.bwdVal, index, F.dinv, nullptr, nullptr, nullptr, nullptr};
+  // launch(columns per workgroup, grid) with the workgroups of one chunk of T
+  auto chunked = [&](const LdltStage& T, auto&& launch) {
+    const unsigned groups = T.wide ? Blocks(T.rowEnd - T.rowBegin, 256 / kWave) : (unsigned)(T.compEnd - T.compBegin);
+    if ((long)groups * K <= (T.wide ? kLdltWideSplit : kLdltNarrowSplit)) launch(std::integral_constant<int, 1>(), dim3(groups, K));
+    else launch(std::integral_constant<int, KC>(), dim3(groups, (K + KC - 1) / KC));
+  };
   for (int k = 0; k <= last; k++) {
     const LdltStage& T = F.stages[k];
     if (T.rowBegin == T.rowEnd) continue;
-    if (!T.wide) {
-      // the first stage has no couplings; the next stages' rows have tens (C2 level 0: 43 on average)
-      const auto kernel = k == 0 ? KLdltNarrow<true, kRhs, 8, KC> : KLdltNarrow<true, kRhs, 16, KC>;
-      kernel<<<dim3(T.compEnd - T.compBegin, chunks), 1024, 0, s>>>(T.compBegin, fwd, src, lds, y, n, nullptr, 0, K);
-      continue;
-    }
-    KLdltCouple<true, kRhs, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, fwd, src, lds, y, n, buf, nWide, K);
-    KLdltWide<true, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.wideRows, fwd, buf, nWide, y, n, k == last ? top : nullptr,
-                                                    nullptr, 0, K);
+    chunked(T, [&](auto columns, dim3 grid) {
+      constexpr int C = decltype(columns)::value;
+      if (!T.wide) {
+        // the first stage has no couplings; the next stages' rows have tens (C2 level 0: 43 on average)
+        const auto kernel = k == 0 ? KLdltNarrow<true, kRhs, 8, C> : KLdltNarrow<true, kRhs, 16, C>;
+        kernel<<<grid, 1024, 0, s>>>(T.compBegin, fwd, src, lds, y, n, nullptr, 0, K);
+        return;
+      }
+      KLdltCouple<true, kRhs, C><<<grid, 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, fwd, src, lds, y, n, buf, nWide, K);
+      KLdltWide<true, C><<<grid, 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.wideRows, fwd, buf, nWide, y, n, k == last ? top : nullptr, nullptr, 0, K);
+    });
   }
   for (int k = last; k >= 0; k--) {
     const LdltStage& T = F.stages[k];
     if (T.rowBegin == T.rowEnd) continue;
-    if (!T.wide) {
-      KLdltNarrow<false, false, 8, KC><<<dim3(T.compEnd - T.compBegin, chunks), 1024, 0, s>>>(T.compBegin, bwd, nullptr, 0, y, n, dst, ldd, K);
-      continue;
-    }
-    if (k < last) KLdltCouple<false, false, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, bwd, nullptr, 0, y, n, buf, nWide, K);
-    KLdltWide<false, KC><<<wideGrid(T), 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.wideRows, bwd, k == last ? top : buf, nWide, y, n, nullptr,
-                                                     dst, ldd, K);
+    chunked(T, [&](auto columns, dim3 grid) {
+      constexpr int C = decltype(columns)::value;
+      if (!T.wide) {
+        KLdltNarrow<false, false, 8, C><<<grid, 1024, 0, s>>>(T.compBegin, bwd, nullptr, 0, y, n, dst, ldd, K);
+        return;
+      }
+      if (k < last) KLdltCouple<false, false, C><<<grid, 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, bwd, nullptr, 0, y, n, buf, nWide, K);
+      KLdltWide<false, C><<<grid, 256, 0, s>>>(T.rowBegin, T.rowEnd, F.wideBegin, F.wideRows, bwd, k == last ? top : buf, nWide, y, n, nullptr, dst, ldd, K);
+    });
   }
 }
 
@@ -1232,7 +1250,7 @@ void ModulatedStiffness(const DevModulation& m, const double* mask, double* out,
 // each block writes one partial per (column, quantity), and a second pass adds the partials of a
 // column in a fixed order, so repeated calls give bitwise identical norms.
 // kPair: column c's operator is w.m[c] M + w.s[c] S (coef, vl: M's; coefS, vlS: S's).  Memory bounds it:
-// both stencils (144 bytes a texel) once per four columns.  (3.3 M texels x 16 columns: 730 us; the two products
+// both stencils (144 bytes a texel) once per four columns.  (3.3 M texels x 16 columns: 710 us; the two products
 // written, combined and summed in passes of their own 3.2 ms.)
 template <int KC>
 struct PairWeights {

@@ -170,9 +170,10 @@ __global__ __launch_bounds__(256) void KMixDeepGs(int q, int nTiles, const MixTi
 // registers (kIt texels per thread and colour), all loaded in one round trip before the first colour; a
 // colour then waits for LDS only.  (A 512^2 cube, three columns, us a launch: 11.7 with e and each
 // colour's operands read through the L2 colour by colour; 3.9 on levels of up to 1024 positions, and 11
-// on the level of 1764, where the one CU's arithmetic bounds a colour.)  A texel
-// whose 3x3 neighbourhood lies inside the chart (every deep texel) loads its stencil, and learns from
-// c4 whether it is deep.  All threads reach every barrier.
+// on the level of 1764, two texels a thread.  That form takes 128 registers and spills 8 of them; vector
+// instructions issue in 32 % of its cycles, and a third of its waves' cycles wait to issue.)  A texel whose
+// 3x3 neighbourhood lies inside the chart (every deep texel) loads its stencil, and learns from c4 whether it
+// is deep.  All threads reach every barrier.
 template <bool kHalf>
 struct ChartOperands {
   typename std::conditional<kHalf, uint4, Stencil9>::type sten;
