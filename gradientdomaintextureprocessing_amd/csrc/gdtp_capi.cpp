@@ -285,6 +285,17 @@ int gdtp_hierarchy_array_i32(const gdtp_hierarchy* h, int level, const char* cna
   else if (name == "tasks.taskSteps") v = L.tasks.taskSteps;
   else if (name == "tasks.lineElem") v = L.tasks.lineElem;
   else if (name == "tasks.elems") v = L.tasks.elems;
+  else if (name == "tasks.bandBlockRow" || name == "tasks.bandRows" || name == "tasks.bandPairs") {
+    BandTables t;
+    try {
+      BuildBandTables(L.tasks, t);
+    } catch (const std::exception& e) {
+      return Fail(GDTP_ERROR_GEOMETRY, e.what());
+    }
+    if (name == "tasks.bandBlockRow") v = t.blockRow;
+    else if (name == "tasks.bandRows") { for (auto& r : t.rows) v.insert(v.end(), {r.base, r.len, r.pair0, r.pairs}); }
+    else { for (auto& p : t.pairs) v.insert(v.end(), {p.texel, p.deep, p.places, p.flags}); }
+  }
   else if (name == "tasks.segments") { for (auto& s : L.tasks.segments) v.insert(v.end(), {s.currentStart, s.currentEnd, s.previousStart, s.nextStart, s.deepStart}); }
   else if (name == "charts") {
     for (auto& c : L.charts)

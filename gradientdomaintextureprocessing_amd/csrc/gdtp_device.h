@@ -48,12 +48,6 @@ struct DevCsr {
   double* val = nullptr;
 };
 
-// One chart row of a band block: the texels its deep rows touch, base .. base + len - 1, and its pairs
-// of neighbouring deep texels.
-struct BandRow {
-  int base, len, pair0, pairs;
-};
-
 struct DevLevel {
   int N = 0, D = 0, B = 0;
   double* coef = nullptr;      // reciprocal (levels < L-1) deep stencil, SoA [10][D]
@@ -69,7 +63,7 @@ struct DevLevel {
   int* taskPtr = nullptr;
   int* blockRow = nullptr;                           // first row of each block in bandRows
   BandRow* bandRows = nullptr;
-  int4* pairs = nullptr;                             // (texel g, deep index, LDS places, 1: starts a segment | 2: g + 1 too)
+  int4* pairs = nullptr;                             // BandPair
   long nPairs = 0;
   int nRaster = 0, nRestr = 0, nProl = 0;
   int *raster = nullptr, *restr = nullptr, *prol = nullptr;  // 5, 5, 6 ints per line

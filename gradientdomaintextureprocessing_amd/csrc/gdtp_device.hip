@@ -3,7 +3,6 @@
 // Vectors are column-major: column c of a level-l vector starts at c*ld.  Deep stencils are
 // stored structure-of-arrays, [10][D], so every stencil slot is a coalesced stream.
 #include <algorithm>
-#include <climits>
 #include <stdexcept>
 
 #include "gdtp_device.h"
@@ -40,7 +39,8 @@ static constexpr int kBandColumns = 3;  // most columns of a band workgroup
 // brings the next rows' stencils into the L2 ahead of the first pass (level 0 865 against 777 then), and
 // nine pass waves of one column each instead of three of three (level 0 1346, level 1 467: the stencil
 // loads of nine waves).  A lane's two neighbouring words as one 16-byte load: level 0 777 to 765.)
-constexpr int kBandRing = 8, kBandRowMax = 136;  // ring rows; texels of a row (132 at most), padded
+constexpr int kBandRing = 8;  // ring rows, of kBandRowMax texels
+static_assert(kBandPairs == kWave, "a pair per lane");
 
 // Wave-wide DPP move of a double; lanes without a source (and rows masked out) get `old`, or with kZero
 // zero (for unmasked moves: no initial value to set up).
@@ -736,45 +736,6 @@ static T* UploadTo(std::vector<void*>& allocs, const V& v) {
   return p;
 }
 
-// The band kernel's tables: for every block the chart rows its deep rows touch (a row without deep
-// texels between two deep ones is a row without pairs), and each row's deep texels in pairs of
-// neighbours (a segment of odd length ends in a pair of one).  Segments of a row are at least one texel
-// apart, so 128 columns hold at most 64 pairs.
-static void BandTables(const BandTasks& T, std::vector<int>& blockRow, std::vector<BandRow>& rows, std::vector<int4>& pairs) {
-  blockRow.assign(1, 0), rows.clear(), pairs.clear();
-  const int nb = (int)T.blockBegin.size();
-  for (int k = 0; k < nb; k++) {
-    const int l0 = T.blockBegin[k], l1 = T.blockDeepEnd[k], y0 = l0 < l1 ? T.lineRow[l0] : 0;
-    const int nr = l0 < l1 ? T.lineRow[l1 - 1] - y0 + 1 : 0;
-    std::vector<int> lo(nr + 2, INT_MAX), hi(nr + 2, -1), line(nr + 2, -1);
-    auto touch = [&](int r, int g) { lo[r] = std::min(lo[r], g - 1), hi[r] = std::max(hi[r], g + 1); };
-    for (int l = l0; l < l1; l++) {
-      const int r = T.lineRow[l] - y0 + 1;
-      if (r < 1 || r > nr || line[r] >= 0) throw std::runtime_error("band block rows out of order");
-      line[r] = l;
-      for (int e = T.lineElem[l]; e < T.lineElem[l + 1]; e++) {
-        const int* E = &T.elems[4 * (size_t)e];
-        touch(r, E[0]), touch(r - 1, E[1]), touch(r + 1, E[2]);
-      }
-    }
-    for (int r = 0; r < nr + 2; r++) {
-      BandRow W{hi[r] < 0 ? 0 : lo[r], hi[r] < 0 ? 0 : hi[r] - lo[r] + 1, (int)pairs.size(), 0};
-      if (line[r] >= 0)
-        for (int e = T.lineElem[line[r]], end = T.lineElem[line[r] + 1]; e < end;) {
-          const int* E = &T.elems[4 * (size_t)e];
-          const bool first = E[3] < 0, two = e + 1 < end && E[7] >= 0;
-          pairs.push_back(make_int4(E[0], first ? -E[3] - 1 : E[3], (E[0] - lo[r]) | (E[1] - 1 - lo[r - 1]) << 8 | (E[2] - 1 - lo[r + 1]) << 16,
-                                    (first ? 1 : 0) | (two ? 2 : 0)));
-          W.pairs++, e += two ? 2 : 1;
-        }
-      // two more texels than a row holds are read (and not used) past a pair of one
-      if (W.len + 2 > kBandRowMax || W.pairs > kWave) throw std::runtime_error("band row wider than its block");
-      rows.push_back(W);
-    }
-    blockRow.push_back((int)rows.size());
-  }
-}
-
 template <class T>
 static T* Upload(DeviceSystem& ds, const std::vector<T>& v) {
   return UploadTo(ds.allocations, v);
@@ -916,12 +877,11 @@ void UploadSystem(const Hierarchy& h, const OperatorHierarchy& oh, const FineOpe
     d.nTasks = (int)H.tasks.taskPtr.size() - 1;
     d.taskPtr = Upload(ds, H.tasks.taskPtr);
     {
-      std::vector<int> blockRow;
-      std::vector<BandRow> rows;
-      std::vector<int4> pairs;
-      BandTables(H.tasks, blockRow, rows, pairs);
-      d.blockRow = Upload(ds, blockRow), d.bandRows = Upload(ds, rows);
-      d.pairs = Upload(ds, pairs), d.nPairs = (long)pairs.size();
+      BandTables t;
+      BuildBandTables(H.tasks, t);
+      d.blockRow = Upload(ds, t.blockRow), d.bandRows = Upload(ds, t.rows);
+      static_assert(sizeof(BandPair) == sizeof(int4), "a pair is loaded as four words");
+      d.pairs = reinterpret_cast<int4*>(Upload(ds, t.pairs)), d.nPairs = (long)t.pairs.size();
     }
     std::vector<int> rl;
     for (auto& x : H.rasterLines) rl.insert(rl.end(), {x.start, x.end, x.prev, x.next, x.coeff});

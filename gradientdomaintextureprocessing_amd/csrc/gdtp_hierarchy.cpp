@@ -8,6 +8,7 @@
 #include <cstring>
 #include <map>
 #include <queue>
+#include <stdexcept>
 
 namespace gdtp {
 
@@ -642,6 +643,42 @@ void BandSchedule(BandTasks& T) {
       steps[t] = std::max(steps[t], s0 + blockSteps(b));
       prev = std::move(cur);
     }
+  }
+}
+
+// Segments of a row are at least one texel apart, so 128 columns hold at most 64 pairs.
+void BuildBandTables(const BandTasks& T, BandTables& t) {
+  t.blockRow.assign(1, 0), t.rows.clear(), t.pairs.clear();
+  const int nb = (int)T.blockBegin.size();
+  for (int k = 0; k < nb; k++) {
+    const int l0 = T.blockBegin[k], l1 = T.blockDeepEnd[k], y0 = l0 < l1 ? T.lineRow[l0] : 0;
+    const int nr = l0 < l1 ? T.lineRow[l1 - 1] - y0 + 1 : 0;
+    std::vector<int> lo(nr + 2, INT32_MAX), hi(nr + 2, -1), line(nr + 2, -1);
+    auto touch = [&](int r, int g) { lo[r] = std::min(lo[r], g - 1), hi[r] = std::max(hi[r], g + 1); };
+    for (int l = l0; l < l1; l++) {
+      const int r = T.lineRow[l] - y0 + 1;
+      if (r < 1 || r > nr || line[r] >= 0) throw std::runtime_error("band block rows out of order");
+      line[r] = l;
+      for (int e = T.lineElem[l]; e < T.lineElem[l + 1]; e++) {
+        const int* E = &T.elems[4 * (size_t)e];
+        touch(r, E[0]), touch(r - 1, E[1]), touch(r + 1, E[2]);
+      }
+    }
+    for (int r = 0; r < nr + 2; r++) {
+      BandRow W{hi[r] < 0 ? 0 : lo[r], hi[r] < 0 ? 0 : hi[r] - lo[r] + 1, (int)t.pairs.size(), 0};
+      if (line[r] >= 0)
+        for (int e = T.lineElem[line[r]], end = T.lineElem[line[r] + 1]; e < end;) {
+          const int* E = &T.elems[4 * (size_t)e];
+          const bool first = E[3] < 0, two = e + 1 < end && E[7] >= 0;
+          t.pairs.push_back({E[0], first ? -E[3] - 1 : E[3], (E[0] - lo[r]) | (E[1] - 1 - lo[r - 1]) << 8 | (E[2] - 1 - lo[r + 1]) << 16,
+                             (first ? 1 : 0) | (two ? 2 : 0)});
+          W.pairs++, e += two ? 2 : 1;
+        }
+      // two more texels than a row holds are read (and not used) past a pair of one
+      if (W.len + 2 > kBandRowMax || W.pairs > kBandPairs) throw std::runtime_error("band row wider than its block");
+      t.rows.push_back(W);
+    }
+    t.blockRow.push_back((int)t.rows.size());
   }
 }
 

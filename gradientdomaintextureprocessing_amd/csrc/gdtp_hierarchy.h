@@ -99,6 +99,28 @@ struct BandTasks {
 // whose steps are short, runs them one after another).  Fills lineElem, elems, blockStart, taskSteps.
 void BandSchedule(BandTasks& T);
 
+// The GPU band kernel's tables.  A block's chart rows are those of its deep rows and one row either side (a
+// row without deep texels between two deep ones has no pairs): block b's are [blockRow[b], blockRow[b + 1]).
+constexpr int kBandRowMax = 136;  // texels of a row (132 at most), padded
+constexpr int kBandPairs = 64;    // pairs of a row
+// One chart row: the texels that the block's deep rows touch in it, base .. base + len - 1, and its pairs of
+// neighbouring deep texels (a segment of odd length ends in a pair of one).
+struct BandRow {
+  int base, len, pair0, pairs;
+};
+// A pair's first texel and its deep index; its place in its row, that of the texel above and to the left in the
+// row above, and of the one below and to the left in the row below (a byte each); 1: it starts a
+// segment, 2: there is a second texel.
+struct BandPair {
+  int texel, deep, places, flags;
+};
+struct BandTables {
+  std::vector<int> blockRow;
+  std::vector<BandRow> rows;
+  std::vector<BandPair> pairs;
+};
+void BuildBandTables(const BandTasks& T, BandTables& t);
+
 struct Level {
   std::vector<GridChart> charts;
   int numTexels = 0, numInterior = 0, numDeep = 0, numBoundary = 0, numCells = 0, numBoundaryCells = 0, numInteriorCells = 0;
